@@ -152,10 +152,11 @@ struct FacesShape {
   static_assert(TX <= 64 && TY <= 64, "a boundary face row or column fits one wave");
   static constexpr int LX = TX + 4, LY = TY + 4, LN = LX * LY;
   static constexpr int NS = (LN + kTileThreads - 1) / kTileThreads;  // slots per thread
-  // LDS (floats): two staged planes of the 8 fields, then the hydro fluxes
-  // of the plane's x-faces [5][TY][TX+1] and y-faces [5][TY+1][TX]
-  static constexpr int kPlanes = 2 * 8 * LN;
-  static constexpr int kFx = kPlanes;
+  // LDS (floats): two staged planes of rho, v, p, B_x, B_y; one plane of the
+  // sums of B_z on the lower and upper z-faces; then the hydro fluxes of the
+  // plane's x-faces [5][TY][TX+1] and y-faces [5][TY+1][TX]
+  static constexpr int kSz = 2 * 7 * LN;
+  static constexpr int kFx = kSz + LN;
   static constexpr int kFy = kFx + 5 * TY * (TX + 1);
   // then the global in-plane offset of every staged slot (int), kept in LDS
   // rather than in registers (read once per plane by the slot's own thread)
@@ -170,12 +171,23 @@ struct FacesShape {
 // hydro divergence of its cells.  Per plane p the workgroup computes the
 // x-faces i in [x0, x0+TX] and the y-faces j in [y0, y0+TY] (the upper
 // boundary faces of the tile, i.e. one face column and one face row more
-// than it owns, spread over the first TY+TX threads), keeps their hydro
-// fluxes in LDS and differences them; the z-faces come from the register
-// queue, one plane of faces beyond zend.  Only the tile's own faces write
-// their B fluxes to memory.  Recon is the box's reconstruction (b.recon: 0
-// minbee2, 1 piecewise constant) as a compile-time constant, so that the
-// scheme costs no per-variable selects; faces_tile_any dispatches on it.
+// than it owns, on the lanes of a rotating wave), keeps their hydro fluxes in
+// LDS and differences them, and every thread its cell's lower z-face; one
+// more pass computes the z-faces below plane zend.  Only the tile's own faces
+// write their B fluxes to memory.  Recon is the box's reconstruction
+// (b.recon: 0 minbee2, 1 piecewise constant) as a compile-time constant, so
+// that the scheme costs no per-variable selects; faces_tile_any dispatches on
+// it.
+//
+// Bound by VALU issue in large boxes, by the latency of a march in small
+// ones.  The z stencil needs only the thread's own column, so its planes
+// z0-2, z0-1 and zend+1 are loaded into registers and never staged: a chunk
+// of zc planes takes zc passes, zc + 1 staged planes and one more z-face.
+// Staging them too (zc + 4 passes over zc + 4 planes) took 496 us at 256^3
+// (periodic) against 478, 20.2 against 18.3 at 64^3 and 13.3 against 11.4 at
+// 32^3.  The column of plane zend+1 is loaded after the march: prefetching it
+// during the last pass keeps the staging registers alive across the loop's
+// end, which costs 14 VGPRs (11 spilled at 4 waves per SIMD).
 template <int TX, int TY, int Recon>
 __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, const FluxSet &Fs,
                                            float h, int x0, int y0, int z0, int zend,
@@ -194,6 +206,7 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
   const bool src = b.source == 1;
   const float idx = b.inv_d[0], idy = b.inv_d[1], idz = b.inv_d[2];
 
+  float *const SZ = lds + S::kSz;  // B_z on the lower + upper z-face, plane p
   // global in-plane byte offset of every LDS slot this thread stages (each
   // thread writes and reads only its own slots)
   unsigned *const GXY = reinterpret_cast<unsigned *>(lds + S::kGxy);
@@ -208,34 +221,65 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
   // start of plane p (wrapped) in an array
   auto plane_of = [&](auto *arr, int p) { return arr + (size_t)wrap(p, nz) * plane; };
   float stage[NS][8];
-  auto load_plane = [&](int p) {
+  auto load_plane = [&](int p, float (&dst)[NS][8]) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       if (tid + s * NT < LN) {
         const unsigned g = opaque(GXY[tid + s * NT]);
 #pragma unroll
-        for (int f = 0; f < 8; ++f) stage[s][f] = *at_byte(plane_of(W.f[f], p), g);
+        for (int f = 0; f < 8; ++f) dst[s][f] = *at_byte(plane_of(W.f[f], p), g);
       }
     }
   };
-  auto store_plane = [&](int buf) {
+  // rho, v, p, B_x, B_y of a plane into buffer buf
+  auto store_plane = [&](int buf, const float (&src)[NS][8]) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       const int li = tid + s * NT;
       if (li < LN) {
 #pragma unroll
-        for (int f = 0; f < 8; ++f) lds[(buf * 8 + f) * LN + li] = stage[s][f];
+        for (int f = 0; f < 7; ++f) lds[(buf * 7 + f) * LN + li] = src[s][f];
       }
     }
   };
+  // B_z of the newest staged plane at this thread's slots, and its sum with
+  // the next plane's
+  float bzs[NS];
+  auto store_bzsum = [&](const float (&src)[NS][8]) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      if (tid + s * NT < LN) SZ[tid + s * NT] = bzs[s] + src[s][7];
+      bzs[s] = src[s][7];
+    }
+  };
+  // the thread's own column of plane p, with the upper B_x and B_y faces:
+  // rho, vx, vy, vz, p, B_x, B_y, B_z | B_x(x+1), B_y(y+1)
+  const unsigned ownc = valid ? own : 0u;
+  auto load_column = [&](int p, float (&dst)[NS][8]) {
+    const unsigned ox = valid ? (unsigned)(y * nx + wrap(x + 1, nx)) * 4u : 0u;
+    const unsigned oy = valid ? (unsigned)(wrap(y + 1, ny) * nx + x) * 4u : 0u;
+#pragma unroll
+    for (int f = 0; f < 7; ++f) dst[0][f] = *at_byte(plane_of(W.f[f], p), ownc);
+    dst[1][0] = *at_byte(plane_of(W.f[5], p), ox);
+    dst[1][1] = *at_byte(plane_of(W.f[6], p), oy);
+  };
+  // z-stencil values of a column: rho, vz, vx, vy, p, Bx_avg, By_avg
+  auto column_vars = [&](const float (&cl)[NS][8], float (&q)[7]) {
+    q[0] = cl[0][0];
+    q[1] = cl[0][3];
+    q[2] = cl[0][1];
+    q[3] = cl[0][2];
+    q[4] = cl[0][4];
+    q[5] = 0.5f * (cl[0][5] + cl[1][0]);
+    q[6] = 0.5f * (cl[0][6] + cl[1][1]);
+  };
 
-  // lower x-face of the cell at LDS index c of plane buffer cb (nb: next plane)
-  auto face_x = [&](int cb, int nb, int c) -> Flux7 {
-    const float *R = lds + (cb * 8 + 0) * LN, *VX = lds + (cb * 8 + 1) * LN;
-    const float *VY = lds + (cb * 8 + 2) * LN, *VZ = lds + (cb * 8 + 3) * LN;
-    const float *PR = lds + (cb * 8 + 4) * LN, *BX = lds + (cb * 8 + 5) * LN;
-    const float *BY = lds + (cb * 8 + 6) * LN, *BZ = lds + (cb * 8 + 7) * LN;
-    const float *BZN = lds + (nb * 8 + 7) * LN;
+  // lower x-face of the cell at LDS index c of plane buffer cb
+  auto face_x = [&](int cb, int c) -> Flux7 {
+    const float *R = lds + (cb * 7 + 0) * LN, *VX = lds + (cb * 7 + 1) * LN;
+    const float *VY = lds + (cb * 7 + 2) * LN, *VZ = lds + (cb * 7 + 3) * LN;
+    const float *PR = lds + (cb * 7 + 4) * LN, *BX = lds + (cb * 7 + 5) * LN;
+    const float *BY = lds + (cb * 7 + 6) * LN;
     float L[7], Rr[7];
     const int s0 = c - 2, s1 = c - 1, s2 = c, s3 = c + 1;
     recon(mode, R[s0], R[s1], R[s2], R[s3], L[0], Rr[0]);
@@ -245,8 +289,7 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
     recon(mode, PR[s0], PR[s1], PR[s2], PR[s3], L[4], Rr[4]);
     recon_bsum(mode, BY[s0] + BY[s0 + LX], BY[s1] + BY[s1 + LX], BY[s2] + BY[s2 + LX],
                BY[s3] + BY[s3 + LX], L[5], Rr[5]);
-    recon_bsum(mode, BZ[s0] + BZN[s0], BZ[s1] + BZN[s1], BZ[s2] + BZN[s2], BZ[s3] + BZN[s3],
-               L[6], Rr[6]);
+    recon_bsum(mode, SZ[s0], SZ[s1], SZ[s2], SZ[s3], L[6], Rr[6]);
     if (src) {
       const float mbv = 0.5f * h * accel_x(b, 0.5f * (VY[s1] + VY[s2]));
       L[1] += mbv;
@@ -256,12 +299,11 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
                 L[4], Rr[4], L[5], Rr[5], L[6], Rr[6]);
   };
   // lower y-face of the cell at LDS index c; yrow = the face's array row
-  auto face_y = [&](int cb, int nb, int c, int yrow) -> Flux7 {
-    const float *R = lds + (cb * 8 + 0) * LN, *VX = lds + (cb * 8 + 1) * LN;
-    const float *VY = lds + (cb * 8 + 2) * LN, *VZ = lds + (cb * 8 + 3) * LN;
-    const float *PR = lds + (cb * 8 + 4) * LN, *BX = lds + (cb * 8 + 5) * LN;
-    const float *BY = lds + (cb * 8 + 6) * LN, *BZ = lds + (cb * 8 + 7) * LN;
-    const float *BZN = lds + (nb * 8 + 7) * LN;
+  auto face_y = [&](int cb, int c, int yrow) -> Flux7 {
+    const float *R = lds + (cb * 7 + 0) * LN, *VX = lds + (cb * 7 + 1) * LN;
+    const float *VY = lds + (cb * 7 + 2) * LN, *VZ = lds + (cb * 7 + 3) * LN;
+    const float *PR = lds + (cb * 7 + 4) * LN, *BX = lds + (cb * 7 + 5) * LN;
+    const float *BY = lds + (cb * 7 + 6) * LN;
     float L[7], Rr[7];
     const int s0 = c - 2 * LX, s1 = c - LX, s2 = c, s3 = c + LX;
     recon(mode, R[s0], R[s1], R[s2], R[s3], L[0], Rr[0]);
@@ -269,8 +311,7 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
     recon(mode, VZ[s0], VZ[s1], VZ[s2], VZ[s3], L[2], Rr[2]);
     recon(mode, VX[s0], VX[s1], VX[s2], VX[s3], L[3], Rr[3]);
     recon(mode, PR[s0], PR[s1], PR[s2], PR[s3], L[4], Rr[4]);
-    recon_bsum(mode, BZ[s0] + BZN[s0], BZ[s1] + BZN[s1], BZ[s2] + BZN[s2], BZ[s3] + BZN[s3],
-               L[5], Rr[5]);
+    recon_bsum(mode, SZ[s0], SZ[s1], SZ[s2], SZ[s3], L[5], Rr[5]);
     recon_bsum(mode, BX[s0] + BX[s0 + 1], BX[s1] + BX[s1 + 1], BX[s2] + BX[s2 + 1],
                BX[s3] + BX[s3 + 1], L[6], Rr[6]);
     if (src) {
@@ -286,15 +327,13 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
   // order, as face_y / face_x, so the two give the same bits.  The five
   // hydro variables are reconstructed in the fixed order (rho, vx, vy, vz, p)
   // and the velocities then permuted into (normal, t1, t2); of the
-  // transverse B averages, the one along z (B_z of this and the next plane)
-  // is common to both and the other (B_y along y for an x-face, B_x along x
+  // transverse B averages, the one along z (the sums of B_z) is common to both and the other (B_y along y for an x-face, B_x along x
   // for a y-face) is read through a per-lane pointer.
-  auto face_xy = [&](int cb, int nb, int c, bool isy, int yrow) -> Flux7 {
-    const float *R = lds + (cb * 8 + 0) * LN, *VX = lds + (cb * 8 + 1) * LN;
-    const float *VY = lds + (cb * 8 + 2) * LN, *VZ = lds + (cb * 8 + 3) * LN;
-    const float *PR = lds + (cb * 8 + 4) * LN, *BX = lds + (cb * 8 + 5) * LN;
-    const float *BY = lds + (cb * 8 + 6) * LN, *BZ = lds + (cb * 8 + 7) * LN;
-    const float *BZN = lds + (nb * 8 + 7) * LN;
+  auto face_xy = [&](int cb, int c, bool isy, int yrow) -> Flux7 {
+    const float *R = lds + (cb * 7 + 0) * LN, *VX = lds + (cb * 7 + 1) * LN;
+    const float *VY = lds + (cb * 7 + 2) * LN, *VZ = lds + (cb * 7 + 3) * LN;
+    const float *PR = lds + (cb * 7 + 4) * LN, *BX = lds + (cb * 7 + 5) * LN;
+    const float *BY = lds + (cb * 7 + 6) * LN;
     const float *OA = isy ? BX : BY, *OB = isy ? BX + 1 : BY + LX;
     const int st = isy ? LX : 1;
     const int s0 = c - 2 * st, s1 = c - st, s2 = c, s3 = c + st;
@@ -305,8 +344,7 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
     recon(mode, VZ[s0], VZ[s1], VZ[s2], VZ[s3], lz, rz);
     recon(mode, PR[s0], PR[s1], PR[s2], PR[s3], L[4], Rr[4]);
     recon_bsum(mode, OA[s0] + OB[s0], OA[s1] + OB[s1], OA[s2] + OB[s2], OA[s3] + OB[s3], lo, ro);
-    recon_bsum(mode, BZ[s0] + BZN[s0], BZ[s1] + BZN[s1], BZ[s2] + BZN[s2], BZ[s3] + BZN[s3], lc,
-               rc);
+    recon_bsum(mode, SZ[s0], SZ[s1], SZ[s2], SZ[s3], lc, rc);
     // x-face: (vx, vy, vz), (B_y, B_z); y-face: (vy, vz, vx), (B_z, B_x)
     L[1] = isy ? ly : lx, Rr[1] = isy ? ry : rx;
     L[2] = isy ? lz : ly, Rr[2] = isy ? rz : ry;
@@ -345,28 +383,95 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
 
   // own cell in the LDS tile
   const int c = (ty + 2) * LX + tx + 2;
-  // z-stencil queue: q[s] holds plane p-3+s: rho, vz, vx, vy, p, Bx_avg, By_avg
-  float q[4][7];
-  // limited z-slope of plane p-2 (carried from the previous plane: it is the
-  // left state's slope of this plane's z-face and the right state's of the
-  // previous one)
-  float zs_prev[7] = {};
-  float bz_prev = 0.0f;  // B_z on the lower z-face of plane p-1
-  float bz_cur = 0.0f;
-  // divergence pipeline: x+y part of planes p-1, p-2; z-flux of the lower
-  // face of plane p-2
-  float pxy1[5] = {}, pxy2[5] = {}, fzl[5] = {};
+  // z march: values of plane p, their difference to plane p-1, and the left
+  // state of the z-face below plane p (all three carried from plane to plane)
+  float qc[7], dm[7], Lz[7];
+  float pxy[5] = {}, fzl[5] = {};  // x+y divergence and lower z-flux of plane p-1
+  float bz;                        // B_z on the lower z-face of plane p, own cell
 
-  const int zs = z0 - 2, zlast = zend + 1;
-  load_plane(zs);
-  store_plane(zs & 1);
-  load_plane(zs + 1);
-  store_plane((zs + 1) & 1);
+  // prologue, all loads in flight together: the own column of planes z0-2,
+  // z0-1; planes z0 and z0+1 staged
+  {
+    float c0[NS][8], c1[NS][8], first[NS][8];
+    load_plane(z0, first);
+    load_plane(z0 + 1, stage);
+    load_column(z0 - 2, c0);
+    load_column(z0 - 1, c1);
+    bz = *at_byte(plane_of(W.f[7], z0), ownc);
+    store_plane(z0 & 1, first);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) bzs[s] = first[s][7];
+    store_plane((z0 + 1) & 1, stage);
+    store_bzsum(stage);
+    column_vars(c0, qc);
+    column_vars(c1, Lz);
+#pragma unroll
+    for (int v = 0; v < 7; ++v) dm[v] = Lz[v] - qc[v];
+  }
   __syncthreads();
+  {
+    const float *P0 = lds + (z0 & 1) * 7 * LN;
+    qc[0] = P0[c];
+    qc[1] = P0[3 * LN + c];
+    qc[2] = P0[1 * LN + c];
+    qc[3] = P0[2 * LN + c];
+    qc[4] = P0[4 * LN + c];
+    qc[5] = 0.5f * (P0[5 * LN + c] + P0[5 * LN + c + 1]);
+    qc[6] = 0.5f * (P0[6 * LN + c] + P0[6 * LN + c + LX]);
+#pragma unroll
+    for (int v = 0; v < 7; ++v) {
+      const float d = qc[v] - Lz[v];
+      if (mode != 1) Lz[v] = Lz[v] + 0.5f * minmod_med3(dm[v], d);
+      dm[v] = d;
+    }
+  }
 
-  for (int p = zs; p <= zlast; ++p) {
+  // the z-face below plane p: its left state was formed with plane p-1, the
+  // right state needs qn, the values of plane p+1; completes plane p-1
+  auto face_z = [&](int p, const float (&qn)[7], float (&fzn)[5], bool inner) {
+    const unsigned ownp = opaque(own);
+    float Rr[7], Ln[7];
+#pragma unroll
+    for (int v = 0; v < 7; ++v) {
+      const float d = qn[v] - qc[v];
+      if (mode == 1) {
+        Rr[v] = qc[v];
+        Ln[v] = qc[v];
+      } else {
+        const float sl = minmod_med3(dm[v], d);
+        Rr[v] = qc[v] - 0.5f * sl;
+        Ln[v] = qc[v] + 0.5f * sl;
+      }
+      dm[v] = d;
+      qc[v] = qn[v];
+    }
+    if (valid) {
+      // the z acceleration is zero: the face predictor adds nothing
+      const Flux7 r = hlld(b.gamma, b.inv_gm1, bz, Lz[0], Rr[0], Lz[1], Rr[1], Lz[2], Rr[2],
+                           Lz[3], Rr[3], Lz[4], Rr[4], Lz[5], Rr[5], Lz[6], Rr[6]);
+      fzn[0] = r.rho;
+      fzn[1] = r.mt1;
+      fzn[2] = r.mt2;
+      fzn[3] = r.mn;
+      fzn[4] = r.e;
+      if (inner) {
+        put_nt(at_byte(plane_of(SB.fb[4], p), ownp), r.bt1);  // B_x
+        put_nt(at_byte(plane_of(SB.fb[5], p), ownp), r.bt2);  // B_y
+      }
+      // plane p-1 complete: its lower z-face (fzl) and upper z-face (fzn)
+      if (p > z0) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k)
+          put_nt(at_byte(plane_of(SB.pace[k], p - 1), ownp), pxy[k] + (fzl[k] - fzn[k]) * idz);
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 7; ++v) Lz[v] = Ln[v];
+  };
+
+  for (int p = z0; p < zend; ++p) {
     const int cb = p & 1, nb = (p + 1) & 1;
-    const bool prefetch = (p + 2 <= zlast);
+    const bool staged = p + 2 <= zend;   // plane p+2 is staged during this pass
     const unsigned ownp = opaque(own);
     if constexpr (TX + TY <= 64) {
       // the wave that also evaluates this plane's boundary faces sets the
@@ -376,29 +481,11 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
       else
         __builtin_amdgcn_s_setprio(0);
     }
-    if (prefetch) load_plane(p + 2);
+    if (staged) load_plane(p + 2, stage);
     {
-      const float *P0 = lds + cb * 8 * LN;
-      // push plane p into the z queue
-#pragma unroll
-      for (int s = 0; s < 3; ++s)
-#pragma unroll
-        for (int v = 0; v < 7; ++v) q[s][v] = q[s + 1][v];
-      q[3][0] = P0[c];
-      q[3][1] = P0[3 * LN + c];
-      q[3][2] = P0[1 * LN + c];
-      q[3][3] = P0[2 * LN + c];
-      q[3][4] = P0[4 * LN + c];
-      q[3][5] = 0.5f * (P0[5 * LN + c] + P0[5 * LN + c + 1]);
-      q[3][6] = 0.5f * (P0[6 * LN + c] + P0[6 * LN + c + LX]);
-      bz_prev = bz_cur;
-      bz_cur = P0[7 * LN + c];
-    }
-    const bool xy_plane = p >= z0 && p < zend;
-    if (xy_plane) {
       const int yrow = y < ny ? y : y - ny;  // the face row y == ny is face 0
       if (y < ny && x <= nx) {
-        const Flux7 r = face_x(cb, nb, c);
+        const Flux7 r = face_x(cb, c);
         put_x(ty, tx, r);
         if (valid) {
           put_nt(at_byte(plane_of(SB.fb[0], p), ownp), r.bt1);  // B_y
@@ -406,7 +493,7 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
         }
       }
       if (x < nx && y <= ny) {
-        const Flux7 r = face_y(cb, nb, c, yrow);
+        const Flux7 r = face_y(cb, c, yrow);
         put_y(ty, tx, r);
         if (valid) {
           put_nt(at_byte(plane_of(SB.fb[2], p), ownp), r.bt1);  // B_z
@@ -428,7 +515,7 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
           const int row = isy ? TY : lane - TX, col = isy ? lane : TX;
           const int yy = y0 + row;
           if (isy ? (x0 + lane < nx && yy <= ny) : (yy < ny && x0 + TX <= nx)) {
-            const Flux7 r = face_xy(cb, nb, (row + 2) * LX + col + 2, isy, yy < ny ? yy : yy - ny);
+            const Flux7 r = face_xy(cb, (row + 2) * LX + col + 2, isy, yy < ny ? yy : yy - ny);
             if (isy)
               put_y(TY, lane, r);
             else
@@ -438,50 +525,32 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
       } else {
         if (wave == ((2 * rot) & 3) && lane < TY) {
           const int yy = y0 + lane;
-          if (yy < ny && x0 + TX <= nx) put_x(lane, TX, face_x(cb, nb, (lane + 2) * LX + TX + 2));
+          if (yy < ny && x0 + TX <= nx) put_x(lane, TX, face_x(cb, (lane + 2) * LX + TX + 2));
         } else if (wave == ((2 * rot + 1) & 3) && lane < TX) {
           const int yy = y0 + TY;
           if (x0 + lane < nx && yy <= ny)
-            put_y(TY, lane, face_y(cb, nb, (TY + 2) * LX + lane + 2, yy < ny ? yy : yy - ny));
+            put_y(TY, lane, face_y(cb, (TY + 2) * LX + lane + 2, yy < ny ? yy : yy - ny));
         }
       }
     }
-    // z-face below plane p-1 (one plane beyond the chunk: the upper face of
-    // its last plane)
+    const float bz_nx = *at_byte(plane_of(W.f[7], p + 1), opaque(ownc));
     float fzn[5] = {};
-    // limited slope of plane p-1, minmod(x_{p-1} - x_{p-2}, x_p - x_{p-1})
-    float zs_cur[7];
-#pragma unroll
-    for (int v = 0; v < 7; ++v) zs_cur[v] = minmod_med3(q[2][v] - q[1][v], q[3][v] - q[2][v]);
-    if (valid && p - 1 >= z0 && p - 1 <= zend) {
-      float L[7], Rr[7];
-#pragma unroll
-      for (int v = 0; v < 7; ++v) {
-        if (mode == 1) {
-          L[v] = q[1][v];
-          Rr[v] = q[2][v];
-        } else {
-          L[v] = q[1][v] + 0.5f * zs_prev[v];
-          Rr[v] = q[2][v] - 0.5f * zs_cur[v];
-        }
-      }
-      // the z acceleration is zero: the face predictor adds nothing
-      const Flux7 r = hlld(b.gamma, b.inv_gm1, bz_prev, L[0], Rr[0], L[1], Rr[1], L[2], Rr[2],
-                           L[3], Rr[3], L[4], Rr[4], L[5], Rr[5], L[6], Rr[6]);
-      fzn[0] = r.rho;
-      fzn[1] = r.mt1;
-      fzn[2] = r.mt2;
-      fzn[3] = r.mn;
-      fzn[4] = r.e;
-      if (p - 1 < zend) {
-        put_nt(at_byte(plane_of(SB.fb[4], p - 1), ownp), r.bt1);  // B_x
-        put_nt(at_byte(plane_of(SB.fb[5], p - 1), ownp), r.bt2);  // B_y
-      }
+    {
+      const float *P1 = lds + nb * 7 * LN;
+      float qn[7];
+      qn[0] = P1[c];
+      qn[1] = P1[3 * LN + c];
+      qn[2] = P1[1 * LN + c];
+      qn[3] = P1[2 * LN + c];
+      qn[4] = P1[4 * LN + c];
+      qn[5] = 0.5f * (P1[5 * LN + c] + P1[5 * LN + c + 1]);
+      qn[6] = 0.5f * (P1[6 * LN + c] + P1[6 * LN + c + LX]);
+      face_z(p, qn, fzn, true);
     }
+    bz = bz_nx;
     __syncthreads();
     // x + y divergence of plane p (X, Y order)
-    float pxy[5] = {};
-    if (valid && xy_plane) {
+    if (valid) {
       constexpr int sx = TY * (TX + 1), sy = (TY + 1) * TX;
 #pragma unroll
       for (int k = 0; k < 5; ++k) {
@@ -492,22 +561,20 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
         pxy[k] = sacc;
       }
     }
-    // plane p-2 complete: its lower z-face (fzl) and upper z-face (fzn)
-    if (valid && p - 2 >= z0 && p - 2 < zend) {
 #pragma unroll
-      for (int k = 0; k < 5; ++k)
-        put_nt(at_byte(plane_of(SB.pace[k], p - 2), ownp), pxy2[k] + (fzl[k] - fzn[k]) * idz);
+    for (int k = 0; k < 5; ++k) fzl[k] = fzn[k];
+    if (staged) {  // plane p is no longer needed
+      store_plane(cb, stage);
+      store_bzsum(stage);
     }
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      pxy2[k] = pxy1[k];
-      pxy1[k] = pxy[k];
-      fzl[k] = fzn[k];
-    }
-#pragma unroll
-    for (int v = 0; v < 7; ++v) zs_prev[v] = zs_cur[v];
-    if (prefetch) store_plane(cb);  // plane p is no longer needed
     __syncthreads();
+  }
+  // the z-faces below plane zend, the upper faces of the chunk's last plane
+  {
+    float qn[7], fzn[5];
+    load_column(zend + 1, stage);
+    column_vars(stage, qn);
+    face_z(zend, qn, fzn, false);
   }
 }
 
