@@ -5,7 +5,9 @@
 // W^{n+1}); a step reads W^n, writes W* in stage 1 and W^{n+1} in stage 2,
 // and the roles rotate, so no kernel updates a field that a neighbouring
 // thread still reads.  dt never leaves the device: the CFL minimum is
-// reduced into a StepState record that the stage kernels read.
+// reduced into a step record; the next step's first kernel commits the record
+// and decides the new step in a second one (the two alternate), which that
+// step's later kernels read.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -85,6 +87,15 @@ void derive_box(const nmhd_desc *d, Box &b, nmhd_geometry &g) {
   b.face_off = (d->fixes & NMHD_FIX_FACE_POSITION) ? 0.0f : 0.5f;
 }
 
+float cfl_minimum(const StepRec &r) {
+  unsigned m = 0x7f800000u;  // the candidates are >= 0: their bits order as they do
+  for (int i = 0; i < kCflSlots; ++i)
+    if (r.cfl[i * kCflStride] < m) m = r.cfl[i * kCflStride];
+  float v;
+  std::memcpy(&v, &m, sizeof(v));
+  return v;
+}
+
 }  // namespace nmhd
 
 namespace {
@@ -131,14 +142,17 @@ struct nmhd_ctx {
   int cur = 0;
   float *flux[3][7] = {};
   float *scratch8[8] = {};
-  StepState *st = nullptr;
-  StepState *diag = nullptr;
+  // step records: rec[r] is the last one enqueued, rec[2] the diagnostics'
+  StepRec *rec = nullptr;
+  int r = 0;
+  bool reset = false;       // the next step starts a new run
+  StepRec *host = nullptr;  // pinned, for reading a record back
   double *diag_part = nullptr;  // run diagnostics: per-block partials, result
   double *diag_out = nullptr;
   int path = NMHD_PATH_TILED;
   // tile shapes of the tiled path (fastest measured at 256^3-512^3 on MI355X)
   int ftile = TV_32x8, utile = TV_64x4;
-  bool cfl_valid = false;  // st->cfl_next_bits holds the CFL minimum of the state
+  bool cfl_valid = false;  // rec[r].cfl holds the CFL minimum of the state (ghost cells aside)
   std::string err;
   bool timing = false;
   std::vector<Pending> pending;
@@ -232,76 +246,80 @@ void update_dispatch(nmhd_ctx *c, FieldPtrs Win, const FluxSet &F, FieldPtrs Wb,
     launch_update(c->stream, c->box, Win, F, Wb, Wo, st, hsel, pace_only);
 }
 
-// One iteration of the proceed() loop (INL:1094-1201), enqueued.
-// after_step: the previous step of the same enqueue call left its commit to
-// this step's opening launch; defer_commit: leave this step's commit to the
-// next one (steps enqueued back to back share one bookkeeping launch).
-void enqueue_step(nmhd_ctx *c, float goal, bool after_step = false, bool defer_commit = false) {
+// One iteration of the proceed() loop (INL:1094-1201), enqueued.  The first
+// kernel that follows the CFL minimum opens the step (open_step).
+void enqueue_step(nmhd_ctx *c, float goal) {
   const Box &b = c->box;
   hipStream_t s = c->stream;
   const int A = c->cur;
   const bool tiled = c->path == NMHD_PATH_TILED;
   const bool full_cfl = !(tiled && c->cfl_valid);
   const bool ghosts = b.m[1] > 0 || b.m[2] > 0;
-  // with the carried CFL minimum and no ghost cells to add to it, dt is
-  // decided in the opening launch
-  const bool dt_in_open = !full_cfl && !ghosts;
-  timed(c, S_BEGIN,
-        [&] { launch_open_step(s, c->st, after_step, full_cfl, dt_in_open, goal); });
-  if (b.m[1] > 0) timed(c, S_GHOST_Y, [&] { launch_ghost_y(s, b, fields(c, A), c->st); });
-  if (b.m[2] > 0) timed(c, S_GHOST_Z, [&] { launch_ghost_z(s, b, fields(c, A), c->st); });
+  StepRec *const in = c->rec + c->r, *const out = c->rec + (c->r ^ 1);
+  const bool reset = c->reset;
+  if (full_cfl) timed(c, S_BEGIN, [&] { launch_clear_cfl(s, in, reset); });
+  if (b.m[1] > 0) timed(c, S_GHOST_Y, [&] { launch_ghost_y(s, b, fields(c, A), in, reset); });
+  if (b.m[2] > 0) timed(c, S_GHOST_Z, [&] { launch_ghost_z(s, b, fields(c, A), in, reset); });
   if (full_cfl)
-    timed(c, S_CFL, [&] { launch_cfl(s, b, fields(c, A), goal, c->st); });
+    timed(c, S_CFL, [&] { launch_cfl(s, b, fields(c, A), goal, in, reset); });
   else if (ghosts)
-    timed(c, S_CFL_GHOSTS, [&] { launch_cfl_ghosts(s, b, fields(c, A), c->st); });
-  if (!dt_in_open) timed(c, S_DT, [&] { launch_dt(s, c->st, goal); });
+    timed(c, S_CFL_GHOSTS, [&] { launch_cfl_ghosts(s, b, fields(c, A), in, reset); });
+  const OpenStep open{in, out, goal, reset};
+  if (!tiled) timed(c, S_DT, [&] { launch_open_step(s, open); });
   const FluxSet F = fluxes(c);
   const int slots[3] = {S_FLUX_X, S_FLUX_Y, S_FLUX_Z};
   // one RK stage: fluxes of W[in], update of the conserved base W[base] into W[out]
-  auto stage = [&](int in, int base, int out, int hsel, bool last) {
+  auto stage = [&](int Win, int base, int Wout, int hsel, bool first, bool last) {
     if (tiled) {
-      timed(c, last ? S_FACES2 : S_FACES1,
-            [&] { launch_faces(s, b, fields(c, in), F, c->st, hsel, c->ftile); });
+      const StageStep ss{out, hsel, 0.0f};
+      timed(c, last ? S_FACES2 : S_FACES1, [&] {
+        launch_faces(s, b, fields(c, Win), F, ss, first ? open : OpenStep{}, c->ftile);
+      });
       timed(c, last ? S_UPDATE2 : S_UPDATE1, [&] {
-        launch_update_tiled(s, b, fields(c, in), F, fields(c, base), fields(c, out), c->st, hsel,
-                            false, last, c->utile);
+        launch_update_tiled(s, b, fields(c, Win), F, fields(c, base), fields(c, Wout), ss, false,
+                            last, c->utile);
       });
       return;
     }
     for (int d = 0; d < 3; ++d)
-      timed(c, slots[d], [&] { flux_dispatch(c, d, fields(c, in), F.dir[d], c->st, hsel); });
+      timed(c, slots[d], [&] { flux_dispatch(c, d, fields(c, Win), F.dir[d], &out->s, hsel); });
     timed(c, last ? S_UPDATE2 : S_UPDATE1, [&] {
-      update_dispatch(c, fields(c, in), F, fields(c, base), fields(c, out), c->st, hsel, false);
+      update_dispatch(c, fields(c, Win), F, fields(c, base), fields(c, Wout), &out->s, hsel, false);
     });
   };
   int next;
   if (c->desc.integrator == NMHD_EULER1) {
     next = (A + 1) % 3;
-    stage(A, A, next, H_FULL, true);
+    stage(A, A, next, H_FULL, true, true);
   } else {
     const int B = (A + 1) % 3;
     next = (A + 2) % 3;
-    stage(A, A, B, H_HALF, false);
-    stage(B, A, next, H_FULL, true);
+    stage(A, A, B, H_HALF, true, false);
+    stage(B, A, next, H_FULL, false, true);
   }
   // an inactive step carries the state into the next buffer: on the tiled
   // path the last stage's update kernel does it, the other paths copy
   if (!tiled)
-    timed(c, S_COPY, [&] { launch_copy_state(s, b, fields(c, A), fields(c, next), c->st); });
-  if (!defer_commit) timed(c, S_COMMIT, [&] { launch_commit(s, c->st); });
+    timed(c, S_COPY, [&] { launch_copy_state(s, b, fields(c, A), fields(c, next), &out->s); });
   c->cur = next;
+  c->r ^= 1;
+  c->reset = false;
   c->cfl_valid = tiled;
 }
 
+// The record as the last enqueued step leaves it, committed.
 int read_step_state(nmhd_ctx *c, StepState *h) {
-  HIPCHECK(c, hipMemcpyAsync(h, c->st, sizeof(StepState), hipMemcpyDeviceToHost, c->stream));
+  HIPCHECK(c, hipMemcpyAsync(&c->host->s, &c->rec[c->r].s, sizeof(StepState),
+                             hipMemcpyDeviceToHost, c->stream));
   HIPCHECK(c, hipStreamSynchronize(c->stream));
-  return NMHD_OK;
-}
-
-int write_step_state(nmhd_ctx *c, const StepState *h) {
-  HIPCHECK(c, hipMemcpyAsync(c->st, h, sizeof(StepState), hipMemcpyHostToDevice, c->stream));
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
+  *h = c->host->s;
+  if (h->active) {
+    h->t = h->t_next;
+    h->generation += 1;
+    h->steps_done += 1;
+    h->active = 0;
+  }
+  if (c->reset) h->finished = h->goal_reached = h->steps_done = 0;
   return NMHD_OK;
 }
 
@@ -321,8 +339,8 @@ void free_all(nmhd_ctx *c) {
       if (p) (void)hipFree(p), p = nullptr;
   for (auto &p : c->scratch8)
     if (p) (void)hipFree(p), p = nullptr;
-  if (c->st) (void)hipFree(c->st), c->st = nullptr;
-  if (c->diag) (void)hipFree(c->diag), c->diag = nullptr;
+  if (c->rec) (void)hipFree(c->rec), c->rec = nullptr;
+  if (c->host) (void)hipHostFree(c->host), c->host = nullptr;
   if (c->diag_part) (void)hipFree(c->diag_part), c->diag_part = nullptr;
   if (c->diag_out) (void)hipFree(c->diag_out), c->diag_out = nullptr;
   for (auto &p : c->pending) c->pool.push_back(p.a), c->pool.push_back(p.b);
@@ -364,17 +382,14 @@ int nmhd_create(const nmhd_desc *desc, nmhd_ctx **out) {
   for (auto &row : c->flux)
     for (auto &p : row)
       if (hipMalloc(&p, bytes) != hipSuccess) return bail(NMHD_ENOMEM, "flux allocation failed");
-  if (hipMalloc(&c->st, sizeof(StepState)) != hipSuccess ||
-      hipMalloc(&c->diag, sizeof(StepState)) != hipSuccess)
+  if (hipMalloc(&c->rec, 3 * sizeof(StepRec)) != hipSuccess ||
+      hipHostMalloc(&c->host, sizeof(StepRec)) != hipSuccess)
     return bail(NMHD_ENOMEM, "step record allocation failed");
   for (int k = 0; k < 3; ++k)
     for (int f = 0; f < 8; ++f)
       if (hipMemsetAsync(c->state[k][f], 0, bytes, c->stream) != hipSuccess)
         return bail(NMHD_EHIP, "state clear failed");
-  StepState h;
-  std::memset(&h, 0, sizeof(h));
-  if (hipMemcpyAsync(c->st, &h, sizeof(h), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-      hipMemcpyAsync(c->diag, &h, sizeof(h), hipMemcpyHostToDevice, c->stream) != hipSuccess ||
+  if (hipMemsetAsync(c->rec, 0, 3 * sizeof(StepRec), c->stream) != hipSuccess ||
       hipStreamSynchronize(c->stream) != hipSuccess)
     return bail(NMHD_EHIP, "step record init failed");
   *out = c;
@@ -395,6 +410,20 @@ int nmhd_get_geometry(const nmhd_ctx *ctx, nmhd_geometry *geo) {
   return NMHD_OK;
 }
 
+// Whether all eight pointers are memory of the context's own device, which a
+// kernel may address (another device's may need a staged copy).
+static bool own_device(const nmhd_ctx *c, const float *const p[8]) {
+  for (int f = 0; f < 8; ++f) {
+    hipPointerAttribute_t a;
+    if ((uintptr_t)p[f] % sizeof(float) || hipPointerGetAttributes(&a, p[f]) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    if (a.type != hipMemoryTypeDevice || a.device != c->device) return false;
+  }
+  return true;
+}
+
 static int copy_state(nmhd_ctx *c, const float *const src[8], float *const dst[8], bool in,
                       hipMemcpyKind kind) {
   if (!c) return NMHD_EINVAL;
@@ -403,13 +432,24 @@ static int copy_state(nmhd_ctx *c, const float *const src[8], float *const dst[8
     if (in && !src[f]) return fail(c, NMHD_EINVAL, "null field pointer");
     if (!in && !dst[f]) return fail(c, NMHD_EINVAL, "null field pointer");
   }
-  HIPCHECK(c, hipStreamSynchronize(c->stream));
   if (in) c->cfl_valid = false;
-  for (int f = 0; f < 8; ++f) {
-    if (in)
-      HIPCHECK(c, hipMemcpyAsync(c->state[c->cur][f], src[f], bytes, kind, c->stream));
-    else
-      HIPCHECK(c, hipMemcpyAsync(dst[f], c->state[c->cur][f], bytes, kind, c->stream));
+  if (kind == hipMemcpyDeviceToDevice && own_device(c, in ? src : dst)) {
+    FieldPtrs from = fields(c, c->cur), to = from;
+    for (int f = 0; f < 8; ++f) {
+      if (in)
+        from.f[f] = const_cast<float *>(src[f]);
+      else
+        to.f[f] = dst[f];
+    }
+    launch_copy_fields(c->stream, c->box.ncell, from, to);
+    HIPCHECK(c, hipGetLastError());
+  } else {
+    for (int f = 0; f < 8; ++f) {
+      if (in)
+        HIPCHECK(c, hipMemcpyAsync(c->state[c->cur][f], src[f], bytes, kind, c->stream));
+      else
+        HIPCHECK(c, hipMemcpyAsync(dst[f], c->state[c->cur][f], bytes, kind, c->stream));
+    }
   }
   HIPCHECK(c, hipStreamSynchronize(c->stream));
   return NMHD_OK;
@@ -434,16 +474,11 @@ int nmhd_get_state_device(nmhd_ctx *ctx, float *const f[8]) {
 
 int nmhd_set_time(nmhd_ctx *ctx, double t, int generation) {
   if (!ctx) return NMHD_EINVAL;
-  HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
-  StepState h;
-  std::memset(&h, 0, sizeof(h));
-  h.t = t;
-  h.t_next = t;
-  h.generation = generation;
-  h.cfl_bits = 0x7f800000u;
-  h.cfl_next_bits = 0x7f800000u;
+  launch_set_time(ctx->stream, ctx->rec + ctx->r, t, generation);
+  HIPCHECK(ctx, hipGetLastError());
   ctx->cfl_valid = false;
-  return write_step_state(ctx, &h);
+  ctx->reset = false;
+  return NMHD_OK;
 }
 
 int nmhd_get_time(nmhd_ctx *ctx, double *t, int *generation) {
@@ -465,23 +500,22 @@ int nmhd_relative_displacement(const nmhd_ctx *ctx, double t, float *normalized,
 
 int nmhd_fill_ghosts(nmhd_ctx *c) {
   if (!c) return NMHD_EINVAL;
-  launch_diag_prepare(c->stream, c->diag, c->st, 0.0f);
-  if (c->box.m[1] > 0) launch_ghost_y(c->stream, c->box, fields(c, c->cur), c->diag);
-  if (c->box.m[2] > 0) launch_ghost_z(c->stream, c->box, fields(c, c->cur), c->diag);
+  StepRec *const diag = c->rec + 2;
+  launch_diag_prepare(c->stream, diag, c->rec + c->r, 0.0f);
+  if (c->box.m[1] > 0) launch_ghost_y(c->stream, c->box, fields(c, c->cur), diag, true);
+  if (c->box.m[2] > 0) launch_ghost_z(c->stream, c->box, fields(c, c->cur), diag, true);
   return sync_and_check(c);
 }
 
 int nmhd_cfl_dt(nmhd_ctx *c, float goal_time, float *dt) {
   if (!c || !dt) return NMHD_EINVAL;
-  launch_diag_prepare(c->stream, c->diag, c->st, 0.0f);
-  launch_cfl(c->stream, c->box, fields(c, c->cur), goal_time, c->diag);
-  StepState h;
-  HIPCHECK(c, hipMemcpyAsync(&h, c->diag, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+  StepRec *const diag = c->rec + 2;
+  launch_diag_prepare(c->stream, diag, c->rec + c->r, 0.0f);
+  launch_cfl(c->stream, c->box, fields(c, c->cur), goal_time, diag, true);
+  HIPCHECK(c, hipMemcpyAsync(c->host, diag, sizeof(StepRec), hipMemcpyDeviceToHost, c->stream));
   int r = sync_and_check(c);
   if (r) return r;
-  float v;
-  std::memcpy(&v, &h.cfl_bits, sizeof(v));
-  *dt = v;
+  *dt = cfl_minimum(*c->host);
   return NMHD_OK;
 }
 
@@ -493,16 +527,18 @@ int nmhd_rhs(nmhd_ctx *c, float h, float *const pace[8]) {
       return fail(c, NMHD_ENOMEM, "scratch allocation failed");
   FieldPtrs out;
   for (int f = 0; f < 8; ++f) out.f[f] = c->scratch8[f];
-  launch_diag_prepare(c->stream, c->diag, c->st, h);
+  StepRec *const diag = c->rec + 2;
+  launch_diag_prepare(c->stream, diag, c->rec + c->r, h);
   const FluxSet F = fluxes(c);
   if (c->path == NMHD_PATH_TILED) {
-    launch_faces(c->stream, c->box, fields(c, c->cur), F, c->diag, H_DIAG, c->ftile);
-    launch_update_tiled(c->stream, c->box, fields(c, c->cur), F, fields(c, c->cur), out, c->diag,
-                        H_DIAG, true, false, c->utile);
+    const StageStep ss{diag, H_DIAG, 0.0f};
+    launch_faces(c->stream, c->box, fields(c, c->cur), F, ss, OpenStep{}, c->ftile);
+    launch_update_tiled(c->stream, c->box, fields(c, c->cur), F, fields(c, c->cur), out, ss, true,
+                        false, c->utile);
   } else {
     for (int d = 0; d < 3; ++d)
-      flux_dispatch(c, d, fields(c, c->cur), F.dir[d], c->diag, H_DIAG);
-    update_dispatch(c, fields(c, c->cur), F, fields(c, c->cur), out, c->diag, H_DIAG, true);
+      flux_dispatch(c, d, fields(c, c->cur), F.dir[d], &diag->s, H_DIAG);
+    update_dispatch(c, fields(c, c->cur), F, fields(c, c->cur), out, &diag->s, H_DIAG, true);
   }
   for (int f = 0; f < 8; ++f)
     HIPCHECK(c, hipMemcpyAsync(pace[f], out.f[f], bytes, hipMemcpyDeviceToHost, c->stream));
@@ -511,29 +547,22 @@ int nmhd_rhs(nmhd_ctx *c, float h, float *const pace[8]) {
 
 int nmhd_reset_run(nmhd_ctx *c) {
   if (!c) return NMHD_EINVAL;
-  StepState h;
-  int r = read_step_state(c, &h);
-  if (r) return r;
-  h.finished = 0;
-  h.active = 0;
-  h.goal_reached = 0;
-  h.steps_done = 0;
-  return write_step_state(c, &h);
+  c->reset = true;
+  return NMHD_OK;
 }
 
 int nmhd_enqueue_steps(nmhd_ctx *c, float goal_time, int nsteps) {
   if (!c || nsteps < 0) return NMHD_EINVAL;
-  for (int k = 0; k < nsteps; ++k) enqueue_step(c, goal_time, k > 0, k + 1 < nsteps);
+  for (int k = 0; k < nsteps; ++k) enqueue_step(c, goal_time);
   HIPCHECK(c, hipGetLastError());
   return NMHD_OK;
 }
 
 int nmhd_synchronize(nmhd_ctx *c, int *steps_taken, int *goal_reached) {
   if (!c) return NMHD_EINVAL;
-  int r = sync_and_check(c);
-  if (r) return r;
   StepState h;
-  r = read_step_state(c, &h);
+  int r = read_step_state(c, &h);
+  if (!r) r = sync_and_check(c);
   if (r) return r;
   if (steps_taken) *steps_taken = h.steps_done;
   if (goal_reached) *goal_reached = h.goal_reached;
@@ -545,10 +574,9 @@ int nmhd_step(nmhd_ctx *c, float goal_time, float *dt, int *goal_reached) {
   int r = nmhd_reset_run(c);
   if (r) return r;
   enqueue_step(c, goal_time);
-  r = sync_and_check(c);
-  if (r) return r;
   StepState h;
   r = read_step_state(c, &h);
+  if (!r) r = sync_and_check(c);
   if (r) return r;
   if (dt) *dt = h.dt;
   if (goal_reached) *goal_reached = h.goal_reached;

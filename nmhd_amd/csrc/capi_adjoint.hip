@@ -18,18 +18,17 @@ using namespace nmhd;
 namespace nmhd {
 
 void enqueue_frozen_step(hipStream_t s, const Box &b, int integrator, FieldPtrs Win,
-                         FieldPtrs Wstar, FieldPtrs Wout, const FluxSet &F, StepState *st,
-                         float dt) {
-  launch_adj_set_dt(s, st, dt);
+                         FieldPtrs Wstar, FieldPtrs Wout, const FluxSet &F, float dt) {
+  const StageStep full{nullptr, H_FIXED, dt}, half{nullptr, H_FIXED, dt / 2};
   if (integrator == NMHD_EULER1) {
-    launch_faces(s, b, Win, F, st, H_FULL);
-    launch_update_tiled(s, b, Win, F, Win, Wout, st, H_FULL, false, false);
+    launch_faces(s, b, Win, F, full);
+    launch_update_tiled(s, b, Win, F, Win, Wout, full, false, false);
     return;
   }
-  launch_faces(s, b, Win, F, st, H_HALF);
-  launch_update_tiled(s, b, Win, F, Win, Wstar, st, H_HALF, false, false);
-  launch_faces(s, b, Wstar, F, st, H_FULL);
-  launch_update_tiled(s, b, Wstar, F, Win, Wout, st, H_FULL, false, false);
+  launch_faces(s, b, Win, F, half);
+  launch_update_tiled(s, b, Win, F, Win, Wstar, half, false, false);
+  launch_faces(s, b, Wstar, F, full);
+  launch_update_tiled(s, b, Wstar, F, Win, Wout, full, false, false);
 }
 
 }  // namespace nmhd
@@ -52,7 +51,7 @@ struct nmhd_adj {
   float *flux[21] = {};   // face fluxes of the forward stages
   float *work[kWork] = {};
   float *scratch_out[8] = {};
-  StepState *st = nullptr;
+  StepRec *rec = nullptr;  // of nmhd_adj_cfl_dt
   std::string err;
 };
 
@@ -94,8 +93,7 @@ FluxSet flux_set(nmhd_adj *a) {
 
 // W_out = S(W_in; dt) with the production stage kernels.
 void enqueue_forward(nmhd_adj *a, FieldPtrs Win, FieldPtrs Wstar, FieldPtrs Wout, float dt) {
-  enqueue_frozen_step(a->stream, a->box, a->desc.integrator, Win, Wstar, Wout, flux_set(a), a->st,
-                      dt);
+  enqueue_frozen_step(a->stream, a->box, a->desc.integrator, Win, Wstar, Wout, flux_set(a), dt);
 }
 
 AdjStageArgs stage_args(nmhd_adj *a) {
@@ -119,7 +117,7 @@ void free_adj(nmhd_adj *a) {
     if (p) (void)hipFree(p), p = nullptr;
   for (auto &p : a->work)
     if (p) (void)hipFree(p), p = nullptr;
-  if (a->st) (void)hipFree(a->st), a->st = nullptr;
+  if (a->rec) (void)hipFree(a->rec), a->rec = nullptr;
   if (a->own) (void)hipStreamDestroy(a->own), a->own = nullptr;
 }
 
@@ -171,11 +169,9 @@ int nmhd_adj_create(const nmhd_desc *desc, nmhd_adj **out) {
     if (hipMalloc(&p, bytes) != hipSuccess) return bail(NMHD_ENOMEM, "allocation failed");
   for (auto &p : a->work)
     if (hipMalloc(&p, bytes) != hipSuccess) return bail(NMHD_ENOMEM, "allocation failed");
-  if (hipMalloc(&a->st, sizeof(StepState)) != hipSuccess)
+  if (hipMalloc(&a->rec, sizeof(StepRec)) != hipSuccess)
     return bail(NMHD_ENOMEM, "allocation failed");
-  StepState h;
-  std::memset(&h, 0, sizeof(h));
-  if (hipMemcpy(a->st, &h, sizeof(h), hipMemcpyHostToDevice) != hipSuccess)
+  if (hipMemset(a->rec, 0, sizeof(StepRec)) != hipSuccess)
     return bail(NMHD_EHIP, "step record init failed");
   *out = a;
   return NMHD_OK;
@@ -218,14 +214,12 @@ int nmhd_adj_synchronize(nmhd_adj *a) {
 
 int nmhd_adj_cfl_dt(nmhd_adj *a, const float *const w[8], float goal_time, float *dt) {
   if (!a || !ptrs_ok(w) || !dt) return afail(a, NMHD_EINVAL, "bad argument");
-  StepState h;
-  std::memset(&h, 0, sizeof(h));
-  h.cfl_bits = 0x7f800000u;
-  AHIP(a, hipMemcpyAsync(a->st, &h, sizeof(h), hipMemcpyHostToDevice, a->stream));
-  launch_cfl(a->stream, a->box, to_fields_c(w), goal_time, a->st);
-  AHIP(a, hipMemcpyAsync(&h, a->st, sizeof(h), hipMemcpyDeviceToHost, a->stream));
+  launch_clear_cfl(a->stream, a->rec, true);
+  launch_cfl(a->stream, a->box, to_fields_c(w), goal_time, a->rec, true);
+  StepRec h;
+  AHIP(a, hipMemcpyAsync(&h, a->rec, sizeof(h), hipMemcpyDeviceToHost, a->stream));
   AHIP(a, hipStreamSynchronize(a->stream));
-  std::memcpy(dt, &h.cfl_bits, sizeof(float));
+  *dt = cfl_minimum(h);
   return NMHD_OK;
 }
 

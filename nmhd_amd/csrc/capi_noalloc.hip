@@ -1,14 +1,12 @@
 // capi_noalloc.hip -- nmhd_adj_forward_noalloc: the frozen-dt step of
 // nmhd_adj_forward for callers that cannot allocate device memory (work
 // under HIP graph capture, tight serving loops, harnesses that forbid
-// hipMalloc).  The step's scratch -- the step record, the midpoint stage
-// state W* and the 11 arrays the face kernel hands to the update kernel --
-// lives in one file-scope device array of fixed size instead of buffers
+// hipMalloc).  The step's scratch -- the midpoint stage state W* and the 11
+// arrays the face kernel hands to the update kernel -- lives in one file-scope device array of fixed size instead of buffers
 // allocated by nmhd_adj_create.  Every GPU the library runs on holds its
 // own copy of the array until the process ends.
 //
-// Layout of the array (floats): [0, 64) the step record (StepState, 256 B
-// slot); then 19 arrays of `stride` floats each (ncell rounded up to a
+// Layout of the array (floats): 19 arrays of `stride` floats each (ncell rounded up to a
 // multiple of 64, so that every array starts 256-byte aligned): W* (8),
 // the hydro divergence (5), the six face B fluxes (6).
 #include <hip/hip_runtime.h>
@@ -22,12 +20,10 @@ using namespace nmhd;
 
 namespace {
 constexpr size_t kAlignFloats = 64;   // 256 bytes
-constexpr size_t kRecordFloats = 64;  // step record slot
 constexpr size_t kArrays = 8 + 11;    // W* + the face -> update hand-off
 constexpr size_t kMaxCells = NMHD_NOALLOC_MAX_CELLS;
-constexpr size_t kScratchFloats = kRecordFloats + kArrays * kMaxCells;
+constexpr size_t kScratchFloats = kArrays * kMaxCells;
 static_assert(kMaxCells % kAlignFloats == 0, "array strides stay within the scratch");
-static_assert(sizeof(StepState) <= kRecordFloats * sizeof(float), "record slot too small");
 }  // namespace
 
 // The scratch.  In host code `scratch` names a host-side stand-in, not the
@@ -94,12 +90,11 @@ int nmhd_adj_forward_noalloc(const nmhd_desc *desc, const float *const w_in[8], 
     return nfail(NMHD_EINVAL, "box of " + std::to_string((long long)b.ncell) +
                                   " cells exceeds the no-allocation scratch (at most " +
                                   std::to_string((long long)kMaxCells) + " cells)");
-  float *base = nullptr;
-  const int rc = scratch_on_current_device(&base);
+  float *arr = nullptr;
+  const int rc = scratch_on_current_device(&arr);
   if (rc != NMHD_OK) return rc;
 
   const size_t stride = ((size_t)b.ncell + kAlignFloats - 1) / kAlignFloats * kAlignFloats;
-  float *arr = base + kRecordFloats;
   auto slot = [&](size_t k) { return arr + k * stride; };
   FieldPtrs Win, Wstar, Wout;
   for (int f = 0; f < 8; ++f) {
@@ -118,10 +113,7 @@ int nmhd_adj_forward_noalloc(const nmhd_desc *desc, const float *const w_in[8], 
   F.dir[2].f[5] = slot(17);
   F.dir[2].f[6] = slot(18);
 
-  // the record: dt, h, active are set by the step's first kernel; nothing
-  // else of it is read, so no clearing is needed
-  StepState *st = reinterpret_cast<StepState *>(base);
-  enqueue_frozen_step((hipStream_t)stream, b, desc->integrator, Win, Wstar, Wout, F, st, dt);
+  enqueue_frozen_step((hipStream_t)stream, b, desc->integrator, Win, Wstar, Wout, F, dt);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return nfail(NMHD_EHIP, std::string("launch: ") + hipGetErrorString(e));
   return NMHD_OK;

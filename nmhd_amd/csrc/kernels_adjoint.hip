@@ -406,22 +406,9 @@ __global__ void __launch_bounds__(256) k_adj_bfinish(Box b, const float *lbb0, c
   }
 }
 
-// Step record of a stage with a frozen dt.
-__global__ void k_adj_set_dt(StepState *st, float dt) {
-  st->dt = dt;
-  st->h = dt / 2;
-  st->h_diag = dt;
-  st->active = 1;
-  st->finished = 0;
-}
-
 }  // namespace
 
 // ------------------------------------------------------------- launchers
-
-void launch_adj_set_dt(hipStream_t s, StepState *st, float dt) {
-  hipLaunchKernelGGL(k_adj_set_dt, dim3(1), dim3(1), 0, s, st, dt);
-}
 
 void launch_adj_stage(hipStream_t s, const Box &b, const AdjStageArgs &A) {
   const dim3 g(grid_for(b.ncell)), blk(kBlock);

@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(256) k_batch_cfl(const BatchBox *boxes, float 
     cell_coords(b, a, x, y, z);
     t = fminf(t, cell_cfl(b, W, a, x, y, z));
   }
-  const float m = tiled::wave_min64(t);
+  const float m = wave_min64(t);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -228,7 +228,7 @@ __global__ void __launch_bounds__(256) k_batch_cfl_ghosts(const BatchBox *boxes,
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n1;
        i += (long)gridDim.x * blockDim.x)
     t = fminf(t, ghost_cfl_cell(bb.b, W, 1, i));
-  const float m = tiled::wave_min64(t);
+  const float m = wave_min64(t);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) {

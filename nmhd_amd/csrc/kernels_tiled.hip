@@ -17,24 +17,24 @@ namespace tiled {
 // Recon = b.recon (the launcher picks the instantiation)
 template <int TX, int TY, int Recon>
 __global__ void __launch_bounds__(kTileThreads, (FacesShape<TX, TY>::kWavesPerSimd))
-    k_faces(Box b, FieldPtrs W, FluxSet F,
-                                                        const StepState *st, int hsel, int zc,
-                                                        int gx, int gy) {
-  if (!st->active) return;
+    k_faces(Box b, FieldPtrs W, FluxSet F, StageStep ss, OpenStep open, int zc, int gx, int gy) {
+  float h;
+  if (!stage_begin(ss, open, h)) return;
   __shared__ float lds[FacesShape<TX, TY>::kLds];
   const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
   const int x0 = (lb % gx) * TX, y0 = ((lb / gx) % gy) * TY, z0 = (lb / gx / gy) * zc;
-  faces_tile<TX, TY, Recon>(b, W, F, stage_h(st, hsel), x0, y0, z0, min(z0 + zc, b.n[2]), lds);
+  faces_tile<TX, TY, Recon>(b, W, F, h, x0, y0, z0, min(z0 + zc, b.n[2]), lds);
 }
 
 template <int TX, int TY, bool PaceOnly, bool Cfl>
 __global__ void __launch_bounds__(kTileThreads) k_update_march(Box b, FieldPtrs Win, FluxSet F,
                                                                FieldPtrs Wb, FieldPtrs Wo,
-                                                               StepState *st, int hsel, int zc,
-                                                               int gx, int gy) {
+                                                               StageStep ss, int zc, int gx,
+                                                               int gy) {
   const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
   const int x0 = (lb % gx) * TX, y0 = ((lb / gx) % gy) * TY, z0 = (lb / gx / gy) * zc;
-  if (!st->active) {
+  float h;
+  if (!stage_begin(ss, OpenStep{}, h)) {
     // a step enqueued after the run reached its goal: the last stage's
     // output carries the step's base state through the buffer rotation
     if (Cfl && !PaceOnly) {
@@ -51,9 +51,9 @@ __global__ void __launch_bounds__(kTileThreads) k_update_march(Box b, FieldPtrs 
   __shared__ float lds[UpdateShape<TX, TY>::kLds];
   __shared__ float red[4];
   float cfl_t = 3.0e38f;
-  update_tile<TX, TY, PaceOnly, Cfl>(b, Win, F, Wb, Wo, stage_h(st, hsel), x0, y0, z0,
-                                     min(z0 + zc, b.n[2]), lds, cfl_t);
-  if (Cfl && !PaceOnly) block_min_into(cfl_t, &st->cfl_next_bits, red);
+  update_tile<TX, TY, PaceOnly, Cfl>(b, Win, F, Wb, Wo, h, x0, y0, z0, min(z0 + zc, b.n[2]), lds,
+                                     cfl_t);
+  if (Cfl && !PaceOnly) block_min_into(cfl_t, cfl_slot(ss.rec, blockIdx.x), red);
 }
 
 }  // namespace tiled
@@ -82,56 +82,56 @@ int tiled_zchunk(const Box &b, int tx, int ty, bool faces) {
 namespace {
 
 template <int TX, int TY>
-void faces_as(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const StepState *st,
-              int hsel) {
+void faces_as(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const StageStep &ss,
+              const OpenStep &open) {
   const int zc = tiled_zchunk(b, TX, TY, true);
   const int gx = (b.n[0] + TX - 1) / TX, gy = (b.n[1] + TY - 1) / TY, gz = (b.n[2] + zc - 1) / zc;
   if (b.recon == 1)
     hipLaunchKernelGGL((tiled::k_faces<TX, TY, 1>), dim3(gx * gy * gz), dim3(tiled::kTileThreads),
-                       0, s, b, W, F, st, hsel, zc, gx, gy);
+                       0, s, b, W, F, ss, open, zc, gx, gy);
   else
     hipLaunchKernelGGL((tiled::k_faces<TX, TY, 0>), dim3(gx * gy * gz), dim3(tiled::kTileThreads),
-                       0, s, b, W, F, st, hsel, zc, gx, gy);
+                       0, s, b, W, F, ss, open, zc, gx, gy);
 }
 
 template <int TX, int TY>
 void update_as(hipStream_t s, const Box &b, FieldPtrs Win, const FluxSet &F, FieldPtrs Wbase,
-               FieldPtrs Wout, StepState *st, int hsel, bool pace_only, bool cfl) {
+               FieldPtrs Wout, const StageStep &ss, bool pace_only, bool cfl) {
   const int zc = tiled_zchunk(b, TX, TY, false);
   const int gx = (b.n[0] + TX - 1) / TX, gy = (b.n[1] + TY - 1) / TY, gz = (b.n[2] + zc - 1) / zc;
   const dim3 grid(gx * gy * gz), blk(tiled::kTileThreads);
   if (pace_only)
     hipLaunchKernelGGL((tiled::k_update_march<TX, TY, true, false>), grid, blk, 0, s, b, Win, F,
-                       Wbase, Wout, st, hsel, zc, gx, gy);
+                       Wbase, Wout, ss, zc, gx, gy);
   else if (cfl)
     hipLaunchKernelGGL((tiled::k_update_march<TX, TY, false, true>), grid, blk, 0, s, b, Win, F,
-                       Wbase, Wout, st, hsel, zc, gx, gy);
+                       Wbase, Wout, ss, zc, gx, gy);
   else
     hipLaunchKernelGGL((tiled::k_update_march<TX, TY, false, false>), grid, blk, 0, s, b, Win, F,
-                       Wbase, Wout, st, hsel, zc, gx, gy);
+                       Wbase, Wout, ss, zc, gx, gy);
 }
 
 }  // namespace
 
-void launch_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const StepState *st,
-                  int hsel, int tile) {
+void launch_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const StageStep &ss,
+                  const OpenStep &open, int tile) {
   if (tile == TV_64x4)
-    faces_as<64, 4>(s, b, W, F, st, hsel);
+    faces_as<64, 4>(s, b, W, F, ss, open);
   else if (tile == TV_16x16)
-    faces_as<16, 16>(s, b, W, F, st, hsel);
+    faces_as<16, 16>(s, b, W, F, ss, open);
   else
-    faces_as<32, 8>(s, b, W, F, st, hsel);
+    faces_as<32, 8>(s, b, W, F, ss, open);
 }
 
 void launch_update_tiled(hipStream_t s, const Box &b, FieldPtrs Win, const FluxSet &F,
-                         FieldPtrs Wbase, FieldPtrs Wout, StepState *st, int hsel, bool pace_only,
-                         bool cfl, int tile) {
+                         FieldPtrs Wbase, FieldPtrs Wout, const StageStep &ss, bool pace_only, bool cfl,
+                         int tile) {
   if (tile == TV_64x4)
-    update_as<64, 4>(s, b, Win, F, Wbase, Wout, st, hsel, pace_only, cfl);
+    update_as<64, 4>(s, b, Win, F, Wbase, Wout, ss, pace_only, cfl);
   else if (tile == TV_16x16)
-    update_as<16, 16>(s, b, Win, F, Wbase, Wout, st, hsel, pace_only, cfl);
+    update_as<16, 16>(s, b, Win, F, Wbase, Wout, ss, pace_only, cfl);
   else
-    update_as<32, 8>(s, b, Win, F, Wbase, Wout, st, hsel, pace_only, cfl);
+    update_as<32, 8>(s, b, Win, F, Wbase, Wout, ss, pace_only, cfl);
 }
 
 }  // namespace nmhd

@@ -21,8 +21,41 @@ struct FluxSet {
   FluxOut dir[3];
 };
 
-// Which stage step a stage kernel uses: StepState::h, ::dt or ::h_diag.
-enum HSel { H_HALF = 0, H_FULL = 1, H_DIAG = 2 };
+// Which stage step a stage kernel uses: StepState::h, ::dt or ::h_diag, or
+// one given by value (StageStep::h).
+enum HSel { H_HALF = 0, H_FULL = 1, H_DIAG = 2, H_FIXED = 3 };
+
+// The step record of a context with the CFL minimum of the state the step
+// produces, spread over slots a cache line apart: the atomics of a few
+// hundred workgroups on one word serialise (about 11 ns each, 6 us at 64^3),
+// on 64 lines they do not.
+constexpr int kCflSlots = 64, kCflStride = 32;
+struct alignas(128) StepRec {
+  StepState s;
+  alignas(128) unsigned cfl[kCflSlots * kCflStride];  // float bits, +inf when empty
+};
+__device__ __forceinline__ unsigned *cfl_slot(StepRec *r, int block) {
+  return &r->cfl[(block & (kCflSlots - 1)) * kCflStride];
+}
+
+// The step a stage kernel belongs to: its record, or (H_FIXED) a step of
+// size h that is always taken.
+struct StageStep {
+  StepRec *rec;
+  int hsel;
+  float h;
+};
+
+// The bookkeeping between two steps, done by the first kernel of a step (every
+// wave computes it, one writes it): commit the step in `in`, decide the next
+// one from its CFL minimum, write it to `out`.  reset: `in` ends a run, start
+// a new one.  in == NULL: the kernel opens no step.
+struct OpenStep {
+  const StepRec *in;
+  StepRec *out;
+  float goal;
+  int reset;
+};
 
 constexpr int kBlock = 256;
 
@@ -86,6 +119,38 @@ __device__ __forceinline__ void step_commit(StepState &s) {
   s.active = 0;
 }
 
+// The time of the state that the step in s leaves behind, and whether the
+// run that it belongs to ended there.
+__device__ __forceinline__ double committed_time(const StepState &s) {
+  return s.active ? s.t_next : s.t;
+}
+__device__ __forceinline__ bool run_ended(const StepState &s, int reset) {
+  return s.finished && !reset;
+}
+
+__device__ __forceinline__ float wave_min64(float v) {
+  for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
+  return v;
+}
+
+// OpenStep by a full wave; every wave of the launch gets the step in flight,
+// the wave with `write` set records it.
+__device__ __forceinline__ StepState open_step(const OpenStep &o, bool write) {
+  const int slot = (threadIdx.x & 63) * kCflStride;
+  const unsigned mine = o.in->cfl[slot];
+  StepState s = o.in->s;
+  step_commit(s);
+  if (o.reset) s.finished = s.goal_reached = s.steps_done = 0;
+  const bool ended = s.finished;
+  s.cfl_bits = __float_as_uint(wave_min64(__uint_as_float(mine)));
+  step_dt(s, o.goal);
+  if (write) {
+    o.out->cfl[slot] = ended ? mine : 0x7f800000u;
+    if ((threadIdx.x & 63) == 0) o.out->s = s;
+  }
+  return s;
+}
+
 // CFL time of one cell (cfl_condition_inner, INL:714-720):
 // min_d C*d_d/|v_d + sqrt((gamma p + b2)/rho)|, b2 = sum_d max(B_lo^2, B_hi^2)
 // (|v_d| + sqrt(..) with fix_cfl), without FMA contraction so that every CFL
@@ -141,22 +206,22 @@ constexpr int kTileTX[TV_COUNT] = {64, 32, 16};
 constexpr int kTileTY[TV_COUNT] = {4, 8, 16};
 
 // kernels_common.hip
-void launch_begin_step(hipStream_t s, StepState *st, bool full);
-// commit the previous step (commit_prev), begin the next (full CFL pass or
-// the carried minimum) and, with dt_too, decide its dt, in one launch
-void launch_open_step(hipStream_t s, StepState *st, bool commit_prev, bool full, bool dt_too,
-                      float goal);
-void launch_cfl_ghosts(hipStream_t s, const Box &b, FieldPtrs W, StepState *st);
-void launch_ghost_y(hipStream_t s, const Box &b, FieldPtrs W, const StepState *st);
-void launch_ghost_z(hipStream_t s, const Box &b, FieldPtrs W, const StepState *st);
-void launch_cfl(hipStream_t s, const Box &b, FieldPtrs W, float goal, StepState *st);
-void launch_dt(hipStream_t s, StepState *st, float goal);
-void launch_commit(hipStream_t s, StepState *st);
+// empty the CFL minimum of rec before a full pass (not when the run that rec
+// ends is finished and goes on: its minimum is still wanted)
+void launch_clear_cfl(hipStream_t s, StepRec *rec, bool reset);
+void launch_open_step(hipStream_t s, const OpenStep &open);
+// the ghost fills and CFL passes of the step that follows rec's
+void launch_cfl_ghosts(hipStream_t s, const Box &b, FieldPtrs W, StepRec *rec, bool reset);
+void launch_ghost_y(hipStream_t s, const Box &b, FieldPtrs W, const StepRec *rec, bool reset);
+void launch_ghost_z(hipStream_t s, const Box &b, FieldPtrs W, const StepRec *rec, bool reset);
+void launch_cfl(hipStream_t s, const Box &b, FieldPtrs W, float goal, StepRec *rec, bool reset);
 void launch_copy_state(hipStream_t s, const Box &b, FieldPtrs src, FieldPtrs dst,
                        const StepState *st);
+void launch_copy_fields(hipStream_t s, long ncell, const FieldPtrs &src, const FieldPtrs &dst);
+void launch_set_time(hipStream_t s, StepRec *rec, double t, int generation);
 void launch_hlld_batch(hipStream_t s, long n, float gamma, bool strict, FluxIn in,
                        FluxOut out);
-void launch_diag_prepare(hipStream_t s, StepState *diag, const StepState *st, float h);
+void launch_diag_prepare(hipStream_t s, StepRec *diag, const StepRec *rec, float h);
 
 // kernels_unfused.hip (fast arithmetic) and kernels_strict.hip (reference
 // rounding, bit-exact against the CPU oracle)
@@ -220,16 +285,16 @@ struct AdjStageArgs {
   // (one 32-bit word per face)
   float *gU[5], *lE[3], *lbb[3], *abn[3], *face[45];
 };
-void launch_adj_set_dt(hipStream_t s, StepState *st, float dt);
 void launch_adj_stage(hipStream_t s, const Box &b, const AdjStageArgs &A);
 
 // kernels_tiled.hip
 int tiled_zchunk(const Box &b, int tx, int ty, bool faces);
 // tile: TileVariant of the z-marching tiles
-void launch_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const StepState *st,
-                  int hsel, int tile = TV_32x8);
+// open: the bookkeeping of the step that this launch begins (in == NULL: none)
+void launch_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const StageStep &ss,
+                  const OpenStep &open = {}, int tile = TV_32x8);
 void launch_update_tiled(hipStream_t s, const Box &b, FieldPtrs Win, const FluxSet &F,
-                         FieldPtrs Wbase, FieldPtrs Wout, StepState *st, int hsel, bool pace_only,
+                         FieldPtrs Wbase, FieldPtrs Wout, const StageStep &ss, bool pace_only,
                          bool cfl, int tile = TV_64x4);
 
 }  // namespace nmhd

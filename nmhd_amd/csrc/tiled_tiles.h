@@ -43,6 +43,22 @@ __device__ __forceinline__ float stage_h(const StepState *st, int hsel) {
   return hsel == H_HALF ? st->h : (hsel == H_FULL ? st->dt : st->h_diag);
 }
 
+// The stage step of a launch, opening the step first when it is the step's
+// first kernel; false: the step is not taken.
+__device__ __forceinline__ bool stage_begin(const StageStep &ss, const OpenStep &open, float &h) {
+  if (open.in) {
+    const StepState s = open_step(open, blockIdx.x == 0 && threadIdx.x < 64);
+    h = stage_h(&s, ss.hsel);
+    return s.active;
+  }
+  if (ss.hsel == H_FIXED) {
+    h = ss.h;
+    return true;
+  }
+  h = stage_h(&ss.rec->s, ss.hsel);
+  return ss.rec->s.active;
+}
+
 // true modulo for staging coordinates, which may lie several box lengths
 // outside [0, n) when a tile is wider than a small box
 __device__ __forceinline__ int pmod(int i, int n) {
@@ -101,11 +117,6 @@ __device__ __forceinline__ void recon_bsum(int mode, float s0, float s1, float s
 
 __device__ __forceinline__ float upwind(float s, float f0, float f1) {
   return s > 0.0f ? f0 : (s < 0.0f ? f1 : 0.5f * (f0 + f1));
-}
-
-__device__ __forceinline__ float wave_min64(float v) {
-  for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
-  return v;
 }
 
 // Minimum of v over the 256-thread workgroup, folded into *target (float
@@ -602,6 +613,99 @@ struct UpdateShape {
   static constexpr int kLds = 16 * RN + 10 * EN;
 };
 
+// The two sweeps' members of the twelve edges of a cell, u and v (0: lower,
+// 1: upper) indexing the edge: XY / YX on x-face u and y-face v, XZ / ZX on
+// x-face u and z-face v, YZ / ZY on y-face u and z-face v.
+struct CellEdges {
+  float XY[2][2], YX[2][2], XZ[2][2], ZX[2][2], YZ[2][2], ZY[2][2];
+};
+
+// The update of the cell at address a, row y, plane r: pc the hydro
+// divergence, wb the base rho, v, p, bb its six base face fields (x lower,
+// x upper, y.., z..).  cfl_t is lowered to the CFL time of the new state.
+template <bool PaceOnly, bool Cfl>
+__device__ __forceinline__ void finish_cell(const Box &b, const CellEdges &ce, const float (&pc)[5],
+                                            const float (&wb)[5], const float (&bb)[6], float h,
+                                            int y, int r, int a, const FieldPtrs &Wo,
+                                            float &cfl_t) {
+  const float idx_ = b.inv_d[0], idy_ = b.inv_d[1], idz_ = b.inv_d[2];
+  const int ny = b.n[1], nz = b.n[2];
+  float pbx[2], pby[2], pbz[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    pbx[u] = 0.5f * ((ce.XY[u][1] - ce.XY[u][0]) * idy_ + (ce.XZ[u][1] - ce.XZ[u][0]) * idz_) -
+             0.5f * (ce.YX[u][1] - ce.YX[u][0]) * idy_ - 0.5f * (ce.ZX[u][1] - ce.ZX[u][0]) * idz_;
+    pby[u] = -0.5f * (ce.XY[1][u] - ce.XY[0][u]) * idx_ +
+             0.5f * ((ce.YZ[u][1] - ce.YZ[u][0]) * idz_ + (ce.YX[1][u] - ce.YX[0][u]) * idx_) -
+             0.5f * (ce.ZY[u][1] - ce.ZY[u][0]) * idz_;
+    pbz[u] = -0.5f * (ce.XZ[1][u] - ce.XZ[0][u]) * idx_ - 0.5f * (ce.YZ[1][u] - ce.YZ[0][u]) * idy_ +
+             0.5f * ((ce.ZX[1][u] - ce.ZX[0][u]) * idx_ + (ce.ZY[1][u] - ce.ZY[0][u]) * idy_);
+  }
+  if (PaceOnly) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) put_nt(&Wo.f[k][a], pc[k]);
+    put_nt(&Wo.f[5][a], pbx[0]);
+    put_nt(&Wo.f[6][a], pby[0]);
+    put_nt(&Wo.f[7][a], pbz[0]);
+  } else {
+    const float rho0 = wb[0];
+    const float vx0 = wb[1], vy0 = wb[2], vz0 = wb[3];
+    const float bxl0 = bb[0], bxh0 = bb[1], byl0 = bb[2], byh0 = bb[3];
+    const float bzl0 = bb[4], bzh0 = bb[5];
+    const float e0 = wb[4] * b.inv_gm1 + 0.5f * rho0 * (vx0 * vx0 + vy0 * vy0 + vz0 * vz0) +
+                     0.25f * (bxl0 * bxl0 + bxh0 * bxh0 + byl0 * byl0 + byh0 * byh0 +
+                              bzl0 * bzl0 + bzh0 * bzh0);
+    const float rho = rho0 + h * pc[0];
+    const float mx = rho0 * vx0 + h * pc[1];
+    const float my = rho0 * vy0 + h * pc[2];
+    const float mz = rho0 * vz0 + h * pc[3];
+    const float e = e0 + h * pc[4];
+    const float bxl = bxl0 + h * pbx[0], bxh = bxh0 + h * pbx[1];
+    const float byl = byl0 + h * pby[0], byh = byh0 + h * pby[1];
+    const float bzl = bzl0 + h * pbz[0], bzh = bzh0 + h * pbz[1];
+    const float irho = frcp(rho);
+    float ux = mx * irho, uy = my * irho;
+    const float uz = mz * irho;
+    const float eint = e - 0.5f * (mx * mx + my * my + mz * mz) * irho -
+                       0.25f * (bxl * bxl + bxh * bxh + byl * byl + byh * byh + bzl * bzl +
+                                bzh * bzh);
+    const float pres = eint * b.gm1;
+    if (b.source == 1) {
+      const float ax_ = accel_x(b, uy);
+      const float ay_ = accel_y(b, ux, y);
+      ux += h * ax_;
+      uy += h * ay_;
+    }
+    put_nt(&Wo.f[0][a], rho);
+    put_nt(&Wo.f[1][a], ux);
+    put_nt(&Wo.f[2][a], uy);
+    put_nt(&Wo.f[3][a], uz);
+    put_nt(&Wo.f[4][a], pres);
+    put_nt(&Wo.f[5][a], bxl);
+    put_nt(&Wo.f[6][a], byl);
+    put_nt(&Wo.f[7][a], bzl);
+    if (Cfl) {
+      // CFL time of the new state for cells the next ghost fill leaves
+      // untouched (interior rows/planes); the ghost cells are reduced
+      // after the fill
+      const bool ghost = (y < b.m[1]) || (y >= ny - b.m[1]) ||
+                         (b.m[2] > 0 && (r < b.m[2] || r >= nz - b.m[2] - 1));
+      if (!ghost) {
+        // same rounding as the full CFL pass (no contraction), so an
+        // incrementally reduced dt equals it bit for bit
+#pragma clang fp contract(off)
+        const float b2 = fmaxf(bxl * bxl, bxh * bxh) + fmaxf(byl * byl, byh * byh) +
+                         fmaxf(bzl * bzl, bzh * bzh);
+        const float cs = sqrtf((b.gamma * pres + b2) / rho);
+        const float t = fminf(b.cfl * b.d[0] / cfl_speed(b, ux, cs),
+                              fminf(b.cfl * b.d[1] / cfl_speed(b, uy, cs),
+                                    b.cfl * b.d[2] / cfl_speed(b, uz, cs)));
+        cfl_t = fminf(cfl_t, t);
+      }
+    }
+  }
+}
+
 // The cell update as a z march: a TX x TY column tile plus a one-cell ring
 // is staged in LDS, one plane ahead (prefetched into registers while the
 // current plane is computed), so that each HBM value is fetched once per tile.
@@ -802,8 +906,6 @@ __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, 
   storez(rz);
   __syncthreads();
 
-  const float idx = b.inv_d[0], idy = b.inv_d[1], idz = b.inv_d[2];
-
   for (int r = z0; r < zend; ++r) {
     const bool more = r + 1 < zend;
     if (more) {  // prefetch the data of the next iteration
@@ -828,93 +930,21 @@ __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, 
       const int a = r * plane + own;
       // E at x-face i+u, y-face j+v (plane r); x-face i+u, z-face r+v; y-face
       // j+u, z-face r+v
-      float EXY[2][2], EYX[2][2], EXZ[2][2], EZX[2][2], EYZ[2][2], EZY[2][2];
+      CellEdges ce;
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
-          EXY[u][v] = E[0 * EN + q0 + u + v * EX];
-          EYX[u][v] = E[1 * EN + q0 + u + v * EX];
+          ce.XY[u][v] = E[0 * EN + q0 + u + v * EX];
+          ce.YX[u][v] = E[1 * EN + q0 + u + v * EX];
           const float *F = E + (2 + 4 * ((r + v) & 1)) * EN + q0;
-          EXZ[u][v] = F[u];
-          EZX[u][v] = F[EN + u];
-          EYZ[u][v] = F[2 * EN + u * EX];
-          EZY[u][v] = F[3 * EN + u * EX];
+          ce.XZ[u][v] = F[u];
+          ce.ZX[u][v] = F[EN + u];
+          ce.YZ[u][v] = F[2 * EN + u * EX];
+          ce.ZY[u][v] = F[3 * EN + u * EX];
         }
-      const float idx_ = idx, idy_ = idy, idz_ = idz;
-      float pbx[2], pby[2], pbz[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        pbx[u] = 0.5f * ((EXY[u][1] - EXY[u][0]) * idy_ + (EXZ[u][1] - EXZ[u][0]) * idz_) -
-                 0.5f * (EYX[u][1] - EYX[u][0]) * idy_ - 0.5f * (EZX[u][1] - EZX[u][0]) * idz_;
-        pby[u] = -0.5f * (EXY[1][u] - EXY[0][u]) * idx_ +
-                 0.5f * ((EYZ[u][1] - EYZ[u][0]) * idz_ + (EYX[1][u] - EYX[0][u]) * idx_) -
-                 0.5f * (EZY[u][1] - EZY[u][0]) * idz_;
-        pbz[u] = -0.5f * (EXZ[1][u] - EXZ[0][u]) * idx_ - 0.5f * (EYZ[1][u] - EYZ[0][u]) * idy_ +
-                 0.5f * ((EZX[1][u] - EZX[0][u]) * idx_ + (EZY[1][u] - EZY[0][u]) * idy_);
-      }
-      if (PaceOnly) {
-#pragma unroll
-        for (int k = 0; k < 5; ++k) put_nt(&Wo.f[k][a], pc[k]);
-        put_nt(&Wo.f[5][a], pbx[0]);
-        put_nt(&Wo.f[6][a], pby[0]);
-        put_nt(&Wo.f[7][a], pbz[0]);
-      } else {
-        const float rho0 = wb[0];
-        const float vx0 = wb[1], vy0 = wb[2], vz0 = wb[3];
-        const float bzl0 = bz_lo, bzh0 = bz_hi;
-        const float e0 = wb[4] * b.inv_gm1 + 0.5f * rho0 * (vx0 * vx0 + vy0 * vy0 + vz0 * vz0) +
-                         0.25f * (bxl0 * bxl0 + bxh0 * bxh0 + byl0 * byl0 + byh0 * byh0 +
-                                  bzl0 * bzl0 + bzh0 * bzh0);
-        const float rho = rho0 + h * pc[0];
-        const float mx = rho0 * vx0 + h * pc[1];
-        const float my = rho0 * vy0 + h * pc[2];
-        const float mz = rho0 * vz0 + h * pc[3];
-        const float e = e0 + h * pc[4];
-        const float bxl = bxl0 + h * pbx[0], bxh = bxh0 + h * pbx[1];
-        const float byl = byl0 + h * pby[0], byh = byh0 + h * pby[1];
-        const float bzl = bzl0 + h * pbz[0], bzh = bzh0 + h * pbz[1];
-        const float irho = frcp(rho);
-        float ux = mx * irho, uy = my * irho;
-        const float uz = mz * irho;
-        const float eint = e - 0.5f * (mx * mx + my * my + mz * mz) * irho -
-                           0.25f * (bxl * bxl + bxh * bxh + byl * byl + byh * byh + bzl * bzl +
-                                    bzh * bzh);
-        const float pres = eint * b.gm1;
-        if (b.source == 1) {
-          const float ax_ = accel_x(b, uy);
-          const float ay_ = accel_y(b, ux, y);
-          ux += h * ax_;
-          uy += h * ay_;
-        }
-        put_nt(&Wo.f[0][a], rho);
-        put_nt(&Wo.f[1][a], ux);
-        put_nt(&Wo.f[2][a], uy);
-        put_nt(&Wo.f[3][a], uz);
-        put_nt(&Wo.f[4][a], pres);
-        put_nt(&Wo.f[5][a], bxl);
-        put_nt(&Wo.f[6][a], byl);
-        put_nt(&Wo.f[7][a], bzl);
-        if (Cfl) {
-          // CFL time of the new state for cells the next ghost fill leaves
-          // untouched (interior rows/planes); the ghost cells are reduced
-          // after the fill
-          const bool ghost = (y < b.m[1]) || (y >= ny - b.m[1]) ||
-                             (b.m[2] > 0 && (r < b.m[2] || r >= nz - b.m[2] - 1));
-          if (!ghost) {
-            // same rounding as the full CFL pass (no contraction), so an
-            // incrementally reduced dt equals it bit for bit
-#pragma clang fp contract(off)
-            const float b2 = fmaxf(bxl * bxl, bxh * bxh) + fmaxf(byl * byl, byh * byh) +
-                             fmaxf(bzl * bzl, bzh * bzh);
-            const float cs = sqrtf((b.gamma * pres + b2) / rho);
-            const float t = fminf(b.cfl * b.d[0] / cfl_speed(b, ux, cs),
-                                  fminf(b.cfl * b.d[1] / cfl_speed(b, uy, cs),
-                                        b.cfl * b.d[2] / cfl_speed(b, uz, cs)));
-            cfl_t = fminf(cfl_t, t);
-          }
-        }
-      }
+      const float bb[6] = {bxl0, bxh0, byl0, byh0, bz_lo, bz_hi};
+      finish_cell<PaceOnly, Cfl>(b, ce, pc, wb, bb, h, y, r, a, Wo, cfl_t);
     }
     if (more) {
       // the rings are not read between the barriers

@@ -1,0 +1,99 @@
+"""Step bookkeeping between enqueued steps and device state transfers (GPU).
+
+The first kernel of a step commits the previous one and decides dt; a run
+must not depend on how its steps were enqueued, nor on steps enqueued after
+it reached its goal.
+"""
+import numpy as np
+import pytest
+
+from nmhd_amd import capi, problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+def boxes():
+    shear = P.config_c2((24, 12, 9))
+    ghosts_z = P.make_config((20, 12, 10), margin=(0, 2, 3), cfl=0.4)
+    euler = P.make_config((17, 9, 5), cfl=0.4, recon=1, integrator=1)
+    return [("shear", shear, P.shearing_box_mri(shear)),
+            ("periodic", P.config_c1(16), P.orszag_tang_noisy(P.config_c1(16))),
+            ("ghost_z", ghosts_z, P.orszag_tang_noisy(ghosts_z)),
+            ("euler", euler, P.orszag_tang_noisy(euler))]
+
+
+@pytest.mark.parametrize("path", [capi.PATH_TILED, capi.PATH_STRICT])
+@pytest.mark.parametrize("box", range(4))
+def test_enqueueing_does_not_matter(gpu_ready, box, path):
+    name, cfg, W = boxes()[box]
+    whole, single, split = (capi.Context(cfg, path=path) for _ in range(3))
+    for c in (whole, single, split):
+        c.set_state(W)
+        c.set_time(0.2)
+    k, reached = whole.run(1e30, 7)
+    assert (k, reached) == (7, False)
+    for _ in range(7):
+        single.step()
+    split.reset_run()
+    split.enqueue_steps(1e30, 3)
+    split.enqueue_steps(1e30, 0)
+    split.enqueue_steps(1e30, 4)
+    assert split.synchronize() == (7, False)
+    t, g = whole.get_time()
+    assert g == 7 and single.get_time() == (t, g) and split.get_time() == (t, g)
+    ref = whole.get_state()
+    for c in (single, split):
+        assert np.array_equal(ref.view(np.uint32), c.get_state().view(np.uint32)), name
+    # a goal reached inside an enqueued group: the rest of it (an even or an
+    # odd number of steps) changes nothing, and the next run goes on from there
+    dt, _ = single.step()
+    goal = float(np.float32(single.get_time()[0] + 1.5 * dt))
+    steps = []
+    for c, extra in ((whole, 8), (split, 9)):
+        c.run(1e30, 1)
+        c.reset_run()
+        c.enqueue_steps(goal, extra)
+        k, reached = c.synchronize()
+        assert reached
+        steps.append(k)
+    n = 0
+    while True:
+        n += 1
+        if single.step(goal)[1]:
+            break
+    assert steps == [n, n]
+    for c in (whole, single, split):
+        assert c.get_time()[0] == pytest.approx(goal, abs=1e-12 + abs(goal) * 2 ** -23)
+        assert c.run(1e30, 3) == (3, False)
+    ref = whole.get_state()
+    for c in (single, split):
+        assert whole.get_time() == c.get_time()
+        assert np.array_equal(ref.view(np.uint32), c.get_state().view(np.uint32)), name
+        assert np.isfinite(ref).all()
+    for c in (whole, single, split):
+        c.close()
+
+
+@pytest.mark.parametrize("n", [(1, 1, 1), (3, 1, 1), (5, 3, 1), (17, 9, 7), (64, 32, 16)])
+@pytest.mark.parametrize("offset", [0, 1, 2, 4])
+def test_device_state_transfer(gpu_ready, n, offset):
+    """set_state_device / get_state_device at every alignment of the fields,
+    with nothing written outside them."""
+    import torch
+    ctx = capi.Context(P.make_config(n))
+    nc = ctx.ncell
+    stride = nc + 5
+    src = torch.rand(8 * stride + 8, device="cuda")
+    dst = torch.full_like(src, -1.0)
+    torch.cuda.synchronize()
+    start = [offset + f * stride for f in range(8)]
+    ctx.set_state_device([src.data_ptr() + 4 * s for s in start])
+    ctx.get_state_device([dst.data_ptr() + 4 * s for s in start])
+    host = ctx.get_state().reshape(8, nc)
+    a, d = src.cpu().numpy(), dst.cpu().numpy()
+    inside = np.zeros(d.size, bool)
+    for f, s in enumerate(start):
+        assert np.array_equal(host[f], a[s:s + nc]) and np.array_equal(d[s:s + nc], a[s:s + nc])
+        inside[s:s + nc] = True
+    assert (d[~inside] == -1.0).all()
+    ctx.close()
