@@ -48,7 +48,9 @@ __device__ __forceinline__ float stage_h(const StepState *st, int hsel) {
 __device__ __forceinline__ bool stage_begin(const StageStep &ss, const OpenStep &open, float &h) {
   if (open.in) {
     const StepState s = open_step(open, blockIdx.x == 0 && threadIdx.x < 64);
-    h = stage_h(&s, ss.hsel);
+    // selected by value: a pointer into the record would keep it in memory
+    const float half = s.h, full = s.dt;
+    h = ss.hsel == H_HALF ? half : full;
     return s.active;
   }
   if (ss.hsel == H_FIXED) {
