@@ -150,8 +150,9 @@ struct nmhd_ctx {
   double *diag_part = nullptr;  // run diagnostics: per-block partials, result
   double *diag_out = nullptr;
   int path = NMHD_PATH_TILED;
-  // tile shapes of the tiled path (fastest measured at 256^3-512^3 on MI355X)
-  int ftile = TV_32x8, utile = TV_64x4;
+  // tile shapes of the tiled path: kernel and shape by the box until
+  // nmhd_set_tiles names one
+  int ftile = kTileAuto, utile = kTileAuto;
   bool cfl_valid = false;  // rec[r].cfl holds the CFL minimum of the state (ghost cells aside)
   std::string err;
   bool timing = false;
@@ -228,6 +229,8 @@ void collect_timing(nmhd_ctx *c) {
   }
   c->pending.clear();
 }
+
+int tile_of(int tile, int otherwise) { return tile == kTileAuto ? otherwise : tile; }
 
 int resolve_path(int p) { return p == NMHD_PATH_AUTO ? NMHD_PATH_TILED : p; }
 
@@ -532,9 +535,9 @@ int nmhd_rhs(nmhd_ctx *c, float h, float *const pace[8]) {
   const FluxSet F = fluxes(c);
   if (c->path == NMHD_PATH_TILED) {
     const StageStep ss{diag, H_DIAG, 0.0f};
-    launch_faces(c->stream, c->box, fields(c, c->cur), F, ss, OpenStep{}, c->ftile);
+    launch_faces(c->stream, c->box, fields(c, c->cur), F, ss, OpenStep{}, tile_of(c->ftile, TV_32x8));
     launch_update_tiled(c->stream, c->box, fields(c, c->cur), F, fields(c, c->cur), out, ss, true,
-                        false, c->utile);
+                        false, tile_of(c->utile, TV_64x4));
   } else {
     for (int d = 0; d < 3; ++d)
       flux_dispatch(c, d, fields(c, c->cur), F.dir[d], &diag->s, H_DIAG);
@@ -689,8 +692,8 @@ int nmhd_set_tiles(nmhd_ctx *c, int faces_tile, int update_tile) {
 
 int nmhd_get_tiles(const nmhd_ctx *c, int *faces_tile, int *update_tile) {
   if (!c) return NMHD_EINVAL;
-  if (faces_tile) *faces_tile = c->ftile;
-  if (update_tile) *update_tile = c->utile;
+  if (faces_tile) *faces_tile = tile_of(c->ftile, TV_32x8);
+  if (update_tile) *update_tile = tile_of(c->utile, TV_64x4);
   return NMHD_OK;
 }
 

@@ -107,11 +107,16 @@ int nmhd_adj_forward_noalloc(const nmhd_desc *desc, const float *const w_in[8], 
   FluxSet F;
   for (int d = 0; d < 3; ++d)
     for (int k = 0; k < 7; ++k) F.dir[d].f[k] = nullptr;
-  for (int k = 0; k < 7; ++k) F.dir[0].f[k] = slot(8 + k);
-  F.dir[1].f[5] = slot(15);
-  F.dir[1].f[6] = slot(16);
-  F.dir[2].f[5] = slot(17);
-  F.dir[2].f[6] = slot(18);
+  if (direct_stage(b)) {  // a small box hands over every flux
+    for (int d = 0; d < 3; ++d)
+      for (int k = 0; k < 7; ++k) F.dir[d].f[k] = slot(8 + 7 * d + k);
+  } else {
+    for (int k = 0; k < 7; ++k) F.dir[0].f[k] = slot(8 + k);
+    F.dir[1].f[5] = slot(15);
+    F.dir[1].f[6] = slot(16);
+    F.dir[2].f[5] = slot(17);
+    F.dir[2].f[6] = slot(18);
+  }
 
   enqueue_frozen_step((hipStream_t)stream, b, desc->integrator, Win, Wstar, Wout, F, dt);
   const hipError_t e = hipGetLastError();

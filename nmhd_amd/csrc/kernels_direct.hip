@@ -1,0 +1,178 @@
+// kernels_direct.hip -- the face fluxes of a box too small to fill the chip
+// with marching tiles: one thread per face, no march, no staging, no barrier.
+//
+//  k_direct_faces   the seven fluxes of one face per thread, three threads
+//                   per cell (x, y and z), into the stage's 21 flux arrays
+//
+// The tiled march solves three or four Riemann problems one after another per
+// plane (3.8 us a plane whatever the box), so a box with few tiles is bound
+// by that chain.  Here every face has its own thread and all its loads are in
+// flight at once; the stencils come from L1 and L2, and the launch is bound by
+// VALU issue from about 50^3 cells on.  It writes 21 arrays instead of the
+// march's 11 (the update then differences the hydro fluxes), which a box this
+// size does into the caches.  The arithmetic of a face is that of the tiles,
+// expression by expression, so the two give the same bits.
+//
+// Reference correspondence: as tiled_tiles.h.
+#include "tiled_tiles.h"
+
+namespace nmhd {
+namespace direct {
+
+using tiled::at_byte;
+using tiled::recon;
+using tiled::recon_bsum;
+
+constexpr int kThreads = 256;
+
+// i (in [-2, n]) brought into [0, n)
+__device__ __forceinline__ int wrap1(int i, int n) {
+  const int j = i < 0 ? i + n : (i >= n ? i - n : i);
+  return n == 1 ? 0 : j;
+}
+
+// What one thread reads for the lower D-face of its cell: the stencil of rho,
+// v (normal first) and p, the sums of the two transverse B on the stencil
+// cells' faces, and the normal B.
+struct Stencil {
+  float q[5][4], e1[4], e2[4], bn;
+};
+
+template <int D>
+__device__ __forceinline__ Stencil load_face(const Box &b, const FieldPtrs &W, int x, int y,
+                                             int z) {
+  constexpr int D1 = (D + 1) % 3, D2 = (D + 2) % 3;
+  // byte offsets of the stencil cells c-2..c+1 along D, and of their upper
+  // neighbours along the two transverse axes
+  unsigned s[4], s1[4], s2[4];
+  const unsigned row = b.n[0] * 4u, plane = row * (unsigned)b.n[1];
+  const unsigned stride[3] = {4u, row, plane};
+  auto at = [&](int d, int i) { return (unsigned)wrap1(i, b.n[d]) * stride[d]; };
+  const int v[3] = {x, y, z};
+  const unsigned o1 = v[D1] * stride[D1], o2 = v[D2] * stride[D2];
+  const unsigned p1 = at(D1, v[D1] + 1), p2 = at(D2, v[D2] + 1);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const unsigned od = at(D, v[D] + k - 2);
+    s[k] = od + (o1 + o2);
+    s1[k] = od + (p1 + o2);
+    s2[k] = od + (o1 + p2);
+  }
+  auto ld = [&](int f, unsigned o) { return *at_byte((const float *)W.f[f], o); };
+  Stencil t;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    t.q[0][k] = ld(0, s[k]);
+    t.q[1][k] = ld(1 + D, s[k]);
+    t.q[2][k] = ld(1 + D1, s[k]);
+    t.q[3][k] = ld(1 + D2, s[k]);
+    t.q[4][k] = ld(4, s[k]);
+    t.e1[k] = ld(5 + D1, s[k]) + ld(5 + D1, s1[k]);
+    t.e2[k] = ld(5 + D2, s[k]) + ld(5 + D2, s2[k]);
+  }
+  t.bn = ld(5 + D, s[2]);
+  return t;
+}
+
+template <int D, int Recon>
+__device__ __forceinline__ Flux7 flux(const Box &b, const Stencil &t, float h, int y) {
+  float L[7], R[7];
+  recon(Recon, t.q[0][0], t.q[0][1], t.q[0][2], t.q[0][3], L[0], R[0]);
+  recon(Recon, t.q[1][0], t.q[1][1], t.q[1][2], t.q[1][3], L[1], R[1]);
+  recon(Recon, t.q[2][0], t.q[2][1], t.q[2][2], t.q[2][3], L[2], R[2]);
+  recon(Recon, t.q[3][0], t.q[3][1], t.q[3][2], t.q[3][3], L[3], R[3]);
+  recon(Recon, t.q[4][0], t.q[4][1], t.q[4][2], t.q[4][3], L[4], R[4]);
+  recon_bsum(Recon, t.e1[0], t.e1[1], t.e1[2], t.e1[3], L[5], R[5]);
+  recon_bsum(Recon, t.e2[0], t.e2[1], t.e2[2], t.e2[3], L[6], R[6]);
+  if (D != 2 && b.source == 1) {
+    // the other in-plane velocity: v_y on an x-face, v_x on a y-face
+    constexpr int o = D == 0 ? 2 : 3;
+    const float va = 0.5f * (t.q[o][1] + t.q[o][2]);
+    const float mbv = 0.5f * h * (D == 0 ? accel_x(b, va) : accel_y_face(b, va, y));
+    L[1] += mbv;
+    R[1] += mbv;
+  }
+  return hlld(b.gamma, b.inv_gm1, t.bn, L[0], R[0], L[1], R[1], L[2], R[2], L[3], R[3], L[4], R[4],
+              L[5], R[5], L[6], R[6]);
+}
+
+// One face per thread: loads, then flux.  The loads come first: the step's
+// record is waited for with them, not before them.
+template <int D, int Recon>
+__device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const FluxOut &F,
+                                         const StageStep &ss, const OpenStep &open, int x, int y,
+                                         int z, bool valid, float *hs) {
+  constexpr int D1 = (D + 1) % 3, D2 = (D + 2) % 3;
+  const Stencil t = load_face<D>(b, W, x, y, z);
+  float h = 0.0f;
+  if (open.in) {
+    // the launch that opens the step: only the face predictor needs its size,
+    // and an untaken step's fluxes are not read, so without a source term
+    // only the first wave looks
+    const bool src = D != 2 && b.source == 1;
+    if (threadIdx.x < 64 && (src || blockIdx.x == 0)) {
+      const StepState s = open_step(open, blockIdx.x == 0);
+      if (threadIdx.x == 0) *hs = tiled::opened_size(s, ss.hsel);
+    }
+    if (src) {
+      __syncthreads();
+      h = *hs;
+    }
+  } else {
+    if (!tiled::stage_active(ss)) return;
+    h = tiled::stage_size(ss);
+  }
+  const Flux7 r = flux<D, Recon>(b, t, h, y);
+  if (!valid) return;
+  const unsigned o = (unsigned)((z * b.n[1] + y) * b.n[0] + x) * 4u;
+  *at_byte(F.f[0], o) = r.rho;
+  *at_byte(F.f[1 + D], o) = r.mn;
+  *at_byte(F.f[1 + D1], o) = r.mt1;
+  *at_byte(F.f[1 + D2], o) = r.mt2;
+  *at_byte(F.f[4], o) = r.e;
+  *at_byte(F.f[5], o) = r.bt1;
+  *at_byte(F.f[6], o) = r.bt2;
+}
+
+// Consecutive workgroups take the three directions of the same cells, and
+// each XCD a contiguous range of cells; a wave takes 64 cells in a row of the
+// arrays (patches of narrower rows, which would spare the division below,
+// touch more cache lines per load: 98 us against 50 at 130x109x75).  Threads
+// past the last cell work on it and store nothing (a whole wave opens the
+// step).
+template <int Recon>
+__global__ void __launch_bounds__(kThreads)
+    k_direct_faces(Box b, FieldPtrs W, FluxSet F, StageStep ss, OpenStep open) {
+  __shared__ float hs;
+  const unsigned lb = xcd_logical_block(blockIdx.x, gridDim.x);
+  const unsigned group = lb / 3, dir = lb - 3 * group;
+  const unsigned i = group * kThreads + threadIdx.x, last = (unsigned)b.ncell - 1;
+  const bool valid = i <= last;
+  int x, y, z;
+  cell_coords(b, valid ? i : last, x, y, z);
+  if (dir == 0)
+    one_face<0, Recon>(b, W, F.dir[0], ss, open, x, y, z, valid, &hs);
+  else if (dir == 1)
+    one_face<1, Recon>(b, W, F.dir[1], ss, open, x, y, z, valid, &hs);
+  else
+    one_face<2, Recon>(b, W, F.dir[2], ss, open, x, y, z, valid, &hs);
+}
+
+}  // namespace direct
+
+// Up to 400,000 cells.  Step times, direct faces against the march: 32^3 26.0
+// / 33.7 us, 64^3 48.5 / 54.3, 64x72x64 68.4 / 77.8, 80^3 102.3 / 97.8, 96^3
+// 139.7 / 135.2, 128^3 304 / 250: the chip is then full of tiles, and the
+// update reads 10 arrays more.
+bool direct_stage(const Box &b) { return b.ncell <= 400000; }
+
+void launch_direct_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F,
+                         const StageStep &ss, const OpenStep &open) {
+  const dim3 grid(3 * grid_for(b.ncell, direct::kThreads)), blk(direct::kThreads);
+  if (b.recon == 1)
+    hipLaunchKernelGGL(direct::k_direct_faces<1>, grid, blk, 0, s, b, W, F, ss, open);
+  else
+    hipLaunchKernelGGL(direct::k_direct_faces<0>, grid, blk, 0, s, b, W, F, ss, open);
+}
+
+}  // namespace nmhd

@@ -2,7 +2,8 @@
 // per RK stage, each a grid of z-marching column tiles (the tile functions
 // are in tiled_tiles.h).
 //
-//  k_faces         all three face fluxes of every cell (21 floats per cell)
+//  k_faces         all three face fluxes of every cell, differenced in the
+//                  tile (k_direct_faces takes its place in small boxes)
 //  k_update_march  divergence, CT, conserved update, primitive recovery, the
 //                  shearing-box kick and (stage 2) the CFL minimum of the
 //                  new state, one atomic per workgroup
@@ -26,8 +27,8 @@ __global__ void __launch_bounds__(kTileThreads, (FacesShape<TX, TY>::kWavesPerSi
   faces_tile<TX, TY, Recon>(b, W, F, h, x0, y0, z0, min(z0 + zc, b.n[2]), lds);
 }
 
-template <int TX, int TY, bool PaceOnly, bool Cfl>
-__global__ void __launch_bounds__(kTileThreads) k_update_march(Box b, FieldPtrs Win, FluxSet F,
+template <int TX, int TY, bool PaceOnly, bool Cfl, bool Raw>
+__global__ void __launch_bounds__(kTileThreads, 4) k_update_march(Box b, FieldPtrs Win, FluxSet F,
                                                                FieldPtrs Wb, FieldPtrs Wo,
                                                                StageStep ss, int zc, int gx,
                                                                int gy) {
@@ -51,7 +52,7 @@ __global__ void __launch_bounds__(kTileThreads) k_update_march(Box b, FieldPtrs 
   __shared__ float lds[UpdateShape<TX, TY>::kLds];
   __shared__ float red[4];
   float cfl_t = 3.0e38f;
-  update_tile<TX, TY, PaceOnly, Cfl>(b, Win, F, Wb, Wo, h, x0, y0, z0, min(z0 + zc, b.n[2]), lds,
+  update_tile<TX, TY, PaceOnly, Cfl, Raw>(b, Win, F, Wb, Wo, h, x0, y0, z0, min(z0 + zc, b.n[2]), lds,
                                      cfl_t);
   if (Cfl && !PaceOnly) block_min_into(cfl_t, cfl_slot(ss.rec, blockIdx.x), red);
 }
@@ -94,27 +95,29 @@ void faces_as(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const 
                        0, s, b, W, F, ss, open, zc, gx, gy);
 }
 
-template <int TX, int TY>
+template <int TX, int TY, bool Raw>
 void update_as(hipStream_t s, const Box &b, FieldPtrs Win, const FluxSet &F, FieldPtrs Wbase,
                FieldPtrs Wout, const StageStep &ss, bool pace_only, bool cfl) {
   const int zc = tiled_zchunk(b, TX, TY, false);
   const int gx = (b.n[0] + TX - 1) / TX, gy = (b.n[1] + TY - 1) / TY, gz = (b.n[2] + zc - 1) / zc;
   const dim3 grid(gx * gy * gz), blk(tiled::kTileThreads);
   if (pace_only)
-    hipLaunchKernelGGL((tiled::k_update_march<TX, TY, true, false>), grid, blk, 0, s, b, Win, F,
-                       Wbase, Wout, ss, zc, gx, gy);
+    hipLaunchKernelGGL((tiled::k_update_march<TX, TY, true, false, false>), grid, blk, 0, s, b,
+                       Win, F, Wbase, Wout, ss, zc, gx, gy);
   else if (cfl)
-    hipLaunchKernelGGL((tiled::k_update_march<TX, TY, false, true>), grid, blk, 0, s, b, Win, F,
-                       Wbase, Wout, ss, zc, gx, gy);
+    hipLaunchKernelGGL((tiled::k_update_march<TX, TY, false, true, Raw>), grid, blk, 0, s, b, Win,
+                       F, Wbase, Wout, ss, zc, gx, gy);
   else
-    hipLaunchKernelGGL((tiled::k_update_march<TX, TY, false, false>), grid, blk, 0, s, b, Win, F,
-                       Wbase, Wout, ss, zc, gx, gy);
+    hipLaunchKernelGGL((tiled::k_update_march<TX, TY, false, false, Raw>), grid, blk, 0, s, b,
+                       Win, F, Wbase, Wout, ss, zc, gx, gy);
 }
 
 }  // namespace
 
 void launch_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const StageStep &ss,
                   const OpenStep &open, int tile) {
+  if (tile == kTileAuto && direct_stage(b)) return launch_direct_faces(s, b, W, F, ss, open);
+  if (tile == kTileAuto) tile = TV_32x8;
   if (tile == TV_64x4)
     faces_as<64, 4>(s, b, W, F, ss, open);
   else if (tile == TV_16x16)
@@ -126,12 +129,18 @@ void launch_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, co
 void launch_update_tiled(hipStream_t s, const Box &b, FieldPtrs Win, const FluxSet &F,
                          FieldPtrs Wbase, FieldPtrs Wout, const StageStep &ss, bool pace_only, bool cfl,
                          int tile) {
-  if (tile == TV_64x4)
-    update_as<64, 4>(s, b, Win, F, Wbase, Wout, ss, pace_only, cfl);
+  const bool raw = tile == kTileAuto && direct_stage(b);
+  if (tile == kTileAuto) tile = TV_64x4;
+  if (raw && tile == TV_64x4)
+    update_as<64, 4, true>(s, b, Win, F, Wbase, Wout, ss, false, cfl);
+  else if (raw)
+    update_as<32, 8, true>(s, b, Win, F, Wbase, Wout, ss, false, cfl);
+  else if (tile == TV_64x4)
+    update_as<64, 4, false>(s, b, Win, F, Wbase, Wout, ss, pace_only, cfl);
   else if (tile == TV_16x16)
-    update_as<16, 16>(s, b, Win, F, Wbase, Wout, ss, pace_only, cfl);
+    update_as<16, 16, false>(s, b, Win, F, Wbase, Wout, ss, pace_only, cfl);
   else
-    update_as<32, 8>(s, b, Win, F, Wbase, Wout, ss, pace_only, cfl);
+    update_as<32, 8, false>(s, b, Win, F, Wbase, Wout, ss, pace_only, cfl);
 }
 
 }  // namespace nmhd

@@ -202,6 +202,7 @@ struct WorkItem {
 
 // Tile shapes of the z-marching kernels (TX x TY, 256 threads each).
 enum TileVariant { TV_64x4 = 0, TV_32x8 = 1, TV_16x16 = 2, TV_COUNT = 3 };
+constexpr int kTileAuto = -1;  // kernel and tile shape by the box
 constexpr int kTileTX[TV_COUNT] = {64, 32, 16};
 constexpr int kTileTY[TV_COUNT] = {4, 8, 16};
 
@@ -287,14 +288,21 @@ struct AdjStageArgs {
 };
 void launch_adj_stage(hipStream_t s, const Box &b, const AdjStageArgs &A);
 
+// kernels_direct.hip (the stage of a small box: a thread per face, a thread
+// per cell; all 21 flux arrays are used)
+bool direct_stage(const Box &b);
+void launch_direct_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F,
+                         const StageStep &ss, const OpenStep &open);
+
 // kernels_tiled.hip
 int tiled_zchunk(const Box &b, int tx, int ty, bool faces);
-// tile: TileVariant of the z-marching tiles
+// tile: TileVariant of the z-marching tiles, or kTileAuto (both launches of a
+// stage then take the same route, direct_stage)
 // open: the bookkeeping of the step that this launch begins (in == NULL: none)
 void launch_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const StageStep &ss,
-                  const OpenStep &open = {}, int tile = TV_32x8);
+                  const OpenStep &open = {}, int tile = kTileAuto);
 void launch_update_tiled(hipStream_t s, const Box &b, FieldPtrs Win, const FluxSet &F,
                          FieldPtrs Wbase, FieldPtrs Wout, const StageStep &ss, bool pace_only,
-                         bool cfl, int tile = TV_64x4);
+                         bool cfl, int tile = kTileAuto);
 
 }  // namespace nmhd

@@ -43,22 +43,31 @@ __device__ __forceinline__ float stage_h(const StepState *st, int hsel) {
   return hsel == H_HALF ? st->h : (hsel == H_FULL ? st->dt : st->h_diag);
 }
 
+// The stage step of a step just opened (selected by value: a pointer into the
+// record would keep it in memory).
+__device__ __forceinline__ float opened_size(const StepState &s, int hsel) {
+  const float half = s.h, full = s.dt;
+  return hsel == H_HALF ? half : full;
+}
+
+// Whether the step that a stage kernel belongs to is taken, and its size.
+__device__ __forceinline__ bool stage_active(const StageStep &ss) {
+  return ss.hsel == H_FIXED || ss.rec->s.active;
+}
+__device__ __forceinline__ float stage_size(const StageStep &ss) {
+  return ss.hsel == H_FIXED ? ss.h : stage_h(&ss.rec->s, ss.hsel);
+}
+
 // The stage step of a launch, opening the step first when it is the step's
 // first kernel; false: the step is not taken.
 __device__ __forceinline__ bool stage_begin(const StageStep &ss, const OpenStep &open, float &h) {
   if (open.in) {
     const StepState s = open_step(open, blockIdx.x == 0 && threadIdx.x < 64);
-    // selected by value: a pointer into the record would keep it in memory
-    const float half = s.h, full = s.dt;
-    h = ss.hsel == H_HALF ? half : full;
+    h = opened_size(s, ss.hsel);
     return s.active;
   }
-  if (ss.hsel == H_FIXED) {
-    h = ss.h;
-    return true;
-  }
-  h = stage_h(&ss.rec->s, ss.hsel);
-  return ss.rec->s.active;
+  h = stage_size(ss);
+  return stage_active(ss);
 }
 
 // true modulo for staging coordinates, which may lie several box lengths
@@ -727,7 +736,9 @@ __device__ __forceinline__ void finish_cell(const Box &b, const CellEdges &ce, c
 // The hydro divergence and the base cell values are the thread's own and
 // stay in registers.  cfl_t is lowered to the CFL time of every interior
 // cell the thread updates (stage 2 with Cfl).
-template <int TX, int TY, bool PaceOnly, bool Cfl>
+// Raw: the hydro fluxes themselves are in Fs (k_direct_faces wrote them) and
+// are differenced here, in the order of the face march.
+template <int TX, int TY, bool PaceOnly, bool Cfl, bool Raw = false>
 __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, const FluxSet &Fs,
                                             const FieldPtrs &Wb, const FieldPtrs &Wo, float h,
                                             int x0, int y0, int z0, int zend, float *lds,
@@ -873,8 +884,10 @@ __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, 
   float pc[5], pc_nx[5], wb[5] = {}, wb_nx[5] = {}, bz_lo = 0.0f, bz_hi = 0.0f, bz_nx = 0.0f;
   auto load_own = [&](int p, float *dpc, float *dwb) {
     const int base = wrap(p, nz) * plane + own;
+    if (!Raw) {
 #pragma unroll
-    for (int k = 0; k < 5; ++k) dpc[k] = get_nt(&SB.pace[k][base]);
+      for (int k = 0; k < 5; ++k) dpc[k] = get_nt(&SB.pace[k][base]);
+    }
     dwb[0] = get_nt(&Wb.f[0][base]);
     dwb[4] = get_nt(&Wb.f[4][base]);
     if (!in_is_base) {
@@ -882,6 +895,27 @@ __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, 
       for (int k = 1; k < 4; ++k) dwb[k] = get_nt(&Wb.f[k][base]);
     }
   };
+
+  // raw hydro fluxes of plane r's cell: x- and y-faces, and the lower z-face,
+  // which is the upper one of the plane before
+  const int ownx = valid ? y * nx + wrap(x + 1, nx) : 0;
+  const int owny = valid ? wrap(y + 1, ny) * nx + x : 0;
+  float fxl[5], fxh[5], fyl[5], fyh[5], fzl[5], fzh[5];
+  auto load_raw = [&](int r) {
+    const int base = r * plane, up = wrap(r + 1, nz) * plane;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      fxl[k] = Fs.dir[0].f[k][base + own];
+      fxh[k] = Fs.dir[0].f[k][base + ownx];
+      fyl[k] = Fs.dir[1].f[k][base + own];
+      fyh[k] = Fs.dir[1].f[k][base + owny];
+      fzh[k] = Fs.dir[2].f[k][up + own];
+    }
+  };
+  if (Raw) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) fzl[k] = Fs.dir[2].f[k][z0 * plane + own];
+  }
 
   // prologue: every load in flight at once; the edges on z-face z0 from
   // planes z0-1 and z0, then plane z0+1 and face z0+1 over them
@@ -910,6 +944,7 @@ __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, 
 
   for (int r = z0; r < zend; ++r) {
     const bool more = r + 1 < zend;
+    if (Raw) load_raw(r);
     if (more) {  // prefetch the data of the next iteration
       load3(r + 2, r3);
       loadz(r + 2, rz);
@@ -946,6 +981,15 @@ __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, 
           ce.ZY[u][v] = F[3 * EN + u * EX];
         }
       const float bb[6] = {bxl0, bxh0, byl0, byh0, bz_lo, bz_hi};
+      if (Raw) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+          float sacc = (fxl[k] - fxh[k]) * b.inv_d[0];
+          sacc += (fyl[k] - fyh[k]) * b.inv_d[1];
+          pc[k] = sacc + (fzl[k] - fzh[k]) * b.inv_d[2];
+          fzl[k] = fzh[k];
+        }
+      }
       finish_cell<PaceOnly, Cfl>(b, ce, pc, wb, bb, h, y, r, a, Wo, cfl_t);
     }
     if (more) {
@@ -953,8 +997,10 @@ __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, 
       store3(r + 2, r3);
       storez(rz);
       storep();
+      if (!Raw) {
 #pragma unroll
-      for (int k = 0; k < 5; ++k) pc[k] = pc_nx[k];
+        for (int k = 0; k < 5; ++k) pc[k] = pc_nx[k];
+      }
 #pragma unroll
       for (int k = 0; k < 5; ++k) wb[k] = wb_nx[k];
       bz_lo = bz_hi;

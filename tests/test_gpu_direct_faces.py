@@ -1,0 +1,70 @@
+"""The small-box route (one thread per face) against the marching tiles, bit
+for bit, and the rules that choose between them (GPU)."""
+import numpy as np
+import pytest
+
+from nmhd_amd import capi, problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+def rough(cfg, seed):
+    """Independent random rho, v, p, B per cell, B = 0 on 1/16 of the faces."""
+    n = cfg["n"]
+    idx = np.arange(n[0] * n[1] * n[2], dtype=np.uint64)
+    u = [P.uniform01(seed, idx, c).reshape(n[2], n[1], n[0]) for c in range(8)]
+    W = np.stack([0.2 + u[0], u[1] - 0.5, u[2] - 0.5, u[3] - 0.5, 0.2 + u[4],
+                  u[5] - 0.5, u[6] - 0.5, u[7] - 0.5]).astype(np.float32)
+    for f in (5, 6, 7):
+        W[f][(idx.reshape(W[f].shape) * np.uint64(2654435761) >> np.uint64(7)) % np.uint64(16)
+             == f] = 0.0
+    return W
+
+
+def run(cfg, W, tiles):
+    """Two frozen-size steps' worth of state: a step, then a goal-clipped one."""
+    ctx = capi.Context(cfg)
+    if tiles:
+        ctx.set_tiles(*tiles)
+    ctx.set_state(W)
+    ctx.set_time(0.3)
+    dt, _ = ctx.step()
+    out = [ctx.get_state()]
+    goal = float(np.float32(ctx.get_time()[0] + 0.25 * dt))
+    assert ctx.run(goal, 3) == (1, True)  # two inactive steps follow
+    out.append(ctx.get_state())
+    t = ctx.get_time()
+    ctx.close()
+    return dt, t, out
+
+
+# one cell, one row, one column, one plane; sizes around a wave, a workgroup
+# and a tile; the last boxes below and above the limit of 400,000 cells
+SIZES = [(1, 1, 1), (3, 1, 1), (1, 1, 5), (64, 1, 1), (1, 67, 1), (1, 1, 70), (17, 15, 1),
+         (2, 2, 2), (7, 9, 4), (33, 9, 3), (16, 16, 1), (31, 33, 35), (64, 72, 33),
+         (100, 80, 50), (101, 80, 50)]
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("recon,integrator", [(0, 0), (1, 0), (0, 1)])
+def test_direct_equals_tiles(gpu_ready, n, recon, integrator):
+    cfg = P.make_config(n, cfl=0.1, recon=recon, integrator=integrator)
+    W = rough(cfg, 11)
+    ref = run(cfg, W, (capi.TILE_32x8, capi.TILE_64x4))
+    got = run(cfg, W, None)
+    assert got[:2] == ref[:2]
+    for a, b in zip(got[2], ref[2]):
+        assert np.isfinite(b).all()
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [(5, 4, 1), (24, 12, 9), (64, 64, 30), (90, 70, 50), (70, 70, 80)])
+@pytest.mark.parametrize("fixes", [0, 7])
+def test_direct_equals_tiles_shearing(gpu_ready, n, fixes):
+    cfg = dict(P.config_c2(n, cfl=0.1), fixes=fixes)
+    W = rough(cfg, 12)
+    ref = run(cfg, W, (capi.TILE_32x8, capi.TILE_64x4))
+    got = run(cfg, W, None)
+    assert got[:2] == ref[:2]
+    for a, b in zip(got[2], ref[2]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
