@@ -31,16 +31,12 @@ __device__ __forceinline__ int wrap1(int i, int n) {
   return n == 1 ? 0 : j;
 }
 
-// What one thread reads for the lower D-face of its cell: the stencil of rho,
-// v (normal first) and p, the sums of the two transverse B on the stencil
-// cells' faces, and the normal B.
-struct Stencil {
-  float q[5][4], e1[4], e2[4], bn;
-};
-
-template <int D>
-__device__ __forceinline__ Stencil load_face(const Box &b, const FieldPtrs &W, int x, int y,
-                                             int z) {
+// One face per thread, the lower D-face of cell (x, y, z).  The loads come
+// first: the step's record is waited for with them, not before them.
+template <int D, int Recon>
+__device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const FluxOut &F,
+                                         const StageStep &ss, const OpenStep &open, int x, int y,
+                                         int z, bool valid, float *hs) {
   constexpr int D1 = (D + 1) % 3, D2 = (D + 2) % 3;
   // byte offsets of the stencil cells c-2..c+1 along D, and of their upper
   // neighbours along the two transverse axes
@@ -58,52 +54,21 @@ __device__ __forceinline__ Stencil load_face(const Box &b, const FieldPtrs &W, i
     s1[k] = od + (p1 + o2);
     s2[k] = od + (o1 + p2);
   }
+  // the stencil of rho, v (normal first) and p, and the sums of the two
+  // transverse B on the stencil cells' faces
+  float q[5][4], e1[4], e2[4];
   auto ld = [&](int f, unsigned o) { return *at_byte((const float *)W.f[f], o); };
-  Stencil t;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    t.q[0][k] = ld(0, s[k]);
-    t.q[1][k] = ld(1 + D, s[k]);
-    t.q[2][k] = ld(1 + D1, s[k]);
-    t.q[3][k] = ld(1 + D2, s[k]);
-    t.q[4][k] = ld(4, s[k]);
-    t.e1[k] = ld(5 + D1, s[k]) + ld(5 + D1, s1[k]);
-    t.e2[k] = ld(5 + D2, s[k]) + ld(5 + D2, s2[k]);
+    q[0][k] = ld(0, s[k]);
+    q[1][k] = ld(1 + D, s[k]);
+    q[2][k] = ld(1 + D1, s[k]);
+    q[3][k] = ld(1 + D2, s[k]);
+    q[4][k] = ld(4, s[k]);
+    e1[k] = ld(5 + D1, s[k]) + ld(5 + D1, s1[k]);
+    e2[k] = ld(5 + D2, s[k]) + ld(5 + D2, s2[k]);
   }
-  t.bn = ld(5 + D, s[2]);
-  return t;
-}
-
-template <int D, int Recon>
-__device__ __forceinline__ Flux7 flux(const Box &b, const Stencil &t, float h, int y) {
-  float L[7], R[7];
-  recon(Recon, t.q[0][0], t.q[0][1], t.q[0][2], t.q[0][3], L[0], R[0]);
-  recon(Recon, t.q[1][0], t.q[1][1], t.q[1][2], t.q[1][3], L[1], R[1]);
-  recon(Recon, t.q[2][0], t.q[2][1], t.q[2][2], t.q[2][3], L[2], R[2]);
-  recon(Recon, t.q[3][0], t.q[3][1], t.q[3][2], t.q[3][3], L[3], R[3]);
-  recon(Recon, t.q[4][0], t.q[4][1], t.q[4][2], t.q[4][3], L[4], R[4]);
-  recon_bsum(Recon, t.e1[0], t.e1[1], t.e1[2], t.e1[3], L[5], R[5]);
-  recon_bsum(Recon, t.e2[0], t.e2[1], t.e2[2], t.e2[3], L[6], R[6]);
-  if (D != 2 && b.source == 1) {
-    // the other in-plane velocity: v_y on an x-face, v_x on a y-face
-    constexpr int o = D == 0 ? 2 : 3;
-    const float va = 0.5f * (t.q[o][1] + t.q[o][2]);
-    const float mbv = 0.5f * h * (D == 0 ? accel_x(b, va) : accel_y_face(b, va, y));
-    L[1] += mbv;
-    R[1] += mbv;
-  }
-  return hlld(b.gamma, b.inv_gm1, t.bn, L[0], R[0], L[1], R[1], L[2], R[2], L[3], R[3], L[4], R[4],
-              L[5], R[5], L[6], R[6]);
-}
-
-// One face per thread: loads, then flux.  The loads come first: the step's
-// record is waited for with them, not before them.
-template <int D, int Recon>
-__device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const FluxOut &F,
-                                         const StageStep &ss, const OpenStep &open, int x, int y,
-                                         int z, bool valid, float *hs) {
-  constexpr int D1 = (D + 1) % 3, D2 = (D + 2) % 3;
-  const Stencil t = load_face<D>(b, W, x, y, z);
+  const float bn = ld(5 + D, s[2]);
   float h = 0.0f;
   if (open.in) {
     // the launch that opens the step: only the face predictor needs its size,
@@ -122,7 +87,24 @@ __device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const
     if (!tiled::stage_active(ss)) return;
     h = tiled::stage_size(ss);
   }
-  const Flux7 r = flux<D, Recon>(b, t, h, y);
+  float L[7], R[7];
+  recon(Recon, q[0][0], q[0][1], q[0][2], q[0][3], L[0], R[0]);
+  recon(Recon, q[1][0], q[1][1], q[1][2], q[1][3], L[1], R[1]);
+  recon(Recon, q[2][0], q[2][1], q[2][2], q[2][3], L[2], R[2]);
+  recon(Recon, q[3][0], q[3][1], q[3][2], q[3][3], L[3], R[3]);
+  recon(Recon, q[4][0], q[4][1], q[4][2], q[4][3], L[4], R[4]);
+  recon_bsum(Recon, e1[0], e1[1], e1[2], e1[3], L[5], R[5]);
+  recon_bsum(Recon, e2[0], e2[1], e2[2], e2[3], L[6], R[6]);
+  if (D != 2 && b.source == 1) {
+    // the other in-plane velocity: v_y on an x-face, v_x on a y-face
+    constexpr int o = D == 0 ? 2 : 3;
+    const float va = 0.5f * (q[o][1] + q[o][2]);
+    const float mbv = 0.5f * h * (D == 0 ? accel_x(b, va) : accel_y_face(b, va, y));
+    L[1] += mbv;
+    R[1] += mbv;
+  }
+  const Flux7 r = hlld(b.gamma, b.inv_gm1, bn, L[0], R[0], L[1], R[1], L[2], R[2], L[3], R[3],
+                       L[4], R[4], L[5], R[5], L[6], R[6]);
   if (!valid) return;
   const unsigned o = (unsigned)((z * b.n[1] + y) * b.n[0] + x) * 4u;
   *at_byte(F.f[0], o) = r.rho;
