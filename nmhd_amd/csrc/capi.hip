@@ -275,6 +275,13 @@ void enqueue_step(nmhd_ctx *c, float goal) {
   auto stage = [&](int Win, int base, int Wout, int hsel, bool first, bool last) {
     if (tiled) {
       const StageStep ss{out, hsel, 0.0f};
+      if (c->ftile == kTileAuto && !(first && last) && tiny_stage(b)) {
+        timed(c, last ? S_UPDATE2 : S_UPDATE1, [&] {
+          launch_tiny_stage(s, b, fields(c, Win), fields(c, base), fields(c, Wout), ss,
+                            first ? open : OpenStep{}, last);
+        });
+        return;
+      }
       timed(c, last ? S_FACES2 : S_FACES1, [&] {
         launch_faces(s, b, fields(c, Win), F, ss, first ? open : OpenStep{}, c->ftile);
       });

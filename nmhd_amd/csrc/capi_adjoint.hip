@@ -20,15 +20,14 @@ namespace nmhd {
 void enqueue_frozen_step(hipStream_t s, const Box &b, int integrator, FieldPtrs Win,
                          FieldPtrs Wstar, FieldPtrs Wout, const FluxSet &F, float dt) {
   const StageStep full{nullptr, H_FIXED, dt}, half{nullptr, H_FIXED, dt / 2};
-  if (integrator == NMHD_EULER1) {
-    launch_faces(s, b, Win, F, full);
-    launch_update_tiled(s, b, Win, F, Win, Wout, full, false, false);
-    return;
-  }
-  launch_faces(s, b, Win, F, half);
-  launch_update_tiled(s, b, Win, F, Win, Wstar, half, false, false);
-  launch_faces(s, b, Wstar, F, full);
-  launch_update_tiled(s, b, Wstar, F, Win, Wout, full, false, false);
+  auto stage = [&](FieldPtrs in, FieldPtrs out, const StageStep &ss) {
+    if (tiny_stage(b)) return launch_tiny_stage(s, b, in, Win, out, ss, OpenStep{}, false);
+    launch_faces(s, b, in, F, ss);
+    launch_update_tiled(s, b, in, F, Win, out, ss, false, false);
+  };
+  if (integrator == NMHD_EULER1) return stage(Win, Wout, full);
+  stage(Win, Wstar, half);
+  stage(Wstar, Wout, full);
 }
 
 }  // namespace nmhd

@@ -10,6 +10,9 @@
 //
 // Tiles are mapped to workgroups XCD-aware (xcd_logical_block) so that
 // neighbouring tiles, which re-read each other's halos, share an L2.
+#include <algorithm>
+#include <cmath>
+
 #include "tiled_tiles.h"
 
 namespace nmhd {
@@ -61,23 +64,68 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_update_march(Box b, FieldPt
 
 // ------------------------------------------------------------- launchers
 
+namespace {
+
+// Microseconds a workgroup takes per plane with 1..4 of them on its CU,
+// measured at 16^3-256^3: latency alone, then more and more issue (faces) or
+// bandwidth (update).
+struct MarchCost {
+  float plane[4];
+  int most;  // longest chunk worth considering
+};
+constexpr MarchCost kFacesCost = {{3.75f, 4.4f, 5.45f, 6.9f}, 32};
+constexpr MarchCost kUpdateCost = {{2.3f, 3.1f, 4.0f, 5.5f}, 16};
+
+}  // namespace
+
+int march_chunk(bool faces, int nz, const std::function<long(int)> &groups_at) {
+  // A march of zc planes costs about one plane more (the prologue and the
+  // last z-face); 1024 workgroups are resident (4 per CU).  In one round a
+  // CU's share decides; past it the rounds blend, except that a small
+  // remainder of the first ones is paid for as a round of its own (at 1050
+  // workgroups 1.5 rounds, at 2112 2.3, at 4224 4.1).
+  const MarchCost &c = faces ? kFacesCost : kUpdateCost;
+  int best = 1;
+  float least = 0.0f;
+  for (int want = 1; want <= c.most && want <= nz; ++want) {
+    const int chunks = (nz + want - 1) / want, zc = (nz + chunks - 1) / chunks;
+    const float rounds = (float)groups_at(zc) / 1024.0f;
+    float cost;
+    if (rounds <= 1.0f) {
+      const int share = (int)std::ceil(rounds * 4.0f);
+      cost = c.plane[share < 1 ? 0 : share - 1] * (float)(zc + 1);
+    } else {
+      const float whole = std::floor(rounds), part = rounds - whole;
+      const float extra = part > 0.0f ? 0.5f * std::max(0.0f, 1.0f - part / 0.4f) / whole : 0.0f;
+      cost = c.plane[3] * (float)(zc + 1) * (rounds + extra);
+    }
+    if (best == 1 && want == 1) least = cost;
+    if (cost < least) least = cost, best = zc;
+  }
+  return best;
+}
+
 int tiled_zchunk(const Box &b, int tx, int ty, bool faces) {
-  // Planes per workgroup march.  Measured on MI355X (256^3 and 512^3): the
-  // update is fastest with 16-plane chunks at both sizes; the face march
-  // with 32 planes once that gives at least 4096 workgroups (4 per CU
-  // resident: enough rounds that the last one is short), else 16.  Smaller
-  // chunks balance the grid better but repeat more prologue planes.  Small
-  // boxes halve the chunk until the grid fills the chip: one full round of
-  // 4 workgroups per CU (1024) for marches of 8 or more planes, half of it
-  // for shorter ones, whose prologue planes weigh more.  Measured step
-  // times (periodic cubes, both kernels at the same chunk): 32^3 best at 1
-  // plane (2.7x faster than 8), 48^3 at 1, 64^3 at 2 (1.8x faster than 8;
-  // 1 plane is 6% slower), 96^3 at 4, 128^3 at 8 (16 is 12% slower).
   const long cols = (long)((b.n[0] + tx - 1) / tx) * ((b.n[1] + ty - 1) / ty);
-  auto groups = [&](int zc) { return cols * ((b.n[2] + zc - 1) / zc); };
-  int zc = faces ? (groups(32) >= 4096 ? 32 : 16) : 16;
-  while (zc > 1 && groups(zc) < (zc >= 8 ? 1024 : 512)) zc /= 2;
-  return zc;
+  return march_chunk(faces, b.n[2], [&](int zc) { return cols * ((b.n[2] + zc - 1) / zc); });
+}
+
+int tiled_shape(int nx, int ny, bool faces) {
+  // Cells that tiles of a shape cover, idle lanes included.  Per covered cell
+  // the face march takes 1.15 times as long on 64x4 and 1.16 on 16x16 tiles
+  // as on 32x8 (256^3: 511 / 444 / 520 us; 80^3, which 16x16 covers exactly:
+  // 38 / 31 / 27).  The update is fastest on 64x4 (256^3: 412 us against 432
+  // on 32x8 and 600 on 16x16), whose idle lanes cost it less: 32x8 wins from
+  // a quarter more on (96^3: 39 against 34).
+  auto covered = [&](int v) {
+    const long tx = kTileTX[v], ty = kTileTY[v];
+    return (float)((nx + tx - 1) / tx * tx) * (float)((ny + ty - 1) / ty * ty);
+  };
+  if (!faces) return covered(TV_64x4) >= 1.25f * covered(TV_32x8) ? TV_32x8 : TV_64x4;
+  int v = TV_32x8;
+  if (1.15f * covered(TV_64x4) < covered(v)) v = TV_64x4;
+  if (1.16f * covered(TV_16x16) < (v == TV_32x8 ? 1.0f : 1.15f) * covered(v)) v = TV_16x16;
+  return v;
 }
 
 namespace {
@@ -117,7 +165,7 @@ void update_as(hipStream_t s, const Box &b, FieldPtrs Win, const FluxSet &F, Fie
 void launch_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const StageStep &ss,
                   const OpenStep &open, int tile) {
   if (tile == kTileAuto && direct_stage(b)) return launch_direct_faces(s, b, W, F, ss, open);
-  if (tile == kTileAuto) tile = TV_32x8;
+  if (tile == kTileAuto) tile = tiled_shape(b.n[0], b.n[1], true);
   if (tile == TV_64x4)
     faces_as<64, 4>(s, b, W, F, ss, open);
   else if (tile == TV_16x16)
@@ -130,7 +178,7 @@ void launch_update_tiled(hipStream_t s, const Box &b, FieldPtrs Win, const FluxS
                          FieldPtrs Wbase, FieldPtrs Wout, const StageStep &ss, bool pace_only, bool cfl,
                          int tile) {
   const bool raw = tile == kTileAuto && direct_stage(b);
-  if (tile == kTileAuto) tile = TV_64x4;
+  if (tile == kTileAuto) tile = tiled_shape(b.n[0], b.n[1], false);
   if (raw && tile == TV_64x4)
     update_as<64, 4, true>(s, b, Win, F, Wbase, Wout, ss, false, cfl);
   else if (raw)

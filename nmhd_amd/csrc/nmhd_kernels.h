@@ -2,6 +2,8 @@
 // kernel translation units.  Not installed; the public ABI is include/nmhd.h.
 #pragma once
 
+#include <functional>
+
 #include "nmhd_device.h"
 
 namespace nmhd {
@@ -288,6 +290,13 @@ struct AdjStageArgs {
 };
 void launch_adj_stage(hipStream_t s, const Box &b, const AdjStageArgs &A);
 
+// kernels_tiny.hip (a whole stage of a very small box in one launch; it may
+// not both open a step and reduce its CFL minimum, as the record is emptied
+// by the launch that opens it)
+bool tiny_stage(const Box &b);
+void launch_tiny_stage(hipStream_t s, const Box &b, FieldPtrs Win, FieldPtrs Wbase, FieldPtrs Wout,
+                       const StageStep &ss, const OpenStep &open, bool cfl);
+
 // kernels_direct.hip (the stage of a small box: a thread per face, a thread
 // per cell; all 21 flux arrays are used)
 bool direct_stage(const Box &b);
@@ -295,7 +304,12 @@ void launch_direct_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet
                          const StageStep &ss, const OpenStep &open);
 
 // kernels_tiled.hip
+// Planes per march of the face or update kernel: the chunk of the least
+// estimated time, groups_at(zc) the workgroups of the launch with chunks of zc.
+int march_chunk(bool faces, int nz, const std::function<long(int)> &groups_at);
 int tiled_zchunk(const Box &b, int tx, int ty, bool faces);
+// Tile shape (TileVariant) of the face or update kernel for a box.
+int tiled_shape(int nx, int ny, bool faces);
 // tile: TileVariant of the z-marching tiles, or kTileAuto (both launches of a
 // stage then take the same route, direct_stage)
 // open: the bookkeeping of the step that this launch begins (in == NULL: none)

@@ -1,5 +1,6 @@
-"""The small-box route (one thread per face) against the marching tiles, bit
-for bit, and the rules that choose between them (GPU)."""
+"""The small-box routes (a fused stage of 4x4x4 tiles; one thread per face)
+against the marching tiles, bit for bit, on both sides of every rule that
+chooses between them (GPU)."""
 import numpy as np
 import pytest
 
@@ -38,11 +39,13 @@ def run(cfg, W, tiles):
     return dt, t, out
 
 
-# one cell, one row, one column, one plane; sizes around a wave, a workgroup
-# and a tile; the last boxes below and above the limit of 400,000 cells
+# one cell, one row, one column, one plane; remainders of the 4x4x4 tiles; the
+# largest fused box (1024 tiles) and one more, sizes around a wave and a
+# workgroup; the last below and above the limit of 400,000 cells
 SIZES = [(1, 1, 1), (3, 1, 1), (1, 1, 5), (64, 1, 1), (1, 67, 1), (1, 1, 70), (17, 15, 1),
-         (2, 2, 2), (7, 9, 4), (33, 9, 3), (16, 16, 1), (31, 33, 35), (64, 72, 33),
-         (100, 80, 50), (101, 80, 50)]
+         (2, 2, 2), (4, 4, 4), (5, 6, 7), (7, 9, 4), (33, 9, 3), (16, 16, 1), (31, 33, 35),
+         (64, 32, 32), (61, 30, 33), (65, 32, 32), (4100, 1, 1), (64, 72, 33), (100, 80, 50),
+         (101, 80, 50)]
 
 
 @pytest.mark.parametrize("n", SIZES)
