@@ -138,6 +138,7 @@ struct nmhd_ctx {
   nmhd_geometry geo;
   int device = 0;
   hipStream_t stream = nullptr;
+  float *arrays = nullptr;  // the 24 state and 21 flux arrays
   float *state[3][8] = {};
   int cur = 0;
   float *flux[3][7] = {};
@@ -341,12 +342,7 @@ int sync_and_check(nmhd_ctx *c) {
 }
 
 void free_all(nmhd_ctx *c) {
-  for (auto &row : c->state)
-    for (auto &p : row)
-      if (p) (void)hipFree(p), p = nullptr;
-  for (auto &row : c->flux)
-    for (auto &p : row)
-      if (p) (void)hipFree(p), p = nullptr;
+  if (c->arrays) (void)hipFree(c->arrays), c->arrays = nullptr;
   for (auto &p : c->scratch8)
     if (p) (void)hipFree(p), p = nullptr;
   if (c->rec) (void)hipFree(c->rec), c->rec = nullptr;
@@ -386,19 +382,19 @@ int nmhd_create(const nmhd_desc *desc, nmhd_ctx **out) {
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess)
     return bail(NMHD_EHIP, "hipStreamCreate failed");
   const size_t bytes = sizeof(float) * (size_t)c->box.ncell;
+  const size_t stride = array_stride(c->box.ncell);
+  if (hipMalloc(&c->arrays, 45 * stride * sizeof(float)) != hipSuccess)
+    return bail(NMHD_ENOMEM, "state allocation failed");
+  float *next = c->arrays;
   for (auto &row : c->state)
-    for (auto &p : row)
-      if (hipMalloc(&p, bytes) != hipSuccess) return bail(NMHD_ENOMEM, "state allocation failed");
+    for (auto &p : row) p = next, next += stride;
   for (auto &row : c->flux)
-    for (auto &p : row)
-      if (hipMalloc(&p, bytes) != hipSuccess) return bail(NMHD_ENOMEM, "flux allocation failed");
+    for (auto &p : row) p = next, next += stride;
   if (hipMalloc(&c->rec, 3 * sizeof(StepRec)) != hipSuccess ||
       hipHostMalloc(&c->host, sizeof(StepRec)) != hipSuccess)
     return bail(NMHD_ENOMEM, "step record allocation failed");
-  for (int k = 0; k < 3; ++k)
-    for (int f = 0; f < 8; ++f)
-      if (hipMemsetAsync(c->state[k][f], 0, bytes, c->stream) != hipSuccess)
-        return bail(NMHD_EHIP, "state clear failed");
+  if (hipMemsetAsync(c->arrays, 0, 24 * stride * sizeof(float), c->stream) != hipSuccess)
+    return bail(NMHD_EHIP, "state clear failed");
   if (hipMemsetAsync(c->rec, 0, 3 * sizeof(StepRec), c->stream) != hipSuccess ||
       hipStreamSynchronize(c->stream) != hipSuccess)
     return bail(NMHD_EHIP, "step record init failed");

@@ -44,12 +44,12 @@ struct nmhd_adj {
   nmhd_geometry geo;
   hipStream_t own = nullptr;
   hipStream_t stream = nullptr;
-  float *wstar[8] = {};   // recomputed stage-1 state
-  float *wnext[8] = {};   // recomputed stage-2 state
-  float *lstar[8] = {};   // dL/dW*
-  float *flux[21] = {};   // face fluxes of the forward stages
+  float *arrays = nullptr;  // the arrays below
+  float *wstar[8] = {};     // recomputed stage-1 state
+  float *wnext[8] = {};     // recomputed stage-2 state
+  float *lstar[8] = {};     // dL/dW*
+  float *flux[21] = {};     // face fluxes of the forward stages
   float *work[kWork] = {};
-  float *scratch_out[8] = {};
   StepRec *rec = nullptr;  // of nmhd_adj_cfl_dt
   std::string err;
 };
@@ -108,14 +108,7 @@ AdjStageArgs stage_args(nmhd_adj *a) {
 }
 
 void free_adj(nmhd_adj *a) {
-  float **groups[] = {a->wstar, a->wnext, a->lstar, a->scratch_out};
-  for (float **g : groups)
-    for (int i = 0; i < 8; ++i)
-      if (g[i]) (void)hipFree(g[i]), g[i] = nullptr;
-  for (auto &p : a->flux)
-    if (p) (void)hipFree(p), p = nullptr;
-  for (auto &p : a->work)
-    if (p) (void)hipFree(p), p = nullptr;
+  if (a->arrays) (void)hipFree(a->arrays), a->arrays = nullptr;
   if (a->rec) (void)hipFree(a->rec), a->rec = nullptr;
   if (a->own) (void)hipStreamDestroy(a->own), a->own = nullptr;
 }
@@ -159,15 +152,18 @@ int nmhd_adj_create(const nmhd_desc *desc, nmhd_adj **out) {
   if (hipStreamCreateWithFlags(&a->own, hipStreamNonBlocking) != hipSuccess)
     return bail(NMHD_EHIP, "hipStreamCreate failed");
   a->stream = a->own;
-  const size_t bytes = sizeof(float) * (size_t)a->box.ncell;
-  float **groups[] = {a->wstar, a->wnext, a->lstar, a->scratch_out};
-  for (float **g : groups)
-    for (int i = 0; i < 8; ++i)
-      if (hipMalloc(&g[i], bytes) != hipSuccess) return bail(NMHD_ENOMEM, "allocation failed");
-  for (auto &p : a->flux)
-    if (hipMalloc(&p, bytes) != hipSuccess) return bail(NMHD_ENOMEM, "allocation failed");
-  for (auto &p : a->work)
-    if (hipMalloc(&p, bytes) != hipSuccess) return bail(NMHD_ENOMEM, "allocation failed");
+  const size_t stride = array_stride(a->box.ncell);
+  if (hipMalloc(&a->arrays, (3 * 8 + 21 + kWork) * stride * sizeof(float)) != hipSuccess)
+    return bail(NMHD_ENOMEM, "allocation failed");
+  float *next = a->arrays;
+  auto take = [&](float **p, int n) {
+    for (int i = 0; i < n; ++i) p[i] = next, next += stride;
+  };
+  take(a->wstar, 8);
+  take(a->wnext, 8);
+  take(a->lstar, 8);
+  take(a->flux, 21);
+  take(a->work, kWork);
   if (hipMalloc(&a->rec, sizeof(StepRec)) != hipSuccess)
     return bail(NMHD_ENOMEM, "allocation failed");
   if (hipMemset(a->rec, 0, sizeof(StepRec)) != hipSuccess)

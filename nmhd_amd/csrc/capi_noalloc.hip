@@ -6,9 +6,10 @@
 // allocated by nmhd_adj_create.  Every GPU the library runs on holds its
 // own copy of the array until the process ends.
 //
-// Layout of the array (floats): 19 arrays of `stride` floats each (ncell rounded up to a
-// multiple of 64, so that every array starts 256-byte aligned): W* (8),
-// the hydro divergence (5), the six face B fluxes (6).
+// Layout: arrays of array_stride(ncell) floats each, so that every array
+// starts 256-byte aligned: W* (8), then the face -> update hand-off: the hydro
+// divergence (5) and the six face B fluxes (6), or for a box on the direct
+// route all 21 face fluxes.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -19,11 +20,11 @@
 using namespace nmhd;
 
 namespace {
-constexpr size_t kAlignFloats = 64;   // 256 bytes
 constexpr size_t kArrays = 8 + 11;    // W* + the face -> update hand-off
 constexpr size_t kMaxCells = NMHD_NOALLOC_MAX_CELLS;
-constexpr size_t kScratchFloats = kArrays * kMaxCells;
-static_assert(kMaxCells % kAlignFloats == 0, "array strides stay within the scratch");
+constexpr size_t kScratchFloats = kArrays * (kMaxCells + 64);  // strides included
+static_assert(kMaxCells % 64 == 0, "a box's stride is at most kMaxCells + 64 floats");
+static_assert((8 + 21) * (kDirectCells + 128) <= kScratchFloats, "all fluxes of a direct box fit");
 }  // namespace
 
 // The scratch.  In host code `scratch` names a host-side stand-in, not the
@@ -94,7 +95,7 @@ int nmhd_adj_forward_noalloc(const nmhd_desc *desc, const float *const w_in[8], 
   const int rc = scratch_on_current_device(&arr);
   if (rc != NMHD_OK) return rc;
 
-  const size_t stride = ((size_t)b.ncell + kAlignFloats - 1) / kAlignFloats * kAlignFloats;
+  const size_t stride = array_stride(b.ncell);
   auto slot = [&](size_t k) { return arr + k * stride; };
   FieldPtrs Win, Wstar, Wout;
   for (int f = 0; f < 8; ++f) {

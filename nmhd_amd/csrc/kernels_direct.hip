@@ -142,11 +142,11 @@ __global__ void __launch_bounds__(kThreads)
 
 }  // namespace direct
 
-// Up to 400,000 cells.  Step times, direct faces against the march: 32^3 26.0
+// Up to 400,000 cells (kDirectCells).  Step times, direct faces against the march: 32^3 26.0
 // / 33.7 us, 64^3 48.5 / 54.3, 64x72x64 68.4 / 77.8, 80^3 102.3 / 97.8, 96^3
 // 139.7 / 135.2, 128^3 304 / 250: the chip is then full of tiles, and the
 // update reads 10 arrays more.
-bool direct_stage(const Box &b) { return b.ncell <= 400000; }
+bool direct_stage(const Box &b) { return b.ncell <= kDirectCells; }
 
 void launch_direct_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F,
                          const StageStep &ss, const OpenStep &open) {
