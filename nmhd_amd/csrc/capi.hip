@@ -262,14 +262,20 @@ void enqueue_step(nmhd_ctx *c, float goal) {
   StepRec *const in = c->rec + c->r, *const out = c->rec + (c->r ^ 1);
   const bool reset = c->reset;
   if (full_cfl) timed(c, S_BEGIN, [&] { launch_clear_cfl(s, in, reset); });
-  if (b.m[1] > 0) timed(c, S_GHOST_Y, [&] { launch_ghost_y(s, b, fields(c, A), in, reset); });
+  // the carried CFL minimum lacks the ghost cells: the fill reduces them as it
+  // writes them, unless a Z fill writes some again
+  const bool fill_cfl = !full_cfl && b.m[1] > 0 && b.m[2] == 0;
+  if (fill_cfl)
+    timed(c, S_GHOST_Y, [&] { launch_ghost_y_cfl(s, b, fields(c, A), in, reset); });
+  else if (b.m[1] > 0)
+    timed(c, S_GHOST_Y, [&] { launch_ghost_y(s, b, fields(c, A), in, reset); });
   if (b.m[2] > 0) timed(c, S_GHOST_Z, [&] { launch_ghost_z(s, b, fields(c, A), in, reset); });
   if (full_cfl)
     timed(c, S_CFL, [&] { launch_cfl(s, b, fields(c, A), goal, in, reset); });
-  else if (ghosts)
+  else if (ghosts && !fill_cfl)
     timed(c, S_CFL_GHOSTS, [&] { launch_cfl_ghosts(s, b, fields(c, A), in, reset); });
   const OpenStep open{in, out, goal, reset};
-  if (!tiled) timed(c, S_DT, [&] { launch_open_step(s, open); });
+  if (!tiled) timed(c, S_DT, [&] { launch_open_step(s, b, open); });
   const FluxSet F = fluxes(c);
   const int slots[3] = {S_FLUX_X, S_FLUX_Y, S_FLUX_Z};
   // one RK stage: fluxes of W[in], update of the conserved base W[base] into W[out]
@@ -480,7 +486,7 @@ int nmhd_get_state_device(nmhd_ctx *ctx, float *const f[8]) {
 
 int nmhd_set_time(nmhd_ctx *ctx, double t, int generation) {
   if (!ctx) return NMHD_EINVAL;
-  launch_set_time(ctx->stream, ctx->rec + ctx->r, t, generation);
+  launch_set_time(ctx->stream, ctx->box, ctx->rec + ctx->r, t, generation);
   HIPCHECK(ctx, hipGetLastError());
   ctx->cfl_valid = false;
   ctx->reset = false;

@@ -13,75 +13,82 @@
 
 namespace nmhd {
 
-// relative_displacement (INL:288-295) with D0 = 0 and
-// relvel = -q*Omega*kLocalExtentY (application/kepler_disk_demo/
-// mhd_solver.curb:46-52), in FP64 as the reference evaluates it.
-__host__ __device__ inline void displacement(const Box &b, double t, float *normalized,
-                                             int *n, float *minor) {
-  const float relvel = -b.qshear * b.omega * b.local_ext[1];
-  const double d0 = 0.0 + t * (double)relvel;
-  const int fold = (int)floor(d0 / (double)b.ext[0]);
-  const double d1 = d0 - (double)((float)fold * b.ext[0]);
-  *normalized = (float)d1;
-  *n = (int)floor(d1 / (double)b.d[0]);
-  *minor = (float)(d1 / (double)b.d[0] - *n);
+// Value of field f that the fill gives cell (x, ghost row j of the lower or
+// upper slab, z); not the first upper ghost By face, which it keeps.
+template <bool Upper>
+__device__ __forceinline__ float ghost_y_value(const Box &b, const FieldPtrs &W,
+                                               const GhostShear &g, int f, int x, int j, int z) {
+#pragma clang fp contract(off)
+  const int nx = b.n[0], M = b.m[1];
+  int i = x;
+  if (b.shear_y) {
+    i = Upper ? x - g.n - 1 : x + g.n;  // |n| < nx
+    i = i < 0 ? i + nx : i;
+    i = i < 0 ? i + nx : (i >= nx ? i - nx : i);
+  }
+  const int row = Upper ? M + j : b.n[1] - 2 * M + j;
+  float v = W.f[f][addr(b, i, row, z)];
+  if (b.shear_y) {
+    // the second source cell (the reference's val_inc1 / val_dec1)
+    const float v1 = b.fix_interp ? W.f[f][addr(b, i + 1 < nx ? i + 1 : 0, row, z)] : v;
+    // (1-d)*v + d*v, exactly as the gather kernel writes it (INL:108-110);
+    // with fix_interp (1-d)*v0 + d*v1 and d*v0 + (1-d)*v1
+    v = Upper ? g.part * v + (1.0f - g.part) * v1 : (1.0f - g.part) * v + g.part * v1;
+    if (f == 1) {
+      const float relvel = -b.qshear * b.omega * b.local_ext[1];
+      v = Upper ? v + relvel : v - relvel;
+    }
+  }
+  return v;
 }
 
-// One (x, row, z) of the M-row Y ghost slab, a in [0, nx * M * nz): the
-// lower ghost row j takes the top interior row j shifted by +n along X, the
-// upper ghost row takes the bottom interior row shifted by -n-1, v_X offset
-// by -/+ relvel; the first upper ghost By face (the outer radial face) is
-// kept.  With fix_interp the shifted values are interpolated between the
-// cells at +n and +n+1 (-n-1 and -n) with the gather kernel's weights
-// (INL:100-110).  t: the box's committed time.
-__device__ __forceinline__ void ghost_y_cell(const Box &b, const FieldPtrs &W, double t, long a) {
-#pragma clang fp contract(off)
-  const int nx = b.n[0], ny = b.n[1], M = b.m[1];
-  // 32-bit index arithmetic: the slab holds fewer than 2^31 cells
-  const unsigned u = (unsigned)a, row = u / (unsigned)nx;
-  const int sx = (int)(u - row * (unsigned)nx);
-  const int sz = (int)(row / (unsigned)M);
-  const int sy = (int)(row - (unsigned)sz * (unsigned)M);
-  int n = 0;
-  float dr = 0.0f, nd, relvel = 0.0f;
-  int ix = sx, dx = sx, ix1 = sx, dx1 = sx;
-  if (b.shear_y) {
-    displacement(b, t, &nd, &n, &dr);
-    relvel = -b.qshear * b.omega * b.local_ext[1];
-    n %= nx;  // same shift, and no int overflow in sx + n for huge t
-    ix = ((sx + n) % nx + nx) % nx;
-    dx = ((sx - n - 1) % nx + nx) % nx;
-    ix1 = ix + 1 < nx ? ix + 1 : 0;
-    dx1 = dx + 1 < nx ? dx + 1 : 0;
+// The fill of cell (x, j, z) of the lower or upper M-row slab.  The first
+// upper ghost By face (the outer radial face) is kept.  Cfl: returns the
+// cell's CFL time, its upper faces formed from the fill's sources (a
+// neighbour's may not be written yet); else +inf.
+template <bool Upper, bool Cfl>
+__device__ __forceinline__ float ghost_y_fill(const Box &b, const FieldPtrs &W, const GhostShear &g,
+                                              int x, int j, int z) {
+  const int nx = b.n[0], ny = b.n[1], nz = b.n[2], M = b.m[1];
+  const long a = addr(b, x, Upper ? ny - M + j : j, z);
+  const bool kept = Upper && j == 0;
+  float v[8];
+  for (int f = 0; f < 8; ++f)
+    v[f] = f == 6 && kept ? W.f[6][a] : ghost_y_value<Upper>(b, W, g, f, x, j, z);
+  float t = __uint_as_float(0x7f800000u);
+  if (Cfl) {
+    const int x1 = x + 1 < nx ? x + 1 : 0, z1 = z + 1 < nz ? z + 1 : 0;
+    float byh;  // the next row: in the slab, or the interior's first, or (wrapped) the array's
+    if (j + 1 < M)
+      byh = ghost_y_value<Upper>(b, W, g, 6, x, j + 1, z);
+    else
+      byh = Upper ? ghost_y_value<false>(b, W, g, 6, x, 0, z) : W.f[6][addr(b, x, M, z)];
+    const float w[5] = {v[0], v[1], v[2], v[3], v[4]}, lo[3] = {v[5], v[6], v[7]};
+    const float hi[3] = {ghost_y_value<Upper>(b, W, g, 5, x1, j, z), byh,
+                         ghost_y_value<Upper>(b, W, g, 7, x, j, z1)};
+    t = cfl_time(b, w, lo, hi);
   }
-  const long src_inc = addr(b, ix, ny - 2 * M + sy, sz);
-  const long src_dec = addr(b, dx, M + sy, sz);
-  const long src_inc1 = addr(b, ix1, ny - 2 * M + sy, sz);
-  const long src_dec1 = addr(b, dx1, M + sy, sz);
-  const long dst_inc = addr(b, sx, sy, sz);
-  const long dst_dec = addr(b, sx, ny - M + sy, sz);
-  const bool interp = b.shear_y && b.fix_interp;
-  for (int f = 0; f < 8; ++f) {
-    float vi = W.f[f][src_inc];
-    float vd = W.f[f][src_dec];
-    // the second source cells (the reference's val_inc1 / val_dec1)
-    const float vi1 = interp ? W.f[f][src_inc1] : vi;
-    const float vd1 = interp ? W.f[f][src_dec1] : vd;
-    if (b.shear_y) {
-      // (1-d)*v + d*v, exactly as the gather kernel writes it (INL:108-110);
-      // with fix_interp (1-d)*v0 + d*v1 and d*v0 + (1-d)*v1
-      float bi = (1.0f - dr) * vi + dr * vi1;
-      float bd = dr * vd + (1.0f - dr) * vd1;
-      if (f == 1) {
-        bi = bi - relvel;
-        bd = bd + relvel;
-      }
-      vi = bi;
-      vd = bd;
-    }
-    W.f[f][dst_inc] = vi;
-    if (!(f == 6 && sy == 0)) W.f[f][dst_dec] = vd;
-  }
+  for (int f = 0; f < 8; ++f)
+    if (!(f == 6 && kept)) W.f[f][a] = v[f];
+  return t;
+}
+
+// The Y ghost cells of a box, i in [0, nx * 2M * nz): lower slab, then upper.
+__device__ __forceinline__ long ghost_y_count(const Box &b) {
+  return (long)b.n[0] * 2 * b.m[1] * b.n[2];
+}
+template <bool Cfl>
+__device__ __forceinline__ float ghost_y_cell(const Box &b, const FieldPtrs &W,
+                                              const GhostShear &g, long i) {
+  // 32-bit index arithmetic: a box holds fewer than 2^31 cells
+  const unsigned slab = (unsigned)(b.n[0] * b.m[1]) * (unsigned)b.n[2];
+  const bool upper = (unsigned)i >= slab;
+  const unsigned u = (unsigned)i - (upper ? slab : 0u), line = u / (unsigned)b.n[0];
+  const int x = (int)(u - line * (unsigned)b.n[0]);
+  const int z = (int)(line / (unsigned)b.m[1]);
+  const int j = (int)(line - (unsigned)z * (unsigned)b.m[1]);
+  return upper ? ghost_y_fill<true, Cfl>(b, W, g, x, j, z)
+               : ghost_y_fill<false, Cfl>(b, W, g, x, j, z);
 }
 
 // Z ghost planes, a in [0, nx * ny * M): [0, M) <- [nz-2M, nz-M),

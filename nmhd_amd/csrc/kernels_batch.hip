@@ -193,11 +193,11 @@ __global__ void k_batch_ghost_y(const BatchBox *boxes, float *state, const StepS
   const BatchBox bb = boxes[box];
   if (bb.b.m[1] == 0 || st[box].finished) return;
   const FieldPtrs W = box_fields(state, bb);
-  const long unit = (long)bb.b.n[0] * bb.b.m[1] * bb.b.n[2];
-  const double t = st[box].t;
+  const long unit = ghost_y_count(bb.b);
+  const GhostShear g = ghost_shear(bb.b, st[box].t);
   for (long a = (long)blockIdx.x * blockDim.x + threadIdx.x; a < unit;
        a += (long)gridDim.x * blockDim.x)
-    ghost_y_cell(bb.b, W, t, a);
+    (void)ghost_y_cell<false>(bb.b, W, g, a);
 }
 
 __global__ void k_batch_ghost_z(const BatchBox *boxes, float *state, const StepState *st) {

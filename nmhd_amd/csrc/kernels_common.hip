@@ -16,7 +16,7 @@ namespace nmhd {
 
 // Bookkeeping as a launch of its own, for the paths whose first kernel does
 // not do it.
-__global__ void k_open_step(OpenStep o) { (void)open_step(o, true); }
+__global__ void k_open_step(Box b, OpenStep o) { (void)open_step(b, o, true); }
 
 __global__ void k_clear_cfl(StepRec *rec, int reset) {
   if (!run_ended(rec->s, reset)) rec->cfl[threadIdx.x * kCflStride] = 0x7f800000u;
@@ -24,15 +24,6 @@ __global__ void k_clear_cfl(StepRec *rec, int reset) {
 
 void host_displacement(const Box &b, double t, float *normalized, int *n, float *minor) {
   displacement(b, t, normalized, n, minor);
-}
-
-// Y ghost rows (ghost_y_cell), one thread per (x, row, z) of the slab.
-__global__ void k_ghost_y(Box b, FieldPtrs W, const StepRec *rec, int reset) {
-  if (run_ended(rec->s, reset)) return;
-  const long unit = (long)b.n[0] * b.m[1] * b.n[2];
-  const long a = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= unit) return;
-  ghost_y_cell(b, W, committed_time(rec->s), a);
 }
 
 // Z ghost planes (ghost_z_cell).
@@ -59,6 +50,22 @@ __device__ __forceinline__ void cfl_block_fold(float t, StepRec *rec) {
     for (int i = 1; i < (int)(blockDim.x >> 6); ++i) m = fminf(m, red[i]);
     atomicMin(cfl_slot(rec, blockIdx.x), __float_as_uint(m));
   }
+}
+
+// Y ghost rows (ghost_y_cell), one thread per ghost cell; with
+// Cfl also the CFL minimum of the rows, from the values just formed.  Bound by
+// latency: as two launches, each thread a lower and an upper cell and the FP64
+// displacement before its loads, a shearing step took 68.4 us at 64^3 and 33.0
+// at 32^3; in one, a thread per cell and the displacement read from the record
+// (the launch that opens a step computes the next fill's), 63.5 and 28.9.
+template <bool Cfl>
+__global__ void __launch_bounds__(256) k_ghost_y(Box b, FieldPtrs W, StepRec *rec, int reset) {
+  if (run_ended(rec->s, reset)) return;
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const GhostShear g = rec->shear;
+  float t = __uint_as_float(0x7f800000u);
+  if (i < ghost_y_count(b)) t = ghost_y_cell<Cfl>(b, W, g, i);
+  if (Cfl) cfl_block_fold(t, rec);
 }
 
 // Grid-stride over the cells with a capped grid.
@@ -133,7 +140,7 @@ __global__ void __launch_bounds__(256) k_copy_fields(long n, FieldPtrs src, Fiel
   for (long i = done + i0; i < n; i += step) d[i] = a[i];
 }
 
-__global__ void k_set_time(StepRec *rec, double t, int generation) {
+__global__ void k_set_time(Box b, StepRec *rec, double t, int generation) {
   rec->cfl[threadIdx.x * kCflStride] = 0x7f800000u;
   if (threadIdx.x != 0) return;
   StepState s = {};
@@ -141,6 +148,7 @@ __global__ void k_set_time(StepRec *rec, double t, int generation) {
   s.generation = generation;
   s.cfl_bits = s.cfl_next_bits = 0x7f800000u;
   rec->s = s;
+  rec->shear = ghost_shear(b, t);
 }
 
 // Diagnostic entry points run on their own step record: current time of the
@@ -154,6 +162,7 @@ __global__ void k_diag_prepare(StepRec *diag, const StepRec *rec, float h) {
   d.active = 1;
   d.cfl_bits = d.cfl_next_bits = 0x7f800000u;
   diag->s = d;
+  diag->shear = rec->shear;
 }
 
 // ------------------------------------------------------------- launchers
@@ -161,8 +170,8 @@ __global__ void k_diag_prepare(StepRec *diag, const StepRec *rec, float h) {
 void launch_clear_cfl(hipStream_t s, StepRec *rec, bool reset) {
   hipLaunchKernelGGL(k_clear_cfl, dim3(1), dim3(kCflSlots), 0, s, rec, (int)reset);
 }
-void launch_open_step(hipStream_t s, const OpenStep &open) {
-  hipLaunchKernelGGL(k_open_step, dim3(1), dim3(64), 0, s, open);
+void launch_open_step(hipStream_t s, const Box &b, const OpenStep &open) {
+  hipLaunchKernelGGL(k_open_step, dim3(1), dim3(64), 0, s, b, open);
 }
 // Blocks of a reduction kernel: one per 1024 cells, at most 512.
 unsigned reduce_grid(long n) {
@@ -183,8 +192,14 @@ void launch_cfl_ghosts(hipStream_t s, const Box &b, FieldPtrs W, StepRec *rec, b
   }
 }
 void launch_ghost_y(hipStream_t s, const Box &b, FieldPtrs W, const StepRec *rec, bool reset) {
-  const long unit = (long)b.n[0] * b.m[1] * b.n[2];
-  hipLaunchKernelGGL(k_ghost_y, dim3(grid_for(unit)), dim3(kBlock), 0, s, b, W, rec, (int)reset);
+  const long unit = (long)b.n[0] * 2 * b.m[1] * b.n[2];
+  hipLaunchKernelGGL(k_ghost_y<false>, dim3(grid_for(unit)), dim3(kBlock), 0, s, b, W,
+                     const_cast<StepRec *>(rec), (int)reset);
+}
+void launch_ghost_y_cfl(hipStream_t s, const Box &b, FieldPtrs W, StepRec *rec, bool reset) {
+  const long unit = (long)b.n[0] * 2 * b.m[1] * b.n[2];
+  hipLaunchKernelGGL(k_ghost_y<true>, dim3(grid_for(unit)), dim3(kBlock), 0, s, b, W, rec,
+                     (int)reset);
 }
 void launch_ghost_z(hipStream_t s, const Box &b, FieldPtrs W, const StepRec *rec, bool reset) {
   const long unit = (long)b.n[0] * b.n[1] * b.m[2];
@@ -211,8 +226,8 @@ void launch_copy_fields(hipStream_t s, long ncell, const FieldPtrs &src, const F
   else
     hipLaunchKernelGGL(k_copy_fields<false>, grid, dim3(kBlock), 0, s, ncell, src, dst);
 }
-void launch_set_time(hipStream_t s, StepRec *rec, double t, int generation) {
-  hipLaunchKernelGGL(k_set_time, dim3(1), dim3(kCflSlots), 0, s, rec, t, generation);
+void launch_set_time(hipStream_t s, const Box &b, StepRec *rec, double t, int generation) {
+  hipLaunchKernelGGL(k_set_time, dim3(1), dim3(kCflSlots), 0, s, b, rec, t, generation);
 }
 void launch_hlld_batch(hipStream_t s, long n, float gamma, bool strict, FluxIn in,
                        FluxOut out) {

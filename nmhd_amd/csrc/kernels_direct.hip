@@ -76,7 +76,7 @@ __device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const
     // only the first wave looks
     const bool src = D != 2 && b.source == 1;
     if (threadIdx.x < 64 && (src || blockIdx.x == 0)) {
-      const StepState s = open_step(open, blockIdx.x == 0);
+      const StepState s = open_step(b, open, blockIdx.x == 0);
       if (threadIdx.x == 0) *hs = tiled::opened_size(s, ss.hsel);
     }
     if (src) {

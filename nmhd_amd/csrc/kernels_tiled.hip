@@ -23,7 +23,7 @@ template <int TX, int TY, int Recon>
 __global__ void __launch_bounds__(kTileThreads, (FacesShape<TX, TY>::kWavesPerSimd))
     k_faces(Box b, FieldPtrs W, FluxSet F, StageStep ss, OpenStep open, int zc, int gx, int gy) {
   float h;
-  if (!stage_begin(ss, open, h)) return;
+  if (!stage_begin(b, ss, open, h)) return;
   __shared__ float lds[FacesShape<TX, TY>::kLds];
   const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
   const int x0 = (lb % gx) * TX, y0 = ((lb / gx) % gy) * TY, z0 = (lb / gx / gy) * zc;
@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_update_march(Box b, FieldPt
   const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
   const int x0 = (lb % gx) * TX, y0 = ((lb / gx) % gy) * TY, z0 = (lb / gx / gy) * zc;
   float h;
-  if (!stage_begin(ss, OpenStep{}, h)) {
+  if (!stage_begin(b, ss, OpenStep{}, h)) {
     // a step enqueued after the run reached its goal: the last stage's
     // output carries the step's base state through the buffer rotation
     if (Cfl && !PaceOnly) {

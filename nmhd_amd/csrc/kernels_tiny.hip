@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(kThreads, 4)
   }
   if (tid < 64) {
     float h;
-    const bool active = tiled::stage_begin(ss, open, h);
+    const bool active = tiled::stage_begin(b, ss, open, h);
     if (tid == 0) {
       S.h = h;
       S.active = active;

@@ -27,6 +27,40 @@ struct FluxSet {
 // one given by value (StageStep::h).
 enum HSel { H_HALF = 0, H_FULL = 1, H_DIAG = 2, H_FIXED = 3 };
 
+// relative_displacement (INL:288-295) with D0 = 0 and
+// relvel = -q*Omega*kLocalExtentY (application/kepler_disk_demo/
+// mhd_solver.curb:46-52), in FP64 as the reference evaluates it.
+__host__ __device__ inline void displacement(const Box &b, double t, float *normalized,
+                                             int *n, float *minor) {
+  const float relvel = -b.qshear * b.omega * b.local_ext[1];
+  const double d0 = 0.0 + t * (double)relvel;
+  const int fold = (int)floor(d0 / (double)b.ext[0]);
+  const double d1 = d0 - (double)((float)fold * b.ext[0]);
+  *normalized = (float)d1;
+  *n = (int)floor(d1 / (double)b.d[0]);
+  *minor = (float)(d1 / (double)b.d[0] - *n);
+}
+
+// The shear of a Y ghost fill: lower ghost row j takes the top interior row j
+// shifted by +n along X, the upper ghost row the bottom interior row shifted
+// by -n-1, v_X offset by -/+ relvel.  With fix_interp the shifted values are
+// interpolated between the cells at +n and +n+1 (-n-1 and -n) with the gather
+// kernel's weights (INL:100-110): part is the fractional displacement.
+struct GhostShear {
+  int n;  // |n| < nx
+  float part;
+};
+// t: the box's committed time
+__device__ __forceinline__ GhostShear ghost_shear(const Box &b, double t) {
+  GhostShear g = {0, 0.0f};
+  if (b.shear_y) {
+    float nd;
+    displacement(b, t, &nd, &g.n, &g.part);
+    g.n %= b.n[0];  // same shift, and no int overflow in x + n for huge t
+  }
+  return g;
+}
+
 // The step record of a context with the CFL minimum of the state the step
 // produces, spread over slots a cache line apart: the atomics of a few
 // hundred workgroups on one word serialise (about 11 ns each, 6 us at 64^3),
@@ -34,6 +68,7 @@ enum HSel { H_HALF = 0, H_FULL = 1, H_DIAG = 2, H_FIXED = 3 };
 constexpr int kCflSlots = 64, kCflStride = 32;
 struct alignas(128) StepRec {
   StepState s;
+  GhostShear shear;  // of the ghost fill that follows the step
   alignas(128) unsigned cfl[kCflSlots * kCflStride];  // float bits, +inf when empty
 };
 __device__ __forceinline__ unsigned *cfl_slot(StepRec *r, int block) {
@@ -137,7 +172,7 @@ __device__ __forceinline__ float wave_min64(float v) {
 
 // OpenStep by a full wave; every wave of the launch gets the step in flight,
 // the wave with `write` set records it.
-__device__ __forceinline__ StepState open_step(const OpenStep &o, bool write) {
+__device__ __forceinline__ StepState open_step(const Box &b, const OpenStep &o, bool write) {
   const int slot = (threadIdx.x & 63) * kCflStride;
   const unsigned mine = o.in->cfl[slot];
   StepState s = o.in->s;
@@ -148,7 +183,11 @@ __device__ __forceinline__ StepState open_step(const OpenStep &o, bool write) {
   step_dt(s, o.goal);
   if (write) {
     o.out->cfl[slot] = ended ? mine : 0x7f800000u;
-    if ((threadIdx.x & 63) == 0) o.out->s = s;
+    const GhostShear g = ghost_shear(b, committed_time(s));
+    if ((threadIdx.x & 63) == 0) {
+      o.out->s = s;
+      o.out->shear = g;
+    }
   }
   return s;
 }
@@ -156,19 +195,26 @@ __device__ __forceinline__ StepState open_step(const OpenStep &o, bool write) {
 // CFL time of one cell (cfl_condition_inner, INL:714-720):
 // min_d C*d_d/|v_d + sqrt((gamma p + b2)/rho)|, b2 = sum_d max(B_lo^2, B_hi^2)
 // (|v_d| + sqrt(..) with fix_cfl), without FMA contraction so that every CFL
-// pass rounds the same way.
+// pass rounds the same way.  w: rho, v, p; lo, hi: the six face fields.
+__device__ __forceinline__ float cfl_time(const Box &b, const float (&w)[5], const float (&lo)[3],
+                                          const float (&hi)[3]) {
+#pragma clang fp contract(off)
+  const float b2 = fmaxf(lo[0] * lo[0], hi[0] * hi[0]) + fmaxf(lo[1] * lo[1], hi[1] * hi[1]) +
+                   fmaxf(lo[2] * lo[2], hi[2] * hi[2]);
+  const float c = sqrtf((b.gamma * w[4] + b2) / w[0]);
+  float t = 3.0e38f;
+  for (int d = 0; d < 3; ++d) t = fminf(t, b.cfl * b.d[d] / cfl_speed(b, w[1 + d], c));
+  return t;
+}
+
 __device__ __forceinline__ float cell_cfl(const Box &b, const FieldPtrs &W, long a, int x, int y,
                                           int z) {
-#pragma clang fp contract(off)
-  const float bxl = W.f[5][a], bxh = W.f[5][addr(b, wrap(x + 1, b.n[0]), y, z)];
-  const float byl = W.f[6][a], byh = W.f[6][addr(b, x, wrap(y + 1, b.n[1]), z)];
-  const float bzl = W.f[7][a], bzh = W.f[7][addr(b, x, y, wrap(z + 1, b.n[2]))];
-  const float b2 = fmaxf(bxl * bxl, bxh * bxh) + fmaxf(byl * byl, byh * byh) +
-                   fmaxf(bzl * bzl, bzh * bzh);
-  const float c = sqrtf((b.gamma * W.f[4][a] + b2) / W.f[0][a]);
-  float t = 3.0e38f;
-  for (int d = 0; d < 3; ++d) t = fminf(t, b.cfl * b.d[d] / cfl_speed(b, W.f[1 + d][a], c));
-  return t;
+  const float w[5] = {W.f[0][a], W.f[1][a], W.f[2][a], W.f[3][a], W.f[4][a]};
+  const float lo[3] = {W.f[5][a], W.f[6][a], W.f[7][a]};
+  const float hi[3] = {W.f[5][addr(b, wrap(x + 1, b.n[0]), y, z)],
+                       W.f[6][addr(b, x, wrap(y + 1, b.n[1]), z)],
+                       W.f[7][addr(b, x, y, wrap(z + 1, b.n[2]))]};
+  return cfl_time(b, w, lo, hi);
 }
 
 // ------------------------------------------------------- multi-box batches
@@ -212,16 +258,18 @@ constexpr int kTileTY[TV_COUNT] = {4, 8, 16};
 // empty the CFL minimum of rec before a full pass (not when the run that rec
 // ends is finished and goes on: its minimum is still wanted)
 void launch_clear_cfl(hipStream_t s, StepRec *rec, bool reset);
-void launch_open_step(hipStream_t s, const OpenStep &open);
+void launch_open_step(hipStream_t s, const Box &b, const OpenStep &open);
 // the ghost fills and CFL passes of the step that follows rec's
 void launch_cfl_ghosts(hipStream_t s, const Box &b, FieldPtrs W, StepRec *rec, bool reset);
 void launch_ghost_y(hipStream_t s, const Box &b, FieldPtrs W, const StepRec *rec, bool reset);
+// the Y fill and the CFL minimum of the rows it writes (boxes without Z ghosts)
+void launch_ghost_y_cfl(hipStream_t s, const Box &b, FieldPtrs W, StepRec *rec, bool reset);
 void launch_ghost_z(hipStream_t s, const Box &b, FieldPtrs W, const StepRec *rec, bool reset);
 void launch_cfl(hipStream_t s, const Box &b, FieldPtrs W, float goal, StepRec *rec, bool reset);
 void launch_copy_state(hipStream_t s, const Box &b, FieldPtrs src, FieldPtrs dst,
                        const StepState *st);
 void launch_copy_fields(hipStream_t s, long ncell, const FieldPtrs &src, const FieldPtrs &dst);
-void launch_set_time(hipStream_t s, StepRec *rec, double t, int generation);
+void launch_set_time(hipStream_t s, const Box &b, StepRec *rec, double t, int generation);
 void launch_hlld_batch(hipStream_t s, long n, float gamma, bool strict, FluxIn in,
                        FluxOut out);
 void launch_diag_prepare(hipStream_t s, StepRec *diag, const StepRec *rec, float h);

@@ -60,9 +60,10 @@ __device__ __forceinline__ float stage_size(const StageStep &ss) {
 
 // The stage step of a launch, opening the step first when it is the step's
 // first kernel; false: the step is not taken.
-__device__ __forceinline__ bool stage_begin(const StageStep &ss, const OpenStep &open, float &h) {
+__device__ __forceinline__ bool stage_begin(const Box &b, const StageStep &ss,
+                                            const OpenStep &open, float &h) {
   if (open.in) {
-    const StepState s = open_step(open, blockIdx.x == 0 && threadIdx.x < 64);
+    const StepState s = open_step(b, open, blockIdx.x == 0 && threadIdx.x < 64);
     h = opened_size(s, ss.hsel);
     return s.active;
   }

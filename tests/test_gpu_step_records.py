@@ -97,3 +97,27 @@ def test_device_state_transfer(gpu_ready, n, offset):
         inside[s:s + nc] = True
     assert (d[~inside] == -1.0).all()
     ctx.close()
+
+
+@pytest.mark.parametrize("n,margin", [((24, 12, 9), 4), ((1, 3, 1), 1), ((5, 2, 2), 2),
+                                      ((70, 4, 3), 4), ((33, 9, 17), 3)])
+@pytest.mark.parametrize("fixes,shear_y", [(0, 1), (7, 1), (2, 1), (1, 0)])
+def test_ghost_fill_reduces_the_cfl_minimum(gpu_ready, n, margin, fixes, shear_y):
+    """The fill adds the ghost cells' CFL times as it writes them: every dt
+    equals that of a full pass over the same state, bit for bit, with the
+    shortest CFL time in the ghost rows (their interior sources are fast
+    where the shear makes them faster still)."""
+    cfg = P.make_config(n, margin=(0, margin, 0), cfl=0.1, source=1, shear_y=shear_y)
+    cfg["fixes"] = fixes
+    W = P.shearing_box_mri(cfg, amp=0.2)
+    a, b = capi.Context(cfg), capi.Context(cfg)
+    a.set_state(W)
+    a.set_time(0.7)
+    for _ in range(4):
+        b.set_state(a.get_state())
+        b.set_time(*a.get_time())
+        dt_full, _ = b.step()  # after set_state: a full pass
+        assert a.step()[0] == dt_full
+        assert np.array_equal(a.get_state().view(np.uint32), b.get_state().view(np.uint32))
+    a.close()
+    b.close()
