@@ -8,8 +8,10 @@
 // (kernels_adjoint.hip) from the last stage to the first.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
+#include <vector>
 
 #include "capi_internal.h"
 
@@ -44,7 +46,7 @@ struct nmhd_adj {
   nmhd_geometry geo;
   hipStream_t own = nullptr;
   hipStream_t stream = nullptr;
-  float *arrays = nullptr;  // the arrays below
+  std::vector<float *> blocks;  // that hold the arrays below
   float *wstar[8] = {};     // recomputed stage-1 state
   float *wnext[8] = {};     // recomputed stage-2 state
   float *lstar[8] = {};     // dL/dW*
@@ -108,7 +110,8 @@ AdjStageArgs stage_args(nmhd_adj *a) {
 }
 
 void free_adj(nmhd_adj *a) {
-  if (a->arrays) (void)hipFree(a->arrays), a->arrays = nullptr;
+  for (float *p : a->blocks) (void)hipFree(p);
+  a->blocks.clear();
   if (a->rec) (void)hipFree(a->rec), a->rec = nullptr;
   if (a->own) (void)hipStreamDestroy(a->own), a->own = nullptr;
 }
@@ -153,21 +156,28 @@ int nmhd_adj_create(const nmhd_desc *desc, nmhd_adj **out) {
     return bail(NMHD_EHIP, "hipStreamCreate failed");
   a->stream = a->own;
   const size_t stride = array_stride(a->box.ncell);
-  if (hipMalloc(&a->arrays, (3 * 8 + 21 + kWork) * stride * sizeof(float)) != hipSuccess)
-    return bail(NMHD_ENOMEM, "allocation failed");
-  float *next = a->arrays;
+  // One block for all arrays, but pieces of under 2 MB where they come to less
+  // than 32 MB: hipMalloc keeps chunks for those (12 us a piece), while a
+  // block of 4 to 30 MB is mapped afresh each time (300 to 700 us).
+  size_t left = 3 * 8 + 21 + kWork, room = 0;
+  const size_t piece = left * stride > (8u << 20) ? left : std::max<size_t>(1, 500000 / stride);
+  float *next = nullptr;
   auto take = [&](float **p, int n) {
-    for (int i = 0; i < n; ++i) p[i] = next, next += stride;
+    for (int i = 0; i < n; ++i, --left, --room, next += stride) {
+      if (!room) {
+        room = std::min(piece, left);
+        if (hipMalloc(&next, room * stride * sizeof(float)) != hipSuccess) return false;
+        a->blocks.push_back(next);
+      }
+      p[i] = next;
+    }
+    return true;
   };
-  take(a->wstar, 8);
-  take(a->wnext, 8);
-  take(a->lstar, 8);
-  take(a->flux, 21);
-  take(a->work, kWork);
+  if (!take(a->wstar, 8) || !take(a->wnext, 8) || !take(a->lstar, 8) || !take(a->flux, 21) ||
+      !take(a->work, kWork))
+    return bail(NMHD_ENOMEM, "allocation failed");
   if (hipMalloc(&a->rec, sizeof(StepRec)) != hipSuccess)
     return bail(NMHD_ENOMEM, "allocation failed");
-  if (hipMemset(a->rec, 0, sizeof(StepRec)) != hipSuccess)
-    return bail(NMHD_EHIP, "step record init failed");
   *out = a;
   return NMHD_OK;
 }
