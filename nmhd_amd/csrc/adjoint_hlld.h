@@ -50,13 +50,14 @@ struct HOut {
 template <class T>
 struct HTape {
   T bx2, abx, sgn;
-  T v2L, v2R, eL, eR, ptL, ptR, gpL, gpR, gpbL, gpbR, sdL, sdR, cf2L, cf2R, cfL, cfR;
+  T ptL, ptR, gpL, gpR, gpbL, gpbR, sdL, sdR, cf2L, cf2R, cfL, cfR;
   T SL, SR, sLu, sRu, den, iden, SMn, SM, ptsn, pts, sLm, sRm, isLm, isRm;
   T rLs, rRs, dL, dR, idL, idR, kvL, kvR, kbLn, kbRn, kbL, kbR;
   T u1Ls, u2Ls, u1Rs, u2Rs, b1Ls, b2Ls, b1Rs, b2Rs;
-  T vbL, vbR, vbLs, vbRs, eLsn, eRsn, eLs, eRs;
-  T srL, srR, SLs, SRs, f, u1ssn, u2ssn, u1ss, u2ss, srLR, b1ssn, b2ssn, b1ss, b2ss, vbss;
-  T eLss, eRss;
+  T srL, srR, f, u1ssn, u2ssn, u1ss, u2ss, srLR, b1ssn, b2ssn, b1ss, b2ss, vbss;
+  // the chosen side's energy chain (no region reads the other side's): v^2,
+  // E, v.B, v*.B*, the numerator of E*, E*, S*, E**
+  T v2, e, vb, vbs, esn, es, Ss, ess;
   bool useL_c, minL, maxL, left;
   int region;  // 0 outer state, 1 single star, 2 double star
 };
@@ -73,10 +74,6 @@ __host__ __device__ inline void hlld_forward(T gamma, T ig, const HIn<T> &in, HT
   t.sgn = bx > T(0) ? T(1) : (bx < T(0) ? T(-1) : T(0));
   const T B2L = t.bx2 + in.b1L * in.b1L + in.b2L * in.b2L;
   const T B2R = t.bx2 + in.b1R * in.b1R + in.b2R * in.b2R;
-  t.v2L = in.unL * in.unL + in.u1L * in.u1L + in.u2L * in.u2L;
-  t.v2R = in.unR * in.unR + in.u1R * in.u1R + in.u2R * in.u2R;
-  t.eL = in.pL * ig + T(0.5) * in.rL * t.v2L + T(0.5) * B2L;
-  t.eR = in.pR * ig + T(0.5) * in.rR * t.v2R + T(0.5) * B2R;
   t.ptL = in.pL + T(0.5) * B2L;
   t.ptR = in.pR + T(0.5) * B2R;
   t.gpL = gamma * in.pL;
@@ -130,18 +127,8 @@ __host__ __device__ inline void hlld_forward(T gamma, T ig, const HIn<T> &in, HT
   t.b2Ls = in.b2L * t.kbL;
   t.b1Rs = in.b1R * t.kbR;
   t.b2Rs = in.b2R * t.kbR;
-  t.vbL = in.unL * bx + in.u1L * in.b1L + in.u2L * in.b2L;
-  t.vbR = in.unR * bx + in.u1R * in.b1R + in.u2R * in.b2R;
-  t.vbLs = t.SM * bx + t.u1Ls * t.b1Ls + t.u2Ls * t.b2Ls;
-  t.vbRs = t.SM * bx + t.u1Rs * t.b1Rs + t.u2Rs * t.b2Rs;
-  t.eLsn = t.sLu * t.eL - t.ptL * in.unL + t.pts * t.SM + bx * (t.vbL - t.vbLs);
-  t.eRsn = t.sRu * t.eR - t.ptR * in.unR + t.pts * t.SM + bx * (t.vbR - t.vbRs);
-  t.eLs = t.eLsn * t.isLm;
-  t.eRs = t.eRsn * t.isRm;
   t.srL = qsqrt(t.rLs);
   t.srR = qsqrt(t.rRs);
-  t.SLs = t.SM - qdiv(t.abx, t.srL);
-  t.SRs = t.SM + qdiv(t.abx, t.srR);
   t.f = qrcp(t.srL + t.srR);
   t.u1ssn = t.srL * t.u1Ls + t.srR * t.u1Rs + (t.b1Rs - t.b1Ls) * t.sgn;
   t.u2ssn = t.srL * t.u2Ls + t.srR * t.u2Rs + (t.b2Rs - t.b2Ls) * t.sgn;
@@ -153,23 +140,34 @@ __host__ __device__ inline void hlld_forward(T gamma, T ig, const HIn<T> &in, HT
   t.b1ss = t.f * t.b1ssn;
   t.b2ss = t.f * t.b2ssn;
   t.vbss = t.SM * bx + t.u1ss * t.b1ss + t.u2ss * t.b2ss;
-  t.eLss = t.eLs - t.srL * (t.vbLs - t.vbss) * t.sgn;
-  t.eRss = t.eRs + t.srR * (t.vbRs - t.vbss) * t.sgn;
 
+  // the side of the contact, and its outer and single-star states
   t.left = t.SM >= T(0);
-  if (t.left)
-    t.region = t.SL > T(0) ? 0 : (T(0) <= t.SLs ? 1 : 2);
-  else
-    t.region = t.SR < T(0) ? 0 : (t.SRs < T(0) ? 1 : 2);
   const bool L = t.left;
   const T r = L ? in.rL : in.rR, un = L ? in.unL : in.unR;
   const T u1 = L ? in.u1L : in.u1R, u2 = L ? in.u2L : in.u2R;
   const T b1 = L ? in.b1L : in.b1R, b2 = L ? in.b2L : in.b2R;
-  const T e = L ? t.eL : t.eR, pt = L ? t.ptL : t.ptR, vb = L ? t.vbL : t.vbR;
-  const T S = L ? t.SL : t.SR, Ss = L ? t.SLs : t.SRs, rs = L ? t.rLs : t.rRs;
+  const T p = L ? in.pL : in.pR, B2 = L ? B2L : B2R, pt = L ? t.ptL : t.ptR;
+  const T S = L ? t.SL : t.SR, sKu = L ? t.sLu : t.sRu, isKm = L ? t.isLm : t.isRm;
+  const T rs = L ? t.rLs : t.rRs;
   const T u1s = L ? t.u1Ls : t.u1Rs, u2s = L ? t.u2Ls : t.u2Rs;
   const T b1s = L ? t.b1Ls : t.b1Rs, b2s = L ? t.b2Ls : t.b2Rs;
-  const T es = L ? t.eLs : t.eRs, ess = L ? t.eLss : t.eRss;
+  t.v2 = un * un + u1 * u1 + u2 * u2;
+  t.e = p * ig + T(0.5) * r * t.v2 + T(0.5) * B2;
+  t.vb = un * bx + u1 * b1 + u2 * b2;
+  t.vbs = t.SM * bx + u1s * b1s + u2s * b2s;
+  t.esn = sKu * t.e - pt * un + t.pts * t.SM + bx * (t.vb - t.vbs);
+  t.es = t.esn * isKm;
+  // S*_K = SM -+ |Bx| / sqrt(rho*_K), E**_K = E*_K -+ sqrt(rho*_K) (..) sgn:
+  // - on the left, + on the right
+  t.Ss = t.SM + qdiv(L ? -t.abx : t.abx, L ? t.srL : t.srR);
+  const T ssr = L ? -t.srL : t.srR;
+  t.ess = t.es + ssr * (t.vbs - t.vbss) * t.sgn;
+  if (t.left)
+    t.region = t.SL > T(0) ? 0 : (T(0) <= t.Ss ? 1 : 2);
+  else
+    t.region = t.SR < T(0) ? 0 : (t.Ss < T(0) ? 1 : 2);
+  const T e = t.e, vb = t.vb, Ss = t.Ss, es = t.es, ess = t.ess;
   F.rho = r * un;
   F.mn = r * un * un + pt - t.bx2;
   F.mt1 = r * u1 * un - bx * b1;
@@ -207,27 +205,28 @@ __host__ __device__ inline void hlld_reverse(T gamma, T ig, const HIn<T> &in, co
   T a_bx = Z, a_bx2 = Z, a_abx = Z;
   T a_rL = Z, a_rR = Z, a_unL = Z, a_unR = Z, a_u1L = Z, a_u1R = Z, a_u2L = Z, a_u2R = Z;
   T a_pL = Z, a_pR = Z, a_b1L = Z, a_b1R = Z, a_b2L = Z, a_b2R = Z;
-  T a_eL = Z, a_eR = Z, a_ptL = Z, a_ptR = Z, a_vbL = Z, a_vbR = Z;
-  T a_SL = Z, a_SR = Z, a_SLs = Z, a_SRs = Z, a_rLs = Z, a_rRs = Z;
+  T a_ptL = Z, a_ptR = Z, a_SL = Z, a_SR = Z, a_rLs = Z, a_rRs = Z;
   T a_u1Ls = Z, a_u2Ls = Z, a_u1Rs = Z, a_u2Rs = Z, a_b1Ls = Z, a_b2Ls = Z, a_b1Rs = Z,
     a_b2Rs = Z;
-  T a_eLs = Z, a_eRs = Z, a_eLss = Z, a_eRss = Z;
   T a_u1ss = Z, a_u2ss = Z, a_b1ss = Z, a_b2ss = Z, a_SM = Z;
 
   // ---- flux of the selected region (side K)
+  const bool L = t.left;
+  const T r = L ? in.rL : in.rR, un = L ? in.unL : in.unR;
+  const T u1 = L ? in.u1L : in.u1R, u2 = L ? in.u2L : in.u2R;
+  const T b1 = L ? in.b1L : in.b1R, b2 = L ? in.b2L : in.b2R;
+  const T e = t.e, pt = L ? t.ptL : t.ptR, vb = t.vb;
+  const T S = L ? t.SL : t.SR, Ss = t.Ss, rs = L ? t.rLs : t.rRs;
+  const T u1s = L ? t.u1Ls : t.u1Rs, u2s = L ? t.u2Ls : t.u2Rs;
+  const T b1s = L ? t.b1Ls : t.b1Rs, b2s = L ? t.b2Ls : t.b2Rs;
+  const T es = t.es, ess = t.ess;
+  // adjoints on side K; the other side's are zero until the double-star
+  // states, which mix the two
+  T ae = Z, avb = Z, apt = Z, ar = Z, aun = Z, au1 = Z, au2 = Z, ab1 = Z, ab2 = Z;
+  T aSs = Z, aes = Z, aess = Z;
   {
-    const bool L = t.left;
     const bool r1 = t.region >= 1, r2 = t.region == 2;
-    const T r = L ? in.rL : in.rR, un = L ? in.unL : in.unR;
-    const T u1 = L ? in.u1L : in.u1R, u2 = L ? in.u2L : in.u2R;
-    const T b1 = L ? in.b1L : in.b1R, b2 = L ? in.b2L : in.b2R;
-    const T e = L ? t.eL : t.eR, pt = L ? t.ptL : t.ptR, vb = L ? t.vbL : t.vbR;
-    const T S = L ? t.SL : t.SR, Ss = L ? t.SLs : t.SRs, rs = L ? t.rLs : t.rRs;
-    const T u1s = L ? t.u1Ls : t.u1Rs, u2s = L ? t.u2Ls : t.u2Rs;
-    const T b1s = L ? t.b1Ls : t.b1Rs, b2s = L ? t.b2Ls : t.b2Rs;
-    const T es = L ? t.eLs : t.eRs, ess = L ? t.eLss : t.eRss;
-    T ar = Z, aun = Z, au1 = Z, au2 = Z, ab1 = Z, ab2 = Z, ae = Z, apt = Z, avb = Z;
-    T aS = Z, aSs = Z, ars = Z, au1s = Z, au2s = Z, ab1s = Z, ab2s = Z, aes = Z, aess = Z;
+    T aS = Z, ars = Z, au1s = Z, au2s = Z, ab1s = Z, ab2s = Z;
     // rho
     ar += aF.rho * un;
     aun += aF.rho * r;
@@ -291,30 +290,25 @@ __host__ __device__ inline void hlld_reverse(T gamma, T ig, const HIn<T> &in, co
       ab1s -= Ss * aF.bt1;
       ab2s -= Ss * aF.bt2;
     }
-    if (L) {
-      a_rL += ar, a_unL += aun, a_u1L += au1, a_u2L += au2, a_b1L += ab1, a_b2L += ab2;
-      a_eL += ae, a_ptL += apt, a_vbL += avb, a_SL += aS, a_SLs += aSs, a_rLs += ars;
-      a_u1Ls += au1s, a_u2Ls += au2s, a_b1Ls += ab1s, a_b2Ls += ab2s, a_eLs += aes,
-          a_eLss += aess;
-    } else {
-      a_rR += ar, a_unR += aun, a_u1R += au1, a_u2R += au2, a_b1R += ab1, a_b2R += ab2;
-      a_eR += ae, a_ptR += apt, a_vbR += avb, a_SR += aS, a_SRs += aSs, a_rRs += ars;
-      a_u1Rs += au1s, a_u2Rs += au2s, a_b1Rs += ab1s, a_b2Rs += ab2s, a_eRs += aes,
-          a_eRss += aess;
-    }
+    a_SL = L ? aS : Z, a_SR = L ? Z : aS;
+    a_rLs = L ? ars : Z, a_rRs = L ? Z : ars;
+    a_u1Ls = L ? au1s : Z, a_u1Rs = L ? Z : au1s;
+    a_u2Ls = L ? au2s : Z, a_u2Rs = L ? Z : au2s;
+    a_b1Ls = L ? ab1s : Z, a_b1Rs = L ? Z : ab1s;
+    a_b2Ls = L ? ab2s : Z, a_b2Rs = L ? Z : ab2s;
   }
 
   // ---- double-star states
-  T a_vbss = Z, a_srL = Z, a_srR = Z, a_f = Z, a_srLR = Z, a_vbLs = Z, a_vbRs = Z;
-  // eLss = eLs - srL (vbLs - vbss) sgn;  eRss = eRs + srR (vbRs - vbss) sgn
-  a_eLs += a_eLss;
-  a_srL -= a_eLss * (t.vbLs - t.vbss) * t.sgn;
-  a_vbLs -= a_eLss * t.srL * t.sgn;
-  a_vbss += a_eLss * t.srL * t.sgn;
-  a_eRs += a_eRss;
-  a_srR += a_eRss * (t.vbRs - t.vbss) * t.sgn;
-  a_vbRs += a_eRss * t.srR * t.sgn;
-  a_vbss -= a_eRss * t.srR * t.sgn;
+  T a_vbss = Z, a_srL = Z, a_srR = Z, a_f = Z, a_srLR = Z, avbs = Z;
+  // ess = es + ssr (vbs - vbss) sgn, ssr = -srL on the left, srR on the right
+  aes += aess;
+  {
+    const T g = aess * (t.vbs - t.vbss) * t.sgn, w = aess * (L ? t.srL : t.srR) * t.sgn;
+    a_srL = L ? -g : Z;
+    a_srR = L ? Z : g;
+    avbs = L ? -w : w;
+    a_vbss = -avbs;
+  }
   // vbss = SM bx + u1ss b1ss + u2ss b2ss
   a_SM += a_vbss * bx;
   a_bx += a_vbss * t.SM;
@@ -362,66 +356,69 @@ __host__ __device__ inline void hlld_reverse(T gamma, T ig, const HIn<T> &in, co
   // f = 1/(srL + srR)
   a_srL -= a_f * t.f * t.f;
   a_srR -= a_f * t.f * t.f;
-  // SLs = SM - abx/srL; SRs = SM + abx/srR
-  a_SM += a_SLs + a_SRs;
-  a_abx += -qdiv(a_SLs, t.srL) + qdiv(a_SRs, t.srR);
-  a_srL += qdiv(a_SLs * t.abx, t.srL * t.srL);
-  a_srR -= qdiv(a_SRs * t.abx, t.srR * t.srR);
+  // Ss = SM - abx/srL on the left, SM + abx/srR on the right
+  a_SM += aSs;
+  {
+    const T sr = L ? t.srL : t.srR;
+    const T g = qdiv(aSs, sr), w = qdiv(aSs * t.abx, sr * sr);
+    a_abx = L ? -g : g;
+    a_srL += L ? w : Z;
+    a_srR -= L ? Z : w;
+  }
   // srL = sqrt(rLs)
   a_rLs += qdiv(a_srL, T(2) * t.srL);
   a_rRs += qdiv(a_srR, T(2) * t.srR);
 
   // ---- single-star states
   T a_sLu = Z, a_sRu = Z, a_isLm = Z, a_isRm = Z, a_pts = Z;
-  {  // eLs = eLsn isLm
-    const T g = a_eLs * t.isLm;
-    a_isLm += a_eLs * t.eLsn;
-    a_sLu += g * t.eL;
-    a_eL += g * t.sLu;
-    a_ptL -= g * in.unL;
-    a_unL -= g * t.ptL;
+  {  // es = esn isKm, esn = sKu e - pt un + pts SM + bx (vb - vbs)
+    const T isKm = L ? t.isLm : t.isRm, sKu = L ? t.sLu : t.sRu;
+    const T g = aes * isKm, w = aes * t.esn, q = g * e;
+    a_isLm = L ? w : Z;
+    a_isRm = L ? Z : w;
+    a_sLu = L ? q : Z;
+    a_sRu = L ? Z : q;
+    ae += g * sKu;
+    apt -= g * un;
+    aun -= g * pt;
     a_pts += g * t.SM;
     a_SM += g * t.pts;
-    a_bx += g * (t.vbL - t.vbLs);
-    a_vbL += g * bx;
-    a_vbLs -= g * bx;
+    a_bx += g * (vb - t.vbs);
+    avb += g * bx;
+    avbs -= g * bx;
   }
-  {  // eRs = eRsn isRm
-    const T g = a_eRs * t.isRm;
-    a_isRm += a_eRs * t.eRsn;
-    a_sRu += g * t.eR;
-    a_eR += g * t.sRu;
-    a_ptR -= g * in.unR;
-    a_unR -= g * t.ptR;
-    a_pts += g * t.SM;
-    a_SM += g * t.pts;
-    a_bx += g * (t.vbR - t.vbRs);
-    a_vbR += g * bx;
-    a_vbRs -= g * bx;
+  // vbs = SM bx + u1s b1s + u2s b2s
+  a_SM += avbs * bx;
+  a_bx += avbs * t.SM;
+  {
+    const T gL = L ? avbs : Z, gR = L ? Z : avbs;
+    a_u1Ls += gL * t.b1Ls;
+    a_b1Ls += gL * t.u1Ls;
+    a_u2Ls += gL * t.b2Ls;
+    a_b2Ls += gL * t.u2Ls;
+    a_u1Rs += gR * t.b1Rs;
+    a_b1Rs += gR * t.u1Rs;
+    a_u2Rs += gR * t.b2Rs;
+    a_b2Rs += gR * t.u2Rs;
   }
-  // vbLs = SM bx + u1Ls b1Ls + u2Ls b2Ls (and R)
-  a_SM += (a_vbLs + a_vbRs) * bx;
-  a_bx += (a_vbLs + a_vbRs) * t.SM;
-  a_u1Ls += a_vbLs * t.b1Ls;
-  a_b1Ls += a_vbLs * t.u1Ls;
-  a_u2Ls += a_vbLs * t.b2Ls;
-  a_b2Ls += a_vbLs * t.u2Ls;
-  a_u1Rs += a_vbRs * t.b1Rs;
-  a_b1Rs += a_vbRs * t.u1Rs;
-  a_u2Rs += a_vbRs * t.b2Rs;
-  a_b2Rs += a_vbRs * t.u2Rs;
-  // vbL = unL bx + u1L b1L + u2L b2L (and R)
-  a_unL += a_vbL * bx;
-  a_bx += a_vbL * in.unL + a_vbR * in.unR;
-  a_u1L += a_vbL * in.b1L;
-  a_b1L += a_vbL * in.u1L;
-  a_u2L += a_vbL * in.b2L;
-  a_b2L += a_vbL * in.u2L;
-  a_unR += a_vbR * bx;
-  a_u1R += a_vbR * in.b1R;
-  a_b1R += a_vbR * in.u1R;
-  a_u2R += a_vbR * in.b2R;
-  a_b2R += a_vbR * in.u2R;
+  // vb = un bx + u1 b1 + u2 b2
+  aun += avb * bx;
+  {
+    const T g = avb * un;  // rounded by itself, as in the two sides' sum
+    a_bx += g;
+  }
+  au1 += avb * b1;
+  ab1 += avb * u1;
+  au2 += avb * b2;
+  ab2 += avb * u2;
+  // side K's adjoints to the states they belong to
+  a_rL = L ? ar : Z, a_rR = L ? Z : ar;
+  a_unL = L ? aun : Z, a_unR = L ? Z : aun;
+  a_u1L = L ? au1 : Z, a_u1R = L ? Z : au1;
+  a_u2L = L ? au2 : Z, a_u2R = L ? Z : au2;
+  a_b1L = L ? ab1 : Z, a_b1R = L ? Z : ab1;
+  a_b2L = L ? ab2 : Z, a_b2R = L ? Z : ab2;
+  a_ptL = L ? apt : Z, a_ptR = L ? Z : apt;
   // b1Ls = b1L kbL, b2Ls = b2L kbL; u1Ls = u1L - b1L kvL, u2Ls = u2L - b2L kvL (and R)
   const T a_kbL = a_b1Ls * in.b1L + a_b2Ls * in.b2L;
   const T a_kbR = a_b1Rs * in.b1R + a_b2Rs * in.b2R;
@@ -534,30 +531,26 @@ __host__ __device__ inline void hlld_reverse(T gamma, T ig, const HIn<T> &in, co
     a_unL += a_SR;
   else
     a_unR += a_SR;
-  T a_cfL = Z, a_cfR = Z;
-  if (t.useL_c)
-    a_cfL += SQ2 * a_cmax;
-  else
-    a_cfR += SQ2 * a_cmax;
-  T a_gpL = Z, a_gpR = Z, a_B2L = Z, a_B2R = Z;
-  {  // cfL = sqrt(cf2L), cf2L = (gpbL + sdL)/(2 rL), sdL = sqrt(gpbL^2 - 4 gpL bx2)
-    const T a_cf2L = t.cfL > Z ? qdiv(a_cfL, T(2) * t.cfL) : Z;
-    const T a_cf2R = t.cfR > Z ? qdiv(a_cfR, T(2) * t.cfR) : Z;
-    T a_gpbL = qdiv(a_cf2L, T(2) * in.rL), a_gpbR = qdiv(a_cf2R, T(2) * in.rR);
-    const T a_sdL = a_gpbL, a_sdR = a_gpbR;
-    a_rL -= qdiv(a_cf2L * t.cf2L, in.rL);
-    a_rR -= qdiv(a_cf2R * t.cf2R, in.rR);
-    const T a_discL = t.sdL > Z ? qdiv(a_sdL, T(2) * t.sdL) : Z;
-    const T a_discR = t.sdR > Z ? qdiv(a_sdR, T(2) * t.sdR) : Z;
-    a_gpbL += a_discL * T(2) * t.gpbL;
-    a_gpbR += a_discR * T(2) * t.gpbR;
-    a_gpL -= a_discL * T(4) * t.bx2;
-    a_gpR -= a_discR * T(4) * t.bx2;
-    a_bx2 -= a_discL * T(4) * t.gpL + a_discR * T(4) * t.gpR;
-    a_gpL += a_gpbL;
-    a_gpR += a_gpbR;
-    a_B2L += a_gpbL;
-    a_B2R += a_gpbR;
+  T a_gpL, a_gpR, a_B2L, a_B2R;
+  {  // on the side of the larger cf: cf = sqrt(cf2), cf2 = (gpb + sd)/(2 r),
+     // sd = sqrt(gpb^2 - 4 gp bx2)
+    const bool C = t.useL_c;
+    const T cf = C ? t.cfL : t.cfR, cf2 = C ? t.cf2L : t.cf2R, sd = C ? t.sdL : t.sdR;
+    const T gp = C ? t.gpL : t.gpR, gpb = C ? t.gpbL : t.gpbR, rc = C ? in.rL : in.rR;
+    const T a_cf = SQ2 * a_cmax;
+    const T a_cf2 = cf > Z ? qdiv(a_cf, T(2) * cf) : Z;
+    T a_gpb = qdiv(a_cf2, T(2) * rc);
+    const T a_sd = a_gpb;
+    const T a_r = qdiv(a_cf2 * cf2, rc);
+    const T a_disc = sd > Z ? qdiv(a_sd, T(2) * sd) : Z;
+    a_gpb += a_disc * T(2) * gpb;
+    const T a_gp0 = a_disc * T(4) * t.bx2, a_b = a_disc * T(4) * gp;
+    a_bx2 -= a_b;
+    const T a_gp = a_gpb - a_gp0;
+    a_rL -= C ? a_r : Z;
+    a_rR -= C ? Z : a_r;
+    a_gpL = C ? a_gp : Z, a_gpR = C ? Z : a_gp;
+    a_B2L = C ? a_gpb : Z, a_B2R = C ? Z : a_gpb;
   }
   a_pL += gamma * a_gpL;
   a_pR += gamma * a_gpR;
@@ -566,21 +559,23 @@ __host__ __device__ inline void hlld_reverse(T gamma, T ig, const HIn<T> &in, co
   a_pR += a_ptR;
   a_B2L += T(0.5) * a_ptL;
   a_B2R += T(0.5) * a_ptR;
-  // eL = pL ig + rL v2L/2 + B2L/2
-  a_pL += a_eL * ig;
-  a_pR += a_eR * ig;
-  a_rL += T(0.5) * a_eL * t.v2L;
-  a_rR += T(0.5) * a_eR * t.v2R;
-  const T a_v2L = T(0.5) * a_eL * in.rL, a_v2R = T(0.5) * a_eR * in.rR;
-  a_B2L += T(0.5) * a_eL;
-  a_B2R += T(0.5) * a_eR;
-  // v2L = unL^2 + u1L^2 + u2L^2
-  a_unL += T(2) * a_v2L * in.unL;
-  a_u1L += T(2) * a_v2L * in.u1L;
-  a_u2L += T(2) * a_v2L * in.u2L;
-  a_unR += T(2) * a_v2R * in.unR;
-  a_u1R += T(2) * a_v2R * in.u1R;
-  a_u2R += T(2) * a_v2R * in.u2R;
+  // e = p ig + r v2/2 + B2/2, v2 = un^2 + u1^2 + u2^2
+  {
+    const T gL = L ? ae : Z, gR = L ? Z : ae;
+    a_pL += gL * ig;
+    a_pR += gR * ig;
+    a_rL += T(0.5) * gL * t.v2;
+    a_rR += T(0.5) * gR * t.v2;
+    const T a_v2L = T(0.5) * gL * in.rL, a_v2R = T(0.5) * gR * in.rR;
+    a_B2L += T(0.5) * gL;
+    a_B2R += T(0.5) * gR;
+    a_unL += T(2) * a_v2L * in.unL;
+    a_u1L += T(2) * a_v2L * in.u1L;
+    a_u2L += T(2) * a_v2L * in.u2L;
+    a_unR += T(2) * a_v2R * in.unR;
+    a_u1R += T(2) * a_v2R * in.u1R;
+    a_u2R += T(2) * a_v2R * in.u2R;
+  }
   // B2L = bx2 + b1L^2 + b2L^2
   a_bx2 += a_B2L + a_B2R;
   a_b1L += T(2) * a_B2L * in.b1L;

@@ -13,7 +13,7 @@
 //                 (3 distinct values per cell: lamE_x, lamE_y, lamE_z) from the
 //                 face-B adjoints of the cell and its lower neighbours, which
 //                 the thread recomputes rather than reading them back
-//   k_adj_faces   per face of the three directions (blockIdx.y): adjoint of
+//   k_adj_faces   per face of the three directions: adjoint of
 //                 the 7 fluxes (divergence + upwinded EMFs, with the forward's
 //                 upwind choice recomputed), then the HLLD reverse sweep
 //                 (adjoint_hlld.h) -> adjoints of the 7 left/right face states
@@ -31,28 +31,45 @@ namespace nmhd {
 
 namespace {
 
-__device__ __forceinline__ long cell_index(const Box &b, int x, int y, int z) {
-  return ((long)z * b.n[1] + y) * b.n[0] + x;
+// Cells by 32-bit byte offset from an array's start (the adjoint's arrays
+// number over a hundred, so a box that fits the GPU has fewer than 2^30
+// cells): loads and stores then take a scalar base and a 32-bit offset, and
+// neighbours are sums of per-axis offsets, with no 64-bit or multiply
+// arithmetic per access.
+__device__ __forceinline__ float ld(const float *p, unsigned o) {
+  return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(p) + o);
+}
+__device__ __forceinline__ float &at(float *p, unsigned o) {
+  return *reinterpret_cast<float *>(reinterpret_cast<char *>(p) + o);
 }
 
-// neighbour of (x, y, z) shifted by s along axis d (periodic)
-__device__ __forceinline__ long nb(const Box &b, int x, int y, int z, int d, int s) {
-  if (d == 0) x = wrap(x + s, b.n[0]);
-  if (d == 1) y = wrap(y + s, b.n[1]);
-  if (d == 2) z = wrap(z + s, b.n[2]);
-  return cell_index(b, x, y, z);
-}
+// The thread's cell, and the offset contributions of its index along each
+// axis and of the neighbours' (periodic).
+struct Place {
+  int v[3];           // x, y, z
+  unsigned stride[3]; // bytes
+  unsigned o[3];      // v * stride
+  __device__ __forceinline__ unsigned own() const { return o[0] + o[1] + o[2]; }
+  // contribution of index v[d] + s (s in -2..2; n: the box's cells along d)
+  __device__ __forceinline__ unsigned to(int d, int s, int n) const {
+    int i = v[d] + s;
+    if (s < 0) i = i < 0 ? i + n : i;
+    if (s > 0) i = i >= n ? i - n : i;
+    // a shift of 2 in a box of one cell wraps twice
+    return (unsigned)(n == 1 ? 0 : i) * stride[d];
+  }
+};
 
-// The thread's cell; 32-bit unsigned index arithmetic (a box holds fewer
-// than 2^31 cells).
-__device__ __forceinline__ bool cell_of(const Box &b, int &x, int &y, int &z, long &a) {
-  a = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (a >= b.ncell) return false;
-  const unsigned u = (unsigned)a, n0 = (unsigned)b.n[0], n1 = (unsigned)b.n[1];
-  const unsigned row = u / n0;
-  x = (int)(u - row * n0);
-  z = (int)(row / n1);
-  y = (int)(row - (unsigned)z * n1);
+// The cell of a thread of workgroup `block` of the cells in order; false
+// beyond the last one.
+__device__ __forceinline__ bool place_of(const Box &b, unsigned block, Place &p) {
+  const unsigned u = block * blockDim.x + threadIdx.x;
+  if (u >= (unsigned)b.ncell) return false;
+  cell_coords(b, u, p.v[0], p.v[1], p.v[2]);
+  p.stride[0] = 4u;
+  p.stride[1] = 4u * (unsigned)b.n[0];
+  p.stride[2] = p.stride[1] * (unsigned)b.n[1];
+  for (int d = 0; d < 3; ++d) p.o[d] = (unsigned)p.v[d] * p.stride[d];
   return true;
 }
 
@@ -60,33 +77,15 @@ __device__ __forceinline__ bool cell_of(const Box &b, int &x, int &y, int &z, lo
 __device__ __forceinline__ float w_lo(float s) { return s > 0.0f ? 1.0f : (s < 0.0f ? 0.0f : 0.5f); }
 __device__ __forceinline__ float w_hi(float s) { return s > 0.0f ? 0.0f : (s < 0.0f ? 1.0f : 0.5f); }
 
-// The forward's sum of four cell velocities around an edge (same order as the
-// stage kernels, so that the sign decision is the same).  The edge lies on
-// the lower p-face and lower q-face of cell (x,y,z) (p < q axes); comp is
-// the velocity component summed.
-__device__ __forceinline__ float edge_sum(const Box &b, const float *v, int x, int y, int z,
-                                          int p, int q, int comp) {
-  const long c = cell_index(b, x, y, z);
-  const long cp = nb(b, x, y, z, p, -1);
-  const long cq = nb(b, x, y, z, q, -1);
-  int xp = x, yp = y, zp = z;
-  if (p == 0) xp = wrap(x - 1, b.n[0]);
-  if (p == 1) yp = wrap(y - 1, b.n[1]);
-  const long cpq = nb(b, xp, yp, zp, q, -1);
-  // winds summed along the first edge axis first when comp is the second
-  // edge axis' component, as the stage kernels do
-  if (comp == q) return v[c] + v[cq] + v[cp] + v[cpq];
-  return v[c] + v[cp] + v[cq] + v[cpq];
-}
-
 // ------------------------------------------------------------- k_adj_prim
 
 // Adjoint of the face value B_d at cell c (its lower d-face) from the stage
 // output: its own adjoint, and through the pressure of the two cells that
 // share the face (c and its lower d-neighbour m).
 __device__ __forceinline__ float face_b_adj(const Box &b, const FieldPtrs &Wout,
-                                            const FieldPtrs &lam, int d, long c, long m) {
-  return lam.f[5 + d][c] - b.gm1 * 0.5f * Wout.f[5 + d][c] * (lam.f[4][c] + lam.f[4][m]);
+                                            const FieldPtrs &lam, int d, unsigned c, unsigned m) {
+  return ld(lam.f[5 + d], c) -
+         b.gm1 * 0.5f * ld(Wout.f[5 + d], c) * (ld(lam.f[4], c) + ld(lam.f[4], m));
 }
 
 // lamE_z = adjoint of the z-edge EMF from the x-sweep (= minus that of the
@@ -99,47 +98,52 @@ __global__ void __launch_bounds__(256) k_adj_prim(Box b, FieldPtrs Wout, FieldPt
                                                   float *gU2, float *gU3, float *gU4, float h,
                                                   float *lEx, float *lEy, float *lEz,
                                                   FieldPtrs lam_base) {
-  int x, y, z;
-  long a;
-  if (!cell_of(b, x, y, z, a)) return;
+  Place p;
+  if (!place_of(b, xcd_logical_block(blockIdx.x, gridDim.x), p)) return;
   const float gm1 = b.gm1, ig = b.inv_gm1;
-  const float rho = Wout.f[0][a];
-  const float v[3] = {Wout.f[1][a], Wout.f[2][a], Wout.f[3][a]};
-  const float lp = lam.f[4][a];
+  const unsigned a = p.own();
+  const float rho = ld(Wout.f[0], a);
+  const float v[3] = {ld(Wout.f[1], a), ld(Wout.f[2], a), ld(Wout.f[3], a)};
+  const float lp = ld(lam.f[4], a);
   const float irho = frcp(rho);
   const float gE = gm1 * lp;
   float gm[3];
-  float grho = lam.f[0][a] + gm1 * lp * 0.5f * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+  float grho = ld(lam.f[0], a) + gm1 * lp * 0.5f * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
   for (int d = 0; d < 3; ++d) {
-    gm[d] = lam.f[1 + d][a] * irho - gm1 * lp * v[d];
-    grho -= lam.f[1 + d][a] * v[d] * irho;
+    const float lv = ld(lam.f[1 + d], a);
+    gm[d] = lv * irho - gm1 * lp * v[d];
+    grho -= lv * v[d] * irho;
   }
-  const long xm = nb(b, x, y, z, 0, -1), ym = nb(b, x, y, z, 1, -1), zm = nb(b, x, y, z, 2, -1);
-  const long mm[3] = {xm, ym, zm};
+  // lower neighbours, one axis and two
+  const unsigned lx = p.to(0, -1, b.n[0]), ly = p.to(1, -1, b.n[1]), lz = p.to(2, -1, b.n[2]);
+  const unsigned xm = lx + (p.o[1] + p.o[2]), ym = p.o[0] + (ly + p.o[2]);
+  const unsigned zm = p.o[0] + (p.o[1] + lz);
+  const unsigned xym = lx + (ly + p.o[2]), xzm = lx + (p.o[1] + lz), yzm = p.o[0] + (ly + lz);
+  const unsigned mm[3] = {xm, ym, zm};
   float gB[3];
   for (int d = 0; d < 3; ++d) gB[d] = face_b_adj(b, Wout, lam, d, a, mm[d]);
-  gU0[a] = grho;
-  gU1[a] = gm[0];
-  gU2[a] = gm[1];
-  gU3[a] = gm[2];
-  gU4[a] = gE;
+  at(gU0, a) = grho;
+  at(gU1, a) = gm[0];
+  at(gU2, a) = gm[1];
+  at(gU3, a) = gm[2];
+  at(gU4, a) = gE;
   // the edge-EMF adjoints: face-B adjoints of the lower x-, y- and
   // z-neighbours, each through its own lower neighbour along its face axis
   {
     const float idx = b.inv_d[0], idy = b.inv_d[1], idz = b.inv_d[2];
-    const float gB0_ym = face_b_adj(b, Wout, lam, 0, ym, nb(b, x, wrap(y - 1, b.n[1]), z, 0, -1));
-    const float gB0_zm = face_b_adj(b, Wout, lam, 0, zm, nb(b, x, y, wrap(z - 1, b.n[2]), 0, -1));
-    const float gB1_xm = face_b_adj(b, Wout, lam, 1, xm, nb(b, wrap(x - 1, b.n[0]), y, z, 1, -1));
-    const float gB1_zm = face_b_adj(b, Wout, lam, 1, zm, nb(b, x, y, wrap(z - 1, b.n[2]), 1, -1));
-    const float gB2_xm = face_b_adj(b, Wout, lam, 2, xm, nb(b, wrap(x - 1, b.n[0]), y, z, 2, -1));
-    const float gB2_ym = face_b_adj(b, Wout, lam, 2, ym, nb(b, x, wrap(y - 1, b.n[1]), z, 2, -1));
-    lEz[a] = h * (0.5f * idy * (gB0_ym - gB[0]) + 0.5f * idx * (gB[1] - gB1_xm));
-    lEy[a] = h * (0.5f * idz * (gB0_zm - gB[0]) + 0.5f * idx * (gB[2] - gB2_xm));
-    lEx[a] = h * (0.5f * idz * (gB1_zm - gB[1]) + 0.5f * idy * (gB[2] - gB2_ym));
+    const float gB0_ym = face_b_adj(b, Wout, lam, 0, ym, xym);
+    const float gB0_zm = face_b_adj(b, Wout, lam, 0, zm, xzm);
+    const float gB1_xm = face_b_adj(b, Wout, lam, 1, xm, xym);
+    const float gB1_zm = face_b_adj(b, Wout, lam, 1, zm, yzm);
+    const float gB2_xm = face_b_adj(b, Wout, lam, 2, xm, xzm);
+    const float gB2_ym = face_b_adj(b, Wout, lam, 2, ym, yzm);
+    at(lEz, a) = h * (0.5f * idy * (gB0_ym - gB[0]) + 0.5f * idx * (gB[1] - gB1_xm));
+    at(lEy, a) = h * (0.5f * idz * (gB0_zm - gB[0]) + 0.5f * idx * (gB[2] - gB2_xm));
+    at(lEx, a) = h * (0.5f * idz * (gB1_zm - gB[1]) + 0.5f * idy * (gB[2] - gB2_ym));
   }
   // cons(W_base): rho, m = rho v, E = p/(g-1) + rho v^2/2 + (B_lo^2 + B_hi^2)/4
-  const float rho0 = Wbase.f[0][a];
-  const float v0[3] = {Wbase.f[1][a], Wbase.f[2][a], Wbase.f[3][a]};
+  const float rho0 = ld(Wbase.f[0], a);
+  const float v0[3] = {ld(Wbase.f[1], a), ld(Wbase.f[2], a), ld(Wbase.f[3], a)};
   float out[8];
   out[0] = grho + 0.5f * gE * (v0[0] * v0[0] + v0[1] * v0[1] + v0[2] * v0[2]);
   for (int d = 0; d < 3; ++d) {
@@ -148,8 +152,9 @@ __global__ void __launch_bounds__(256) k_adj_prim(Box b, FieldPtrs Wout, FieldPt
   }
   out[4] = gE * ig;
   for (int d = 0; d < 3; ++d)
-    out[5 + d] = gB[d] + 0.5f * Wbase.f[5 + d][a] * (gE + gm1 * lam.f[4][mm[d]]);
-  for (int f = 0; f < 8; ++f) lam_base.f[f][a] = AccBase ? lam_base.f[f][a] + out[f] : out[f];
+    out[5 + d] = gB[d] + 0.5f * ld(Wbase.f[5 + d], a) * (gE + gm1 * ld(lam.f[4], mm[d]));
+  for (int f = 0; f < 8; ++f)
+    at(lam_base.f[f], a) = AccBase ? ld(lam_base.f[f], a) + out[f] : out[f];
 }
 
 // ------------------------------------------------------------- k_adj_face
@@ -159,11 +164,10 @@ __global__ void __launch_bounds__(256) k_adj_prim(Box b, FieldPtrs Wout, FieldPt
 //
 // The face reverse hands the gather the adjoints of its two reconstructed
 // states, aL[k] and aR[k] (variable k), and the limiter branches the
-// forward took for them, 4 bits per variable in one word: bit 4k (4k+1)
-// when the left state's limited slope took its lower (upper) difference,
-// bit 4k+2 (4k+3) likewise for the right state's; no bit for a zero slope.
-// The gather then spreads the adjoints over the stencil cells without
-// reading the stencils again.
+// forward took for them, 4 bits per variable in one word: bits 4k, 4k+1 the
+// left state's limited slope, 4k+2, 4k+3 the right state's, each a two-bit
+// signed number (limiter_branch).  The gather then spreads the adjoints over
+// the stencil cells without reading the stencils again.
 struct AdjFaceOut {
   float *aL[7];
   float *aR[7];
@@ -171,13 +175,11 @@ struct AdjFaceOut {
   float *abn;
 };
 
-// Derivative of minmod(a, b) with respect to a and b on the branch the
-// forward took (ties and sign changes as minmod takes them).
-__device__ __forceinline__ void mm_grad(float a, float b, float &da, float &db) {
-  const bool nz = !(a * b <= 0.0f);
-  const bool pick_a = fabsf(a) < fabsf(b);
-  da = (nz && pick_a) ? 1.0f : 0.0f;
-  db = (nz && !pick_a) ? 1.0f : 0.0f;
+// The branch of minmod(a, b) that the forward took, as a two-bit signed
+// number: 1 for a, -1 for b, 0 for a zero slope (ties and sign changes as
+// minmod takes them).
+__device__ __forceinline__ unsigned limiter_branch(float a, float b) {
+  return a * b <= 0.0f ? 0u : (fabsf(a) < fabsf(b) ? 1u : 3u);
 }
 
 template <int D>
@@ -185,85 +187,73 @@ __device__ __forceinline__ void adj_face(const Box &b, const FieldPtrs &W, const
                                          const float *gU1, const float *gU2, const float *gU3,
                                          const float *gU4, const float *lEx, const float *lEy,
                                          const float *lEz, float h, const AdjFaceOut &out,
-                                         int x, int y, int z, long a) {
+                                         const Place &pl) {
   constexpr int D1 = (D + 1) % 3, D2 = (D + 2) % 3;
   const float *gU[5] = {gU0, gU1, gU2, gU3, gU4};
-  const long m1 = nb(b, x, y, z, D, -1);
+  // stencil cells c-2..c+1 along D, and the cells next to them along the
+  // transverse axes: s1, s2 above, r1, r2 (of c-1 and c) below
+  const unsigned o1 = pl.o[D1], o2 = pl.o[D2];
+  const unsigned up1 = pl.to(D1, 1, b.n[D1]), up2 = pl.to(D2, 1, b.n[D2]);
+  const unsigned dn1 = pl.to(D1, -1, b.n[D1]), dn2 = pl.to(D2, -1, b.n[D2]);
+  unsigned cs[4], s1[4], s2[4], r1[2], r2[2];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const unsigned od = pl.to(D, k - 2, b.n[D]);
+    cs[k] = od + (o1 + o2);
+    s1[k] = od + (up1 + o2);
+    s2[k] = od + (o1 + up2);
+    if (k == 1 || k == 2) {
+      r1[k - 1] = od + (dn1 + o2);
+      r2[k - 1] = od + (o1 + dn2);
+    }
+  }
+  const unsigned a = cs[2], m1 = cs[1];
+  // the stencil's variables in the face's order
+  float q[7][4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    q[0][s] = ld(W.f[0], cs[s]);
+    q[1][s] = ld(W.f[1 + D], cs[s]);
+    q[2][s] = ld(W.f[1 + D1], cs[s]);
+    q[3][s] = ld(W.f[1 + D2], cs[s]);
+    q[4][s] = ld(W.f[4], cs[s]);
+    // cell-centred transverse B: the average of the cell's two faces
+    q[5][s] = 0.5f * (ld(W.f[5 + D1], cs[s]) + ld(W.f[5 + D1], s1[s]));
+    q[6][s] = 0.5f * (ld(W.f[5 + D2], cs[s]) + ld(W.f[5 + D2], s2[s]));
+  }
   const float id = b.inv_d[D];
   adj::HOut<float> aF;
-  aF.rho = h * (gU[0][a] - gU[0][m1]) * id;
-  aF.mn = h * (gU[1 + D][a] - gU[1 + D][m1]) * id;
-  aF.mt1 = h * (gU[1 + D1][a] - gU[1 + D1][m1]) * id;
-  aF.mt2 = h * (gU[1 + D2][a] - gU[1 + D2][m1]) * id;
-  aF.e = h * (gU[4][a] - gU[4][m1]) * id;
+  aF.rho = h * (ld(gU[0], a) - ld(gU[0], m1)) * id;
+  aF.mn = h * (ld(gU[1 + D], a) - ld(gU[1 + D], m1)) * id;
+  aF.mt1 = h * (ld(gU[1 + D1], a) - ld(gU[1 + D1], m1)) * id;
+  aF.mt2 = h * (ld(gU[1 + D2], a) - ld(gU[1 + D2], m1)) * id;
+  aF.e = h * (ld(gU[4], a) - ld(gU[4], m1)) * id;
   // B fluxes through the upwinded edge EMFs.  For the x-sweep: F(B_y) feeds
   // the z-edges on y-faces j (as the upper candidate) and j+1 (lower one),
   // upwinded by the y-velocity; F(B_z) the y-edges on z-faces k and k+1.
-  const float *v[3] = {W.f[1], W.f[2], W.f[3]};
   {
-    // component bt1 = B_D1 flux, used by edges along D2 on D1-faces
-    // component bt2 = B_D2 flux, used by edges along D1 on D2-faces
-    auto edge_adj = [&](int q, int xx, int yy, int zz) -> float {
-      // lam of the edge on the lower D-face and lower q-face of cell (xx,yy,zz),
-      // with the sign of the D-sweep's member of the pair
-      const long e = cell_index(b, xx, yy, zz);
-      const int other = 3 - D - q;  // the edge's axis
+    // adjoint of the edge on the lower D- and q-faces of a cell, with the sign
+    // of the D-sweep's member of the pair: the x-sweep (or, for x-edges, the
+    // y-sweep) member carries +lam, the other sweep's -lam
+    auto edge_adj = [&](int q_, unsigned e) -> float {
+      const int other = 3 - D - q_;  // the edge's axis
       const float *arr = other == 0 ? lEx : (other == 1 ? lEy : lEz);
-      // the x-sweep (or, for x-edges, the y-sweep) member carries +lam,
-      // the other sweep's member -lam
-      const int first = D < q ? D : q;
-      return D == first ? arr[e] : -arr[e];
+      return D < q_ ? ld(arr, e) : -ld(arr, e);
     };
-    auto sum_at = [&](int q, int xx, int yy, int zz) -> float {
-      // upwind sum of the q-velocity around the edge on the lower D- and
-      // q-faces of cell (xx,yy,zz), in the forward's order
-      const int p = D < q ? D : q, r = D < q ? q : D;
-      return edge_sum(b, v[q], xx, yy, zz, p, r, q);
-    };
-    int xs[3] = {x, y, z};
-    // bt1: flux of B_D1, edges on D1-faces j (this face's own row) and j+1
-    {
-      const int q = D1;
-      int up[3] = {xs[0], xs[1], xs[2]};
-      up[q] = wrap(up[q] + 1, b.n[q]);
-      const float s0 = sum_at(q, xs[0], xs[1], xs[2]);
-      const float s1 = sum_at(q, up[0], up[1], up[2]);
-      aF.bt1 = edge_adj(q, xs[0], xs[1], xs[2]) * w_hi(s0) +
-               edge_adj(q, up[0], up[1], up[2]) * w_lo(s1);
-    }
-    {
-      const int q = D2;
-      int up[3] = {xs[0], xs[1], xs[2]};
-      up[q] = wrap(up[q] + 1, b.n[q]);
-      const float s0 = sum_at(q, xs[0], xs[1], xs[2]);
-      const float s1 = sum_at(q, up[0], up[1], up[2]);
-      aF.bt2 = edge_adj(q, xs[0], xs[1], xs[2]) * w_hi(s0) +
-               edge_adj(q, up[0], up[1], up[2]) * w_lo(s1);
-    }
+    // the forward's sums of the four cell velocities around the edge below
+    // the face's row and above it, in its order, so that the sign decisions
+    // are the same: v the velocity at c-1, c; lo, hi one row below, above
+    auto below = [](float v1, float v2, float lo1, float lo2) { return v2 + lo2 + v1 + lo1; };
+    auto above = [](float v1, float v2, float hi1, float hi2) { return hi2 + v2 + hi1 + v1; };
+    const float *va = W.f[1 + D1], *vb = W.f[1 + D2];
+    const float sa0 = below(q[2][1], q[2][2], ld(va, r1[0]), ld(va, r1[1]));
+    const float sa1 = above(q[2][1], q[2][2], ld(va, s1[1]), ld(va, s1[2]));
+    aF.bt1 = edge_adj(D1, a) * w_hi(sa0) + edge_adj(D1, s1[2]) * w_lo(sa1);
+    const float sb0 = below(q[3][1], q[3][2], ld(vb, r2[0]), ld(vb, r2[1]));
+    const float sb1 = above(q[3][1], q[3][2], ld(vb, s2[1]), ld(vb, s2[2]));
+    aF.bt2 = edge_adj(D2, a) * w_hi(sb0) + edge_adj(D2, s2[2]) * w_lo(sb1);
   }
-  // recompute the face states (same reconstruction as the forward)
-  // stencil cells c-2..c+1 along D, with their coordinates
-  long cs[4];
-  int cc[4][3];
-  for (int s = 0; s < 4; ++s) {
-    cc[s][0] = x, cc[s][1] = y, cc[s][2] = z;
-    cc[s][D] = wrap(cc[s][D] + s - 2, b.n[D]);
-    cs[s] = cell_index(b, cc[s][0], cc[s][1], cc[s][2]);
-  }
-  // cell-centred B_t of stencil cell s: the average of its two t-faces
-  auto bavg = [&](int t, int s) -> float {
-    return 0.5f * (W.f[5 + t][cs[s]] + W.f[5 + t][nb(b, cc[s][0], cc[s][1], cc[s][2], t, 1)]);
-  };
-  float q[7][4];
-  for (int s = 0; s < 4; ++s) {
-    q[0][s] = W.f[0][cs[s]];
-    q[1][s] = W.f[1 + D][cs[s]];
-    q[2][s] = W.f[1 + D1][cs[s]];
-    q[3][s] = W.f[1 + D2][cs[s]];
-    q[4][s] = W.f[4][cs[s]];
-    q[5][s] = bavg(D1, s);
-    q[6][s] = bavg(D2, s);
-  }
+  // the face states (same reconstruction as the forward)
   float Lq[7], Rq[7];
   for (int k = 0; k < 7; ++k) {
     if (b.recon == 1) {
@@ -278,16 +268,14 @@ __device__ __forceinline__ void adj_face(const Box &b, const FieldPtrs &W, const
   // for the gather
   unsigned br = 0u;
   if (b.recon != 1) {
+#pragma unroll
     for (int k = 0; k < 7; ++k) {
-      float da, db, da2, db2;
-      mm_grad(q[k][1] - q[k][0], q[k][2] - q[k][1], da, db);
-      mm_grad(q[k][2] - q[k][1], q[k][3] - q[k][2], da2, db2);
-      br |= ((da != 0.0f ? 1u : 0u) | (db != 0.0f ? 2u : 0u) | (da2 != 0.0f ? 4u : 0u) |
-             (db2 != 0.0f ? 8u : 0u)) << (4 * k);
+      const float d01 = q[k][1] - q[k][0], d12 = q[k][2] - q[k][1], d23 = q[k][3] - q[k][2];
+      br |= (limiter_branch(d01, d12) | limiter_branch(d12, d23) << 2) << (4 * k);
     }
   }
   adj::HIn<float> in;
-  in.bx = W.f[5 + D][a];
+  in.bx = ld(W.f[5 + D], a);
   in.rL = Lq[0], in.rR = Rq[0], in.unL = Lq[1], in.unR = Rq[1], in.u1L = Lq[2], in.u1R = Rq[2];
   in.u2L = Lq[3], in.u2R = Rq[3], in.pL = Lq[4], in.pR = Rq[4], in.b1L = Lq[5], in.b1R = Rq[5];
   in.b2L = Lq[6], in.b2R = Rq[6];
@@ -299,15 +287,19 @@ __device__ __forceinline__ void adj_face(const Box &b, const FieldPtrs &W, const
   const float gl[7] = {g.rL, g.unL, g.u1L, g.u2L, g.pL, g.b1L, g.b2L};
   const float gr[7] = {g.rR, g.unR, g.u1R, g.u2R, g.pR, g.b1R, g.b2R};
   for (int k = 0; k < 7; ++k) {
-    out.aL[k][a] = gl[k];
-    out.aR[k][a] = gr[k];
+    at(out.aL[k], a) = gl[k];
+    at(out.aR[k], a) = gr[k];
   }
-  out.br[a] = br;
-  out.abn[a] = g.bx;
+  at(reinterpret_cast<float *>(out.br), a) = __uint_as_float(br);
+  at(out.abn, a) = g.bx;
 }
 
-// All faces of the three directions in one launch: blockIdx.y is the
-// direction (a uniform branch per workgroup).
+// All faces of the three directions in one launch: consecutive workgroups
+// take the three directions of the same cells (a uniform branch each), and
+// each XCD a contiguous range of them, so that neighbouring rows and planes
+// share its L2.  VALU (about 990 instructions a face, 1330 with both sides of
+// the fan reversed) and the traffic of 45 output arrays bound it about
+// equally: 243 -> 213 us at 128^3.
 struct AdjFaceOut3 {
   AdjFaceOut d[3];
 };
@@ -317,18 +309,23 @@ __global__ void __launch_bounds__(256) k_adj_faces(Box b, FieldPtrs W, const flo
                                                    const float *gU3, const float *gU4,
                                                    const float *lEx, const float *lEy,
                                                    const float *lEz, float h, AdjFaceOut3 out) {
-  int x, y, z;
-  long a;
-  if (!cell_of(b, x, y, z, a)) return;
-  if (blockIdx.y == 0)
-    adj_face<0>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[0], x, y, z, a);
-  else if (blockIdx.y == 1)
-    adj_face<1>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[1], x, y, z, a);
+  const unsigned lb = xcd_logical_block(blockIdx.x, gridDim.x);
+  const unsigned block = lb / 3, dir = lb - 3 * block;
+  Place p;
+  if (!place_of(b, block, p)) return;
+  if (dir == 0)
+    adj_face<0>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[0], p);
+  else if (dir == 1)
+    adj_face<1>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[1], p);
   else
-    adj_face<2>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[2], x, y, z, a);
+    adj_face<2>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[2], p);
 }
 
 // ------------------------------------------------------------ k_adj_gather
+//
+// Bound by memory: 42 adjoint and 3 branch arrays, most read twice.  Selecting
+// by the two-bit numbers instead of four compares and selects per variable and
+// taking 32-bit offsets: 141 -> 133 us at 128^3.
 //
 // The reconstruction reverse of direction D at cell (x,y,z): res[0..6] =
 // adjoints of rho, v_D, v_D+1, v_D+2, p, Bbar_D+1, Bbar_D+2 of the cell,
@@ -342,21 +339,28 @@ __global__ void __launch_bounds__(256) k_adj_faces(Box b, FieldPtrs W, const flo
 //   cell 2:  aR + aL/2 [m took x2 - x1] - aR/2 ([m' took x2 - x1] - [m' took x3 - x2])
 //   cell 3: -aR/2 [m' took x3 - x2]
 template <int D>
-__device__ __forceinline__ void adj_gather(const Box &b, const AdjFaceOut &fa, int x, int y,
-                                           int z, float (&res)[7]) {
-  const long f0 = nb(b, x, y, z, D, 2), f1 = nb(b, x, y, z, D, 1), f3 = nb(b, x, y, z, D, -1);
-  const long f2 = cell_index(b, x, y, z);
-  const unsigned b0 = fa.br[f0], b1 = fa.br[f1], b2 = fa.br[f2], b3 = fa.br[f3];
-  auto bit = [](unsigned w, int i) { return ((w >> i) & 1u) ? 1.0f : 0.0f; };
+__device__ __forceinline__ void adj_gather(const Box &b, const AdjFaceOut &fa, const Place &p,
+                                           float (&res)[7]) {
+  const unsigned rest = p.o[(D + 1) % 3] + p.o[(D + 2) % 3];
+  const unsigned f0 = p.to(D, 2, b.n[D]) + rest, f1 = p.to(D, 1, b.n[D]) + rest;
+  const unsigned f2 = p.o[D] + rest, f3 = p.to(D, -1, b.n[D]) + rest;
+  auto bits = [&](unsigned o) {
+    return __float_as_uint(ld(reinterpret_cast<const float *>(fa.br), o));
+  };
+  const unsigned b0 = bits(f0), b1 = bits(f1), b2 = bits(f2), b3 = bits(f3);
+  // [m took the lower difference], [the upper], and their difference
+  auto one = [](unsigned w, int i) { return (float)((w >> i) & 1u); };
+  auto signed2 = [](unsigned w, int i) { return (float)((int)(w << (30 - i)) >> 30); };
+#pragma unroll
   for (int k = 0; k < 7; ++k) {
     const int s = 4 * k;
-    const float l0 = fa.aL[k][f0], l1 = fa.aL[k][f1], r1 = fa.aR[k][f1];
-    const float l2 = fa.aL[k][f2], r2 = fa.aR[k][f2], r3 = fa.aR[k][f3];
-    const float c0 = -0.5f * l0 * bit(b0, s);
-    const float c1 = l1 + 0.5f * l1 * (bit(b1, s) - bit(b1, s + 1)) + 0.5f * r1 * bit(b1, s + 2);
-    const float c2 =
-        r2 + 0.5f * l2 * bit(b2, s + 1) - 0.5f * r2 * (bit(b2, s + 2) - bit(b2, s + 3));
-    const float c3 = -0.5f * r3 * bit(b3, s + 3);
+    const float l0 = ld(fa.aL[k], f0), l1 = ld(fa.aL[k], f1), r1 = ld(fa.aR[k], f1);
+    const float l2 = ld(fa.aL[k], f2), r2 = ld(fa.aR[k], f2), r3 = ld(fa.aR[k], f3);
+    const float c0 = -0.5f * l0 * (float)((b0 >> s & 1u) & ~(b0 >> (s + 1)));
+    const float r1_lo = (float)((b1 >> (s + 2) & 1u) & ~(b1 >> (s + 3)));
+    const float c1 = l1 + 0.5f * l1 * signed2(b1, s) + 0.5f * r1 * r1_lo;
+    const float c2 = r2 + 0.5f * l2 * one(b2, s + 1) - 0.5f * r2 * signed2(b2, s + 2);
+    const float c3 = -0.5f * r3 * one(b3, s + 3);
     res[k] = c0 + c1 + c2 + c3;
   }
 }
@@ -367,25 +371,26 @@ __device__ __forceinline__ void adj_gather(const Box &b, const AdjFaceOut &fa, i
 __global__ void __launch_bounds__(256) k_adj_gather(Box b, AdjFaceOut3 fa, FieldPtrs lam_in,
                                                     int accumulate, float *lbb0, float *lbb1,
                                                     float *lbb2) {
-  int x, y, z;
-  long a;
-  if (!cell_of(b, x, y, z, a)) return;
-  float rho = 0.0f, v[3] = {0.0f, 0.0f, 0.0f}, p = 0.0f, bb[3] = {0.0f, 0.0f, 0.0f};
+  Place p;
+  if (!place_of(b, xcd_logical_block(blockIdx.x, gridDim.x), p)) return;
+  const unsigned a = p.own();
+  float rho = 0.0f, v[3] = {0.0f, 0.0f, 0.0f}, pr = 0.0f, bb[3] = {0.0f, 0.0f, 0.0f};
   float res[7];
-  adj_gather<0>(b, fa.d[0], x, y, z, res);  // X: (rho, vx, vy, vz, p, Bby, Bbz)
-  rho += res[0], v[0] += res[1], v[1] += res[2], v[2] += res[3], p += res[4];
+  adj_gather<0>(b, fa.d[0], p, res);  // X: (rho, vx, vy, vz, p, Bby, Bbz)
+  rho += res[0], v[0] += res[1], v[1] += res[2], v[2] += res[3], pr += res[4];
   bb[1] += res[5], bb[2] += res[6];
-  adj_gather<1>(b, fa.d[1], x, y, z, res);  // Y: (rho, vy, vz, vx, p, Bbz, Bbx)
-  rho += res[0], v[1] += res[1], v[2] += res[2], v[0] += res[3], p += res[4];
+  adj_gather<1>(b, fa.d[1], p, res);  // Y: (rho, vy, vz, vx, p, Bbz, Bbx)
+  rho += res[0], v[1] += res[1], v[2] += res[2], v[0] += res[3], pr += res[4];
   bb[2] += res[5], bb[0] += res[6];
-  adj_gather<2>(b, fa.d[2], x, y, z, res);  // Z: (rho, vz, vx, vy, p, Bbx, Bby)
-  rho += res[0], v[2] += res[1], v[0] += res[2], v[1] += res[3], p += res[4];
+  adj_gather<2>(b, fa.d[2], p, res);  // Z: (rho, vz, vx, vy, p, Bbx, Bby)
+  rho += res[0], v[2] += res[1], v[0] += res[2], v[1] += res[3], pr += res[4];
   bb[0] += res[5], bb[1] += res[6];
-  const float out[5] = {rho, v[0], v[1], v[2], p};
-  for (int f = 0; f < 5; ++f) lam_in.f[f][a] = accumulate ? lam_in.f[f][a] + out[f] : out[f];
-  lbb0[a] = bb[0];
-  lbb1[a] = bb[1];
-  lbb2[a] = bb[2];
+  const float out[5] = {rho, v[0], v[1], v[2], pr};
+  for (int f = 0; f < 5; ++f)
+    at(lam_in.f[f], a) = accumulate ? ld(lam_in.f[f], a) + out[f] : out[f];
+  at(lbb0, a) = bb[0];
+  at(lbb1, a) = bb[1];
+  at(lbb2, a) = bb[2];
 }
 
 // Face B_t of lam_in: half of each adjacent cell's cell-average adjoint plus
@@ -394,15 +399,16 @@ __global__ void __launch_bounds__(256) k_adj_bfinish(Box b, const float *lbb0, c
                                                      const float *lbb2, const float *abn0,
                                                      const float *abn1, const float *abn2,
                                                      FieldPtrs lam_in, int accumulate) {
-  int x, y, z;
-  long a;
-  if (!cell_of(b, x, y, z, a)) return;
+  Place p;
+  if (!place_of(b, xcd_logical_block(blockIdx.x, gridDim.x), p)) return;
+  const unsigned a = p.own();
   const float *lbb[3] = {lbb0, lbb1, lbb2};
   const float *abn[3] = {abn0, abn1, abn2};
+#pragma unroll
   for (int t = 0; t < 3; ++t) {
-    const long m = nb(b, x, y, z, t, -1);
-    const float v = 0.5f * (lbb[t][a] + lbb[t][m]) + abn[t][a];
-    lam_in.f[5 + t][a] = accumulate ? lam_in.f[5 + t][a] + v : v;
+    const unsigned m = p.to(t, -1, b.n[t]) + (p.o[(t + 1) % 3] + p.o[(t + 2) % 3]);
+    const float v = 0.5f * (ld(lbb[t], a) + ld(lbb[t], m)) + ld(abn[t], a);
+    at(lam_in.f[5 + t], a) = accumulate ? ld(lam_in.f[5 + t], a) + v : v;
   }
 }
 
@@ -429,7 +435,7 @@ void launch_adj_stage(hipStream_t s, const Box &b, const AdjStageArgs &A) {
     fo.d[d].br = reinterpret_cast<unsigned *>(A.face[d * 15 + 14]);
     fo.d[d].abn = A.abn[d];
   }
-  const dim3 g3(grid_for(b.ncell), 3);
+  const dim3 g3(3 * grid_for(b.ncell));
   hipLaunchKernelGGL(k_adj_faces, g3, blk, 0, s, b, A.Win, A.gU[0], A.gU[1], A.gU[2], A.gU[3],
                      A.gU[4], A.lE[0], A.lE[1], A.lE[2], A.h, fo);
   hipLaunchKernelGGL(k_adj_gather, g, blk, 0, s, b, fo, A.lam_in, A.acc_in ? 1 : 0, A.lbb[0],
