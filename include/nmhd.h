@@ -242,7 +242,7 @@ int nmhd_get_tiles(const nmhd_ctx *ctx, int *faces_tile, int *update_tile);
  * equivalent is one MHDSolver::proceed (INL:1086-1204) per box, run one
  * after another.  Every box keeps its own time, CFL dt and goal clipping;
  * its results are bit-identical to the same box advanced alone by an
- * nmhd_ctx on NMHD_PATH_TILED.  Each RK stage is two persistent launches
+ * nmhd_ctx on NMHD_PATH_TILED.  Each RK stage is two launches
  * over a work table of tiles from all boxes; runs replay the step as a HIP
  * graph.  Any descriptor a context accepts may be batched (periodic and
  * shearing boxes, ghost layers, sources and quirk corrections per box), at
@@ -270,9 +270,10 @@ int nmhd_batch_get_status(nmhd_batch *batch, int box, int *steps_taken, int *goa
 
 /* Tiling: tile shape (enum nmhd_tile) of box's face and update kernels
  * (box = -1: every box); z chunk (planes per work item) and workgroups per
- * CU of the two persistent launches, where 0 (the default) launches one
- * workgroup per work item instead, one launch per tile shape.  Results do
- * not depend on the tiling or the launch mode. */
+ * CU that walk the work table of the two kernels, where 0 (the default)
+ * launches one workgroup per work item instead.  Until a chunk is set, each
+ * kernel takes the one that a cost model expects to be fastest for the boxes
+ * of the batch.  Results do not depend on the tiling or the launch mode. */
 int nmhd_batch_set_tiles(nmhd_batch *batch, int box, int faces_tile, int update_tile);
 int nmhd_batch_set_launch(nmhd_batch *batch, int faces_zchunk, int update_zchunk,
                           int faces_wg_per_cu, int update_wg_per_cu);

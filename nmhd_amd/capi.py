@@ -346,7 +346,7 @@ def hlld_batch(inputs, gamma=5.0 / 3.0, strict=False):
 
 class Batch:
     """Many independent periodic boxes advanced together (nmhd_batch_*):
-    per-box time and dt, persistent tile launches, HIP-graph replay."""
+    per-box time and dt, launches over every box's tiles, HIP-graph replay."""
 
     def __init__(self, cfgs):
         L = load()

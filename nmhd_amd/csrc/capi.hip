@@ -387,7 +387,6 @@ int nmhd_create(const nmhd_desc *desc, nmhd_ctx **out) {
   if (hipGetDevice(&c->device) != hipSuccess) return bail(NMHD_EHIP, "no HIP device");
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess)
     return bail(NMHD_EHIP, "hipStreamCreate failed");
-  const size_t bytes = sizeof(float) * (size_t)c->box.ncell;
   const size_t stride = array_stride(c->box.ncell);
   if (hipMalloc(&c->arrays, 45 * stride * sizeof(float)) != hipSuccess)
     return bail(NMHD_ENOMEM, "state allocation failed");

@@ -1,10 +1,9 @@
 // capi_batch.hip -- the nmhd_batch_* entry points of include/nmhd.h: many
 // independent boxes (periodic or shearing) in shared pools, per-box step
 // records, per-box ghost fills, a work
-// table of tiles for the stage kernels (grouped by tile shape: one launch per
-// shape with a workgroup per tile, or one persistent launch over the whole
-// table), HIP-graph replay of the step, and the autotuner of tile shapes and
-// launch parameters.
+// table of tiles for the stage kernels (a workgroup per tile, or workgroups
+// that walk the table), HIP-graph replay of the step, and the autotuner of
+// tile shapes and launch parameters.
 //
 // Pools: state[k] (k = 0..2, the rotating W^n / W* / W^{n+1} copies) holds
 // the 8 fields of every box back to back (box b at BatchBox::off8, field f at
@@ -51,22 +50,19 @@ struct nmhd_batch {
   long total8 = 0, total21 = 0;
   float *state[3] = {};
   float *flux = nullptr;
-  StepState *st = nullptr;
+  // step records: rec + k * nbox holds those of the steps that left state[k]
+  StepState *rec = nullptr;
   StepState *st_tune = nullptr;
   float *d_goal = nullptr;
   int cur = 0;
   int integrator = NMHD_MIDPOINT2;
   std::vector<int> ftile, utile;
-  // workgroups per CU of the persistent launches; 0: one workgroup per work
-  // item, one launch per tile shape
-  int fzc = 16, uzc = 16, fwg = 0, uwg = 0;
+  // z chunks (0: by default_chunk) and workgroups per CU that walk the table
+  // (0: one workgroup per work item)
+  int fzc = 0, uzc = 0, fwg = 0, uwg = 0;
   WorkItem *d_fitems = nullptr, *d_uitems = nullptr, *d_titems = nullptr;
   int nf = 0, nu = 0;
-  int nfv[TV_COUNT] = {}, nuv[TV_COUNT] = {};  // items per tile shape (the lists are grouped)
-  // side streams and events that let the launches of different tile shapes
-  // run concurrently (forked from and joined back into stream)
-  hipStream_t side[TV_COUNT - 1] = {};
-  hipEvent_t ev_fork = nullptr, ev_join[TV_COUNT - 1] = {};
+  bool fwide = false;  // 64x4 tiles among the face items
   size_t cap_f = 0, cap_u = 0, cap_t = 0;
   bool items_dirty = true;
   bool cfl_valid = false;
@@ -95,13 +91,11 @@ int bfail(nmhd_batch *b, int code, const std::string &msg) {
   } while (0)
 
 // Work items of the given boxes: tiles of tile shape tile[box], z chunks of
-// zc planes, grouped by tile shape, then box by box, x fastest, then y, then
-// z; counts[v] (optional) receives the number of items of shape v.
+// zc planes, grouped by tile shape, then box by box, x fastest, then y, then z.
 std::vector<WorkItem> make_items(const nmhd_batch *b, const std::vector<int> &tile, int zc,
-                                 const std::vector<int> &which, int *counts = nullptr) {
+                                 const std::vector<int> &which) {
   std::vector<WorkItem> out;
   for (int v = 0; v < TV_COUNT; ++v) {
-    const size_t start = out.size();
     const int TX = kTileTX[v], TY = kTileTY[v];
     for (int box : which) {
       if (tile[box] != v) continue;
@@ -117,10 +111,36 @@ std::vector<WorkItem> make_items(const nmhd_batch *b, const std::vector<int> &ti
             out.push_back(w);
           }
     }
-    if (counts) counts[v] = (int)(out.size() - start);
   }
   return out;
 }
+
+bool has_wide(const std::vector<WorkItem> &items) {
+  for (const WorkItem &w : items)
+    if (w.variant == TV_64x4) return true;
+  return false;
+}
+
+// The chunk at which march_chunk expects a launch over every box's tiles to
+// end first.  Chunks of 16 planes, as a large box would take, left 14 boxes of
+// 16..96 cells per edge with one workgroup per CU: 291 us a step against 169;
+// 64 such boxes, which fill the GPU either way, get them still.
+int default_chunk(const nmhd_batch *b, bool faces) {
+  const std::vector<int> &tile = faces ? b->ftile : b->utile;
+  int nz = 1;
+  for (const BatchBox &bb : b->boxes) nz = std::max(nz, bb.b.n[2]);
+  return march_chunk(faces, nz, [&](int zc) {
+    long n = 0;
+    for (int i = 0; i < b->nbox; ++i) {
+      const Box &x = b->boxes[i].b;
+      const long tx = kTileTX[tile[i]], ty = kTileTY[tile[i]];
+      n += (x.n[0] + tx - 1) / tx * ((x.n[1] + ty - 1) / ty) * ((x.n[2] + zc - 1) / zc);
+    }
+    return n;
+  });
+}
+int faces_chunk(const nmhd_batch *b) { return b->fzc ? b->fzc : default_chunk(b, true); }
+int update_chunk(const nmhd_batch *b) { return b->uzc ? b->uzc : default_chunk(b, false); }
 
 std::vector<int> all_boxes(const nmhd_batch *b) {
   std::vector<int> v(b->nbox);
@@ -152,110 +172,54 @@ void drop_graphs(nmhd_batch *b) {
 int refresh_items(nmhd_batch *b) {
   if (!b->items_dirty) return NMHD_OK;
   const std::vector<int> all = all_boxes(b);
-  const std::vector<WorkItem> f = make_items(b, b->ftile, b->fzc, all, b->nfv);
-  const std::vector<WorkItem> u = make_items(b, b->utile, b->uzc, all, b->nuv);
+  const std::vector<WorkItem> f = make_items(b, b->ftile, faces_chunk(b), all);
+  const std::vector<WorkItem> u = make_items(b, b->utile, update_chunk(b), all);
   int r = upload_items(b, f, &b->d_fitems, &b->cap_f);
   if (r) return r;
   r = upload_items(b, u, &b->d_uitems, &b->cap_u);
   if (r) return r;
   b->nf = (int)f.size();
   b->nu = (int)u.size();
+  b->fwide = has_wide(f);
   drop_graphs(b);
   b->items_dirty = false;
   return NMHD_OK;
 }
 
-int grid_of(int nitems, int wg_per_cu, int cus) {
-  return std::max(1, std::min(nitems, wg_per_cu * cus));
-}
-
-// One launch per tile shape that has items, launch(stream, shape, offset):
-// the first on s, the others on side streams forked from s and joined back
-// into it.  The shapes' items belong to different boxes, so the launches are
-// independent, and running them side by side fills the GPU where a small
-// launch alone would not (and hides each launch's tail).  Works eagerly and
-// under graph capture.
-template <class F>
-int over_shapes(nmhd_batch *b, hipStream_t s, const int *counts, F &&launch) {
-  int used[TV_COUNT], off[TV_COUNT], nused = 0;
-  for (int v = 0, o = 0; v < TV_COUNT; o += counts[v], ++v)
-    if (counts[v] > 0) used[nused] = v, off[nused++] = o;
-  if (nused == 0) return NMHD_OK;
-  if (nused > 1) BHIP(b, hipEventRecord(b->ev_fork, s));
-  launch(s, used[0], off[0]);
-  for (int k = 1; k < nused; ++k) {
-    hipStream_t t = b->side[k - 1];
-    BHIP(b, hipStreamWaitEvent(t, b->ev_fork, 0));
-    launch(t, used[k], off[k]);
-    BHIP(b, hipEventRecord(b->ev_join[k - 1], t));
-    BHIP(b, hipStreamWaitEvent(s, b->ev_join[k - 1], 0));
-  }
-  return NMHD_OK;
-}
-
-// The face / update launches of one stage over a grouped item list: the
-// persistent kernel with wg workgroups per CU, or (wg == 0) one launch per
-// tile shape with one workgroup per item.
-int faces_over(nmhd_batch *b, hipStream_t s, int wg, const WorkItem *items, int n,
-               const int *counts, float *state, const StepState *st, int hsel) {
-  if (wg > 0) {
-    launch_batch_faces(s, grid_of(n, wg, b->cus), b->d_boxes, items, n, state, b->flux, st, hsel);
-    return NMHD_OK;
-  }
-  return over_shapes(b, s, counts, [&](hipStream_t t, int v, int off) {
-    launch_batch_faces_items(t, v, b->d_boxes, items + off, counts[v], state, b->flux, st, hsel);
-  });
-}
-
-int update_over(nmhd_batch *b, hipStream_t s, int wg, const WorkItem *items, int n,
-                const int *counts, float *in, float *base, float *out, StepState *st, int hsel,
-                bool cfl) {
-  if (wg > 0) {
-    launch_batch_update(s, grid_of(n, wg, b->cus), b->d_boxes, items, n, in, b->flux, base, out,
-                        st, hsel, cfl);
-    return NMHD_OK;
-  }
-  return over_shapes(b, s, counts, [&](hipStream_t t, int v, int off) {
-    launch_batch_update_items(t, v, b->d_boxes, items + off, counts[v], in, b->flux, base, out,
-                              st, hsel, cfl);
-  });
+// workgroups that walk a table of nitems; 0 (wg_per_cu == 0): one per item
+int grid_of(const nmhd_batch *b, int nitems, int wg_per_cu) {
+  return std::min(nitems, wg_per_cu * b->cus);
 }
 
 // One iteration of the proceed() loop for every box.
-int enqueue_step(nmhd_batch *b, bool full_cfl, float goal) {
+void enqueue_step(nmhd_batch *b, bool full_cfl, float goal) {
   hipStream_t s = b->stream;
   const int A = b->cur, n = b->nbox;
-  launch_batch_begin(s, b->st, n, full_cfl);
+  const int B = (A + 1) % 3, next = b->integrator == NMHD_EULER1 ? B : (A + 2) % 3;
+  StepState *const in = b->rec + A * n, *const rec = b->rec + next * n;
   // ghost fills of the boxes that have ghost layers, then the CFL minimum:
   // a full pass, or the ghost cells added to the stage-2 epilogue's minimum
-  if (b->grid_gy) launch_batch_ghost_y(s, b->d_boxes, n, b->grid_gy, b->state[A], b->st);
-  if (b->grid_gz) launch_batch_ghost_z(s, b->d_boxes, n, b->grid_gz, b->state[A], b->st);
+  if (b->grid_gy) launch_batch_ghost_y(s, b->d_boxes, n, b->grid_gy, b->state[A], in);
+  if (b->grid_gz) launch_batch_ghost_z(s, b->d_boxes, n, b->grid_gz, b->state[A], in);
   if (full_cfl)
-    launch_batch_cfl(s, b->d_boxes, n, b->state[A], goal, b->st);
+    launch_batch_cfl(s, b->d_boxes, n, b->state[A], goal, in);
   else if (b->grid_gcfl)
-    launch_batch_cfl_ghosts(s, b->d_boxes, n, b->grid_gcfl, b->state[A], b->st);
-  launch_batch_dt(s, b->st, n, b->d_goal);
-  auto stage = [&](int in, int base, int out, int hsel, bool last) {
-    const int r = faces_over(b, s, b->fwg, b->d_fitems, b->nf, b->nfv, b->state[in], b->st, hsel);
-    if (r) return r;
-    return update_over(b, s, b->uwg, b->d_uitems, b->nu, b->nuv, b->state[in], b->state[base],
-                       b->state[out], b->st, hsel, last);
+    launch_batch_cfl_ghosts(s, b->d_boxes, n, b->grid_gcfl, b->state[A], in);
+  auto stage = [&](int from, int base, int to, int hsel, bool first, bool last) {
+    launch_batch_faces(s, grid_of(b, b->nf, b->fwg), b->d_boxes, b->d_fitems, b->nf,
+                       b->state[from], b->flux,
+                       BatchStep{rec, first ? in : nullptr, b->d_goal, hsel}, b->fwide);
+    launch_batch_update(s, grid_of(b, b->nu, b->uwg), b->d_boxes, b->d_uitems, b->nu,
+                        b->state[from], b->flux, b->state[base], b->state[to],
+                        BatchStep{rec, nullptr, nullptr, hsel}, last);
   };
-  int next, r;
   if (b->integrator == NMHD_EULER1) {
-    next = (A + 1) % 3;
-    r = stage(A, A, next, H_FULL, true);
+    stage(A, A, next, H_FULL, true, true);
   } else {
-    const int B = (A + 1) % 3;
-    next = (A + 2) % 3;
-    r = stage(A, A, B, H_HALF, false);
-    if (!r) r = stage(B, A, next, H_FULL, true);
+    stage(A, A, B, H_HALF, true, false);
+    stage(B, A, next, H_FULL, false, true);
   }
-  if (r) return r;
-  launch_batch_copy(s, b->d_boxes, n, b->state[A], b->state[next], b->st);
-  launch_batch_commit(s, b->st, n);
   b->cur = next;
-  return NMHD_OK;
 }
 
 int ensure_graph(nmhd_batch *b) {
@@ -263,13 +227,9 @@ int ensure_graph(nmhd_batch *b) {
   if (b->exec[phase]) return NMHD_OK;
   hipGraph_t g = nullptr;
   BHIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-  const int re = enqueue_step(b, false, 0.0f);
+  enqueue_step(b, false, 0.0f);
   const hipError_t e = hipStreamEndCapture(b->stream, &g);
   b->cur = phase;  // capture records; it does not advance the state
-  if (re) {
-    if (g) (void)hipGraphDestroy(g);
-    return re;
-  }
   if (e != hipSuccess)
     return bfail(b, NMHD_EHIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
   const hipError_t ei = hipGraphInstantiate(&b->exec[phase], g, nullptr, nullptr, 0);
@@ -281,17 +241,25 @@ int ensure_graph(nmhd_batch *b) {
   return NMHD_OK;
 }
 
+// The records as the last enqueued step leaves them, committed.
 int read_records(nmhd_batch *b, std::vector<StepState> &h) {
   h.resize(b->nbox);
-  BHIP(b, hipMemcpyAsync(h.data(), b->st, sizeof(StepState) * b->nbox, hipMemcpyDeviceToHost,
-                         b->stream));
+  BHIP(b, hipMemcpyAsync(h.data(), b->rec + b->cur * b->nbox, sizeof(StepState) * b->nbox,
+                         hipMemcpyDeviceToHost, b->stream));
   BHIP(b, hipStreamSynchronize(b->stream));
+  for (StepState &s : h)
+    if (s.active) {
+      s.t = s.t_next;
+      s.generation += 1;
+      s.steps_done += 1;
+      s.active = 0;
+    }
   return NMHD_OK;
 }
 
 int write_records(nmhd_batch *b, const std::vector<StepState> &h) {
-  BHIP(b, hipMemcpyAsync(b->st, h.data(), sizeof(StepState) * b->nbox, hipMemcpyHostToDevice,
-                         b->stream));
+  BHIP(b, hipMemcpyAsync(b->rec + b->cur * b->nbox, h.data(), sizeof(StepState) * b->nbox,
+                         hipMemcpyHostToDevice, b->stream));
   BHIP(b, hipStreamSynchronize(b->stream));
   return NMHD_OK;
 }
@@ -300,24 +268,17 @@ void free_batch(nmhd_batch *b) {
   drop_graphs(b);
   for (auto &p : b->state)
     if (p) (void)hipFree(p), p = nullptr;
-  void *ptrs[] = {b->flux, b->st, b->st_tune, b->d_goal, b->d_boxes,
+  void *ptrs[] = {b->flux, b->rec, b->st_tune, b->d_goal, b->d_boxes,
                   b->d_fitems, b->d_uitems, b->d_titems};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   b->flux = nullptr;
-  b->st = b->st_tune = nullptr;
+  b->rec = b->st_tune = nullptr;
   b->d_goal = nullptr;
   b->d_boxes = nullptr;
   b->d_fitems = b->d_uitems = b->d_titems = nullptr;
-  for (auto &t : b->side)
-    if (t) (void)hipStreamDestroy(t), t = nullptr;
-  for (auto &e : b->ev_join)
-    if (e) (void)hipEventDestroy(e), e = nullptr;
-  if (b->ev_fork) (void)hipEventDestroy(b->ev_fork), b->ev_fork = nullptr;
   if (b->stream) (void)hipStreamDestroy(b->stream), b->stream = nullptr;
 }
-
-int default_tile(int nx) { return nx >= 64 ? TV_64x4 : (nx >= 32 ? TV_32x8 : TV_16x16); }
 
 // ------------------------------------------------------------ autotuner
 
@@ -425,6 +386,7 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
   if (r) return r;
   float *in = b->state[b->cur];
   float *scratch = b->state[(b->cur + 1) % 3];
+  const BatchStep step{b->st_tune, nullptr, nullptr, H_HALF};
   int ntimed = 0;
 
   // per shape: the workgroup-time of each tile shape
@@ -448,8 +410,8 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
         r = time_launch(
             b,
             [&] {
-              launch_batch_faces(b->stream, 1, b->d_boxes, b->d_titems, n, in, b->flux,
-                                 b->st_tune, H_HALF);
+              launch_batch_faces(b->stream, 1, b->d_boxes, b->d_titems, n, in, b->flux, step,
+                                 true);
             },
             &msf);
         if (r) return r;
@@ -457,7 +419,7 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
             b,
             [&] {
               launch_batch_update(b->stream, 1, b->d_boxes, b->d_titems, n, in, b->flux, in,
-                                  scratch, b->st_tune, H_HALF, false);
+                                  scratch, step, false);
             },
             &msu);
         if (r) return r;
@@ -474,7 +436,7 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
     }
   }
 
-  // whole batch: z chunk and workgroups per CU of each persistent launch
+  // whole batch: z chunk and workgroups per CU of each launch
   const std::string lkey = launch_key(b);
   auto hit = cache.entries.find(lkey);
   if (hit == cache.entries.end() || hit->second.size() != 4) {
@@ -482,40 +444,35 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
     float best_f = 1e30f, best_u = 1e30f;
     int fzc = 16, uzc = 16, fwg = 0, uwg = 0;
     for (int zc : kZChunks) {
-      int cf[TV_COUNT], cu[TV_COUNT];
-      const std::vector<WorkItem> fi = make_items(b, b->ftile, zc, all, cf);
+      const std::vector<WorkItem> fi = make_items(b, b->ftile, zc, all);
       r = upload_items(b, fi, &b->d_titems, &b->cap_t);
       if (r) return r;
       for (int wg : kWgPerCu) {
         float ms = 0.0f;
         const int n = (int)fi.size();
-        int rl = NMHD_OK;
         r = time_launch(
             b,
             [&] {
-              if (!rl) rl = faces_over(b, b->stream, wg, b->d_titems, n, cf, in, b->st_tune, H_HALF);
+              launch_batch_faces(b->stream, grid_of(b, n, wg), b->d_boxes, b->d_titems, n, in,
+                                 b->flux, step, has_wide(fi));
             },
             &ms);
-        if (!r) r = rl;
         if (r) return r;
         if (ms < best_f) best_f = ms, fzc = zc, fwg = wg;
       }
-      const std::vector<WorkItem> ui = make_items(b, b->utile, zc, all, cu);
+      const std::vector<WorkItem> ui = make_items(b, b->utile, zc, all);
       r = upload_items(b, ui, &b->d_titems, &b->cap_t);
       if (r) return r;
       for (int wg : kWgPerCu) {
         float ms = 0.0f;
         const int n = (int)ui.size();
-        int rl = NMHD_OK;
         r = time_launch(
             b,
             [&] {
-              if (!rl)
-                rl = update_over(b, b->stream, wg, b->d_titems, n, cu, in, in, scratch,
-                                 b->st_tune, H_HALF, false);
+              launch_batch_update(b->stream, grid_of(b, n, wg), b->d_boxes, b->d_titems, n, in,
+                                  b->flux, in, scratch, step, false);
             },
             &ms);
-        if (!r) r = rl;
         if (r) return r;
         if (ms < best_u) best_u = ms, uzc = zc, uwg = wg;
       }
@@ -577,8 +534,8 @@ int nmhd_batch_create(const nmhd_desc *descs, int nbox, nmhd_batch **out) {
     b->boxes[i].off21 = off21;
     off8 += 8 * b->boxes[i].b.ncell;
     off21 += 21 * b->boxes[i].b.ncell;
-    b->ftile[i] = default_tile(b->boxes[i].b.n[0]);
-    b->utile[i] = b->boxes[i].b.n[0] >= 32 ? TV_32x8 : TV_16x16;
+    b->ftile[i] = tiled_shape(b->boxes[i].b.n[0], b->boxes[i].b.n[1], true);
+    b->utile[i] = tiled_shape(b->boxes[i].b.n[0], b->boxes[i].b.n[1], false);
   }
   b->total8 = off8;
   b->total21 = off21;
@@ -612,20 +569,12 @@ int nmhd_batch_create(const nmhd_desc *descs, int nbox, nmhd_batch **out) {
   if (colon != std::string::npos) b->arch = b->arch.substr(0, colon);
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
     return bail(NMHD_EHIP, "hipStreamCreate failed");
-  for (auto &t : b->side)
-    if (hipStreamCreateWithFlags(&t, hipStreamNonBlocking) != hipSuccess)
-      return bail(NMHD_EHIP, "hipStreamCreate failed");
-  if (hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) != hipSuccess)
-    return bail(NMHD_EHIP, "hipEventCreate failed");
-  for (auto &e : b->ev_join)
-    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
-      return bail(NMHD_EHIP, "hipEventCreate failed");
   for (auto &p : b->state)
     if (hipMalloc(&p, sizeof(float) * (size_t)off8) != hipSuccess)
       return bail(NMHD_ENOMEM, "state pool allocation failed");
   if (hipMalloc(&b->flux, sizeof(float) * (size_t)off21) != hipSuccess)
     return bail(NMHD_ENOMEM, "flux pool allocation failed");
-  if (hipMalloc(&b->st, sizeof(StepState) * nbox) != hipSuccess ||
+  if (hipMalloc(&b->rec, 3 * sizeof(StepState) * nbox) != hipSuccess ||
       hipMalloc(&b->st_tune, sizeof(StepState) * nbox) != hipSuccess ||
       hipMalloc(&b->d_goal, sizeof(float)) != hipSuccess ||
       hipMalloc(&b->d_boxes, sizeof(BatchBox) * nbox) != hipSuccess)
@@ -636,7 +585,7 @@ int nmhd_batch_create(const nmhd_desc *descs, int nbox, nmhd_batch **out) {
   std::vector<StepState> h(nbox);
   std::memset(h.data(), 0, sizeof(StepState) * nbox);
   for (auto &s : h) s.cfl_bits = s.cfl_next_bits = 0x7f800000u;
-  if (hipMemcpyAsync(b->st, h.data(), sizeof(StepState) * nbox, hipMemcpyHostToDevice,
+  if (hipMemcpyAsync(b->rec, h.data(), sizeof(StepState) * nbox, hipMemcpyHostToDevice,
                      b->stream) != hipSuccess ||
       hipMemcpyAsync(b->d_boxes, b->boxes.data(), sizeof(BatchBox) * nbox,
                      hipMemcpyHostToDevice, b->stream) != hipSuccess ||
@@ -748,8 +697,8 @@ int nmhd_batch_set_launch(nmhd_batch *b, int fzc, int uzc, int fwg, int uwg) {
 
 int nmhd_batch_get_launch(const nmhd_batch *b, int *fzc, int *uzc, int *fwg, int *uwg) {
   if (!b) return NMHD_EINVAL;
-  if (fzc) *fzc = b->fzc;
-  if (uzc) *uzc = b->uzc;
+  if (fzc) *fzc = faces_chunk(b);
+  if (uzc) *uzc = update_chunk(b);
   if (fwg) *fwg = b->fwg;
   if (uwg) *uwg = b->uwg;
   return NMHD_OK;
@@ -767,7 +716,10 @@ int nmhd_batch_run(nmhd_batch *b, float goal_time, int nsteps, int use_graph, in
   std::vector<StepState> h;
   int r = read_records(b, h);
   if (r) return r;
-  for (auto &s : h) s.finished = s.active = s.goal_reached = s.steps_done = 0;
+  for (auto &s : h) {
+    s.finished = s.goal_reached = s.steps_done = 0;
+    if (!b->cfl_valid) s.cfl_next_bits = 0x7f800000u;  // for the full pass
+  }
   r = write_records(b, h);
   if (r) return r;
   r = refresh_items(b);
@@ -776,8 +728,7 @@ int nmhd_batch_run(nmhd_batch *b, float goal_time, int nsteps, int use_graph, in
                          b->stream));
   for (int k = 0; k < nsteps; ++k) {
     if (!b->cfl_valid) {
-      r = enqueue_step(b, true, goal_time);
-      if (r) return r;
+      enqueue_step(b, true, goal_time);
       b->cfl_valid = true;
     } else if (use_graph) {
       r = ensure_graph(b);
@@ -785,8 +736,7 @@ int nmhd_batch_run(nmhd_batch *b, float goal_time, int nsteps, int use_graph, in
       BHIP(b, hipGraphLaunch(b->exec[b->cur], b->stream));
       b->cur = b->integrator == NMHD_EULER1 ? (b->cur + 1) % 3 : (b->cur + 2) % 3;
     } else {
-      r = enqueue_step(b, false, goal_time);
-      if (r) return r;
+      enqueue_step(b, false, goal_time);
     }
   }
   BHIP(b, hipGetLastError());

@@ -102,12 +102,6 @@ inline unsigned grid_for(long n, int block = kBlock) {
 
 void host_displacement(const Box &b, double t, float *normalized, int *n, float *minor);
 
-// ------------------------------------------------ step record transitions
-// (shared by the single-box and the multi-box bookkeeping kernels)
-
-// Start a step.  full: the CFL minimum is rebuilt over every cell by a full
-// CFL pass; otherwise it starts from the stage-2 epilogue's minimum of the
-// current state (plus, with ghosts, the cells the ghost fill rewrote).
 // (x, y, z) of the cell at linear index a (x fastest), in 32-bit unsigned
 // arithmetic: a box holds fewer than 2^31 cells.
 __device__ __forceinline__ void cell_coords(const Box &b, long a, int &x, int &y, int &z) {
@@ -118,14 +112,8 @@ __device__ __forceinline__ void cell_coords(const Box &b, long a, int &x, int &y
   y = (int)(row - (unsigned)z * n1);
 }
 
-// A step enqueued after the run reached its goal is inactive and leaves the
-// record alone: cfl_next_bits then still holds the last active step's
-// minimum, which the first step of the next run starts from.
-__device__ __forceinline__ void step_begin(StepState &s, int full) {
-  if (s.finished) return;
-  s.cfl_bits = full ? 0x7f800000u : s.cfl_next_bits;
-  s.cfl_next_bits = 0x7f800000u;  // +inf
-}
+// ------------------------------------------------ step record transitions
+// (shared by the single-box and the multi-box kernels)
 
 // Decide the step: dt = CFL minimum, clipped so that t + dt <= goal
 // (proceed(), INL:1126-1137).
@@ -240,7 +228,7 @@ __host__ __device__ inline FluxSet box_fluxes(float *pool, const BatchBox &bb) {
   return F;
 }
 
-// One tile of a persistent launch: box, tile origin, z range, tile shape.
+// One tile of a batch launch: box, tile origin, z range, tile shape.
 struct WorkItem {
   int box;
   int xy;       // x0 | y0 << 16
@@ -288,35 +276,37 @@ void launch_update(hipStream_t s, const Box &b, FieldPtrs Win, const FluxSet &F,
                    FieldPtrs Wbase, FieldPtrs Wout, const StepState *st, int hsel,
                    bool pace_only);
 
-// kernels_batch.hip (persistent multi-box launches over a work table)
-void launch_batch_begin(hipStream_t s, StepState *st, int nbox, bool full);
+// The step a stage launch over a batch belongs to.  rec[box] is its record,
+// whose cfl_next_bits collects the CFL minimum of the state it produces.  The
+// step's first launch opens it from the records `in` of the step before (open_step's
+// transitions, per box; *goal in device memory, so that a captured step serves
+// any); in == NULL: the launch opens no step.
+struct BatchStep {
+  StepState *rec;
+  const StepState *in;
+  const float *goal;
+  int hsel;
+};
+
+// kernels_batch.hip (multi-box launches over a work table)
 void launch_batch_cfl(hipStream_t s, const BatchBox *boxes, int nbox, float *state, float goal,
-                      StepState *st);
-void launch_batch_dt(hipStream_t s, StepState *st, int nbox, const float *goal);
-void launch_batch_commit(hipStream_t s, StepState *st, int nbox);
-void launch_batch_copy(hipStream_t s, const BatchBox *boxes, int nbox, float *src, float *dst,
-                       const StepState *st);
-// ghost fills and their CFL minimum for the boxes with ghost layers (grid
-// blocks per box, blockIdx.y the box; boxes without return at once)
+                      StepState *rec);
+// ghost fills of the step that follows rec's, and their CFL minimum, for the
+// boxes with ghost layers (grid blocks per box, blockIdx.y the box; boxes
+// without return at once)
 void launch_batch_ghost_y(hipStream_t s, const BatchBox *boxes, int nbox, int grid, float *state,
-                          const StepState *st);
+                          const StepState *rec);
 void launch_batch_ghost_z(hipStream_t s, const BatchBox *boxes, int nbox, int grid, float *state,
-                          const StepState *st);
+                          const StepState *rec);
 void launch_batch_cfl_ghosts(hipStream_t s, const BatchBox *boxes, int nbox, int grid,
-                             float *state, StepState *st);
+                             float *state, StepState *rec);
+// grid: workgroups that walk the table, 0: one per item.  wide: items of
+// 64x4 tiles among them
 void launch_batch_faces(hipStream_t s, int grid, const BatchBox *boxes, const WorkItem *items,
-                        int nitems, float *state, float *flux, const StepState *st, int hsel);
+                        int nitems, float *state, float *flux, const BatchStep &step, bool wide);
 void launch_batch_update(hipStream_t s, int grid, const BatchBox *boxes, const WorkItem *items,
                          int nitems, float *state_in, float *flux, float *state_base,
-                         float *state_out, StepState *st, int hsel, bool cfl);
-// One workgroup per item, all items of one tile shape (variant).
-void launch_batch_faces_items(hipStream_t s, int variant, const BatchBox *boxes,
-                              const WorkItem *items, int nitems, float *state, float *flux,
-                              const StepState *st, int hsel);
-void launch_batch_update_items(hipStream_t s, int variant, const BatchBox *boxes,
-                               const WorkItem *items, int nitems, float *state_in, float *flux,
-                               float *state_base, float *state_out, StepState *st, int hsel,
-                               bool cfl);
+                         float *state_out, const BatchStep &step, bool cfl);
 
 // kernels_diag.hip (run diagnostics: 12 FP64 values, see k_diag_partial)
 constexpr int kDiagVals = 12;

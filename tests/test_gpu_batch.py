@@ -350,3 +350,43 @@ def test_batch_second_run_after_goal(gpu_ready):
     assert_batch_equals(B, ref)
     for i in range(B.nbox):
         assert B.status(i)[0] == ref[i][2], i
+
+
+@pytest.mark.parametrize("integrator", [0, 1])
+@pytest.mark.parametrize("ft,launch", [(None, None), (capi.TILE_64x4, (1, 1, 0, 0)),
+                                       (capi.TILE_16x16, (5, 3, 0, 0)), (None, (2, 3, 1, 1))])
+def test_batch_opened_steps_and_carried_boxes(gpu_ready, integrator, ft, launch):
+    """Steps opened inside the first face launch, boxes that stop at the goal
+    carried by the last update, at tile edges and chunk remainders, both
+    reconstructions in one table; eager and graph steps alternate over the
+    three rotation phases, and a second run goes on."""
+    announce("batch steps, integrator %d, tiles %s, launch %s" % (integrator, ft, launch))
+    shapes = [(17, 9, 1), (33, 8, 5), (16, 16, 16), (64, 4, 3), (1, 40, 7)]
+    boxes = []
+    for i, n in enumerate(shapes):
+        cfg = P.make_config(n, cfl=0.4, integrator=integrator, recon=i % 2)
+        boxes.append((cfg, P.orszag_tang_noisy(cfg, seed=40 + i, b0=0.3)))
+    probe = make_batch(boxes)
+    probe.run(1e30, 1, use_graph=False)
+    dts = sorted(probe.status(i)[2] for i in range(probe.nbox))
+    g1 = float(np.float32(2.5 * dts[len(dts) // 2]))
+    ref = []
+    for cfg, W in boxes:
+        g = capi.Context(cfg, path=capi.PATH_TILED)
+        g.set_state(W)
+        g.run(g1, 5)
+        k, _ = g.run(2 * g1, 6)
+        ref.append((g.get_state(), g.get_time(), k))
+        g.close()
+    B = make_batch(boxes)
+    if ft is not None:
+        B.set_tiles(ft, ft)
+    if launch is not None:
+        B.set_launch(*launch)
+        assert B.get_launch() == launch
+    B.run(g1, 5, use_graph=True)
+    reached = [B.status(i)[1] for i in range(B.nbox)]
+    assert any(reached)
+    B.run(2 * g1, 6, use_graph=False)
+    assert_batch_equals(B, ref)
+    assert [B.status(i)[0] for i in range(B.nbox)] == [k for _, _, k in ref]
