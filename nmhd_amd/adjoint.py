@@ -253,12 +253,16 @@ def reverse_segment(stepper, W_a, a, b, dts, lam, slots, counter=None):
 
 class _Rollout(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, W0, stepper, dts, checkpoint, every, snapshots):
-        n = len(dts)
+    def forward(ctx, W0, stepper, dts, n, checkpoint, every, snapshots):
+        # dts: the n step sizes, or an empty list that receives them
         keep = {0: W0.detach()}
         stage = {}
         W = W0.detach()
+        t = 0.0
         for k in range(n):
+            if k == len(dts):
+                dts.append(_next_dt(stepper, W, t))
+                t += dts[k]
             if checkpoint == "all":
                 stage[k], W = stepper.forward_stages(W, dts[k])
             else:
@@ -321,7 +325,13 @@ class _Rollout(torch.autograd.Function):
                     states[j - a + 1] = stages[j - a] = None
                 del states, stages
         ctx.keep = ctx.stage = None
-        return lam, None, None, None, None, None
+        return lam, None, None, None, None, None, None
+
+
+def _next_dt(stepper, W, t, goal=1e30):
+    """The CFL dt of the step from W at time t, clipped to the goal."""
+    dt = stepper.cfl_dt(W, goal)
+    return float(goal - t) if t + dt > goal else dt
 
 
 def record_dts(W0, stepper, nsteps, goal=1e30):
@@ -330,9 +340,7 @@ def record_dts(W0, stepper, nsteps, goal=1e30):
     W = W0.detach()
     t = 0.0
     for _ in range(nsteps):
-        dt = stepper.cfl_dt(W, goal)
-        if t + dt > goal:
-            dt = float(goal - t)
+        dt = _next_dt(stepper, W, t, goal)
         dts.append(dt)
         W = stepper.forward(W, dt)
         t += dt
@@ -344,22 +352,21 @@ def rollout(W0, stepper, nsteps=None, dts=None, checkpoint="uniform", every=None
     """W_N = S(...S(W0; dt_0)...; dt_{N-1}), differentiable w.r.t. W0.
 
     dts: the step sizes (frozen); when None they are recorded from the CFL
-    condition along the trajectory (an extra forward pass without grad).
-    Returns (W_N, dts)."""
+    condition as the trajectory is computed.  Returns (W_N, dts)."""
+    if dts is None and nsteps is None:
+        raise ValueError("give nsteps or dts")
+    n = len(range(nsteps)) if dts is None else len(dts)
     if dts is None:
-        if nsteps is None:
-            raise ValueError("give nsteps or dts")
-        with torch.no_grad():
-            dts = record_dts(W0, stepper, nsteps)
-    n = len(dts)
+        _ptrs(W0)  # recording takes no copy of a strided W0
+    dts = [] if dts is None else list(dts)
     if checkpoint not in ("all", "uniform", "revolve"):
         raise ValueError("checkpoint must be 'all', 'uniform' or 'revolve'")
     if every is None:
         every = max(1, int(round(math.sqrt(n))))
     if snapshots is None:
         snapshots = max(1, int(math.ceil(math.log2(max(n, 2)))))
-    return _Rollout.apply(W0.contiguous(), stepper, tuple(dts), checkpoint, every,
-                          snapshots), list(dts)
+    WN = _Rollout.apply(W0.contiguous(), stepper, dts, n, checkpoint, every, snapshots)
+    return WN, dts
 
 
 def finite_difference_check(stepper, W0, dts, directions, grad, loss, eps=1e-3, nperturb=8,
