@@ -33,6 +33,7 @@ thread_local std::string g_batch_create_error;
 
 constexpr int kZChunks[5] = {2, 4, 8, 16, 32};
 constexpr int kWgPerCu[5] = {0, 1, 2, 3, 4};  // 0: one workgroup per item
+constexpr size_t kStage = 1 << 18;  // floats of a half of the copy-out buffer
 constexpr int kTuneItems = 48;  // work items timed per shape and tile shape
 
 }  // namespace
@@ -70,6 +71,10 @@ struct nmhd_batch {
   // that ghost layer)
   int grid_gy = 0, grid_gz = 0, grid_gcfl = 0;
   hipGraphExec_t exec[3] = {};
+  // pinned halves through which get_state copies, with an event each (made by
+  // its first call)
+  float *stage[2] = {};
+  hipEvent_t staged[2] = {};
   std::string err;
 };
 
@@ -277,6 +282,10 @@ void free_batch(nmhd_batch *b) {
   b->d_goal = nullptr;
   b->d_boxes = nullptr;
   b->d_fitems = b->d_uitems = b->d_titems = nullptr;
+  for (int i = 0; i < 2; ++i) {
+    if (b->stage[i]) (void)hipHostFree(b->stage[i]), b->stage[i] = nullptr;
+    if (b->staged[i]) (void)hipEventDestroy(b->staged[i]), b->staged[i] = nullptr;
+  }
   if (b->stream) (void)hipStreamDestroy(b->stream), b->stream = nullptr;
 }
 
@@ -627,12 +636,34 @@ int nmhd_batch_get_state(nmhd_batch *b, int box, float *const fields[8]) {
   if (!box_ok(b, box) || !fields) return bfail(b, NMHD_EINVAL, "bad argument");
   for (int f = 0; f < 8; ++f)
     if (!fields[f]) return bfail(b, NMHD_EINVAL, "null field pointer");
-  BHIP(b, hipStreamSynchronize(b->stream));
-  const FieldPtrs W = box_fields(b->state[b->cur], b->boxes[box]);
-  const size_t bytes = sizeof(float) * (size_t)b->boxes[box].b.ncell;
-  for (int f = 0; f < 8; ++f)
-    BHIP(b, hipMemcpyAsync(fields[f], W.f[f], bytes, hipMemcpyDeviceToHost, b->stream));
-  BHIP(b, hipStreamSynchronize(b->stream));
+  for (int i = 0; i < 2; ++i) {
+    if (!b->stage[i]) BHIP(b, hipHostMalloc(&b->stage[i], kStage * sizeof(float)));
+    if (!b->staged[i]) BHIP(b, hipEventCreateWithFlags(&b->staged[i], hipEventDisableTiming));
+  }
+  // The eight fields lie back to back: they come over in pieces, the next one
+  // in flight while the last is spread over the caller's arrays.  A copy per
+  // field into pageable memory took 30 us each whatever its size, 3.4 ms for
+  // 14 boxes of 1.02M cells together; this takes 1.8 ms.
+  const size_t n = (size_t)b->boxes[box].b.ncell, total = 8 * n;
+  const float *src = b->state[b->cur] + b->boxes[box].off8;
+  auto piece = [&](size_t k) { return std::min(kStage, total - k * kStage); };
+  auto fetch = [&](size_t k) {
+    const hipError_t e = hipMemcpyAsync(b->stage[k & 1], src + k * kStage,
+                                        piece(k) * sizeof(float), hipMemcpyDeviceToHost, b->stream);
+    return e == hipSuccess ? hipEventRecord(b->staged[k & 1], b->stream) : e;
+  };
+  const size_t pieces = (total + kStage - 1) / kStage;
+  for (size_t k = 0; k < pieces && k < 2; ++k) BHIP(b, fetch(k));
+  for (size_t k = 0; k < pieces; ++k) {
+    BHIP(b, hipEventSynchronize(b->staged[k & 1]));
+    const float *from = b->stage[k & 1];
+    for (size_t at = k * kStage, end = at + piece(k); at < end;) {
+      const size_t f = at / n, len = std::min((f + 1) * n, end) - at;
+      std::memcpy(fields[f] + (at - f * n), from, len * sizeof(float));
+      from += len, at += len;
+    }
+    if (k + 2 < pieces) BHIP(b, fetch(k + 2));
+  }
   return NMHD_OK;
 }
 
