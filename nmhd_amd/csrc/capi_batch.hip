@@ -210,13 +210,14 @@ void enqueue_step(nmhd_batch *b, bool full_cfl, float goal) {
     launch_batch_cfl(s, b->d_boxes, n, b->state[A], goal, in);
   else if (b->grid_gcfl)
     launch_batch_cfl_ghosts(s, b->d_boxes, n, b->grid_gcfl, b->state[A], in);
+  const bool nt = streamed(b->total8 / 8);
   auto stage = [&](int from, int base, int to, int hsel, bool first, bool last) {
     launch_batch_faces(s, grid_of(b, b->nf, b->fwg), b->d_boxes, b->d_fitems, b->nf,
                        b->state[from], b->flux,
-                       BatchStep{rec, first ? in : nullptr, b->d_goal, hsel}, b->fwide);
+                       BatchStep{rec, first ? in : nullptr, b->d_goal, hsel}, b->fwide, nt);
     launch_batch_update(s, grid_of(b, b->nu, b->uwg), b->d_boxes, b->d_uitems, b->nu,
                         b->state[from], b->flux, b->state[base], b->state[to],
-                        BatchStep{rec, nullptr, nullptr, hsel}, last);
+                        BatchStep{rec, nullptr, nullptr, hsel}, last, nt);
   };
   if (b->integrator == NMHD_EULER1) {
     stage(A, A, next, H_FULL, true, true);
@@ -396,6 +397,7 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
   float *in = b->state[b->cur];
   float *scratch = b->state[(b->cur + 1) % 3];
   const BatchStep step{b->st_tune, nullptr, nullptr, H_HALF};
+  const bool nt = streamed(b->total8 / 8);
   int ntimed = 0;
 
   // per shape: the workgroup-time of each tile shape
@@ -420,7 +422,7 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
             b,
             [&] {
               launch_batch_faces(b->stream, 1, b->d_boxes, b->d_titems, n, in, b->flux, step,
-                                 true);
+                                 true, nt);
             },
             &msf);
         if (r) return r;
@@ -428,7 +430,7 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
             b,
             [&] {
               launch_batch_update(b->stream, 1, b->d_boxes, b->d_titems, n, in, b->flux, in,
-                                  scratch, step, false);
+                                  scratch, step, false, nt);
             },
             &msu);
         if (r) return r;
@@ -463,7 +465,7 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
             b,
             [&] {
               launch_batch_faces(b->stream, grid_of(b, n, wg), b->d_boxes, b->d_titems, n, in,
-                                 b->flux, step, has_wide(fi));
+                                 b->flux, step, has_wide(fi), nt);
             },
             &ms);
         if (r) return r;
@@ -479,7 +481,7 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
             b,
             [&] {
               launch_batch_update(b->stream, grid_of(b, n, wg), b->d_boxes, b->d_titems, n, in,
-                                  b->flux, in, scratch, step, false);
+                                  b->flux, in, scratch, step, false, nt);
             },
             &ms);
         if (r) return r;

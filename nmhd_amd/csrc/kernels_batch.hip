@@ -70,7 +70,7 @@ __device__ __forceinline__ bool batch_begin(const BatchStep &step, int box, floa
   return s->active;
 }
 
-template <bool Wide>
+template <bool Wide, bool Nt>
 __device__ __forceinline__ void faces_item(const BatchBox *boxes, const WorkItem &w, float *state,
                                            float *flux, const BatchStep &step, float *lds) {
   float h;
@@ -83,11 +83,11 @@ __device__ __forceinline__ void faces_item(const BatchBox *boxes, const WorkItem
   if (!active)
     ;
   else if (Wide && w.variant == TV_64x4)
-    tiled::faces_tile_any<64, 4>(bb.b, W, F, h, x0, y0, z0, zend, lds);
+    tiled::faces_tile_any<64, 4, Nt>(bb.b, W, F, h, x0, y0, z0, zend, lds);
   else if (w.variant == TV_32x8)
-    tiled::faces_tile_any<32, 8>(bb.b, W, F, h, x0, y0, z0, zend, lds);
+    tiled::faces_tile_any<32, 8, Nt>(bb.b, W, F, h, x0, y0, z0, zend, lds);
   else
-    tiled::faces_tile_any<16, 16>(bb.b, W, F, h, x0, y0, z0, zend, lds);
+    tiled::faces_tile_any<16, 16, Nt>(bb.b, W, F, h, x0, y0, z0, zend, lds);
   // the box's first item records the step it opened (after the tile: a store
   // before it would keep the box's parameters out of scalar registers)
   if (step.in && w.xy == 0 && z0 == 0 && threadIdx.x == 0) step.rec[w.box] = batch_open(step, w.box);
@@ -96,12 +96,13 @@ __device__ __forceinline__ void faces_item(const BatchBox *boxes, const WorkItem
 // A workgroup per item.  64x4 tiles need more registers and LDS than the other
 // two shapes, of which four workgroups fit a CU: tables without them take the
 // narrow instantiation.
-template <bool Wide>
+template <bool Wide, bool Nt>
 __global__ void __launch_bounds__(tiled::kTileThreads, Wide ? 3 : 4)
     k_batch_faces_items(const BatchBox *boxes, const WorkItem *items, float *state, float *flux,
                         BatchStep step) {
   __shared__ float lds[kFacesLds<Wide>];
-  faces_item<Wide>(boxes, items[xcd_logical_block(blockIdx.x, gridDim.x)], state, flux, step, lds);
+  faces_item<Wide, Nt>(boxes, items[xcd_logical_block(blockIdx.x, gridDim.x)], state, flux, step,
+                       lds);
 }
 
 // Workgroups that walk the table.
@@ -111,10 +112,10 @@ __global__ void __launch_bounds__(tiled::kTileThreads)
   __shared__ float lds[kFacesLds<true>];
   const int G = gridDim.x;
   for (int it = xcd_logical_block(blockIdx.x, G); it < nitems; it += G)
-    faces_item<true>(boxes, items[it], state, flux, step, lds);
+    faces_item<true, true>(boxes, items[it], state, flux, step, lds);
 }
 
-template <int TX, int TY, bool Cfl>
+template <int TX, int TY, bool Cfl, bool Nt>
 __device__ __forceinline__ void update_tile_of(const Box &b, const WorkItem &w, bool active,
                                                const FieldPtrs &Win, const FluxSet &F,
                                                const FieldPtrs &Wb, const FieldPtrs &Wo, float h,
@@ -122,7 +123,8 @@ __device__ __forceinline__ void update_tile_of(const Box &b, const WorkItem &w, 
   int x0, y0, z0, zend;
   item_tile(w, x0, y0, z0, zend);
   if (active) {
-    tiled::update_tile<TX, TY, false, Cfl>(b, Win, F, Wb, Wo, h, x0, y0, z0, zend, lds, cfl_t);
+    tiled::update_tile<TX, TY, false, Cfl, false, Nt>(b, Win, F, Wb, Wo, h, x0, y0, z0, zend, lds,
+                                                      cfl_t);
     return;
   }
   // a box that takes no step: the last stage's output carries its state
@@ -135,7 +137,7 @@ __device__ __forceinline__ void update_tile_of(const Box &b, const WorkItem &w, 
     }
 }
 
-template <bool Cfl>
+template <bool Cfl, bool Nt>
 __device__ __forceinline__ void update_item(const BatchBox *boxes, const WorkItem &w,
                                             float *state_in, float *flux, float *state_base,
                                             float *state_out, const BatchStep &step, float *lds,
@@ -149,21 +151,21 @@ __device__ __forceinline__ void update_item(const BatchBox *boxes, const WorkIte
   const FluxSet F = box_fluxes(flux, bb);
   float cfl_t = 3.0e38f;
   if (w.variant == TV_64x4)
-    update_tile_of<64, 4, Cfl>(bb.b, w, active, Win, F, Wb, Wo, h, lds, cfl_t);
+    update_tile_of<64, 4, Cfl, Nt>(bb.b, w, active, Win, F, Wb, Wo, h, lds, cfl_t);
   else if (w.variant == TV_32x8)
-    update_tile_of<32, 8, Cfl>(bb.b, w, active, Win, F, Wb, Wo, h, lds, cfl_t);
+    update_tile_of<32, 8, Cfl, Nt>(bb.b, w, active, Win, F, Wb, Wo, h, lds, cfl_t);
   else
-    update_tile_of<16, 16, Cfl>(bb.b, w, active, Win, F, Wb, Wo, h, lds, cfl_t);
+    update_tile_of<16, 16, Cfl, Nt>(bb.b, w, active, Win, F, Wb, Wo, h, lds, cfl_t);
   if (Cfl && active) tiled::block_min_into(cfl_t, &step.rec[w.box].cfl_next_bits, red);
 }
 
-template <bool Cfl>
+template <bool Cfl, bool Nt>
 __global__ void __launch_bounds__(tiled::kTileThreads, 4)
     k_batch_update_items(const BatchBox *boxes, const WorkItem *items, float *state_in,
                          float *flux, float *state_base, float *state_out, BatchStep step) {
   __shared__ float lds[kUpdateLds];
   __shared__ float red[4];
-  update_item<Cfl>(boxes, items[xcd_logical_block(blockIdx.x, gridDim.x)], state_in, flux,
+  update_item<Cfl, Nt>(boxes, items[xcd_logical_block(blockIdx.x, gridDim.x)], state_in, flux,
                    state_base, state_out, step, lds, red);
 }
 
@@ -175,7 +177,7 @@ __global__ void __launch_bounds__(tiled::kTileThreads)
   __shared__ float red[4];
   const int G = gridDim.x;
   for (int it = xcd_logical_block(blockIdx.x, G); it < nitems; it += G)
-    update_item<Cfl>(boxes, items[it], state_in, flux, state_base, state_out, step, lds, red);
+    update_item<Cfl, true>(boxes, items[it], state_in, flux, state_base, state_out, step, lds, red);
 }
 
 // Full CFL pass: blockIdx.y is the box, blocks stride over its cells.
@@ -273,39 +275,42 @@ void launch_batch_cfl_ghosts(hipStream_t s, const BatchBox *boxes, int nbox, int
   hipLaunchKernelGGL(k_batch_cfl_ghosts, dim3(grid, nbox), dim3(256), 0, s, boxes, state, rec);
 }
 void launch_batch_faces(hipStream_t s, int grid, const BatchBox *boxes, const WorkItem *items,
-                        int nitems, float *state, float *flux, const BatchStep &step, bool wide) {
+                        int nitems, float *state, float *flux, const BatchStep &step, bool wide,
+                        bool nt) {
   const dim3 blk(tiled::kTileThreads);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nitems), blk, 0, s, boxes, items, state, flux, step);
+  };
   if (grid)
     hipLaunchKernelGGL(k_batch_faces, dim3(grid), blk, 0, s, boxes, items, nitems, state, flux,
                        step);
-  else if (wide)
-    hipLaunchKernelGGL(k_batch_faces_items<true>, dim3(nitems), blk, 0, s, boxes, items, state,
-                       flux, step);
+  else if (nt)
+    wide ? go(k_batch_faces_items<true, true>) : go(k_batch_faces_items<false, true>);
   else
-    hipLaunchKernelGGL(k_batch_faces_items<false>, dim3(nitems), blk, 0, s, boxes, items, state,
-                       flux, step);
+    wide ? go(k_batch_faces_items<true, false>) : go(k_batch_faces_items<false, false>);
 }
 
 template <bool Cfl>
 void update_as(hipStream_t s, int grid, const BatchBox *boxes, const WorkItem *items, int nitems,
                float *state_in, float *flux, float *state_base, float *state_out,
-               const BatchStep &step) {
+               const BatchStep &step, bool nt) {
   const dim3 blk(tiled::kTileThreads);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nitems), blk, 0, s, boxes, items, state_in, flux, state_base,
+                       state_out, step);
+  };
   if (grid)
     hipLaunchKernelGGL(k_batch_update<Cfl>, dim3(grid), blk, 0, s, boxes, items, nitems, state_in,
                        flux, state_base, state_out, step);
   else
-    hipLaunchKernelGGL(k_batch_update_items<Cfl>, dim3(nitems), blk, 0, s, boxes, items, state_in,
-                       flux, state_base, state_out, step);
+    nt ? go(k_batch_update_items<Cfl, true>) : go(k_batch_update_items<Cfl, false>);
 }
 
 void launch_batch_update(hipStream_t s, int grid, const BatchBox *boxes, const WorkItem *items,
                          int nitems, float *state_in, float *flux, float *state_base,
-                         float *state_out, const BatchStep &step, bool cfl) {
-  if (cfl)
-    update_as<true>(s, grid, boxes, items, nitems, state_in, flux, state_base, state_out, step);
-  else
-    update_as<false>(s, grid, boxes, items, nitems, state_in, flux, state_base, state_out, step);
+                         float *state_out, const BatchStep &step, bool cfl, bool nt) {
+  auto as = cfl ? update_as<true> : update_as<false>;
+  as(s, grid, boxes, items, nitems, state_in, flux, state_base, state_out, step, nt);
 }
 
 }  // namespace nmhd

@@ -19,7 +19,7 @@ namespace nmhd {
 namespace tiled {
 
 // Recon = b.recon (the launcher picks the instantiation)
-template <int TX, int TY, int Recon>
+template <int TX, int TY, int Recon, bool Nt>
 __global__ void __launch_bounds__(kTileThreads, (FacesShape<TX, TY>::kWavesPerSimd))
     k_faces(Box b, FieldPtrs W, FluxSet F, StageStep ss, OpenStep open, int zc, int gx, int gy) {
   float h;
@@ -27,10 +27,10 @@ __global__ void __launch_bounds__(kTileThreads, (FacesShape<TX, TY>::kWavesPerSi
   __shared__ float lds[FacesShape<TX, TY>::kLds];
   const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
   const int x0 = (lb % gx) * TX, y0 = ((lb / gx) % gy) * TY, z0 = (lb / gx / gy) * zc;
-  faces_tile<TX, TY, Recon>(b, W, F, h, x0, y0, z0, min(z0 + zc, b.n[2]), lds);
+  faces_tile<TX, TY, Recon, Nt>(b, W, F, h, x0, y0, z0, min(z0 + zc, b.n[2]), lds);
 }
 
-template <int TX, int TY, bool PaceOnly, bool Cfl, bool Raw>
+template <int TX, int TY, bool PaceOnly, bool Cfl, bool Raw, bool Nt>
 __global__ void __launch_bounds__(kTileThreads, 4) k_update_march(Box b, FieldPtrs Win, FluxSet F,
                                                                FieldPtrs Wb, FieldPtrs Wo,
                                                                StageStep ss, int zc, int gx,
@@ -55,14 +55,23 @@ __global__ void __launch_bounds__(kTileThreads, 4) k_update_march(Box b, FieldPt
   __shared__ float lds[UpdateShape<TX, TY>::kLds];
   __shared__ float red[4];
   float cfl_t = 3.0e38f;
-  update_tile<TX, TY, PaceOnly, Cfl, Raw>(b, Win, F, Wb, Wo, h, x0, y0, z0, min(z0 + zc, b.n[2]), lds,
-                                     cfl_t);
+  update_tile<TX, TY, PaceOnly, Cfl, Raw, Nt>(b, Win, F, Wb, Wo, h, x0, y0, z0,
+                                              min(z0 + zc, b.n[2]), lds, cfl_t);
   if (Cfl && !PaceOnly) block_min_into(cfl_t, cfl_slot(ss.rec, blockIdx.x), red);
 }
 
 }  // namespace tiled
 
 // ------------------------------------------------------------- launchers
+
+// A stage reads and writes 27 arrays (35 in the second), of which the next
+// kernel wants most at once: boxes whose hand-off and states the 256 MB
+// last-level cache holds for a good part keep them there.  Step times through
+// the caches / past them: 80^3 90 / 96 us, 112^3 184 / 211, 130x109x75 180 /
+// 205, 128^3 220 / 240, 170x158x120 (3.2M cells) 429 / 477; from 160^3 (4.1M)
+// on the halo planes matter more: 469 / 451, 192^3 800 / 759, 256x264x256
+// 1888 / 1820.
+bool streamed(long cells) { return cells > 3500000; }
 
 namespace {
 
@@ -116,12 +125,12 @@ int tiled_shape(int nx, int ny, bool faces) {
   // as on 32x8 (256^3: 511 / 444 / 520 us; 80^3, which 16x16 covers exactly:
   // 38 / 31 / 27).  The update is fastest on 64x4 (256^3: 412 us against 432
   // on 32x8 and 600 on 16x16), whose idle lanes cost it less: 32x8 wins from
-  // a quarter more on (96^3: 39 against 34).
+  // a fifth more on (130x109x75: 36 against 34, 160x120x100: 58 / 53).
   auto covered = [&](int v) {
     const long tx = kTileTX[v], ty = kTileTY[v];
     return (float)((nx + tx - 1) / tx * tx) * (float)((ny + ty - 1) / ty * ty);
   };
-  if (!faces) return covered(TV_64x4) >= 1.25f * covered(TV_32x8) ? TV_32x8 : TV_64x4;
+  if (!faces) return covered(TV_64x4) >= 1.19f * covered(TV_32x8) ? TV_32x8 : TV_64x4;
   int v = TV_32x8;
   if (1.15f * covered(TV_64x4) < covered(v)) v = TV_64x4;
   if (1.16f * covered(TV_16x16) < (v == TV_32x8 ? 1.0f : 1.15f) * covered(v)) v = TV_16x16;
@@ -135,12 +144,14 @@ void faces_as(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F, const 
               const OpenStep &open) {
   const int zc = tiled_zchunk(b, TX, TY, true);
   const int gx = (b.n[0] + TX - 1) / TX, gy = (b.n[1] + TY - 1) / TY, gz = (b.n[2] + zc - 1) / zc;
-  if (b.recon == 1)
-    hipLaunchKernelGGL((tiled::k_faces<TX, TY, 1>), dim3(gx * gy * gz), dim3(tiled::kTileThreads),
-                       0, s, b, W, F, ss, open, zc, gx, gy);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(gx * gy * gz), dim3(tiled::kTileThreads), 0, s, b, W, F, ss,
+                       open, zc, gx, gy);
+  };
+  if (streamed(b.ncell))
+    b.recon == 1 ? go(tiled::k_faces<TX, TY, 1, true>) : go(tiled::k_faces<TX, TY, 0, true>);
   else
-    hipLaunchKernelGGL((tiled::k_faces<TX, TY, 0>), dim3(gx * gy * gz), dim3(tiled::kTileThreads),
-                       0, s, b, W, F, ss, open, zc, gx, gy);
+    b.recon == 1 ? go(tiled::k_faces<TX, TY, 1, false>) : go(tiled::k_faces<TX, TY, 0, false>);
 }
 
 template <int TX, int TY, bool Raw>
@@ -148,16 +159,18 @@ void update_as(hipStream_t s, const Box &b, FieldPtrs Win, const FluxSet &F, Fie
                FieldPtrs Wout, const StageStep &ss, bool pace_only, bool cfl) {
   const int zc = tiled_zchunk(b, TX, TY, false);
   const int gx = (b.n[0] + TX - 1) / TX, gy = (b.n[1] + TY - 1) / TY, gz = (b.n[2] + zc - 1) / zc;
-  const dim3 grid(gx * gy * gz), blk(tiled::kTileThreads);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(gx * gy * gz), dim3(tiled::kTileThreads), 0, s, b, Win, F,
+                       Wbase, Wout, ss, zc, gx, gy);
+  };
   if (pace_only)
-    hipLaunchKernelGGL((tiled::k_update_march<TX, TY, true, false, false>), grid, blk, 0, s, b,
-                       Win, F, Wbase, Wout, ss, zc, gx, gy);
-  else if (cfl)
-    hipLaunchKernelGGL((tiled::k_update_march<TX, TY, false, true, Raw>), grid, blk, 0, s, b, Win,
-                       F, Wbase, Wout, ss, zc, gx, gy);
+    go(tiled::k_update_march<TX, TY, true, false, false, false>);
+  else if (!Raw && streamed(b.ncell))
+    cfl ? go(tiled::k_update_march<TX, TY, false, true, false, true>)
+        : go(tiled::k_update_march<TX, TY, false, false, false, true>);
   else
-    hipLaunchKernelGGL((tiled::k_update_march<TX, TY, false, false, Raw>), grid, blk, 0, s, b,
-                       Win, F, Wbase, Wout, ss, zc, gx, gy);
+    cfl ? go(tiled::k_update_march<TX, TY, false, true, Raw, false>)
+        : go(tiled::k_update_march<TX, TY, false, false, Raw, false>);
 }
 
 }  // namespace

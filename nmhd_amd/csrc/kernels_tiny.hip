@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(kThreads, 4)
         ce.YZ[u][w] = S.edge[2][0][yz];
         ce.ZY[u][w] = S.edge[2][1][yz];
       }
-    tiled::finish_cell<false, Cfl>(b, ce, pc, wb, bb, h, y, z, own, Wo, cfl_t);
+    tiled::finish_cell<false, Cfl, false>(b, ce, pc, wb, bb, h, y, z, own, Wo, cfl_t);
   }
   if (Cfl) {
     cfl_t = wave_min64(cfl_t);

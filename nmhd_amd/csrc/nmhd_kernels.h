@@ -301,12 +301,14 @@ void launch_batch_ghost_z(hipStream_t s, const BatchBox *boxes, int nbox, int gr
 void launch_batch_cfl_ghosts(hipStream_t s, const BatchBox *boxes, int nbox, int grid,
                              float *state, StepState *rec);
 // grid: workgroups that walk the table, 0: one per item.  wide: items of
-// 64x4 tiles among them
+// 64x4 tiles among them; nt: streamed() of all boxes together
 void launch_batch_faces(hipStream_t s, int grid, const BatchBox *boxes, const WorkItem *items,
-                        int nitems, float *state, float *flux, const BatchStep &step, bool wide);
+                        int nitems, float *state, float *flux, const BatchStep &step, bool wide,
+                        bool nt);
 void launch_batch_update(hipStream_t s, int grid, const BatchBox *boxes, const WorkItem *items,
                          int nitems, float *state_in, float *flux, float *state_base,
-                         float *state_out, const BatchStep &step, bool cfl);
+                         float *state_out, const BatchStep &step, bool cfl,
+                         bool nt);
 
 // kernels_diag.hip (run diagnostics: 12 FP64 values, see k_diag_partial)
 constexpr int kDiagVals = 12;
@@ -345,6 +347,8 @@ void launch_direct_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet
 // kernels_tiled.hip
 // Planes per march of the face or update kernel: the chunk of the least
 // estimated time, groups_at(zc) the workgroups of the launch with chunks of zc.
+// whether the stage kernels over that many cells store past the caches
+bool streamed(long cells);
 int march_chunk(bool faces, int nz, const std::function<long(int)> &groups_at);
 int tiled_zchunk(const Box &b, int tx, int ty, bool faces);
 // Tile shape (TileVariant) of the face or update kernel for a box.

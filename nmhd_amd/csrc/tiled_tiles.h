@@ -78,12 +78,21 @@ __device__ __forceinline__ int pmod(int i, int n) {
   return r < 0 ? r + n : r;
 }
 
-// Results that the next kernel reads are stored non-temporally: written
-// once per step, they would otherwise displace the halo planes that
-// neighbouring tiles re-read from L2 (1-3% faster per kernel, measured).
-__device__ __forceinline__ void put_nt(float *dst, float v) { __builtin_nontemporal_store(v, dst); }
-// Likewise for values that only the loading thread reads (no halo reuse).
-__device__ __forceinline__ float get_nt(const float *src) { return __builtin_nontemporal_load(src); }
+// Results that the next kernel reads, and values that only the loading thread
+// reads.  Nt: past the caches, where they would displace the halo planes that
+// neighbouring tiles re-read from L2; otherwise through them, where the next
+// kernel finds them (streamed() decides).
+template <bool Nt>
+__device__ __forceinline__ void put(float *dst, float v) {
+  if (Nt)
+    __builtin_nontemporal_store(v, dst);
+  else
+    *dst = v;
+}
+template <bool Nt>
+__device__ __forceinline__ float get(const float *src) {
+  return Nt ? __builtin_nontemporal_load(src) : *src;
+}
 
 // The element at byte offset boff (32-bit) from a workgroup-uniform base:
 // loads and stores through it take the scalar-base + 32-bit vector-offset
@@ -211,7 +220,7 @@ struct FacesShape {
 // 32^3.  The column of plane zend+1 is loaded after the march: prefetching it
 // during the last pass keeps the staging registers alive across the loop's
 // end, which costs 14 VGPRs (11 spilled at 4 waves per SIMD).
-template <int TX, int TY, int Recon>
+template <int TX, int TY, int Recon, bool Nt>
 __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, const FluxSet &Fs,
                                            float h, int x0, int y0, int z0, int zend,
                                            float *lds) {
@@ -478,14 +487,14 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
       fzn[3] = r.mn;
       fzn[4] = r.e;
       if (inner) {
-        put_nt(at_byte(plane_of(SB.fb[4], p), ownp), r.bt1);  // B_x
-        put_nt(at_byte(plane_of(SB.fb[5], p), ownp), r.bt2);  // B_y
+        put<Nt>(at_byte(plane_of(SB.fb[4], p), ownp), r.bt1);  // B_x
+        put<Nt>(at_byte(plane_of(SB.fb[5], p), ownp), r.bt2);  // B_y
       }
       // plane p-1 complete: its lower z-face (fzl) and upper z-face (fzn)
       if (p > z0) {
 #pragma unroll
         for (int k = 0; k < 5; ++k)
-          put_nt(at_byte(plane_of(SB.pace[k], p - 1), ownp), pxy[k] + (fzl[k] - fzn[k]) * idz);
+          put<Nt>(at_byte(plane_of(SB.pace[k], p - 1), ownp), pxy[k] + (fzl[k] - fzn[k]) * idz);
       }
     }
 #pragma unroll
@@ -511,16 +520,16 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
         const Flux7 r = face_x(cb, c);
         put_x(ty, tx, r);
         if (valid) {
-          put_nt(at_byte(plane_of(SB.fb[0], p), ownp), r.bt1);  // B_y
-          put_nt(at_byte(plane_of(SB.fb[1], p), ownp), r.bt2);  // B_z
+          put<Nt>(at_byte(plane_of(SB.fb[0], p), ownp), r.bt1);  // B_y
+          put<Nt>(at_byte(plane_of(SB.fb[1], p), ownp), r.bt2);  // B_z
         }
       }
       if (x < nx && y <= ny) {
         const Flux7 r = face_y(cb, c, yrow);
         put_y(ty, tx, r);
         if (valid) {
-          put_nt(at_byte(plane_of(SB.fb[2], p), ownp), r.bt1);  // B_z
-          put_nt(at_byte(plane_of(SB.fb[3], p), ownp), r.bt2);  // B_x
+          put<Nt>(at_byte(plane_of(SB.fb[2], p), ownp), r.bt1);  // B_z
+          put<Nt>(at_byte(plane_of(SB.fb[3], p), ownp), r.bt2);  // B_x
         }
       }
       // the tile's upper boundary faces, the y-faces of row y0+TY and the
@@ -603,14 +612,14 @@ __device__ __forceinline__ void faces_tile(const Box &b, const FieldPtrs &W, con
 
 // faces_tile for the box's reconstruction (a uniform branch: two copies of
 // the march, each without scheme selects).
-template <int TX, int TY>
+template <int TX, int TY, bool Nt>
 __device__ __forceinline__ void faces_tile_any(const Box &b, const FieldPtrs &W,
                                                const FluxSet &Fs, float h, int x0, int y0,
                                                int z0, int zend, float *lds) {
   if (b.recon == 1)
-    faces_tile<TX, TY, 1>(b, W, Fs, h, x0, y0, z0, zend, lds);
+    faces_tile<TX, TY, 1, Nt>(b, W, Fs, h, x0, y0, z0, zend, lds);
   else
-    faces_tile<TX, TY, 0>(b, W, Fs, h, x0, y0, z0, zend, lds);
+    faces_tile<TX, TY, 0, Nt>(b, W, Fs, h, x0, y0, z0, zend, lds);
 }
 
 template <int TX, int TY>
@@ -635,7 +644,7 @@ struct CellEdges {
 // The update of the cell at address a, row y, plane r: pc the hydro
 // divergence, wb the base rho, v, p, bb its six base face fields (x lower,
 // x upper, y.., z..).  cfl_t is lowered to the CFL time of the new state.
-template <bool PaceOnly, bool Cfl>
+template <bool PaceOnly, bool Cfl, bool Nt>
 __device__ __forceinline__ void finish_cell(const Box &b, const CellEdges &ce, const float (&pc)[5],
                                             const float (&wb)[5], const float (&bb)[6], float h,
                                             int y, int r, int a, const FieldPtrs &Wo,
@@ -655,10 +664,10 @@ __device__ __forceinline__ void finish_cell(const Box &b, const CellEdges &ce, c
   }
   if (PaceOnly) {
 #pragma unroll
-    for (int k = 0; k < 5; ++k) put_nt(&Wo.f[k][a], pc[k]);
-    put_nt(&Wo.f[5][a], pbx[0]);
-    put_nt(&Wo.f[6][a], pby[0]);
-    put_nt(&Wo.f[7][a], pbz[0]);
+    for (int k = 0; k < 5; ++k) put<Nt>(&Wo.f[k][a], pc[k]);
+    put<Nt>(&Wo.f[5][a], pbx[0]);
+    put<Nt>(&Wo.f[6][a], pby[0]);
+    put<Nt>(&Wo.f[7][a], pbz[0]);
   } else {
     const float rho0 = wb[0];
     const float vx0 = wb[1], vy0 = wb[2], vz0 = wb[3];
@@ -688,14 +697,14 @@ __device__ __forceinline__ void finish_cell(const Box &b, const CellEdges &ce, c
       ux += h * ax_;
       uy += h * ay_;
     }
-    put_nt(&Wo.f[0][a], rho);
-    put_nt(&Wo.f[1][a], ux);
-    put_nt(&Wo.f[2][a], uy);
-    put_nt(&Wo.f[3][a], uz);
-    put_nt(&Wo.f[4][a], pres);
-    put_nt(&Wo.f[5][a], bxl);
-    put_nt(&Wo.f[6][a], byl);
-    put_nt(&Wo.f[7][a], bzl);
+    put<Nt>(&Wo.f[0][a], rho);
+    put<Nt>(&Wo.f[1][a], ux);
+    put<Nt>(&Wo.f[2][a], uy);
+    put<Nt>(&Wo.f[3][a], uz);
+    put<Nt>(&Wo.f[4][a], pres);
+    put<Nt>(&Wo.f[5][a], bxl);
+    put<Nt>(&Wo.f[6][a], byl);
+    put<Nt>(&Wo.f[7][a], bzl);
     if (Cfl) {
       // CFL time of the new state for cells the next ghost fill leaves
       // untouched (interior rows/planes); the ghost cells are reduced
@@ -739,7 +748,7 @@ __device__ __forceinline__ void finish_cell(const Box &b, const CellEdges &ce, c
 // cell the thread updates (stage 2 with Cfl).
 // Raw: the hydro fluxes themselves are in Fs (k_direct_faces wrote them) and
 // are differenced here, in the order of the face march.
-template <int TX, int TY, bool PaceOnly, bool Cfl, bool Raw = false>
+template <int TX, int TY, bool PaceOnly, bool Cfl, bool Raw, bool Nt>
 __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, const FluxSet &Fs,
                                             const FieldPtrs &Wb, const FieldPtrs &Wo, float h,
                                             int x0, int y0, int z0, int zend, float *lds,
@@ -887,13 +896,13 @@ __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, 
     const int base = wrap(p, nz) * plane + own;
     if (!Raw) {
 #pragma unroll
-      for (int k = 0; k < 5; ++k) dpc[k] = get_nt(&SB.pace[k][base]);
+      for (int k = 0; k < 5; ++k) dpc[k] = get<Nt>(&SB.pace[k][base]);
     }
-    dwb[0] = get_nt(&Wb.f[0][base]);
-    dwb[4] = get_nt(&Wb.f[4][base]);
+    dwb[0] = get<Nt>(&Wb.f[0][base]);
+    dwb[4] = get<Nt>(&Wb.f[4][base]);
     if (!in_is_base) {
 #pragma unroll
-      for (int k = 1; k < 4; ++k) dwb[k] = get_nt(&Wb.f[k][base]);
+      for (int k = 1; k < 4; ++k) dwb[k] = get<Nt>(&Wb.f[k][base]);
     }
   };
 
@@ -951,7 +960,7 @@ __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, 
       loadz(r + 2, rz);
       loadp(r + 1);
       load_own(r + 1, pc_nx, wb_nx);
-      bz_nx = get_nt(&Wb.f[7][wrap(r + 2, nz) * plane + own]);
+      bz_nx = get<Nt>(&Wb.f[7][wrap(r + 2, nz) * plane + own]);
     }
     edges(r, r + 1, true);
     const float *BXB = SP + 2 * RN, *BYB = SP + 3 * RN;
@@ -991,7 +1000,7 @@ __device__ __forceinline__ void update_tile(const Box &b, const FieldPtrs &Win, 
           fzl[k] = fzh[k];
         }
       }
-      finish_cell<PaceOnly, Cfl>(b, ce, pc, wb, bb, h, y, r, a, Wo, cfl_t);
+      finish_cell<PaceOnly, Cfl, Nt>(b, ce, pc, wb, bb, h, y, r, a, Wo, cfl_t);
     }
     if (more) {
       // the rings are not read between the barriers
