@@ -43,6 +43,14 @@ __device__ __forceinline__ float &at(float *p, unsigned o) {
   return *reinterpret_cast<float *>(reinterpret_cast<char *>(p) + o);
 }
 
+template <bool Nt>
+__device__ __forceinline__ void put(float *p, float v) {
+  if (Nt)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
+
 // The thread's cell, and the offset contributions of its index along each
 // axis and of the neighbours' (periodic).
 struct Place {
@@ -182,7 +190,7 @@ __device__ __forceinline__ unsigned limiter_branch(float a, float b) {
   return a * b <= 0.0f ? 0u : (fabsf(a) < fabsf(b) ? 1u : 3u);
 }
 
-template <int D>
+template <int D, bool Nt>
 __device__ __forceinline__ void adj_face(const Box &b, const FieldPtrs &W, const float *gU0,
                                          const float *gU1, const float *gU2, const float *gU3,
                                          const float *gU4, const float *lEx, const float *lEy,
@@ -287,23 +295,31 @@ __device__ __forceinline__ void adj_face(const Box &b, const FieldPtrs &W, const
   const float gl[7] = {g.rL, g.unL, g.u1L, g.u2L, g.pL, g.b1L, g.b2L};
   const float gr[7] = {g.rR, g.unR, g.u1R, g.u2R, g.pR, g.b1R, g.b2R};
   for (int k = 0; k < 7; ++k) {
-    at(out.aL[k], a) = gl[k];
-    at(out.aR[k], a) = gr[k];
+    put<Nt>(&at(out.aL[k], a), gl[k]);
+    put<Nt>(&at(out.aR[k], a), gr[k]);
   }
   at(reinterpret_cast<float *>(out.br), a) = __uint_as_float(br);
   at(out.abn, a) = g.bx;
 }
+
+// Cells up to which the faces' 42 adjoint arrays (168 bytes a cell) are stored
+// through the caches for the gather to find; past that they only displace the
+// stencils' neighbours there.  One reverse step through / past the caches: 64^3
+// 144 / 149 us, 72^3 200 / 207, 100x90x80 (720k cells) 371 / 387, 96^3 (885k)
+// 443 / 430, 112^3 750 / 705, 128^3 1078 / 1019, 224^3 5690 / 5630.
+constexpr long kAdjCached = 800000;
 
 // All faces of the three directions in one launch: consecutive workgroups
 // take the three directions of the same cells (a uniform branch each), and
 // each XCD a contiguous range of them, so that neighbouring rows and planes
 // share its L2.  VALU (about 990 instructions a face, 1330 with both sides of
 // the fan reversed) and the traffic of 45 output arrays bound it about
-// equally: 243 -> 213 us at 128^3.
+// equally: 243 -> 213 us at 128^3, 198 past the caches.
 struct AdjFaceOut3 {
   AdjFaceOut d[3];
 };
 
+template <bool Nt>
 __global__ void __launch_bounds__(256) k_adj_faces(Box b, FieldPtrs W, const float *gU0,
                                                    const float *gU1, const float *gU2,
                                                    const float *gU3, const float *gU4,
@@ -314,18 +330,19 @@ __global__ void __launch_bounds__(256) k_adj_faces(Box b, FieldPtrs W, const flo
   Place p;
   if (!place_of(b, block, p)) return;
   if (dir == 0)
-    adj_face<0>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[0], p);
+    adj_face<0, Nt>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[0], p);
   else if (dir == 1)
-    adj_face<1>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[1], p);
+    adj_face<1, Nt>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[1], p);
   else
-    adj_face<2>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[2], p);
+    adj_face<2, Nt>(b, W, gU0, gU1, gU2, gU3, gU4, lEx, lEy, lEz, h, out.d[2], p);
 }
 
 // ------------------------------------------------------------ k_adj_gather
 //
 // Bound by memory: 42 adjoint and 3 branch arrays, most read twice.  Selecting
 // by the two-bit numbers instead of four compares and selects per variable and
-// taking 32-bit offsets: 141 -> 133 us at 128^3.
+// taking 32-bit offsets: 141 -> 133 us at 128^3, 122 when the faces store past
+// the caches.
 //
 // The reconstruction reverse of direction D at cell (x,y,z): res[0..6] =
 // adjoints of rho, v_D, v_D+1, v_D+2, p, Bbar_D+1, Bbar_D+2 of the cell,
@@ -436,8 +453,9 @@ void launch_adj_stage(hipStream_t s, const Box &b, const AdjStageArgs &A) {
     fo.d[d].abn = A.abn[d];
   }
   const dim3 g3(3 * grid_for(b.ncell));
-  hipLaunchKernelGGL(k_adj_faces, g3, blk, 0, s, b, A.Win, A.gU[0], A.gU[1], A.gU[2], A.gU[3],
-                     A.gU[4], A.lE[0], A.lE[1], A.lE[2], A.h, fo);
+  auto faces = b.ncell > kAdjCached ? k_adj_faces<true> : k_adj_faces<false>;
+  hipLaunchKernelGGL(faces, g3, blk, 0, s, b, A.Win, A.gU[0], A.gU[1], A.gU[2], A.gU[3], A.gU[4],
+                     A.lE[0], A.lE[1], A.lE[2], A.h, fo);
   hipLaunchKernelGGL(k_adj_gather, g, blk, 0, s, b, fo, A.lam_in, A.acc_in ? 1 : 0, A.lbb[0],
                      A.lbb[1], A.lbb[2]);
   hipLaunchKernelGGL(k_adj_bfinish, g, blk, 0, s, b, A.lbb[0], A.lbb[1], A.lbb[2], A.abn[0],

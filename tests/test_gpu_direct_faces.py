@@ -71,3 +71,21 @@ def test_direct_equals_tiles_shearing(gpu_ready, n, fixes):
     assert got[:2] == ref[:2]
     for a, b in zip(got[2], ref[2]):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("recon", [0, 1])
+@pytest.mark.parametrize("integrator", [0, 1])
+def test_large_box_equals_its_periodic_cell(gpu_ready, recon, integrator):
+    """3.51M cells, just past the size from which the tiles store past the
+    caches: 4x4x4 copies of a 38^3 box do what the box does, bit for bit."""
+    print("\n[case] 152^3 of 4x4x4 copies, recon %d, integrator %d" % (recon, integrator),
+          flush=True)
+    kw = dict(cfl=0.3, recon=recon, integrator=integrator)
+    small = P.make_config((38, 38, 38), global_extent=(38 / 64,) * 3, **kw)
+    large = P.make_config((152, 152, 152), global_extent=(152 / 64,) * 3, **kw)
+    W = rough(small, 5)
+    dt, t, out = run(small, W, None)
+    dt4, t4, out4 = run(large, np.tile(W, (1, 4, 4, 4)), None)
+    assert (dt, t) == (dt4, t4)
+    for a, b in zip(out, out4):
+        assert np.array_equal(np.tile(a, (1, 4, 4, 4)).view(np.uint32), b.view(np.uint32))
