@@ -22,7 +22,7 @@ The JSON line also carries
   batched      -- 64 periodic boxes of uneven sizes (edges from
                   {16,24,32,48,64,96}, seed 1004; Orszag-Tang and blast
                   states) advanced 100 steps with per-box dt by the batched
-                  path (persistent tile launches, HIP-graph replay, autotuned
+                  path (launches over every box's tiles, HIP graphs, autotuned
                   tiles), against the same boxes advanced one after another
                   by single-box contexts;
   adjoint      -- the hand-written adjoint on the 64^3 Orszag-Tang box with
@@ -384,10 +384,10 @@ def adjoint_leg(a, torch):
 
 def stage_rates(cfg, tim, kbytes, zones):
     """Algorithmic GB/s of each stage of the step: reconstruction + HLLD (the
-    face kernels), CT + update (the update kernels), CFL reduction (the
-    ghost-cell pass; the interior is reduced in the update's epilogue) and the
-    boundary (shearing-periodic ghost fill, 8 fields read + written per ghost
-    cell)."""
+    face kernels), CT + update (the update kernels), CFL reduction (a
+    ghost-cell pass; None where there is none: the interior is reduced in the
+    update's epilogue, the rows of a Y fill as it writes them) and the boundary
+    (shearing-periodic ghost fill, 8 fields read + written per ghost cell)."""
     m = cfg["m"][1]
     ghost_cells = 2 * m * cfg["n"][0] * cfg["n"][2]
 

@@ -231,8 +231,8 @@ int nmhd_timing_get(nmhd_ctx *ctx, int i, const char **name, double *total_ms,
 int nmhd_set_path(nmhd_ctx *ctx, int path);
 int nmhd_get_path(const nmhd_ctx *ctx, int *path);
 /* Tile shapes (enum nmhd_tile) of the face and update kernels of
- * NMHD_PATH_TILED (default NMHD_TILE_32x8 and NMHD_TILE_64x4); results do
- * not depend on them. */
+ * NMHD_PATH_TILED (by default kernel and shape follow the box's size);
+ * results do not depend on them. */
 int nmhd_set_tiles(nmhd_ctx *ctx, int faces_tile, int update_tile);
 int nmhd_get_tiles(const nmhd_ctx *ctx, int *faces_tile, int *update_tile);
 
@@ -281,7 +281,7 @@ int nmhd_batch_get_launch(const nmhd_batch *batch, int *faces_zchunk, int *updat
                           int *faces_wg_per_cu, int *update_wg_per_cu);
 /* Autotuner: per distinct box shape, time every tile shape of both kernels
  * (one workgroup walking that shape's tiles, i.e. the workgroup-time the
- * shape costs in a persistent launch) and keep the fastest; then time the
+ * shape costs in a launch that walks a table) and keep the fastest; then time the
  * z chunk and workgroups per CU of the whole batch.  Results are cached in
  * the text file cache_path (NULL: $NMHD_TUNE_CACHE, else
  * $HOME/.cache/nmhd_amd/batch_tuning.txt), keyed by the GPU architecture

@@ -1,14 +1,13 @@
 // tiled_tiles.h -- the two stage kernels of the production path as tile
 // functions, shared by the single-box launches (kernels_tiled.hip) and the
-// persistent multi-box launches (kernels_batch.hip).
+// multi-box launches (kernels_batch.hip).
 //
 //  faces_tile   all three face fluxes of every cell of a TX x TY column tile
 //               over planes [z0, zend), one HLLD per face plus the tile's
 //               upper boundary faces.  The x and y stencils (cells i-2..i+1)
 //               are read from an LDS ring of two planes that the workgroup
-//               stages cooperatively; the z stencil (planes k-2..k+1) lives
-//               in a per-thread register queue filled as the march passes
-//               each plane.  Differences the hydro fluxes in the tile (LDS
+//               stages cooperatively; the z stencil is the thread's own
+//               column, carried in registers.  Differences the hydro fluxes in the tile (LDS
 //               for x and y, registers for z) and writes the hydro
 //               divergence of every cell (5 floats) and the six B fluxes the
 //               CT needs (6 floats).
@@ -20,7 +19,7 @@
 //               thread's cells (interior cells only).
 //
 // Both run on 256-thread workgroups (TX * TY == 256, 1-D thread index) and
-// take their LDS as a pointer so that one persistent kernel can run tiles of
+// take their LDS as a pointer so that one kernel can run tiles of
 // several shapes out of one buffer.  The arithmetic of a cell does not depend
 // on the tile shape or the z chunk, so every tiling gives bit-identical
 // results.

@@ -9,6 +9,7 @@ every counter found (FETCH_SIZE / WRITE_SIZE are KiB per dispatch).
 """
 import argparse
 import collections
+import re
 import sqlite3
 
 
@@ -37,10 +38,10 @@ def counters(db):
 
 
 # rocprof kernel names -> per-launch slots of the tiled step (the stage-2
-# update is the instantiation with the CFL epilogue: <TX, TY, false, true>)
-SLOTS = ((("k_faces<", ""), ("faces_s1", "faces_s2")),
-         (("k_update_march<", ", false, true>"), ("update_s2",)),
-         (("k_update_march<", ", false, false>"), ("update_s1",)))
+# update is the instantiation with the CFL epilogue: <TX, TY, false, true, ...>)
+SLOTS = ((r"k_faces<", ("faces_s1", "faces_s2")),
+         (r"k_update_march<\d+, \d+, false, true,", ("update_s2",)),
+         (r"k_update_march<\d+, \d+, false, false,", ("update_s1",)))
 
 
 def traffic(fetch_db, write_db, fetch_scale, write_scale, valu_db=None):
@@ -52,9 +53,9 @@ def traffic(fetch_db, write_db, fetch_scale, write_scale, valu_db=None):
     w = counters(write_db)
     v = counters(valu_db) if valu_db else {}
     out = {}
-    for (pat, suffix), slots in SLOTS:
+    for pat, slots in SLOTS:
         for k in f:
-            if pat in k and k.endswith(suffix) and k in w:
+            if re.search(pat, k) and k in w:
                 fk = f[k]["FETCH_SIZE"]
                 wk = w[k]["WRITE_SIZE"]
                 rec = {"rocprof_kernel": k, "fetch_kib": fk, "write_kib": wk,
