@@ -111,8 +111,10 @@ __global__ void __launch_bounds__(tiled::kTileThreads)
                   float *flux, BatchStep step) {
   __shared__ float lds[kFacesLds<true>];
   const int G = gridDim.x;
-  for (int it = xcd_logical_block(blockIdx.x, G); it < nitems; it += G)
+  for (int it = xcd_logical_block(blockIdx.x, G); it < nitems; it += G) {
     faces_item<true, true>(boxes, items[it], state, flux, step, lds);
+    __syncthreads();  // the next tile's shape lays the LDS out anew
+  }
 }
 
 template <int TX, int TY, bool Cfl, bool Nt>
@@ -176,8 +178,10 @@ __global__ void __launch_bounds__(tiled::kTileThreads)
   __shared__ float lds[kUpdateLds];
   __shared__ float red[4];
   const int G = gridDim.x;
-  for (int it = xcd_logical_block(blockIdx.x, G); it < nitems; it += G)
+  for (int it = xcd_logical_block(blockIdx.x, G); it < nitems; it += G) {
     update_item<Cfl, true>(boxes, items[it], state_in, flux, state_base, state_out, step, lds, red);
+    __syncthreads();
+  }
 }
 
 // Full CFL pass: blockIdx.y is the box, blocks stride over its cells.
