@@ -24,6 +24,7 @@
 //                 face reverse recorded) -> lam_in of rho, v, p and of the
 //                 cell-averaged B
 //   k_adj_bfinish face B: cell-average and normal-field adjoints -> lam_in B
+//                 (in small boxes the gather does it)
 #include "adjoint_hlld.h"
 #include "nmhd_kernels.h"
 
@@ -355,36 +356,66 @@ __global__ void __launch_bounds__(256) k_adj_faces(Box b, FieldPtrs W, const flo
 //   cell 1:  aL + aL/2 ([m took x1 - x0] - [m took x2 - x1]) + aR/2 [m' took x2 - x1]
 //   cell 2:  aR + aL/2 [m took x2 - x1] - aR/2 ([m' took x2 - x1] - [m' took x3 - x2])
 //   cell 3: -aR/2 [m' took x3 - x2]
+
+// The four faces along D around a cell, and their limiter branches.
+struct GatherFaces {
+  unsigned f[4], br[4];
+};
 template <int D>
-__device__ __forceinline__ void adj_gather(const Box &b, const AdjFaceOut &fa, const Place &p,
-                                           float (&res)[7]) {
+__device__ __forceinline__ GatherFaces gather_faces(const Box &b, const AdjFaceOut &fa,
+                                                    const Place &p) {
   const unsigned rest = p.o[(D + 1) % 3] + p.o[(D + 2) % 3];
-  const unsigned f0 = p.to(D, 2, b.n[D]) + rest, f1 = p.to(D, 1, b.n[D]) + rest;
-  const unsigned f2 = p.o[D] + rest, f3 = p.to(D, -1, b.n[D]) + rest;
-  auto bits = [&](unsigned o) {
-    return __float_as_uint(ld(reinterpret_cast<const float *>(fa.br), o));
-  };
-  const unsigned b0 = bits(f0), b1 = bits(f1), b2 = bits(f2), b3 = bits(f3);
+  GatherFaces g;
+  g.f[0] = p.to(D, 2, b.n[D]) + rest, g.f[1] = p.to(D, 1, b.n[D]) + rest;
+  g.f[2] = p.o[D] + rest, g.f[3] = p.to(D, -1, b.n[D]) + rest;
+  for (int q = 0; q < 4; ++q)
+    g.br[q] = __float_as_uint(ld(reinterpret_cast<const float *>(fa.br), g.f[q]));
+  return g;
+}
+__device__ __forceinline__ float gather_var(const AdjFaceOut &fa, const GatherFaces &g, int k) {
+  const unsigned f0 = g.f[0], f1 = g.f[1], f2 = g.f[2], f3 = g.f[3];
+  const unsigned b0 = g.br[0], b1 = g.br[1], b2 = g.br[2], b3 = g.br[3];
   // [m took the lower difference], [the upper], and their difference
   auto one = [](unsigned w, int i) { return (float)((w >> i) & 1u); };
   auto signed2 = [](unsigned w, int i) { return (float)((int)(w << (30 - i)) >> 30); };
+  const int s = 4 * k;
+  const float l0 = ld(fa.aL[k], f0), l1 = ld(fa.aL[k], f1), r1 = ld(fa.aR[k], f1);
+  const float l2 = ld(fa.aL[k], f2), r2 = ld(fa.aR[k], f2), r3 = ld(fa.aR[k], f3);
+  const float c0 = -0.5f * l0 * (float)((b0 >> s & 1u) & ~(b0 >> (s + 1)));
+  const float r1_lo = (float)((b1 >> (s + 2) & 1u) & ~(b1 >> (s + 3)));
+  const float c1 = l1 + 0.5f * l1 * signed2(b1, s) + 0.5f * r1 * r1_lo;
+  const float c2 = r2 + 0.5f * l2 * one(b2, s + 1) - 0.5f * r2 * signed2(b2, s + 2);
+  const float c3 = -0.5f * r3 * one(b3, s + 3);
+  return c0 + c1 + c2 + c3;
+}
+template <int D>
+__device__ __forceinline__ void adj_gather(const Box &b, const AdjFaceOut &fa, const Place &p,
+                                           float (&res)[7]) {
+  const GatherFaces g = gather_faces<D>(b, fa, p);
 #pragma unroll
-  for (int k = 0; k < 7; ++k) {
-    const int s = 4 * k;
-    const float l0 = ld(fa.aL[k], f0), l1 = ld(fa.aL[k], f1), r1 = ld(fa.aR[k], f1);
-    const float l2 = ld(fa.aL[k], f2), r2 = ld(fa.aR[k], f2), r3 = ld(fa.aR[k], f3);
-    const float c0 = -0.5f * l0 * (float)((b0 >> s & 1u) & ~(b0 >> (s + 1)));
-    const float r1_lo = (float)((b1 >> (s + 2) & 1u) & ~(b1 >> (s + 3)));
-    const float c1 = l1 + 0.5f * l1 * signed2(b1, s) + 0.5f * r1 * r1_lo;
-    const float c2 = r2 + 0.5f * l2 * one(b2, s + 1) - 0.5f * r2 * signed2(b2, s + 2);
-    const float c3 = -0.5f * r3 * one(b3, s + 3);
-    res[k] = c0 + c1 + c2 + c3;
-  }
+  for (int k = 0; k < 7; ++k) res[k] = gather_var(fa, g, k);
+}
+
+// The cell-average B_T adjoint of the cell below p along T, as k_adj_gather
+// sums it for that cell.
+template <int T>
+__device__ __forceinline__ float lower_bbar(const Box &b, const AdjFaceOut3 &fa, const Place &p) {
+  Place q = p;
+  q.o[T] = p.to(T, -1, b.n[T]);
+  // the sweeps along the other two axes, x before y before z; B_T is variable
+  // 5 of the sweep along the axis before T, 6 of that after
+  constexpr int A = T == 0 ? 1 : 0, C = T == 2 ? 1 : 2;
+  float m = 0.0f;
+  m += gather_var(fa.d[A], gather_faces<A>(b, fa.d[A], q), (A + 1) % 3 == T ? 5 : 6);
+  m += gather_var(fa.d[C], gather_faces<C>(b, fa.d[C], q), (C + 1) % 3 == T ? 5 : 6);
+  return m;
 }
 
 // lam_in of rho, v, p from the three directions' reconstruction reverses
 // (written, or added to with accumulate), and the cell-average B adjoints
-// lbb[t] (written).
+// lbb[t] (written), or with Finish the face B of lam_in (k_adj_bfinish), the
+// lower neighbours' averages then gathered again.
+template <bool Finish>
 __global__ void __launch_bounds__(256) k_adj_gather(Box b, AdjFaceOut3 fa, FieldPtrs lam_in,
                                                     int accumulate, float *lbb0, float *lbb1,
                                                     float *lbb2) {
@@ -405,10 +436,26 @@ __global__ void __launch_bounds__(256) k_adj_gather(Box b, AdjFaceOut3 fa, Field
   const float out[5] = {rho, v[0], v[1], v[2], pr};
   for (int f = 0; f < 5; ++f)
     at(lam_in.f[f], a) = accumulate ? ld(lam_in.f[f], a) + out[f] : out[f];
+  if (Finish) {
+    const float low[3] = {lower_bbar<0>(b, fa, p), lower_bbar<1>(b, fa, p),
+                          lower_bbar<2>(b, fa, p)};
+    for (int t = 0; t < 3; ++t) {
+      const float f = 0.5f * (bb[t] + low[t]) + ld(fa.d[t].abn, a);
+      at(lam_in.f[5 + t], a) = accumulate ? ld(lam_in.f[5 + t], a) + f : f;
+    }
+    return;
+  }
   at(lbb0, a) = bb[0];
   at(lbb1, a) = bb[1];
   at(lbb2, a) = bb[2];
 }
+
+// Cells up to which the gather finishes the face B itself: it then reads 60
+// values more a cell, mostly cached, and saves a launch and the averages' way
+// through memory.  One reverse step folded / with k_adj_bfinish: 20^3 42 / 47
+// us, 35x30x28 52 / 55, 48^3 88 / 92, 64^3 138 / 142, 72^3 192 / 191, 96^3 438 /
+// 432, 128^3 1040 / 1027.
+constexpr long kAdjFold = 300000;
 
 // Face B_t of lam_in: half of each adjacent cell's cell-average adjoint plus
 // the normal-field adjoint of the t-sweep's face.
@@ -456,10 +503,13 @@ void launch_adj_stage(hipStream_t s, const Box &b, const AdjStageArgs &A) {
   auto faces = b.ncell > kAdjCached ? k_adj_faces<true> : k_adj_faces<false>;
   hipLaunchKernelGGL(faces, g3, blk, 0, s, b, A.Win, A.gU[0], A.gU[1], A.gU[2], A.gU[3], A.gU[4],
                      A.lE[0], A.lE[1], A.lE[2], A.h, fo);
-  hipLaunchKernelGGL(k_adj_gather, g, blk, 0, s, b, fo, A.lam_in, A.acc_in ? 1 : 0, A.lbb[0],
-                     A.lbb[1], A.lbb[2]);
-  hipLaunchKernelGGL(k_adj_bfinish, g, blk, 0, s, b, A.lbb[0], A.lbb[1], A.lbb[2], A.abn[0],
-                     A.abn[1], A.abn[2], A.lam_in, A.acc_in ? 1 : 0);
+  const bool fold = b.ncell <= kAdjFold;
+  auto gather = fold ? k_adj_gather<true> : k_adj_gather<false>;
+  hipLaunchKernelGGL(gather, g, blk, 0, s, b, fo, A.lam_in, A.acc_in ? 1 : 0, A.lbb[0], A.lbb[1],
+                     A.lbb[2]);
+  if (!fold)
+    hipLaunchKernelGGL(k_adj_bfinish, g, blk, 0, s, b, A.lbb[0], A.lbb[1], A.lbb[2], A.abn[0],
+                       A.abn[1], A.abn[2], A.lam_in, A.acc_in ? 1 : 0);
 }
 
 }  // namespace nmhd
