@@ -90,9 +90,12 @@ constexpr MarchCost kUpdateCost = {{2.3f, 3.1f, 4.0f, 5.5f}, 16};
 int march_chunk(bool faces, int nz, const std::function<long(int)> &groups_at) {
   // A march of zc planes costs about one plane more (the prologue and the
   // last z-face); 1024 workgroups are resident (4 per CU).  In one round a
-  // CU's share decides; past it the rounds blend, except that a small
-  // remainder of the first ones is paid for as a round of its own (at 1050
-  // workgroups 1.5 rounds, at 2112 2.3, at 4224 4.1).
+  // CU's share decides; past it the rounds blend, except that a remainder of
+  // the first ones costs more than its share, a small one nearly a round of its
+  // own (1050 workgroups 1.5 rounds, 1216 1.4, 1408 1.5, 1664 1.7, 2112 2.3,
+  // 4224 4.1).  With the remainders past 0.4 at their share alone, 16 boxes of
+  // 16..96 cells per edge took 214 us a step against 203, 112^3 185 / 181,
+  // 170x158x120 428 / 418; 144^3 377 / 381 is the one the other way.
   const MarchCost &c = faces ? kFacesCost : kUpdateCost;
   int best = 1;
   float least = 0.0f;
@@ -105,7 +108,9 @@ int march_chunk(bool faces, int nz, const std::function<long(int)> &groups_at) {
       cost = c.plane[share < 1 ? 0 : share - 1] * (float)(zc + 1);
     } else {
       const float whole = std::floor(rounds), part = rounds - whole;
-      const float extra = part > 0.0f ? 0.5f * std::max(0.0f, 1.0f - part / 0.4f) / whole : 0.0f;
+      const float extra =
+          part > 0.0f ? (0.4f * std::max(0.0f, 1.0f - part / 0.3f) + 0.15f * (1.0f - part)) / whole
+                      : 0.0f;
       cost = c.plane[3] * (float)(zc + 1) * (rounds + extra);
     }
     if (best == 1 && want == 1) least = cost;
