@@ -261,7 +261,7 @@ void enqueue_step(nmhd_ctx *c, float goal) {
   const bool ghosts = b.m[1] > 0 || b.m[2] > 0;
   StepRec *const in = c->rec + c->r, *const out = c->rec + (c->r ^ 1);
   const bool reset = c->reset;
-  if (full_cfl) timed(c, S_BEGIN, [&] { launch_clear_cfl(s, in, reset); });
+  if (full_cfl) timed(c, S_BEGIN, [&] { launch_clear_cfl(s, in); });
   // the carried CFL minimum lacks the ghost cells: the fill reduces them as it
   // writes them, unless a Z fill writes some again
   const bool fill_cfl = !full_cfl && b.m[1] > 0 && b.m[2] == 0;
@@ -271,7 +271,7 @@ void enqueue_step(nmhd_ctx *c, float goal) {
     timed(c, S_GHOST_Y, [&] { launch_ghost_y(s, b, fields(c, A), in, reset); });
   if (b.m[2] > 0) timed(c, S_GHOST_Z, [&] { launch_ghost_z(s, b, fields(c, A), in, reset); });
   if (full_cfl)
-    timed(c, S_CFL, [&] { launch_cfl(s, b, fields(c, A), goal, in, reset); });
+    timed(c, S_CFL, [&] { launch_cfl(s, b, fields(c, A), goal, in, reset, tiled); });
   else if (ghosts && !fill_cfl)
     timed(c, S_CFL_GHOSTS, [&] { launch_cfl_ghosts(s, b, fields(c, A), in, reset); });
   const OpenStep open{in, out, goal, reset};

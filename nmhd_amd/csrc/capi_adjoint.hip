@@ -219,7 +219,7 @@ int nmhd_adj_synchronize(nmhd_adj *a) {
 
 int nmhd_adj_cfl_dt(nmhd_adj *a, const float *const w[8], float goal_time, float *dt) {
   if (!a || !ptrs_ok(w) || !dt) return afail(a, NMHD_EINVAL, "bad argument");
-  launch_clear_cfl(a->stream, a->rec, true);
+  launch_clear_cfl(a->stream, a->rec);
   launch_cfl(a->stream, a->box, to_fields_c(w), goal_time, a->rec, true);
   StepRec h;
   AHIP(a, hipMemcpyAsync(&h, a->rec, sizeof(h), hipMemcpyDeviceToHost, a->stream));

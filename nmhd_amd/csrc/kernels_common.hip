@@ -18,9 +18,7 @@ namespace nmhd {
 // not do it.
 __global__ void k_open_step(Box b, OpenStep o) { (void)open_step(b, o, true); }
 
-__global__ void k_clear_cfl(StepRec *rec, int reset) {
-  if (!run_ended(rec->s, reset)) rec->cfl[threadIdx.x * kCflStride] = 0x7f800000u;
-}
+__global__ void k_clear_cfl(StepRec *rec) { rec->cfl[threadIdx.x * kCflStride] = 0x7f800000u; }
 
 void host_displacement(const Box &b, double t, float *normalized, int *n, float *minor) {
   displacement(b, t, normalized, n, minor);
@@ -70,13 +68,15 @@ __global__ void __launch_bounds__(256) k_ghost_y(Box b, FieldPtrs W, StepRec *re
 
 // Grid-stride over the cells with a capped grid.
 __global__ void __launch_bounds__(256) k_cfl(Box b, FieldPtrs W, float goal, StepRec *rec,
-                                             int reset) {
-  if (run_ended(rec->s, reset)) return;
-  float t = goal;
+                                             int reset, int carry) {
+  const bool ended = run_ended(rec->s, reset);
+  if (ended && !carry) return;
+  float t = ended ? 3.0e38f : goal;
   for (long a = (long)blockIdx.x * blockDim.x + threadIdx.x; a < b.ncell;
        a += (long)gridDim.x * blockDim.x) {
     int x, y, z;
     cell_coords(b, a, x, y, z);
+    if (ended && refilled(b, y, z)) continue;
     t = fminf(t, cell_cfl(b, W, a, x, y, z));
   }
   cfl_block_fold(t, rec);
@@ -167,8 +167,8 @@ __global__ void k_diag_prepare(StepRec *diag, const StepRec *rec, float h) {
 
 // ------------------------------------------------------------- launchers
 
-void launch_clear_cfl(hipStream_t s, StepRec *rec, bool reset) {
-  hipLaunchKernelGGL(k_clear_cfl, dim3(1), dim3(kCflSlots), 0, s, rec, (int)reset);
+void launch_clear_cfl(hipStream_t s, StepRec *rec) {
+  hipLaunchKernelGGL(k_clear_cfl, dim3(1), dim3(kCflSlots), 0, s, rec);
 }
 void launch_open_step(hipStream_t s, const Box &b, const OpenStep &open) {
   hipLaunchKernelGGL(k_open_step, dim3(1), dim3(64), 0, s, b, open);
@@ -205,9 +205,10 @@ void launch_ghost_z(hipStream_t s, const Box &b, FieldPtrs W, const StepRec *rec
   const long unit = (long)b.n[0] * b.n[1] * b.m[2];
   hipLaunchKernelGGL(k_ghost_z, dim3(grid_for(unit)), dim3(kBlock), 0, s, b, W, rec, (int)reset);
 }
-void launch_cfl(hipStream_t s, const Box &b, FieldPtrs W, float goal, StepRec *rec, bool reset) {
+void launch_cfl(hipStream_t s, const Box &b, FieldPtrs W, float goal, StepRec *rec, bool reset,
+                bool carry) {
   hipLaunchKernelGGL(k_cfl, dim3(reduce_grid(b.ncell)), dim3(kBlock), 0, s, b, W, goal, rec,
-                     (int)reset);
+                     (int)reset, (int)carry);
 }
 void launch_copy_state(hipStream_t s, const Box &b, FieldPtrs src, FieldPtrs dst,
                        const StepState *st) {

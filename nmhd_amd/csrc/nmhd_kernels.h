@@ -195,6 +195,14 @@ __device__ __forceinline__ float cfl_time(const Box &b, const float (&w)[5], con
   return t;
 }
 
+// Whether a ghost fill changes the CFL time of a cell of row y, plane z: it
+// rewrites the ghost cells, and the upper B_z face of the last interior plane.
+// The minimum that a step carries to the next leaves these cells out.
+__device__ __forceinline__ bool refilled(const Box &b, int y, int z) {
+  return y < b.m[1] || y >= b.n[1] - b.m[1] ||
+         (b.m[2] > 0 && (z < b.m[2] || z >= b.n[2] - b.m[2] - 1));
+}
+
 __device__ __forceinline__ float cell_cfl(const Box &b, const FieldPtrs &W, long a, int x, int y,
                                           int z) {
   const float w[5] = {W.f[0][a], W.f[1][a], W.f[2][a], W.f[3][a], W.f[4][a]};
@@ -243,9 +251,8 @@ constexpr int kTileTX[TV_COUNT] = {64, 32, 16};
 constexpr int kTileTY[TV_COUNT] = {4, 8, 16};
 
 // kernels_common.hip
-// empty the CFL minimum of rec before a full pass (not when the run that rec
-// ends is finished and goes on: its minimum is still wanted)
-void launch_clear_cfl(hipStream_t s, StepRec *rec, bool reset);
+// empty the CFL minimum of rec before a full pass
+void launch_clear_cfl(hipStream_t s, StepRec *rec);
 void launch_open_step(hipStream_t s, const Box &b, const OpenStep &open);
 // the ghost fills and CFL passes of the step that follows rec's
 void launch_cfl_ghosts(hipStream_t s, const Box &b, FieldPtrs W, StepRec *rec, bool reset);
@@ -253,7 +260,12 @@ void launch_ghost_y(hipStream_t s, const Box &b, FieldPtrs W, const StepRec *rec
 // the Y fill and the CFL minimum of the rows it writes (boxes without Z ghosts)
 void launch_ghost_y_cfl(hipStream_t s, const Box &b, FieldPtrs W, StepRec *rec, bool reset);
 void launch_ghost_z(hipStream_t s, const Box &b, FieldPtrs W, const StepRec *rec, bool reset);
-void launch_cfl(hipStream_t s, const Box &b, FieldPtrs W, float goal, StepRec *rec, bool reset);
+// the full pass; for a step that is not taken (the run that rec ends is
+// finished and goes on) it does nothing, or with carry it leaves the minimum
+// that the step is to hand on: without the cells that the next fill rewrites
+// and without the goal
+void launch_cfl(hipStream_t s, const Box &b, FieldPtrs W, float goal, StepRec *rec, bool reset,
+                bool carry = false);
 void launch_copy_state(hipStream_t s, const Box &b, FieldPtrs src, FieldPtrs dst,
                        const StepState *st);
 void launch_copy_fields(hipStream_t s, long ncell, const FieldPtrs &src, const FieldPtrs &dst);

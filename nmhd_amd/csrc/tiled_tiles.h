@@ -649,7 +649,6 @@ __device__ __forceinline__ void finish_cell(const Box &b, const CellEdges &ce, c
                                             int y, int r, int a, const FieldPtrs &Wo,
                                             float &cfl_t) {
   const float idx_ = b.inv_d[0], idy_ = b.inv_d[1], idz_ = b.inv_d[2];
-  const int ny = b.n[1], nz = b.n[2];
   float pbx[2], pby[2], pbz[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
@@ -708,9 +707,7 @@ __device__ __forceinline__ void finish_cell(const Box &b, const CellEdges &ce, c
       // CFL time of the new state for cells the next ghost fill leaves
       // untouched (interior rows/planes); the ghost cells are reduced
       // after the fill
-      const bool ghost = (y < b.m[1]) || (y >= ny - b.m[1]) ||
-                         (b.m[2] > 0 && (r < b.m[2] || r >= nz - b.m[2] - 1));
-      if (!ghost) {
+      if (!refilled(b, y, r)) {
         // same rounding as the full CFL pass (no contraction), so an
         // incrementally reduced dt equals it bit for bit
 #pragma clang fp contract(off)

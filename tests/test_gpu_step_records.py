@@ -74,6 +74,39 @@ def test_enqueueing_does_not_matter(gpu_ready, box, path):
         c.close()
 
 
+@pytest.mark.parametrize("path", [capi.PATH_TILED, capi.PATH_STRICT])
+@pytest.mark.parametrize("box", range(4))
+def test_state_loaded_after_the_goal(gpu_ready, box, path):
+    """Steps enqueued without a new run after the goal was reached do nothing,
+    also where a state was loaded in between: the next run's dt is that of the
+    loaded state alone, not of the one before it, of the ghost rows it came
+    with, of those steps' goal, nor (after the strict path) none at all."""
+    name, cfg, W = boxes()[box]
+    a, b = capi.Context(cfg, path=path), capi.Context(cfg, path=capi.PATH_TILED)
+    a.set_state(W)
+    dt, _ = a.step()
+    assert a.run(float(np.float32(a.get_time()[0] + 0.5 * dt)), 1) == (1, True)
+    a.set_path(capi.PATH_TILED)
+    X = W.copy()
+    X[4] *= 2.0
+    m = cfg["m"]
+    ny, nz = cfg["n"][1], cfg["n"][2]
+    X[4][nz // 2, ny // 2] *= 4.0  # rows that no ghost row copies
+    X[4][:, [y for y in range(ny) if y < m[1] or y >= ny - m[1]], :] *= 100.0
+    X[4][[z for z in range(nz) if z < m[2] or z >= nz - m[2]]] *= 100.0
+    a.set_state(X)
+    a.enqueue_steps(1e-6, 3)
+    a.synchronize()
+    assert np.array_equal(a.get_state().view(np.uint32), X.view(np.uint32)), name
+    b.set_state(X)
+    b.set_time(*a.get_time())
+    for _ in range(2):
+        assert a.step()[0] == b.step()[0], name
+    assert np.array_equal(a.get_state().view(np.uint32), b.get_state().view(np.uint32)), name
+    a.close()
+    b.close()
+
+
 @pytest.mark.parametrize("n", [(1, 1, 1), (3, 1, 1), (5, 3, 1), (17, 9, 7), (64, 32, 16)])
 @pytest.mark.parametrize("offset", [0, 1, 2, 4])
 def test_device_state_transfer(gpu_ready, n, offset):
