@@ -452,6 +452,7 @@ static int copy_state(nmhd_ctx *c, const float *const src[8], float *const dst[8
       else
         to.f[f] = dst[f];
     }
+    (void)hipGetLastError();  // an earlier call's, which no copy would report
     launch_copy_fields(c->stream, c->box.ncell, from, to);
     HIPCHECK(c, hipGetLastError());
   } else {
@@ -485,6 +486,7 @@ int nmhd_get_state_device(nmhd_ctx *ctx, float *const f[8]) {
 
 int nmhd_set_time(nmhd_ctx *ctx, double t, int generation) {
   if (!ctx) return NMHD_EINVAL;
+  (void)hipGetLastError();  // an earlier call's
   launch_set_time(ctx->stream, ctx->box, ctx->rec + ctx->r, t, generation);
   HIPCHECK(ctx, hipGetLastError());
   ctx->cfl_valid = false;

@@ -132,6 +132,23 @@ def test_device_state_transfer(gpu_ready, n, offset):
     ctx.close()
 
 
+def test_device_state_transfer_after_another_call_failed(gpu_ready):
+    """An error that an earlier HIP call of the program left behind is not that
+    of a transfer or of set_time."""
+    ctx = capi.Context(P.make_config((4, 2, 2)))
+    import torch
+    W = torch.rand(8, 16, device="cuda")
+    torch.cuda.synchronize()
+    ptrs = [W[f].data_ptr() for f in range(8)]
+    for call in (lambda: ctx.set_state_device(ptrs), lambda: ctx.get_state_device(ptrs),
+                 lambda: ctx.set_time(0.5, 3)):
+        assert capi.load().hipSetDevice(10000) != 0
+        call()
+    assert np.array_equal(ctx.get_state().reshape(8, 16), W.cpu().numpy())
+    assert ctx.get_time() == (0.5, 3)
+    ctx.close()
+
+
 @pytest.mark.parametrize("n,margin", [((24, 12, 9), 4), ((1, 3, 1), 1), ((5, 2, 2), 2),
                                       ((70, 4, 3), 4), ((33, 9, 17), 3)])
 @pytest.mark.parametrize("fixes,shear_y", [(0, 1), (7, 1), (2, 1), (1, 0)])
