@@ -421,16 +421,26 @@ int nmhd_get_geometry(const nmhd_ctx *ctx, nmhd_geometry *geo) {
   return NMHD_OK;
 }
 
-// Whether all eight pointers are memory of the context's own device, which a
-// kernel may address (another device's may need a staged copy).
-static bool own_device(const nmhd_ctx *c, const float *const p[8]) {
+// Whether one kernel may do what a copy per field does to the caller's eight
+// arrays: they are memory of the context's own device (another device's may
+// need a staged copy), and each lies whole in the allocation that it points into
+// (a copy refuses one that does not).
+static bool one_kernel_copies(const nmhd_ctx *c, const float *const p[8]) {
+  const size_t bytes = sizeof(float) * (size_t)c->box.ncell;
   for (int f = 0; f < 8; ++f) {
+    const uintptr_t at = (uintptr_t)p[f];
     hipPointerAttribute_t a;
-    if ((uintptr_t)p[f] % sizeof(float) || hipPointerGetAttributes(&a, p[f]) != hipSuccess) {
+    hipDeviceptr_t base;
+    size_t size;
+    if (at % sizeof(float) || hipPointerGetAttributes(&a, p[f]) != hipSuccess ||
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)at) != hipSuccess) {
       (void)hipGetLastError();
       return false;
     }
     if (a.type != hipMemoryTypeDevice || a.device != c->device) return false;
+    if (at < (uintptr_t)base || at - (uintptr_t)base > size ||
+        size - (at - (uintptr_t)base) < bytes)
+      return false;
   }
   return true;
 }
@@ -444,7 +454,7 @@ static int copy_state(nmhd_ctx *c, const float *const src[8], float *const dst[8
     if (!in && !dst[f]) return fail(c, NMHD_EINVAL, "null field pointer");
   }
   if (in) c->cfl_valid = false;
-  if (kind == hipMemcpyDeviceToDevice && own_device(c, in ? src : dst)) {
+  if (kind == hipMemcpyDeviceToDevice && one_kernel_copies(c, in ? src : dst)) {
     FieldPtrs from = fields(c, c->cur), to = from;
     for (int f = 0; f < 8; ++f) {
       if (in)

@@ -149,6 +149,37 @@ def test_device_state_transfer_after_another_call_failed(gpu_ready):
     ctx.close()
 
 
+def test_device_state_transfer_outside_an_allocation(gpu_ready):
+    """A field that runs past the end of its allocation is refused, as a copy
+    refuses it: here by half its 64 bytes, which still lie in the page."""
+    import ctypes
+    ctx = capi.Context(P.make_config((4, 2, 2)))
+    W = np.arange(8 * 16, dtype=np.float32).reshape(8, 2, 2, 4) + 1.0
+    ctx.set_state(W)
+    L = capi.load()
+    buf = ctypes.c_void_p()
+    size = 3584
+    assert L.hipMalloc(ctypes.byref(buf), ctypes.c_size_t(size)) == 0
+    whole = [buf.value + 64 * f for f in range(8)]
+    ctx.get_state_device(whole)
+    for f in (0, 7):
+        ptrs = list(whole)
+        ptrs[f] = buf.value + size - 32
+        with pytest.raises(capi.NmhdError):
+            ctx.set_state_device(ptrs)
+        ctx.set_state(W)
+        with pytest.raises(capi.NmhdError):
+            ctx.get_state_device(ptrs)
+    # the last place where it fits
+    ptrs = whole[:7] + [buf.value + size - 64]
+    ctx.get_state_device(ptrs)
+    ctx.set_state(W + 1.0)
+    ctx.set_state_device(ptrs)
+    assert np.array_equal(ctx.get_state(), W)
+    ctx.close()
+    assert L.hipFree(buf) == 0
+
+
 @pytest.mark.parametrize("n,margin", [((24, 12, 9), 4), ((1, 3, 1), 1), ((5, 2, 2), 2),
                                       ((70, 4, 3), 4), ((33, 9, 17), 3)])
 @pytest.mark.parametrize("fixes,shear_y", [(0, 1), (7, 1), (2, 1), (1, 0)])
