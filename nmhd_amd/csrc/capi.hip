@@ -423,9 +423,10 @@ int nmhd_get_geometry(const nmhd_ctx *ctx, nmhd_geometry *geo) {
 
 // Whether one kernel may do what a copy per field does to the caller's eight
 // arrays: they are memory of the context's own device (another device's may
-// need a staged copy), and each lies whole in the allocation that it points into
-// (a copy refuses one that does not).
-static bool one_kernel_copies(const nmhd_ctx *c, const float *const p[8]) {
+// need a staged copy), each lies whole in the allocation that it points into
+// (a copy refuses one that does not), and none that is written overlaps another
+// (the copies leave the later field's values there).
+static bool one_kernel_copies(const nmhd_ctx *c, const float *const p[8], bool written) {
   const size_t bytes = sizeof(float) * (size_t)c->box.ncell;
   for (int f = 0; f < 8; ++f) {
     const uintptr_t at = (uintptr_t)p[f];
@@ -441,6 +442,10 @@ static bool one_kernel_copies(const nmhd_ctx *c, const float *const p[8]) {
     if (at < (uintptr_t)base || at - (uintptr_t)base > size ||
         size - (at - (uintptr_t)base) < bytes)
       return false;
+    for (int g = 0; written && g < f; ++g) {
+      const uintptr_t other = (uintptr_t)p[g];
+      if ((at > other ? at - other : other - at) < bytes) return false;
+    }
   }
   return true;
 }
@@ -454,7 +459,7 @@ static int copy_state(nmhd_ctx *c, const float *const src[8], float *const dst[8
     if (!in && !dst[f]) return fail(c, NMHD_EINVAL, "null field pointer");
   }
   if (in) c->cfl_valid = false;
-  if (kind == hipMemcpyDeviceToDevice && one_kernel_copies(c, in ? src : dst)) {
+  if (kind == hipMemcpyDeviceToDevice && one_kernel_copies(c, in ? src : dst, !in)) {
     FieldPtrs from = fields(c, c->cur), to = from;
     for (int f = 0; f < 8; ++f) {
       if (in)

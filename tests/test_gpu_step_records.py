@@ -180,6 +180,29 @@ def test_device_state_transfer_outside_an_allocation(gpu_ready):
     assert L.hipFree(buf) == 0
 
 
+@pytest.mark.parametrize("shift", [0, 3, 15, 16])
+def test_device_state_fields_that_overlap(gpu_ready, shift):
+    """Fields fetched into arrays that overlap: the later field's values stay,
+    as after a copy per field in turn."""
+    import torch
+    ctx = capi.Context(P.make_config((4, 2, 2)))
+    W = np.arange(8 * 16, dtype=np.float32).reshape(8, 2, 2, 4) + 1.0
+    ctx.set_state(W)
+    dst = torch.full((8 * 16,), -1.0, device="cuda")
+    torch.cuda.synchronize()
+    ctx.get_state_device([dst.data_ptr() + 4 * shift * f for f in range(8)])
+    want = np.full(8 * 16, -1.0, np.float32)
+    for f in range(8):
+        want[shift * f:shift * f + 16] = W[f].reshape(-1)
+    assert np.array_equal(dst.cpu().numpy(), want)
+    # the same arrays may all be read
+    ctx.set_state_device([dst.data_ptr() + 4 * shift * f for f in range(8)])
+    got = ctx.get_state().reshape(8, 16)
+    for f in range(8):
+        assert np.array_equal(got[f], want[shift * f:shift * f + 16])
+    ctx.close()
+
+
 @pytest.mark.parametrize("n,margin", [((24, 12, 9), 4), ((1, 3, 1), 1), ((5, 2, 2), 2),
                                       ((70, 4, 3), 4), ((33, 9, 17), 3)])
 @pytest.mark.parametrize("fixes,shear_y", [(0, 1), (7, 1), (2, 1), (1, 0)])
