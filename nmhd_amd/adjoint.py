@@ -258,14 +258,16 @@ def reverse_segment(stepper, W_a, a, b, dts, lam, slots, counter=None):
 class _Rollout(torch.autograd.Function):
     @staticmethod
     def forward(ctx, W0, stepper, dts, n, checkpoint, every, snapshots):
-        # dts: the n step sizes, or an empty list that receives them
+        # dts: the n step sizes, or the first of them: the list receives the rest
         keep = {0: W0.detach()}
         stage = {}
         W = W0.detach()
         t = 0.0
+        record = len(dts) < n
         for k in range(n):
-            if k == len(dts):
-                dts.append(_next_dt(stepper, W, t))
+            if record:
+                if k == len(dts):
+                    dts.append(_next_dt(stepper, W, t))
                 t += dts[k]
             if checkpoint == "all":
                 stage[k], W = stepper.forward_stages(W, dts[k])
@@ -360,9 +362,11 @@ def rollout(W0, stepper, nsteps=None, dts=None, checkpoint="uniform", every=None
     if dts is None and nsteps is None:
         raise ValueError("give nsteps or dts")
     n = len(range(nsteps)) if dts is None else len(dts)
-    if dts is None:
-        _ptrs(W0)  # recording takes no copy of a strided W0
-    dts = [] if dts is None else list(dts)
+    if dts is not None:
+        dts = list(dts)
+    else:
+        with torch.no_grad():  # from W0 itself: what the stepper refuses, a copy is not either
+            dts = [_next_dt(stepper, W0.detach(), 0.0)] if n else []
     if checkpoint not in ("all", "uniform", "revolve"):
         raise ValueError("checkpoint must be 'all', 'uniform' or 'revolve'")
     if every is None:

@@ -236,3 +236,57 @@ def test_transcription_differentiable_regime():
     e5 = fd_vs_autograd(cfg, Wb, 6, 1e-5)
     assert e5 < 1e-3 and e5 < e4 / 5  # converges (first order: the fan's kinks)
     assert fd_vs_autograd(cfg, W, 6, 1e-5) > 1e-1
+
+
+class DecayStepper:
+    """A stepper on CPU tensors: S(W; dt) = W (1 - dt), dt = min W / 8, for
+    contiguous (8, 2, 3, 4) states as the GPU's."""
+
+    def cfl_dt(self, W, goal=1e30):
+        if tuple(W.shape) != (8, 2, 3, 4) or not W.is_contiguous():
+            raise ValueError("state")
+        return min(goal, float(W.min()) / 8)
+
+    def forward(self, W, dt):
+        return W * (1.0 - dt)
+
+    def reverse(self, W, dt, lam):
+        return lam * (1.0 - dt)
+
+    def forward_stages(self, W, dt):
+        return W, self.forward(W, dt)
+
+    def reverse_stages(self, W, Ws, Wout, dt, lam):
+        return self.reverse(W, dt, lam)
+
+
+@pytest.mark.parametrize("checkpoint", ["all", "revolve"])
+@pytest.mark.parametrize("n", [0, 1, 2, 5])
+def test_rollout_records_with_the_stepper_alone(n, checkpoint):
+    """Recorded step sizes are the stepper's own along the trajectory, whatever
+    it takes for a state."""
+    torch.manual_seed(3)
+    W0 = (torch.rand(8, 2, 3, 4) + 1.0).requires_grad_(True)
+    S = DecayStepper()
+    W, dts = A.rollout(W0, S, nsteps=n, checkpoint=checkpoint)
+    assert dts == A.record_dts(W0, S, n) and len(dts) == n
+    again, given = A.rollout(W0, S, dts=dts, checkpoint=checkpoint)
+    assert torch.equal(W, again) and given == dts
+    if n == 0:
+        return
+    W.sum().backward()
+    want = torch.ones_like(W0)
+    for dt in reversed(dts):
+        want = want * (1.0 - dt)
+    assert torch.equal(W0.grad, want)
+
+
+def test_rollout_takes_the_states_the_stepper_takes():
+    S = DecayStepper()
+    strided = (torch.rand(4, 3, 2, 8) + 1.0).permute(3, 2, 1, 0)
+    for W0 in (strided, torch.ones(7, 2, 3, 4)):
+        # no step asks the stepper about the state
+        W, dts = A.rollout(W0, S, nsteps=0)
+        assert dts == [] and torch.equal(W, W0)
+        with pytest.raises(ValueError, match="state"):
+            A.rollout(W0, S, nsteps=2)
