@@ -501,6 +501,21 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
   return NMHD_OK;
 }
 
+// Whether a field is memory that the CPU reaches like any other, and whether it
+// is pinned (its copies then need no buffer between).
+struct HostMemory {
+  bool plain, pinned;
+};
+HostMemory host_memory(const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return {true, false};
+  }
+  if (a.type == hipMemoryTypeUnregistered) return {true, false};
+  return {a.type == hipMemoryTypeHost, a.type == hipMemoryTypeHost};
+}
+
 bool box_ok(const nmhd_batch *b, int box) { return b && box >= 0 && box < b->nbox; }
 
 }  // namespace
@@ -638,6 +653,24 @@ int nmhd_batch_get_state(nmhd_batch *b, int box, float *const fields[8]) {
   if (!box_ok(b, box) || !fields) return bfail(b, NMHD_EINVAL, "bad argument");
   for (int f = 0; f < 8; ++f)
     if (!fields[f]) return bfail(b, NMHD_EINVAL, "null field pointer");
+  // Copies straight into the caller's arrays: where the CPU may not write them
+  // and, from half a megabyte a field, where they are pinned (96^3 580 us against
+  // 992 through the buffer, 256^3 9.5 ms against 18.2; 48^3 143 against 134).
+  const size_t cells = (size_t)b->boxes[box].b.ncell;
+  bool plain = true, pinned = true;
+  for (int f = 0; f < 8; ++f) {
+    const HostMemory m = host_memory(fields[f]);
+    plain = plain && m.plain;
+    pinned = pinned && m.pinned;
+  }
+  if (!plain || (pinned && 8 * cells > 4 * kStage)) {
+    const FieldPtrs W = box_fields(b->state[b->cur], b->boxes[box]);
+    for (int f = 0; f < 8; ++f)
+      BHIP(b, hipMemcpyAsync(fields[f], W.f[f], sizeof(float) * cells, hipMemcpyDeviceToHost,
+                             b->stream));
+    BHIP(b, hipStreamSynchronize(b->stream));
+    return NMHD_OK;
+  }
   for (int i = 0; i < 2; ++i) {
     if (!b->stage[i]) BHIP(b, hipHostMalloc(&b->stage[i], kStage * sizeof(float)));
     if (!b->staged[i]) BHIP(b, hipEventCreateWithFlags(&b->staged[i], hipEventDisableTiming));
@@ -646,7 +679,7 @@ int nmhd_batch_get_state(nmhd_batch *b, int box, float *const fields[8]) {
   // in flight while the last is spread over the caller's arrays.  A copy per
   // field into pageable memory took 30 us each whatever its size, 3.4 ms for
   // 14 boxes of 1.02M cells together; this takes 1.8 ms.
-  const size_t n = (size_t)b->boxes[box].b.ncell, total = 8 * n;
+  const size_t n = cells, total = 8 * n;
   const float *src = b->state[b->cur] + b->boxes[box].off8;
   auto piece = [&](size_t k) { return std::min(kStage, total - k * kStage); };
   auto fetch = [&](size_t k) {
