@@ -95,6 +95,7 @@ enum nmhd_fix {
 
 /* Tile shapes (TX x TY columns marched along z) of the tiled kernels. */
 enum nmhd_tile {
+  NMHD_TILE_AUTO = -1, /* kernel and shape by the box's size (the default) */
   NMHD_TILE_64x4 = 0,
   NMHD_TILE_32x8 = 1,
   NMHD_TILE_16x16 = 2
@@ -231,8 +232,9 @@ int nmhd_timing_get(nmhd_ctx *ctx, int i, const char **name, double *total_ms,
 int nmhd_set_path(nmhd_ctx *ctx, int path);
 int nmhd_get_path(const nmhd_ctx *ctx, int *path);
 /* Tile shapes (enum nmhd_tile) of the face and update kernels of
- * NMHD_PATH_TILED (by default kernel and shape follow the box's size);
- * results do not depend on them. */
+ * NMHD_PATH_TILED; results do not depend on them.  NMHD_TILE_AUTO for both
+ * also lets small boxes take kernels without tiles; for one of them it picks
+ * that kernel's shape.  nmhd_get_tiles returns what was set. */
 int nmhd_set_tiles(nmhd_ctx *ctx, int faces_tile, int update_tile);
 int nmhd_get_tiles(const nmhd_ctx *ctx, int *faces_tile, int *update_tile);
 
@@ -268,12 +270,12 @@ int nmhd_batch_get_time(nmhd_batch *batch, int box, double *t, int *generation);
 int nmhd_batch_get_status(nmhd_batch *batch, int box, int *steps_taken, int *goal_reached,
                           float *last_dt);
 
-/* Tiling: tile shape (enum nmhd_tile) of box's face and update kernels
- * (box = -1: every box); z chunk (planes per work item) and workgroups per
+/* Tiling: tile shape (enum nmhd_tile; NMHD_TILE_AUTO: by the box's size, as
+ * after creation) of box's face and update kernels (box = -1: every box); z chunk (planes per work item) and workgroups per
  * CU that walk the work table of the two kernels, where 0 (the default)
- * launches one workgroup per work item instead.  Until a chunk is set, each
- * kernel takes the one that a cost model expects to be fastest for the boxes
- * of the batch.  Results do not depend on the tiling or the launch mode. */
+ * launches one workgroup per work item instead.  A chunk of 0 (the default)
+ * stands for the one that a cost model expects to be fastest for the boxes of
+ * the batch; nmhd_batch_get_launch returns the chunks in use.  Results do not depend on the tiling or the launch mode. */
 int nmhd_batch_set_tiles(nmhd_batch *batch, int box, int faces_tile, int update_tile);
 int nmhd_batch_set_launch(nmhd_batch *batch, int faces_zchunk, int update_zchunk,
                           int faces_wg_per_cu, int update_wg_per_cu);

@@ -35,7 +35,7 @@ EXPORTS = (
     "nmhd_adj_reverse", "nmhd_adj_forward_stages", "nmhd_adj_reverse_stages",
     "nmhd_adj_forward_noalloc",
 )
-TILE_64x4, TILE_32x8, TILE_16x16 = 0, 1, 2
+TILE_AUTO, TILE_64x4, TILE_32x8, TILE_16x16 = -1, 0, 1, 2
 # enum nmhd_fix: corrections of reference quirks (0 = the reference's behaviour)
 FIX_CFL_SPEED, FIX_SHEAR_INTERP, FIX_FACE_POSITION, FIX_ALL = 1, 2, 4, 7
 

@@ -151,8 +151,7 @@ struct nmhd_ctx {
   double *diag_part = nullptr;  // run diagnostics: per-block partials, result
   double *diag_out = nullptr;
   int path = NMHD_PATH_TILED;
-  // tile shapes of the tiled path: kernel and shape by the box until
-  // nmhd_set_tiles names one
+  // tile shapes of the tiled path, as nmhd_set_tiles names them
   int ftile = kTileAuto, utile = kTileAuto;
   bool cfl_valid = false;  // rec[r].cfl holds the CFL minimum of the state (ghost cells aside)
   std::string err;
@@ -233,6 +232,17 @@ void collect_timing(nmhd_ctx *c) {
 
 int tile_of(int tile, int otherwise) { return tile == kTileAuto ? otherwise : tile; }
 
+// The tile arguments of a stage's launches: kTileAuto only for both, as the
+// routes of small boxes take both.
+int faces_tile(const nmhd_ctx *c) {
+  return c->utile == kTileAuto ? c->ftile
+                               : tile_of(c->ftile, tiled_shape(c->box.n[0], c->box.n[1], true));
+}
+int update_tile(const nmhd_ctx *c) {
+  return c->ftile == kTileAuto ? c->utile
+                               : tile_of(c->utile, tiled_shape(c->box.n[0], c->box.n[1], false));
+}
+
 int resolve_path(int p) { return p == NMHD_PATH_AUTO ? NMHD_PATH_TILED : p; }
 
 void flux_dispatch(nmhd_ctx *c, int d, FieldPtrs W, FluxOut F, const StepState *st, int hsel) {
@@ -282,7 +292,7 @@ void enqueue_step(nmhd_ctx *c, float goal) {
   auto stage = [&](int Win, int base, int Wout, int hsel, bool first, bool last) {
     if (tiled) {
       const StageStep ss{out, hsel, 0.0f};
-      if (c->ftile == kTileAuto && !(first && last) && tiny_stage(b)) {
+      if (faces_tile(c) == kTileAuto && !(first && last) && tiny_stage(b)) {
         timed(c, last ? S_UPDATE2 : S_UPDATE1, [&] {
           launch_tiny_stage(s, b, fields(c, Win), fields(c, base), fields(c, Wout), ss,
                             first ? open : OpenStep{}, last);
@@ -290,11 +300,12 @@ void enqueue_step(nmhd_ctx *c, float goal) {
         return;
       }
       timed(c, last ? S_FACES2 : S_FACES1, [&] {
-        launch_faces(s, b, fields(c, Win), F, ss, first ? open : OpenStep{}, c->ftile);
+        launch_faces(s, b, fields(c, Win), F, ss, first ? open : OpenStep{},
+                     faces_tile(c));
       });
       timed(c, last ? S_UPDATE2 : S_UPDATE1, [&] {
         launch_update_tiled(s, b, fields(c, Win), F, fields(c, base), fields(c, Wout), ss, false,
-                            last, c->utile);
+                            last, update_tile(c));
       });
       return;
     }
@@ -706,7 +717,7 @@ int nmhd_get_diagnostics(nmhd_ctx *c, nmhd_diagnostics *out) {
 }
 
 int nmhd_set_tiles(nmhd_ctx *c, int faces_tile, int update_tile) {
-  if (!c || faces_tile < 0 || faces_tile >= TV_COUNT || update_tile < 0 ||
+  if (!c || faces_tile < kTileAuto || faces_tile >= TV_COUNT || update_tile < kTileAuto ||
       update_tile >= TV_COUNT)
     return NMHD_EINVAL;
   int r = sync_and_check(c);
@@ -717,8 +728,8 @@ int nmhd_set_tiles(nmhd_ctx *c, int faces_tile, int update_tile) {
 
 int nmhd_get_tiles(const nmhd_ctx *c, int *faces_tile, int *update_tile) {
   if (!c) return NMHD_EINVAL;
-  if (faces_tile) *faces_tile = tile_of(c->ftile, TV_32x8);
-  if (update_tile) *update_tile = tile_of(c->utile, TV_64x4);
+  if (faces_tile) *faces_tile = c->ftile;
+  if (update_tile) *update_tile = c->utile;
   return NMHD_OK;
 }
 

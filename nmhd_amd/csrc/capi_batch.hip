@@ -147,6 +147,12 @@ int default_chunk(const nmhd_batch *b, bool faces) {
 int faces_chunk(const nmhd_batch *b) { return b->fzc ? b->fzc : default_chunk(b, true); }
 int update_chunk(const nmhd_batch *b) { return b->uzc ? b->uzc : default_chunk(b, false); }
 
+void set_tiles(nmhd_batch *b, int box, int faces, int update) {
+  const Box &x = b->boxes[box].b;
+  b->ftile[box] = faces == kTileAuto ? tiled_shape(x.n[0], x.n[1], true) : faces;
+  b->utile[box] = update == kTileAuto ? tiled_shape(x.n[0], x.n[1], false) : update;
+}
+
 std::vector<int> all_boxes(const nmhd_batch *b) {
   std::vector<int> v(b->nbox);
   for (int i = 0; i < b->nbox; ++i) v[i] = i;
@@ -560,8 +566,7 @@ int nmhd_batch_create(const nmhd_desc *descs, int nbox, nmhd_batch **out) {
     b->boxes[i].off21 = off21;
     off8 += 8 * b->boxes[i].b.ncell;
     off21 += 21 * b->boxes[i].b.ncell;
-    b->ftile[i] = tiled_shape(b->boxes[i].b.n[0], b->boxes[i].b.n[1], true);
-    b->utile[i] = tiled_shape(b->boxes[i].b.n[0], b->boxes[i].b.n[1], false);
+    set_tiles(b, i, kTileAuto, kTileAuto);
   }
   b->total8 = off8;
   b->total21 = off21;
@@ -740,17 +745,17 @@ int nmhd_batch_get_status(nmhd_batch *b, int box, int *steps_taken, int *goal_re
 }
 
 int nmhd_batch_set_tiles(nmhd_batch *b, int box, int faces_tile, int update_tile) {
-  if (!b || box < -1 || box >= b->nbox || faces_tile < 0 || faces_tile >= TV_COUNT ||
-      update_tile < 0 || update_tile >= TV_COUNT)
+  if (!b || box < -1 || box >= b->nbox || faces_tile < kTileAuto || faces_tile >= TV_COUNT ||
+      update_tile < kTileAuto || update_tile >= TV_COUNT)
     return bfail(b, NMHD_EINVAL, "bad tile selection");
   for (int i = 0; i < b->nbox; ++i)
-    if (box == -1 || box == i) b->ftile[i] = faces_tile, b->utile[i] = update_tile;
+    if (box == -1 || box == i) set_tiles(b, i, faces_tile, update_tile);
   b->items_dirty = true;
   return NMHD_OK;
 }
 
 int nmhd_batch_set_launch(nmhd_batch *b, int fzc, int uzc, int fwg, int uwg) {
-  if (!b || fzc < 1 || uzc < 1 || fzc > 32767 || uzc > 32767 || fwg < 0 || uwg < 0 || fwg > 64 ||
+  if (!b || fzc < 0 || uzc < 0 || fzc > 32767 || uzc > 32767 || fwg < 0 || uwg < 0 || fwg > 64 ||
       uwg > 64)
     return bfail(b, NMHD_EINVAL, "bad launch parameters");
   b->fzc = fzc;

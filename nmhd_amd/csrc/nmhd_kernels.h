@@ -246,7 +246,7 @@ struct WorkItem {
 
 // Tile shapes of the z-marching kernels (TX x TY, 256 threads each).
 enum TileVariant { TV_64x4 = 0, TV_32x8 = 1, TV_16x16 = 2, TV_COUNT = 3 };
-constexpr int kTileAuto = -1;  // kernel and tile shape by the box
+constexpr int kTileAuto = -1;  // NMHD_TILE_AUTO: kernel and tile shape by the box
 constexpr int kTileTX[TV_COUNT] = {64, 32, 16};
 constexpr int kTileTY[TV_COUNT] = {4, 8, 16};
 

@@ -435,3 +435,29 @@ def test_batch_state_into_pinned_memory_is_one_copy(gpu_ready):
     print("pageable %.0f us, pinned %.0f us" % (best[0] * 1e6, best[1] * 1e6), flush=True)
     assert best[1] < 0.8 * best[0]
     B.close()
+
+
+def test_batch_default_tiling_can_be_set_again(gpu_ready):
+    """Chunks of 0 and automatic tiles give back the tiling of a new batch."""
+    announce("batch tiling set and set back")
+    boxes = small_boxes(seed=17)
+    ref = single_runs(boxes, 1e30, 4)
+    B = make_batch(boxes)
+    fresh = B.get_launch()
+    B.set_tiles(capi.TILE_64x4, capi.TILE_16x16)
+    B.set_launch(29, 31, 1, 0)
+    assert B.get_launch() == (29, 31, 1, 0)
+    B.run(1e30, 2)
+    B.set_launch(0, 7, 0, 0)
+    assert B.get_launch()[1:] == (7, 0, 0)
+    B.set_launch(0, 0, 0, 0)
+    B.set_tiles(capi.TILE_AUTO, capi.TILE_AUTO)
+    assert B.get_launch() == fresh
+    B.run(1e30, 2)
+    assert_batch_equals(B, ref)
+    for bad in ((-1, 1, 0, 0), (1, -1, 0, 0)):
+        with pytest.raises(capi.NmhdError):
+            B.set_launch(*bad)
+    with pytest.raises(capi.NmhdError):
+        B.set_tiles(-2, 0)
+    B.close()

@@ -89,3 +89,49 @@ def test_large_box_equals_its_periodic_cell(gpu_ready, recon, integrator):
     assert (dt, t) == (dt4, t4)
     for a, b in zip(out, out4):
         assert np.array_equal(np.tile(a, (1, 4, 4, 4)).view(np.uint32), b.view(np.uint32))
+
+
+AUTO = capi.TILE_AUTO
+T328, T644 = capi.TILE_32x8, capi.TILE_64x4
+
+
+def test_automatic_tiles_can_be_set_again(gpu_ready):
+    """get_tiles returns what set_tiles takes: setting it back changes nothing,
+    and the small-box kernels, left by naming a shape, can be had again."""
+    cfg = P.make_config((16, 16, 16), cfl=0.1)
+    ctx = capi.Context(cfg)
+    ctx.set_state(rough(cfg, 3))
+    ctx.timing_enable()
+
+    def fused():
+        ctx.timing_reset()
+        ctx.run(1e30, 2)
+        t = ctx.timing()
+        assert t["update_s2"][1] == 2
+        return t["faces_s2"][1] == 0
+
+    assert ctx.get_tiles() == (AUTO, AUTO) and fused()
+    ctx.set_tiles(*ctx.get_tiles())
+    assert fused()
+    for tiles in ((T328, T644), (AUTO, T644), (T328, AUTO)):
+        ctx.set_tiles(*tiles)
+        assert ctx.get_tiles() == tiles and not fused()
+    ctx.set_tiles(AUTO, AUTO)
+    assert fused()
+    for bad in ((-2, 0), (0, -2), (3, 0), (AUTO, 3)):
+        with pytest.raises(capi.NmhdError):
+            ctx.set_tiles(*bad)
+    assert ctx.get_tiles() == (AUTO, AUTO)
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [(16, 16, 16), (65, 32, 32), (101, 80, 50)])
+@pytest.mark.parametrize("tiles", [(AUTO, T644), (T328, AUTO), (AUTO, capi.TILE_16x16)])
+def test_one_automatic_tile(gpu_ready, n, tiles):
+    """A shape for one kernel alone: the other takes a tile too."""
+    cfg = P.make_config(n, cfl=0.1)
+    W = rough(cfg, 11)
+    ref, got = run(cfg, W, (T328, T644)), run(cfg, W, tiles)
+    assert got[:2] == ref[:2]
+    for a, b in zip(got[2], ref[2]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
