@@ -461,3 +461,37 @@ def test_batch_default_tiling_can_be_set_again(gpu_ready):
     with pytest.raises(capi.NmhdError):
         B.set_tiles(-2, 0)
     B.close()
+
+
+@pytest.fixture(scope="module")
+def large_mix():
+    """3.61M cells, just past the 3.5M from which the batch kernels store past
+    the caches: a periodic, a shearing and a small first-order box, with their
+    single-box results after 3 steps."""
+    boxes = []
+    cfg = P.make_config((128, 128, 128), cfl=0.4)
+    boxes.append((cfg, P.orszag_tang_noisy(cfg, seed=51)))
+    cfg = P.config_c2((112, 112, 112))
+    boxes.append((cfg, P.shearing_box_mri(cfg, seed=52)))
+    cfg = P.make_config((33, 20, 17), cfl=0.4, recon=1)
+    boxes.append((cfg, P.orszag_tang_noisy(cfg, seed=53)))
+    assert sum(P.ncell(c) for c, _ in boxes) > 3500000
+    return boxes, single_runs(boxes, 1e30, 3)
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("launch", [(0, 0, 0, 0), (16, 7, 2, 3), (5, 16, 0, 3), (16, 16, 4, 0)])
+def test_batch_past_the_caches(gpu_ready, large_mix, launch, wide):
+    """A workgroup per item and walking workgroups, with and without 64x4 face
+    tiles, in a batch past the size from which results go past the caches
+    (small_boxes' tests run the same launches through them)."""
+    announce("large batch, launch %s, 64x4 face tiles %s" % (launch, wide))
+    boxes, ref = large_mix
+    B = make_batch(boxes)
+    B.set_tiles(capi.TILE_16x16, capi.TILE_64x4, box=1)
+    B.set_tiles(capi.TILE_64x4 if wide else capi.TILE_32x8, capi.TILE_32x8, box=2)
+    B.set_launch(*launch)
+    B.run(1e30, 1, use_graph=False)
+    B.run(1e30, 2, use_graph=True)
+    assert_batch_equals(B, ref)
+    B.close()
