@@ -134,7 +134,8 @@ int default_chunk(const nmhd_batch *b, bool faces) {
   const std::vector<int> &tile = faces ? b->ftile : b->utile;
   int nz = 1;
   for (const BatchBox &bb : b->boxes) nz = std::max(nz, bb.b.n[2]);
-  return march_chunk(faces, nz, [&](int zc) {
+  const bool wide = std::find(tile.begin(), tile.end(), (int)TV_64x4) != tile.end();
+  return march_chunk(faces, nz, march_per_cu(faces, wide), [&](int zc) {
     long n = 0;
     for (int i = 0; i < b->nbox; ++i) {
       const Box &x = b->boxes[i].b;

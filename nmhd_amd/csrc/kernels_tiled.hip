@@ -87,9 +87,17 @@ constexpr MarchCost kUpdateCost = {{2.3f, 3.1f, 4.0f, 5.5f}, 16};
 
 }  // namespace
 
-int march_chunk(bool faces, int nz, const std::function<long(int)> &groups_at) {
+// Counted as four, 64x4 face tiles (and all face tiles of a batch with any)
+// took chunks with a second round: 64x4x2000 cells 35 us a face launch against
+// 30, 640x12x400 130 / 117, a step of 18 boxes of 2.39M cells 382 / 352, of 17
+// of 0.83M 188 / 167.
+int march_per_cu(bool faces, bool wide) {
+  return faces && wide ? tiled::FacesShape<64, 4>::kWavesPerSimd : 4;
+}
+
+int march_chunk(bool faces, int nz, int per_cu, const std::function<long(int)> &groups_at) {
   // A march of zc planes costs about one plane more (the prologue and the
-  // last z-face); 1024 workgroups are resident (4 per CU).  In one round a
+  // last z-face); 256 per_cu workgroups are resident.  In one round a
   // CU's share decides; past it the rounds blend, except that a remainder of
   // the first ones costs more than its share, a small one nearly a round of its
   // own (1050 workgroups 1.5 rounds, 1216 1.4, 1408 1.5, 1664 1.7, 2112 2.3,
@@ -101,17 +109,17 @@ int march_chunk(bool faces, int nz, const std::function<long(int)> &groups_at) {
   float least = 0.0f;
   for (int want = 1; want <= c.most && want <= nz; ++want) {
     const int chunks = (nz + want - 1) / want, zc = (nz + chunks - 1) / chunks;
-    const float rounds = (float)groups_at(zc) / 1024.0f;
+    const float rounds = (float)groups_at(zc) / (256.0f * (float)per_cu);
     float cost;
     if (rounds <= 1.0f) {
-      const int share = (int)std::ceil(rounds * 4.0f);
+      const int share = (int)std::ceil(rounds * (float)per_cu);
       cost = c.plane[share < 1 ? 0 : share - 1] * (float)(zc + 1);
     } else {
       const float whole = std::floor(rounds), part = rounds - whole;
       const float extra =
           part > 0.0f ? (0.4f * std::max(0.0f, 1.0f - part / 0.3f) + 0.15f * (1.0f - part)) / whole
                       : 0.0f;
-      cost = c.plane[3] * (float)(zc + 1) * (rounds + extra);
+      cost = c.plane[per_cu - 1] * (float)(zc + 1) * (rounds + extra);
     }
     if (best == 1 && want == 1) least = cost;
     if (cost < least) least = cost, best = zc;
@@ -119,10 +127,15 @@ int march_chunk(bool faces, int nz, const std::function<long(int)> &groups_at) {
   return best;
 }
 
+namespace {
+
 int tiled_zchunk(const Box &b, int tx, int ty, bool faces) {
   const long cols = (long)((b.n[0] + tx - 1) / tx) * ((b.n[1] + ty - 1) / ty);
-  return march_chunk(faces, b.n[2], [&](int zc) { return cols * ((b.n[2] + zc - 1) / zc); });
+  return march_chunk(faces, b.n[2], march_per_cu(faces, tx == 64),
+                     [&](int zc) { return cols * ((b.n[2] + zc - 1) / zc); });
 }
+
+}  // namespace
 
 int tiled_shape(int nx, int ny, bool faces) {
   // Cells that tiles of a shape cover, idle lanes included.  Per covered cell

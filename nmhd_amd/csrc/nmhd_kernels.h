@@ -358,11 +358,12 @@ void launch_direct_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet
 
 // kernels_tiled.hip
 // Planes per march of the face or update kernel: the chunk of the least
-// estimated time, groups_at(zc) the workgroups of the launch with chunks of zc.
+// estimated time, groups_at(zc) the workgroups of the launch with chunks of zc,
+// per_cu how many of them a CU holds (march_per_cu).
 // whether the stage kernels over that many cells store past the caches
 bool streamed(long cells);
-int march_chunk(bool faces, int nz, const std::function<long(int)> &groups_at);
-int tiled_zchunk(const Box &b, int tx, int ty, bool faces);
+int march_chunk(bool faces, int nz, int per_cu, const std::function<long(int)> &groups_at);
+int march_per_cu(bool faces, bool wide);  // wide: 64x4 tiles in the launch
 // Tile shape (TileVariant) of the face or update kernel for a box.
 int tiled_shape(int nx, int ny, bool faces);
 // tile: TileVariant of the z-marching tiles, or kTileAuto (both launches of a

@@ -495,3 +495,16 @@ def test_batch_past_the_caches(gpu_ready, large_mix, launch, wide):
     B.run(1e30, 2, use_graph=True)
     assert_batch_equals(B, ref)
     B.close()
+
+
+def test_batch_chunks_fill_the_rounds_of_64x4_tiles(gpu_ready):
+    """Three workgroups of 64x4 face tiles share a CU, four of the other
+    shapes: 768 are resident, and a chunk that makes 1000 of them waits for a
+    second round (64x4x2000 cells: the faces take 35 us, 30 with 667)."""
+    announce("face chunk of 64x4 tiles")
+    B = capi.Batch([P.make_config((64, 4, 2000))])
+    B.set_tiles(capi.TILE_64x4, capi.TILE_64x4)
+    assert 512 < -(-2000 // B.get_launch()[0]) <= 768
+    B.set_tiles(capi.TILE_32x8, capi.TILE_64x4)
+    assert 768 < 2 * -(-2000 // B.get_launch()[0]) <= 1024
+    B.close()
