@@ -283,14 +283,15 @@ int nmhd_batch_get_launch(const nmhd_batch *batch, int *faces_zchunk, int *updat
                           int *faces_wg_per_cu, int *update_wg_per_cu);
 /* Autotuner: per distinct box shape, time every tile shape of both kernels
  * (one workgroup walking that shape's tiles, i.e. the workgroup-time the
- * shape costs in a launch that walks a table) and keep the fastest; then time the
- * z chunk and workgroups per CU of the whole batch.  Results are cached in
- * the text file cache_path (NULL: $NMHD_TUNE_CACHE, else
- * $HOME/.cache/nmhd_amd/batch_tuning.txt), keyed by the GPU architecture
- * and the box shape (and, for the launch parameters, the batch's shapes);
- * cached entries are reused without timing.  *timed_shapes (may be NULL)
- * returns how many shapes were timed.  Overwrites the batch's scratch
- * buffers, not the boxes' states. */
+ * shape costs) and keep the fastest; then time, for the whole batch, both
+ * kernels with these and with the default shapes at several z chunks and
+ * workgroups per CU.  The default tiling stays unless another is faster.
+ * Results are cached in the text file cache_path (NULL: $NMHD_TUNE_CACHE, else
+ * $HOME/.cache/nmhd_amd/batch_tuning.txt), keyed by the GPU architecture with
+ * the version of the kernels and the box shape (and, for the launch
+ * parameters, the batch's shapes); cached entries are reused without timing.
+ * *timed_shapes (may be NULL) returns how many shapes were timed.  Overwrites
+ * the batch's scratch buffers, not the boxes' states. */
 int nmhd_batch_autotune(nmhd_batch *batch, const char *cache_path, int *timed_shapes);
 
 /* MHDSolver::proceed for every box: at most nsteps steps toward goal_time

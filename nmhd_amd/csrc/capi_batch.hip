@@ -31,9 +31,12 @@ namespace {
 // per thread: the message of the calling thread's last failed create
 thread_local std::string g_batch_create_error;
 
-constexpr int kZChunks[5] = {2, 4, 8, 16, 32};
+constexpr int kZChunks[6] = {0, 2, 4, 8, 16, 32};  // 0: by default_chunk
 constexpr int kWgPerCu[5] = {0, 1, 2, 3, 4};  // 0: one workgroup per item
 constexpr size_t kStage = 1 << 18;  // floats of a half of the copy-out buffer
+// Raised with any change of the batch kernels or of the default tiling, so that
+// entries of other kernels are not found.
+constexpr int kTuneVersion = 2;
 constexpr int kTuneItems = 48;  // work items timed per shape and tile shape
 
 }  // namespace
@@ -203,6 +206,17 @@ int grid_of(const nmhd_batch *b, int nitems, int wg_per_cu) {
   return std::min(nitems, wg_per_cu * b->cus);
 }
 
+// The two launches of a stage over the work tables, the states by their slots.
+void enqueue_faces(nmhd_batch *b, int from, const BatchStep &step) {
+  launch_batch_faces(b->stream, grid_of(b, b->nf, b->fwg), b->d_boxes, b->d_fitems, b->nf,
+                     b->state[from], b->flux, step, b->fwide, streamed(b->total8 / 8));
+}
+void enqueue_update(nmhd_batch *b, int from, int base, int to, const BatchStep &step, bool last) {
+  launch_batch_update(b->stream, grid_of(b, b->nu, b->uwg), b->d_boxes, b->d_uitems, b->nu,
+                      b->state[from], b->flux, b->state[base], b->state[to], step, last,
+                      streamed(b->total8 / 8));
+}
+
 // One iteration of the proceed() loop for every box.
 void enqueue_step(nmhd_batch *b, bool full_cfl, float goal) {
   hipStream_t s = b->stream;
@@ -217,14 +231,9 @@ void enqueue_step(nmhd_batch *b, bool full_cfl, float goal) {
     launch_batch_cfl(s, b->d_boxes, n, b->state[A], goal, in);
   else if (b->grid_gcfl)
     launch_batch_cfl_ghosts(s, b->d_boxes, n, b->grid_gcfl, b->state[A], in);
-  const bool nt = streamed(b->total8 / 8);
   auto stage = [&](int from, int base, int to, int hsel, bool first, bool last) {
-    launch_batch_faces(s, grid_of(b, b->nf, b->fwg), b->d_boxes, b->d_fitems, b->nf,
-                       b->state[from], b->flux,
-                       BatchStep{rec, first ? in : nullptr, b->d_goal, hsel}, b->fwide, nt);
-    launch_batch_update(s, grid_of(b, b->nu, b->uwg), b->d_boxes, b->d_uitems, b->nu,
-                        b->state[from], b->flux, b->state[base], b->state[to],
-                        BatchStep{rec, nullptr, nullptr, hsel}, last, nt);
+    enqueue_faces(b, from, BatchStep{rec, first ? in : nullptr, b->d_goal, hsel});
+    enqueue_update(b, from, base, to, BatchStep{rec, nullptr, nullptr, hsel}, last);
   };
   if (b->integrator == NMHD_EULER1) {
     stage(A, A, next, H_FULL, true, true);
@@ -306,6 +315,10 @@ std::string shape_key(const nmhd_batch *b, int box) {
   return o.str();
 }
 
+std::string kernels_key(const nmhd_batch *b) {
+  return b->arch + "/" + std::to_string(kTuneVersion) + " ";
+}
+
 std::string cache_file(const char *path) {
   if (path && *path) return path;
   const char *env = std::getenv("NMHD_TUNE_CACHE");
@@ -320,7 +333,16 @@ void make_parent_dirs(const std::string &file) {
 }
 
 // Cache lines: "shape <arch> <nx> <ny> <nz> <recon> <source> : <faces> <update>"
-// and "launch <arch> <hash> : <fzc> <uzc> <fwg> <uwg>".
+// and "launch <arch> <hash> : <fzc> <uzc> <fwg> <uwg> <ftuned> <utuned>", the
+// last two whether a kernel takes the tuned tile shapes (1) or the default ones;
+// <arch> ends in the version of the kernels timed (kTuneVersion).
+// Whether an entry read back holds as many values, each in 0..most.
+bool within(const std::vector<int> &v, const std::vector<int> &most) {
+  if (v.size() != most.size()) return false;
+  for (size_t i = 0; i < v.size(); ++i)
+    if (v[i] < 0 || v[i] > most[i]) return false;
+  return true;
+}
 struct TuneCache {
   std::map<std::string, std::vector<int>> entries;
   void load(const std::string &file) {
@@ -359,25 +381,50 @@ std::string launch_key(const nmhd_batch *b) {
     for (char c : s + ";") h = (h ^ (unsigned char)c) * 1099511628211ull;
   char buf[64];
   std::snprintf(buf, sizeof(buf), "%016llx", h);
-  return "launch " + b->arch + " " + buf;
+  return "launch " + kernels_key(b) + buf;
 }
 
-// Milliseconds of one launch of fn (after one untimed warm-up launch).
+// Milliseconds of one launch of fn (after one untimed warm-up launch), the
+// least of reps.
 template <class F>
-int time_launch(nmhd_batch *b, F &&fn, float *ms) {
+int time_launch(nmhd_batch *b, F &&fn, float *ms, int reps = 1) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   BHIP(b, hipEventCreate(&e0));
   BHIP(b, hipEventCreate(&e1));
   fn();
-  BHIP(b, hipEventRecord(e0, b->stream));
-  fn();
-  BHIP(b, hipEventRecord(e1, b->stream));
-  BHIP(b, hipEventSynchronize(e1));
-  BHIP(b, hipGetLastError());
-  BHIP(b, hipEventElapsedTime(ms, e0, e1));
+  *ms = 1e30f;
+  for (int i = 0; i < reps; ++i) {
+    float t = 0.0f;
+    BHIP(b, hipEventRecord(e0, b->stream));
+    fn();
+    BHIP(b, hipEventRecord(e1, b->stream));
+    BHIP(b, hipEventSynchronize(e1));
+    BHIP(b, hipGetLastError());
+    BHIP(b, hipEventElapsedTime(&t, e0, e1));
+    *ms = std::min(*ms, t);
+  }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   return NMHD_OK;
+}
+
+const std::vector<int> kLaunchMost = {32767, 32767, 64, 64, 1, 1};
+
+// How a batch is tiled (nmhd_batch's members of these names).
+struct Tiling {
+  std::vector<int> ftile, utile;
+  int fzc = 0, uzc = 0, fwg = 0, uwg = 0;
+  int ftuned = 0, utuned = 0;  // tile shapes: the timed ones
+};
+
+void set_tiling(nmhd_batch *b, const Tiling &t) {
+  b->ftile = t.ftile;
+  b->utile = t.utile;
+  b->fzc = t.fzc;
+  b->uzc = t.uzc;
+  b->fwg = t.fwg;
+  b->uwg = t.uwg;
+  b->items_dirty = true;
 }
 
 int prepare_tune_records(nmhd_batch *b) {
@@ -407,13 +454,20 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
   const bool nt = streamed(b->total8 / 8);
   int ntimed = 0;
 
+  // the default tiling, and the tile shapes timed as the best
+  Tiling plain, tuned;
+  for (int i = 0; i < b->nbox; ++i) set_tiles(b, i, kTileAuto, kTileAuto);
+  plain.ftile = tuned.ftile = b->ftile;
+  plain.utile = tuned.utile = b->utile;
+  tuned.ftuned = tuned.utuned = 1;
+
   // per shape: the workgroup-time of each tile shape
   std::map<std::string, std::vector<int>> groups;
   for (int i = 0; i < b->nbox; ++i) groups[shape_key(b, i)].push_back(i);
   for (auto &g : groups) {
-    const std::string key = "shape " + b->arch + " " + g.first;
+    const std::string key = "shape " + kernels_key(b) + g.first;
     auto hit = cache.entries.find(key);
-    if (hit == cache.entries.end() || hit->second.size() != 2) {
+    if (hit == cache.entries.end() || !within(hit->second, {TV_COUNT - 1, TV_COUNT - 1})) {
       float best_f = 1e30f, best_u = 1e30f;
       int vf = TV_16x16, vu = TV_16x16;
       for (int v = 0; v < TV_COUNT; ++v) {
@@ -449,60 +503,78 @@ int tune(nmhd_batch *b, const char *path, int *timed) {
       ++ntimed;
     }
     for (int box : g.second) {
-      b->ftile[box] = cache.entries[key][0];
-      b->utile[box] = cache.entries[key][1];
+      tuned.ftile[box] = cache.entries[key][0];
+      tuned.utile[box] = cache.entries[key][1];
     }
   }
 
-  // whole batch: z chunk and workgroups per CU of each launch
+  // whole batch: tile shapes, z chunk and workgroups per CU of each kernel, the
+  // faces' first, then the update's.  Each is timed as a step runs it: the
+  // stages' launches, the last update with its CFL epilogue.  The default tiling
+  // is kept unless another takes less than 0.99 of its time, of the kernel and
+  // then of the whole step (timings of one tiling differ by that).
   const std::string lkey = launch_key(b);
   auto hit = cache.entries.find(lkey);
-  if (hit == cache.entries.end() || hit->second.size() != 4) {
-    const std::vector<int> all = all_boxes(b);
-    float best_f = 1e30f, best_u = 1e30f;
-    int fzc = 16, uzc = 16, fwg = 0, uwg = 0;
-    for (int zc : kZChunks) {
-      const std::vector<WorkItem> fi = make_items(b, b->ftile, zc, all);
-      r = upload_items(b, fi, &b->d_titems, &b->cap_t);
+  if (hit == cache.entries.end() || !within(hit->second, kLaunchMost)) {
+    const int cur = b->cur, one = (cur + 1) % 3, two = (cur + 2) % 3;
+    const bool euler = b->integrator == NMHD_EULER1;
+    auto faces = [&] {
+      enqueue_faces(b, cur, step);
+      if (!euler) enqueue_faces(b, one, step);
+    };
+    auto update = [&] {
+      if (!euler) enqueue_update(b, cur, cur, one, step, false);
+      enqueue_update(b, euler ? cur : one, cur, two, step, true);
+    };
+    auto whole = [&] {
+      enqueue_faces(b, cur, step);
+      enqueue_update(b, cur, cur, one, step, euler);
+      if (euler) return;
+      enqueue_faces(b, one, step);
+      enqueue_update(b, one, cur, two, step, true);
+    };
+    auto time_tiling = [&](const Tiling &t, auto &&launches, float *ms) {
+      set_tiling(b, t);
+      const int rc = refresh_items(b);
+      return rc ? rc : time_launch(b, launches, ms, 3);
+    };
+    Tiling best = plain;
+    float whole_plain, whole_best, least;
+    r = time_tiling(plain, whole, &whole_plain);
+    if (r) return r;
+    for (int kernel = 0; kernel < 2; ++kernel) {
+      auto time_kernel = [&](const Tiling &t, float *ms) {
+        return kernel == 0 ? time_tiling(t, faces, ms) : time_tiling(t, update, ms);
+      };
+      r = time_kernel(best, &least);
       if (r) return r;
-      for (int wg : kWgPerCu) {
-        float ms = 0.0f;
-        const int n = (int)fi.size();
-        r = time_launch(
-            b,
-            [&] {
-              launch_batch_faces(b->stream, grid_of(b, n, wg), b->d_boxes, b->d_titems, n, in,
-                                 b->flux, step, has_wide(fi), nt);
-            },
-            &ms);
-        if (r) return r;
-        if (ms < best_f) best_f = ms, fzc = zc, fwg = wg;
-      }
-      const std::vector<WorkItem> ui = make_items(b, b->utile, zc, all);
-      r = upload_items(b, ui, &b->d_titems, &b->cap_t);
-      if (r) return r;
-      for (int wg : kWgPerCu) {
-        float ms = 0.0f;
-        const int n = (int)ui.size();
-        r = time_launch(
-            b,
-            [&] {
-              launch_batch_update(b->stream, grid_of(b, n, wg), b->d_boxes, b->d_titems, n, in,
-                                  b->flux, in, scratch, step, false, nt);
-            },
-            &ms);
-        if (r) return r;
-        if (ms < best_u) best_u = ms, uzc = zc, uwg = wg;
-      }
+      least *= 0.99f;
+      for (const Tiling *tiles : {&plain, &tuned})
+        for (int zc : kZChunks) {
+          if (tiles == &tuned && (kernel == 0 ? tuned.ftile == plain.ftile
+                                              : tuned.utile == plain.utile))
+            break;
+          for (int wg : kWgPerCu) {
+            Tiling t = best;
+            if (kernel == 0)
+              t.ftile = tiles->ftile, t.fzc = zc, t.fwg = wg, t.ftuned = tiles->ftuned;
+            else
+              t.utile = tiles->utile, t.uzc = zc, t.uwg = wg, t.utuned = tiles->utuned;
+            float ms;
+            r = time_kernel(t, &ms);
+            if (r) return r;
+            if (ms < least) least = ms, best = t;
+          }
+        }
     }
-    cache.entries[lkey] = {fzc, uzc, fwg, uwg};
+    r = time_tiling(best, whole, &whole_best);
+    if (r) return r;
+    if (!(whole_best < 0.99f * whole_plain)) best = plain;
+    cache.entries[lkey] = {best.fzc, best.uzc, best.fwg, best.uwg, best.ftuned, best.utuned};
   }
   const std::vector<int> &lp = cache.entries[lkey];
-  b->fzc = lp[0];
-  b->uzc = lp[1];
-  b->fwg = lp[2];
-  b->uwg = lp[3];
-  b->items_dirty = true;
+  set_tiling(b, Tiling{lp[4] ? tuned.ftile : plain.ftile, lp[5] ? tuned.utile : plain.utile,
+                       lp[0], lp[1], lp[2], lp[3], lp[4], lp[5]});
   (void)cache.save(file);  // a read-only cache location only costs a re-tune
   if (timed) *timed = ntimed;
   return NMHD_OK;
