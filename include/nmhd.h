@@ -353,9 +353,9 @@ int nmhd_adj_reverse_stages(nmhd_adj *adj, const float *const w_in[8],
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (work under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): w_out = S(w_in; dt) as nmhd_adj_forward computes it,
- * with the same kernels and bit-identical results, but with no nmhd_adj
- * object and no allocation.  The step's scratch (step record, midpoint
- * stage state, the face-to-update hand-off) is a fixed device array of the
+ * with the same arithmetic and bit-identical results, but with no nmhd_adj
+ * object and no allocation.  The step's scratch (midpoint stage state
+ * and the face-to-update hand-off) is a fixed device array of the
  * library, one per GPU, held until the process ends (76 MiB): boxes of at
  * most NMHD_NOALLOC_MAX_CELLS cells; larger ones are rejected (NMHD_EINVAL).
  * Periodic boxes only, as nmhd_adj_create.  Work is enqueued on `stream` (a

@@ -22,10 +22,15 @@ namespace nmhd {
 void enqueue_frozen_step(hipStream_t s, const Box &b, int integrator, FieldPtrs Win,
                          FieldPtrs Wstar, FieldPtrs Wout, const FluxSet &F, float dt) {
   const StageStep full{nullptr, H_FIXED, dt}, half{nullptr, H_FIXED, dt / 2};
+  bool all = true;  // 21 arrays
+  for (const FluxOut &d : F.dir)
+    for (const float *p : d.f) all = all && p;
+  const int ftile = all ? kTileAuto : tiled_shape(b.n[0], b.n[1], true);
+  const int utile = all ? kTileAuto : tiled_shape(b.n[0], b.n[1], false);
   auto stage = [&](FieldPtrs in, FieldPtrs out, const StageStep &ss) {
     if (tiny_stage(b)) return launch_tiny_stage(s, b, in, Win, out, ss, OpenStep{}, false);
-    launch_faces(s, b, in, F, ss);
-    launch_update_tiled(s, b, in, F, Win, out, ss, false, false);
+    launch_faces(s, b, in, F, ss, OpenStep{}, ftile);
+    launch_update_tiled(s, b, in, F, Win, out, ss, false, false, utile);
   };
   if (integrator == NMHD_EULER1) return stage(Win, Wout, full);
   stage(Win, Wstar, half);

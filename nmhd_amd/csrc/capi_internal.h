@@ -18,8 +18,9 @@ void derive_box(const nmhd_desc *d, Box &b, nmhd_geometry &g);
 
 // The frozen-dt step W_out = S(W_in; dt) of a periodic box with the
 // production stage kernels, enqueued on s: Wstar holds the midpoint stage
-// state (unused for NMHD_EULER1), and of F only the 11 arrays the face kernel
-// hands to the update kernel (tiled::stage_buf) are used.
+// state (unused for NMHD_EULER1).  F: the 11 arrays that the face march hands
+// to the update (tiled::stage_buf), the others null, or all 21, which the
+// kernels of small boxes (direct_stage) need.
 void enqueue_frozen_step(hipStream_t s, const Box &b, int integrator, FieldPtrs Win,
                          FieldPtrs Wstar, FieldPtrs Wout, const FluxSet &F, float dt);
 

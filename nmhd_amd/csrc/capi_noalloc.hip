@@ -1,15 +1,16 @@
 // capi_noalloc.hip -- nmhd_adj_forward_noalloc: the frozen-dt step of
 // nmhd_adj_forward for callers that cannot allocate device memory (work
 // under HIP graph capture, tight serving loops, harnesses that forbid
-// hipMalloc).  The step's scratch -- the midpoint stage state W* and the 11
-// arrays the face kernel hands to the update kernel -- lives in one file-scope device array of fixed size instead of buffers
-// allocated by nmhd_adj_create.  Every GPU the library runs on holds its
+// hipMalloc).  The step's scratch -- the midpoint stage state W* and the
+// arrays the face kernel hands to the update kernel -- lives in one file-scope
+// device array of fixed size instead of buffers allocated by nmhd_adj_create.
+// Every GPU the library runs on holds its
 // own copy of the array until the process ends.
 //
 // Layout: arrays of array_stride(ncell) floats each, so that every array
 // starts 256-byte aligned: W* (8), then the face -> update hand-off: the hydro
 // divergence (5) and the six face B fluxes (6), or for a box on the direct
-// route all 21 face fluxes.
+// route all 21 face fluxes where they fit.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -24,7 +25,6 @@ constexpr size_t kArrays = 8 + 11;    // W* + the face -> update hand-off
 constexpr size_t kMaxCells = NMHD_NOALLOC_MAX_CELLS;
 constexpr size_t kScratchFloats = kArrays * (kMaxCells + 64);  // strides included
 static_assert(kMaxCells % 64 == 0, "a box's stride is at most kMaxCells + 64 floats");
-static_assert((8 + 21) * (kDirectCells + 128) <= kScratchFloats, "all fluxes of a direct box fit");
 }  // namespace
 
 // The scratch.  In host code `scratch` names a host-side stand-in, not the
@@ -108,7 +108,7 @@ int nmhd_adj_forward_noalloc(const nmhd_desc *desc, const float *const w_in[8], 
   FluxSet F;
   for (int d = 0; d < 3; ++d)
     for (int k = 0; k < 7; ++k) F.dir[d].f[k] = nullptr;
-  if (direct_stage(b)) {  // a small box hands over every flux
+  if (direct_stage(b) && (8 + 21) * stride <= kScratchFloats) {  // to 687,000 cells
     for (int d = 0; d < 3; ++d)
       for (int k = 0; k < 7; ++k) F.dir[d].f[k] = slot(8 + 7 * d + k);
   } else {

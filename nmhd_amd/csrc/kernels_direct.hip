@@ -142,11 +142,14 @@ __global__ void __launch_bounds__(kThreads)
 
 }  // namespace direct
 
-// Up to 400,000 cells (kDirectCells).  Step times, direct faces against the march: 32^3 26.0
-// / 33.7 us, 64^3 48.5 / 54.3, 64x72x64 68.4 / 77.8, 80^3 102.3 / 97.8, 96^3
-// 139.7 / 135.2, 128^3 304 / 250: the chip is then full of tiles, and the
-// update reads 10 arrays more.
-bool direct_stage(const Box &b) { return b.ncell <= kDirectCells; }
+// Up to 850,000 cells.  Step times, direct faces against the march: 32^3 26.0 /
+// 33.7 us, 64^3 47.0 / 54.2, 75^3 69.7 / 79.6, 80^3 80.3 / 87.1, 90^3 103 / 116,
+// 100x100x60 85 / 111, 64x64x192 (which the tiles fit) 96.4 / 101.2, shearing
+// 64x64x150 98.9 / 108.4, first-order 64x64x192 90.4 / 96.2.  Past that the
+// update's ten more arrays cost flat boxes that the tiles fit more than the
+// tiles' prologues: 256x256x14 (0.92M) 121 / 118, 512x64x30 (0.98M) 125 / 118,
+// 128x128x64 122.5 / 121.6, though ragged ones gain to 1.4M (112^3 167 / 178).
+bool direct_stage(const Box &b) { return b.ncell <= 850000; }
 
 void launch_direct_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F,
                          const StageStep &ss, const OpenStep &open) {

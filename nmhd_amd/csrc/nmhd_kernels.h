@@ -351,7 +351,6 @@ void launch_tiny_stage(hipStream_t s, const Box &b, FieldPtrs Win, FieldPtrs Wba
 
 // kernels_direct.hip (the stage of a small box: a thread per face, a thread
 // per cell; all 21 flux arrays are used)
-constexpr long kDirectCells = 400000;  // largest box on this route
 bool direct_stage(const Box &b);
 void launch_direct_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet &F,
                          const StageStep &ss, const OpenStep &open);

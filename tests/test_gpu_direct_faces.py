@@ -135,3 +135,58 @@ def test_one_automatic_tile(gpu_ready, n, tiles):
     assert got[:2] == ref[:2]
     for a, b in zip(got[2], ref[2]):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+# 850,000 cells is the last size that takes a thread per face; the frozen step
+# without allocation has room for its fluxes to 687,000
+@pytest.mark.parametrize("n", [(85, 100, 100), (100, 85, 101)])
+@pytest.mark.parametrize("recon,integrator", [(0, 0), (1, 1)])
+def test_direct_equals_tiles_at_its_limit(gpu_ready, n, recon, integrator):
+    cfg = P.make_config(n, cfl=0.1, recon=recon, integrator=integrator)
+    W = rough(cfg, 11)
+    ref, got = run(cfg, W, (T328, T644)), run(cfg, W, None)
+    assert got[:2] == ref[:2]
+    for a, b in zip(got[2], ref[2]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [(100, 67, 102), (100, 67, 103), (85, 100, 100), (100, 85, 101)])
+@pytest.mark.parametrize("integrator", [0, 1])
+def test_noalloc_step_at_the_limits_of_direct_faces(gpu_ready, n, integrator):
+    import torch
+    from nmhd_amd import adjoint as A
+    cfg = P.make_config(n, cfl=0.1, integrator=integrator)
+    W = torch.tensor(rough(cfg, 4), device="cuda")
+    S = A.Stepper(cfg)
+    dt = S.cfl_dt(W)
+    ref = S.forward(W, dt)
+    got = A.forward_noalloc(cfg, W, dt, torch.full_like(W, float("nan")))
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), ref.cpu().numpy().view(np.uint32))
+    S.close()
+
+
+@pytest.mark.parametrize("n", [(75, 75, 75), (90, 90, 90), (100, 100, 80)])
+def test_boxes_below_the_limit_are_faster_than_on_tiles(gpu_ready, n):
+    """The limit lies where the faces' threads stop to pay (75^3 70 us a step
+    against 80 on tiles, 90^3 103 against 116)."""
+    import time
+    cfg = P.make_config(n, cfl=0.1)
+    W = P.orszag_tang(cfg)
+    W[4] += 1.0
+    ctx = [capi.Context(cfg) for _ in range(3)]
+    ctx[1].set_tiles(T328, T644)
+    ctx[2].set_tiles(T328, T328)
+    best = [1e9] * 3
+    for c in ctx:
+        c.set_state(W)
+        c.run(1e30, 32)
+    for rep in range(6):
+        for i, c in enumerate(ctx):
+            t = time.perf_counter()
+            c.run(1e30, 64)
+            best[i] = min(best[i], time.perf_counter() - t)
+    print("\n[case] %s us a step: default %.1f, tiles %.1f, %.1f" % ((n,) + tuple(
+        b / 64 * 1e6 for b in best)), flush=True)
+    assert best[0] < 0.97 * min(best[1:])
+    for c in ctx:
+        c.close()
