@@ -68,6 +68,21 @@ KERNEL_BYTES = {
         "cfl": 32.0,
     },
 }
+# small boxes on the tiled path: a thread per face up to DIRECT_CELLS array cells
+# (all 21 fluxes between the kernels), a whole stage per launch below that
+DIRECT_CELLS = 850000
+KERNEL_BYTES["direct"] = {
+    "faces_s1": 116.0,   # read W (8), write 21 fluxes
+    "faces_s2": 116.0,
+    "update_s1": 148.0,  # read 21 fluxes, W^n (8); write 8
+    "update_s2": 160.0,  # read 21 fluxes, winds of W* (3), W^n (8); write 8
+    "cfl": 32.0,
+}
+KERNEL_BYTES["fused"] = {
+    "update_s1": 64.0,   # read W^n (8), write 8
+    "update_s2": 96.0,   # read W* (8), W^n (8); write 8
+    "cfl": 32.0,
+}
 KERNEL_BYTES["strict"] = KERNEL_BYTES["unfused"]
 KERNEL_BYTES["auto"] = KERNEL_BYTES["tiled"]
 
@@ -382,6 +397,18 @@ def adjoint_leg(a, torch):
     }
 
 
+def kernel_bytes(path_name, cfg, tim):
+    """Bytes per cell of the kernels that a step of this box launched; tim: the
+    context's timing of it."""
+    if path_name == "tiled":
+        n = cfg["n"]
+        if not tim["faces_s1"][1]:
+            path_name = "fused"
+        elif n[0] * n[1] * n[2] <= DIRECT_CELLS:
+            path_name = "direct"
+    return KERNEL_BYTES[path_name]
+
+
 def stage_rates(cfg, tim, kbytes, zones):
     """Algorithmic GB/s of each stage of the step: reconstruction + HLLD (the
     face kernels), CT + update (the update kernels), CFL reduction (a
@@ -397,7 +424,7 @@ def stage_rates(cfg, tim, kbytes, zones):
         return None if not n else nbytes * n / (ms * 1e-3) / 1e9
 
     return {
-        "reconstruct_hlld": rate(["faces_s1", "faces_s2"], kbytes["faces_s1"] * zones),
+        "reconstruct_hlld": rate(["faces_s1", "faces_s2"], kbytes.get("faces_s1", 0.0) * zones),
         "ct_update": rate(["update_s1", "update_s2"],
                           0.5 * (kbytes["update_s1"] + kbytes["update_s2"]) * zones),
         "cfl_reduce": rate(["cfl_ghosts"], 32.0 * ghost_cells),
@@ -467,7 +494,7 @@ def main():
     tim = ctx.timing()
     ctx.timing_enable(False)
     path_name = ["auto", "unfused", "tiled", "strict"][ctx.get_path()]
-    kbytes = KERNEL_BYTES[path_name]
+    kbytes = kernel_bytes(path_name, cfg, tim)
     kern = {k: v for k, v in tim.items() if v[1] > 0 and k in kbytes}
     dom = max(kern, key=lambda k: kern[k][0])
     mean_s = kern[dom][0] / kern[dom][1] / 1e3

@@ -112,7 +112,7 @@ enum Slot {
   S_UPDATE1,
   S_UPDATE2,
   S_COPY,
-  S_COMMIT,
+  S_COMMIT,  // no launch of its own any more; the slots keep their numbers
   S_FACES1,
   S_FACES2,
   S_CFL_GHOSTS,
