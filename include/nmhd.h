@@ -175,7 +175,8 @@ int nmhd_cfl_dt(nmhd_ctx *ctx, float goal_time, float *dt);
 /* clear_pace_kernel + add_flux_kernel_caller (INL:741-755, 918-988): the
  * right-hand side P(W) of the current state with stage step h (used by the
  * face predictor 0.5*h*a), written to host arrays in the order rho, mx, my,
- * mz, E, Bx, By, Bz.  Synchronises. */
+ * mz, E, Bx, By, Bz.  On NMHD_PATH_TILED by the marching tiles, whatever the
+ * box's size (the step's other kernels give the same bits).  Synchronises. */
 int nmhd_rhs(nmhd_ctx *ctx, float h, float *const pace[8]);
 
 /* One iteration of MHDSolver::proceed's loop (INL:1094-1201): ghost fill,
@@ -260,7 +261,8 @@ int nmhd_batch_destroy(nmhd_batch *batch);
 const char *nmhd_batch_last_error(const nmhd_batch *batch);
 int nmhd_batch_get_geometry(const nmhd_batch *batch, int box, nmhd_geometry *geo);
 
-/* State and time of one box, as nmhd_set_state / nmhd_set_time. */
+/* State and time of one box, as nmhd_set_state / nmhd_set_time (the state is
+ * fetched into pageable, pinned or device memory). */
 int nmhd_batch_set_state(nmhd_batch *batch, int box, const float *const fields[8]);
 int nmhd_batch_get_state(nmhd_batch *batch, int box, float *const fields[8]);
 int nmhd_batch_set_time(nmhd_batch *batch, int box, double t, int generation);
