@@ -190,3 +190,37 @@ def test_boxes_below_the_limit_are_faster_than_on_tiles(gpu_ready, n):
     assert best[0] < 0.97 * min(best[1:])
     for c in ctx:
         c.close()
+
+
+@pytest.mark.parametrize("n", [(64, 64, 64), (90, 90, 90)])
+def test_steps_past_the_goal_are_cheap(gpu_ready, n):
+    """A step enqueued past the goal solves no faces (64^3: 16 us, 27 when its
+    first launch did; a taken one 46)."""
+    import time
+    cfg = P.make_config(n, cfl=0.1)
+    W = P.orszag_tang(cfg)
+    W[4] += 1.0
+    ctx = capi.Context(cfg)
+    ctx.set_state(W)
+    ctx.run(1e30, 32)
+
+    def best(goal):
+        out = []
+        for rep in range(8):
+            ctx.reset_run()
+            t = time.perf_counter()
+            ctx.enqueue_steps(goal, 32)
+            k, reached = ctx.synchronize()
+            out.append(time.perf_counter() - t)
+        assert (k, reached) == ((32, False) if goal > 1e29 else (1, True))
+        return min(out)
+
+    taken = best(1e30)
+    state = ctx.get_state()
+    past = best(ctx.get_time()[0])
+    print("\n[case] %s: 32 steps taken %.0f us, past the goal %.0f" % (n, taken * 1e6, past * 1e6),
+          flush=True)
+    assert past < 0.45 * taken
+    # the one taken is of size zero, or what t lacks to the goal in float
+    assert np.allclose(ctx.get_state(), state, rtol=1e-3, atol=1e-4)
+    ctx.close()
