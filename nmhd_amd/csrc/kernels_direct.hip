@@ -75,7 +75,7 @@ __device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const
     if (Open && blockIdx.x == 0 && threadIdx.x < 64) (void)open_step(b, open, true);
     return;
   }
-  if (Open) {
+  if (Open || open.in) {
     // the launch that opens the step: only the face predictor needs its size,
     // so without a source term only the first wave forms it
     const bool src = D != 2 && b.source == 1;
@@ -88,6 +88,7 @@ __device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const
       h = *hs;
     }
   } else {
+    if (!tiled::stage_active(ss)) return;
     h = tiled::stage_size(ss);
   }
   float L[7], R[7];
@@ -126,16 +127,19 @@ __device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const
 // past the last cell work on it and store nothing (a whole wave opens the
 // step).
 //
-// Whether the step is taken is read with the loads, the opening launch an
-// instantiation of its own: 32 steps of 64^3 enqueued past the end of a run take
-// 500 us (860 where the opening launch solved its faces before it knew), taken
-// ones as long as without (periodic 44^3 to 94^3 -0.6 to +0.2%, shearing boxes
-// +0.4%).
+// Open: the launch opens a step, and solves nothing where the step is not taken
+// (past the end of a run): a run to a goal 4.5 steps away, whose other 27 steps
+// are such, takes 760 us at 64^3 and 1504 at 90^3, against 955 and 1950 where
+// they solved their first faces.  Tested in one instantiation for all launches it
+// cost steps taken 1.4% at 64^3, in two nothing.  The other instantiation keeps
+// the branch on open.in though its launches open nothing: without it the compiler
+// gives it 53 VGPRs instead of 73, and 30 frozen steps of 92^3 take 3055 us
+// against 3000.
 template <int Recon, bool Open>
 __global__ void __launch_bounds__(kThreads)
     k_direct_faces(Box b, FieldPtrs W, FluxSet F, StageStep ss, OpenStep open) {
   __shared__ float hs;
-  const bool skip = Open ? run_ended(open.in->s, open.reset) : !tiled::stage_active(ss);
+  const bool skip = Open && run_ended(open.in->s, open.reset);
   const unsigned lb = xcd_logical_block(blockIdx.x, gridDim.x);
   const unsigned group = lb / 3, dir = lb - 3 * group;
   const unsigned i = group * kThreads + threadIdx.x, last = (unsigned)b.ncell - 1;
