@@ -25,6 +25,10 @@ using tiled::recon_bsum;
 
 constexpr int kThreads = 256;
 
+// What a launch does with its step: opens it, follows the launch that did, or
+// takes one of a given size.
+enum Role { kFrozen, kOpens, kFollows };
+
 // i (in [-2, n]) brought into [0, n)
 __device__ __forceinline__ int wrap1(int i, int n) {
   const int j = i < 0 ? i + n : (i >= n ? i - n : i);
@@ -33,8 +37,8 @@ __device__ __forceinline__ int wrap1(int i, int n) {
 
 // One face per thread, the lower D-face of cell (x, y, z), and nothing of it
 // (but the opening of the step) with skip, the step not being taken.  The loads
-// come first: the step's record is waited for with them, not before them.
-template <int D, int Recon, bool Open>
+// come first: the size of the step is waited for with them, not before them.
+template <int D, int Recon, int Role>
 __device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const FluxOut &F,
                                          const StageStep &ss, const OpenStep &open, bool skip, int x,
                                          int y, int z, bool valid, float *hs) {
@@ -72,10 +76,10 @@ __device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const
   const float bn = ld(5 + D, s[2]);
   float h = 0.0f;
   if (skip) {
-    if (Open && blockIdx.x == 0 && threadIdx.x < 64) (void)open_step(b, open, true);
+    if (Role == kOpens && blockIdx.x == 0 && threadIdx.x < 64) (void)open_step(b, open, true);
     return;
   }
-  if (Open || open.in) {
+  if (Role == kOpens || (Role == kFrozen && open.in)) {
     // the launch that opens the step: only the face predictor needs its size,
     // so without a source term only the first wave forms it
     const bool src = D != 2 && b.source == 1;
@@ -88,7 +92,7 @@ __device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const
       h = *hs;
     }
   } else {
-    if (!tiled::stage_active(ss)) return;
+    if (Role == kFrozen && !tiled::stage_active(ss)) return;
     h = tiled::stage_size(ss);
   }
   float L[7], R[7];
@@ -127,19 +131,21 @@ __device__ __forceinline__ void one_face(const Box &b, const FieldPtrs &W, const
 // past the last cell work on it and store nothing (a whole wave opens the
 // step).
 //
-// Open: the launch opens a step, and solves nothing where the step is not taken
-// (past the end of a run): a run to a goal 4.5 steps away, whose other 27 steps
-// are such, takes 760 us at 64^3 and 1504 at 90^3, against 955 and 1950 where
-// they solved their first faces.  Tested in one instantiation for all launches it
-// cost steps taken 1.4% at 64^3, in two nothing.  The other instantiation keeps
-// the branch on open.in though its launches open nothing: without it the compiler
-// gives it 53 VGPRs instead of 73, and 30 frozen steps of 92^3 take 3055 us
-// against 3000.
-template <int Recon, bool Open>
+// The launches of a step that may not be taken (past the end of a run) find that
+// out first and then do nothing: a run to a goal 4.5 steps away, whose other 27
+// steps are such, takes 668 us at 64^3 and 1285 at 90^3, against 958 and 1945
+// where they solved their first faces and loaded for the others.  One
+// instantiation for all roles cost steps taken 1.4% at 64^3, these nothing.
+// kFrozen keeps the branch on open.in though its launches open nothing: without
+// it the compiler gives it 53 VGPRs instead of 73, and 30 frozen steps of 92^3
+// take 3055 us against 3000.
+template <int Recon, int Role>
 __global__ void __launch_bounds__(kThreads)
     k_direct_faces(Box b, FieldPtrs W, FluxSet F, StageStep ss, OpenStep open) {
   __shared__ float hs;
-  const bool skip = Open && run_ended(open.in->s, open.reset);
+  const bool skip = Role == kOpens     ? run_ended(open.in->s, open.reset)
+                    : Role == kFollows ? !tiled::stage_active(ss)
+                                       : false;
   const unsigned lb = xcd_logical_block(blockIdx.x, gridDim.x);
   const unsigned group = lb / 3, dir = lb - 3 * group;
   const unsigned i = group * kThreads + threadIdx.x, last = (unsigned)b.ncell - 1;
@@ -147,11 +153,11 @@ __global__ void __launch_bounds__(kThreads)
   int x, y, z;
   cell_coords(b, valid ? i : last, x, y, z);
   if (dir == 0)
-    one_face<0, Recon, Open>(b, W, F.dir[0], ss, open, skip, x, y, z, valid, &hs);
+    one_face<0, Recon, Role>(b, W, F.dir[0], ss, open, skip, x, y, z, valid, &hs);
   else if (dir == 1)
-    one_face<1, Recon, Open>(b, W, F.dir[1], ss, open, skip, x, y, z, valid, &hs);
+    one_face<1, Recon, Role>(b, W, F.dir[1], ss, open, skip, x, y, z, valid, &hs);
   else
-    one_face<2, Recon, Open>(b, W, F.dir[2], ss, open, skip, x, y, z, valid, &hs);
+    one_face<2, Recon, Role>(b, W, F.dir[2], ss, open, skip, x, y, z, valid, &hs);
 }
 
 }  // namespace direct
@@ -169,10 +175,13 @@ void launch_direct_faces(hipStream_t s, const Box &b, FieldPtrs W, const FluxSet
                          const StageStep &ss, const OpenStep &open) {
   const dim3 grid(3 * grid_for(b.ncell, direct::kThreads)), blk(direct::kThreads);
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, blk, 0, s, b, W, F, ss, open); };
+  using namespace direct;
   if (open.in)
-    b.recon == 1 ? go(direct::k_direct_faces<1, true>) : go(direct::k_direct_faces<0, true>);
+    b.recon == 1 ? go(k_direct_faces<1, kOpens>) : go(k_direct_faces<0, kOpens>);
+  else if (ss.hsel == H_FIXED)
+    b.recon == 1 ? go(k_direct_faces<1, kFrozen>) : go(k_direct_faces<0, kFrozen>);
   else
-    b.recon == 1 ? go(direct::k_direct_faces<1, false>) : go(direct::k_direct_faces<0, false>);
+    b.recon == 1 ? go(k_direct_faces<1, kFollows>) : go(k_direct_faces<0, kFollows>);
 }
 
 }  // namespace nmhd
